@@ -35,6 +35,7 @@ struct Item {
 
 constexpr int kItemEdges = 256;   // elements staged in LDS per wavefront at a time
 constexpr int kItemRows = 64;     // most rows one multi-row item may hold
+constexpr int kMaxPieces = 8192;  // most pieces (per partition) for which a plan cuts rows finer than on a large graph
 
 // A row segment that was split: pieces partial[slot0 .. slot0 + n_pieces) add up to it.
 struct Fixup {
@@ -58,6 +59,7 @@ struct fg_spmm_plan {
     // per partition: [item_begin, item_end) and [fixup_begin, fixup_end)
     std::vector<int64_t> item_off, fixup_off;
     int64_t n_items = 0, n_fixups = 0, n_slots = 0, max_slots_in_partition = 0;
+    int64_t default_pieces = 0;          // pieces of a partition at 1024 elements each (or the caller's threshold): what fg_spmm_csr_noalloc_f32's limit counts
     fg::Item *items_dev = nullptr;
     int64_t *item_off_dev = nullptr;     // item_off on the device (num_col_partitions + 1 entries)
     fg::Fixup *fixups_dev = nullptr;

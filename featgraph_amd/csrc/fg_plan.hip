@@ -15,7 +15,39 @@ using fg::Fixup;
 using fg::Item;
 
 namespace {
-constexpr int kDefaultSplit = 1024;   // elements per wavefront piece of a long row
+constexpr int kDefaultSplit = 1024;   // elements per wavefront piece of a long row, on a large graph
+
+// How finely a plan of `nnz` elements is cut when the caller leaves it open.  A wavefront works through its item serially,
+// so on a graph that does not fill the chip (8,192 wavefront slots) the longest item is what a launch takes, and on
+// any graph a long row's last piece is what a launch ends with.  Row pieces of 128 elements below 2^20 elements, 256
+// below 2^23, 512 below 2^25; several rows share an item up to about nnz / 4096 elements (a power of two of 16 .. 256).
+// Measured, operator pairs and training steps, microseconds of kernel time at (1024, 256) -> at the rule's
+// (split, item): 10,500 edges (128, 16) weighted sum F=64 with gradients 47 -> 30, edge softmax H=4 33 -> 8;
+// 169,867 edges (128, 32) 53 -> 39 and 17 -> 16; 400,000 edges (128, 64) 89 -> 60 and 68 -> 41; 2 M edges (256, 256)
+// 154 -> 132; 6 M (256, 256) 367 -> 343, max F=64 822 -> 734; 12.5 M (512, 256) 692 -> 664, 1243 -> 1159.  Smaller items
+// than the rule's lose the one-lane-group-per-row walk of many short rows: 1.5 M edges of degree 15, F=64, 156 at 256,
+// 200 at 64.
+void default_cut(int64_t nnz, int *split, int *item_edges) {
+    *split = nnz < (1 << 20) ? 128 : nnz < (1 << 23) ? 256 : nnz < (1 << 25) ? 512 : kDefaultSplit;
+    int item = 16;
+    while (item < fg::kItemEdges && (int64_t)item * 2 * 4096 <= nnz) item *= 2;
+    *item_edges = nnz < (1 << 20) ? item : fg::kItemEdges;
+}
+
+// Pieces of all rows longer than `split` in the partition that has most of them.
+int64_t most_pieces(const int32_t *pos, int64_t n_dst, int P, int split) {
+    int64_t most = 0;
+    for (int p = 0; p < P; ++p) {
+        const int32_t *pp = pos + p * (n_dst + 1);
+        int64_t pieces = 0;
+        for (int64_t r = 0; r < n_dst; ++r) {
+            const int32_t len = pp[r + 1] - pp[r];
+            if (len > split) pieces += (len + split - 1) / split;
+        }
+        most = std::max(most, pieces);
+    }
+    return most;
+}
 }
 
 extern "C" int fg_spmm_plan_create(const int32_t *pos, int64_t n_dst, int64_t n_src, int P,
@@ -25,10 +57,6 @@ extern "C" int fg_spmm_plan_create(const int32_t *pos, int64_t n_dst, int64_t n_
     if (!pos || n_dst < 0 || n_src < 0) return fail(FG_ERR_ARG, "fg_spmm_plan_create: bad argument");
     if (P < 1) return fail(FG_ERR_ARG, "num_col_partitions should be larger than or equal to 1");
     if (n_dst >= INT32_MAX || n_src >= INT32_MAX) return fail(FG_ERR_SHAPE, "vertex count does not fit int32");
-    int split = (opts && opts->split_threshold > 0) ? opts->split_threshold : kDefaultSplit;
-    int item_edges = (opts && opts->item_edges > 0) ? opts->item_edges : fg::kItemEdges;
-    if (item_edges > fg::kItemEdges) item_edges = fg::kItemEdges;
-    if (item_edges > split) item_edges = split;
     const int64_t d2 = n_dst + 1;
 
     // structure check: one non-decreasing run of positions across all partitions
@@ -41,6 +69,16 @@ extern "C" int fg_spmm_plan_create(const int32_t *pos, int64_t n_dst, int64_t n_
                             p, (long long)r);
             prev = v;
         }
+
+    int split = kDefaultSplit, item_edges = fg::kItemEdges;
+    if (opts && opts->split_threshold > 0) split = opts->split_threshold;
+    else {
+        default_cut(prev, &split, &item_edges);
+        // (kMaxPieces bounds the scratch and what fg_spmm_csr_noalloc_f32 has to fit into its fixed array)
+        while (split < kDefaultSplit && most_pieces(pos, n_dst, P, split) > fg::kMaxPieces) split *= 2;
+    }
+    if (opts && opts->item_edges > 0) item_edges = std::min(opts->item_edges, fg::kItemEdges);
+    if (item_edges > split) item_edges = split;
 
     auto *pl = new fg_spmm_plan();
     pl->n_dst = n_dst; pl->n_src = n_src; pl->nnz = prev;
@@ -107,6 +145,7 @@ extern "C" int fg_spmm_plan_create(const int32_t *pos, int64_t n_dst, int64_t n_
     }
     pl->n_items = (int64_t)items.size();
     pl->n_fixups = (int64_t)fixups.size();
+    pl->default_pieces = (opts && opts->split_threshold > 0) ? pl->max_slots_in_partition : most_pieces(pos, n_dst, P, kDefaultSplit);
 
     hipError_t e = hipGetDevice(&pl->device);
     if (e == hipSuccess && P == 1) fg::prepare_fixed_scratch(pl->device);

@@ -65,7 +65,8 @@ struct SpmmArgs {
     uint32_t x_row_bytes;
     uint32_t x_tile_bytes;
     float *out;
-    float *partial;
+    float *partial;        // pieces of split rows: columns [partial_f0, partial_f0 + partial_ld) of each
+    int partial_ld, partial_f0 = 0;
     int F;                 // row stride of x / out in floats
     int tile_w;            // floats per requested feature tile (F / num_feat_partitions)
     int sub_per_tile;      // kernel tiles (V*L*K floats each) per requested tile
@@ -432,7 +433,7 @@ __device__ __forceinline__ void spmm_items_body(const SpmmArgs &a) {
 
     // one row, or one piece of a long row: 256 elements at a time, the next 256 on their way
     // while the current ones are used
-    float *dst = (it.info < 0 ? out_p + (int64_t)it.row * F : partial_p + (int64_t)it.info * F) + f_lo;
+    float *dst = (it.info < 0 ? out_p + (int64_t)it.row * F : partial_p + (int64_t)it.info * a.partial_ld - a.partial_f0) + f_lo;
     const bool add = ACC && it.info < 0;
 #pragma unroll
     for (int k = 0; k < K; ++k) acc[k] = vzero(vec());
@@ -603,7 +604,7 @@ __global__ __launch_bounds__(kBlock) void gspmm_extreme_kernel(const SpmmArgs a)
         wave_lds_sync();
         walk(0, n);
     }
-    float *dst = (it.info < 0 ? a.out + (int64_t)it.row * F : a.partial + (int64_t)it.info * F) + f_lo;
+    float *dst = (it.info < 0 ? a.out + (int64_t)it.row * F : a.partial + (int64_t)it.info * a.partial_ld - a.partial_f0) + f_lo;
     finish(dst, it.len == 0);
 }
 
@@ -803,25 +804,27 @@ int launch_arg_v(int L, int K, bool full, dim3 grid, hipStream_t st, const SpmmA
     return FG_ERR_SHAPE;
 }
 
-// out[row, :] (+)= sum of the row's pieces, in piece order.  One lane per V columns.
+// out[row, f0 : f0 + width] (+)= sum of the row's pieces, in piece order.  One lane per V columns.
+// Pieces lie partial_ld floats apart and hold columns f0 and up (partial_ld = F, f0 = 0, width = F unless the pieces go
+// to an array of fixed size, a range of columns at a time).
 // part_stride / out_stride (floats; 0 for a launch over one partition's fix-ups): with every pass in a buffer of
 // its own, partition p's pieces start at partial + p * part_stride and its rows at out + p * out_stride.
 template <int V>
 __global__ __launch_bounds__(256) void spmm_fixup_kernel(const Fixup *fixups, int64_t n_fixups,
-                                                         const float *partial, float *out, int F,
+                                                         const float *partial, int partial_ld, float *out, int F, int f0, int width,
                                                          int accumulate, int64_t part_stride, int64_t out_stride) {
     using vec = typename Vec<V>::type;
-    const int per_row = F / V;
+    const int per_row = width / V;
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n_fixups * per_row) return;
     const Fixup fx = fixups[t / per_row];
     const int f = (int)(t % per_row) * V;
     partial += fx.part * part_stride;
     out += fx.part * out_stride;
-    vec sum = *reinterpret_cast<const vec *>(partial + (int64_t)fx.slot0 * F + f);
+    vec sum = *reinterpret_cast<const vec *>(partial + (int64_t)fx.slot0 * partial_ld + f);
     for (int p = 1; p < fx.n_pieces; ++p)
-        vadd(sum, *reinterpret_cast<const vec *>(partial + (int64_t)(fx.slot0 + p) * F + f));
-    vec *o = reinterpret_cast<vec *>(out + (int64_t)fx.row * F + f);
+        vadd(sum, *reinterpret_cast<const vec *>(partial + (int64_t)(fx.slot0 + p) * partial_ld + f));
+    vec *o = reinterpret_cast<vec *>(out + (int64_t)fx.row * F + f0 + f);
     if (accumulate) vadd(sum, *o);
     *o = sum;
 }
@@ -1059,7 +1062,8 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
     // X is gathered from the caller's matrix (no tile-by-tile copy), and nothing is allocated.
     fg::ScratchNeed need = scratch_need(pl, c, F, reduce);
     if (fixed_partial) {
-        need.partial = piece_floats(pl, F);
+        // the limit counts pieces of 1024 elements; a plan cut finer than that fills the buffer a range of columns at a time
+        need.partial = (((size_t)pl->default_pieces * (size_t)F) + 3) & ~(size_t)3;
         if (need.partial > fixed_partial_floats)
             return fail(FG_ERR_SHAPE, "the split rows of this plan need %zu floats of scratch at feature length %d; "
                         "the fixed buffer of this entry point holds %zu", need.partial, F, fixed_partial_floats);
@@ -1097,7 +1101,7 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
         a.x_row_bytes = (uint32_t)(tiled ? ft : F) * 4u;
         a.x_tile_bytes = tiled ? (uint32_t)((uint64_t)pl->n_src * ft * 4u) : 0u;
         a.out = pass_buf; a.out_stride = (int64_t)pass_stride;
-        a.partial = partial; a.partial_stride = (int64_t)piece;
+        a.partial = partial; a.partial_ld = F; a.partial_stride = (int64_t)piece;
         a.F = F; a.tile_w = c.tile_w; a.sub_per_tile = c.sub_per_tile;
         a.heads = heads; a.head_len = F / heads;
         a.vstride = head_major ? 1 : heads; a.head_stride = head_major ? pl->nnz : 1;
@@ -1116,10 +1120,19 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
         const int fv = (aligned16 && F % 4 == 0) ? 4 : 1;
         const int64_t threads = pl->n_fixups * (F / fv);
         const unsigned blocks = (unsigned)((threads + 255) / 256);
-        if (fv == 4) hipLaunchKernelGGL(spmm_fixup_kernel<4>, dim3(blocks), dim3(256), 0, st, pl->fixups_dev, pl->n_fixups, partial, pass_buf, F, 0, (int64_t)piece, (int64_t)pass_stride);
-        else hipLaunchKernelGGL(spmm_fixup_kernel<1>, dim3(blocks), dim3(256), 0, st, pl->fixups_dev, pl->n_fixups, partial, pass_buf, F, 0, (int64_t)piece, (int64_t)pass_stride);
+        if (fv == 4) hipLaunchKernelGGL(spmm_fixup_kernel<4>, dim3(blocks), dim3(256), 0, st, pl->fixups_dev, pl->n_fixups, partial, F, pass_buf, F, 0, F, 0, (int64_t)piece, (int64_t)pass_stride);
+        else hipLaunchKernelGGL(spmm_fixup_kernel<1>, dim3(blocks), dim3(256), 0, st, pl->fixups_dev, pl->n_fixups, partial, F, pass_buf, F, 0, F, 0, (int64_t)piece, (int64_t)pass_stride);
     }
-    for (int p = 0; p < P && !pass_buf; ++p) {
+    // Kernel tiles [cb, ce) at a time: all of them, unless the pieces' columns have to fit an array of fixed size (a plan
+    // cut finer than 1024 elements per piece has at most kMaxPieces pieces, so one kernel tile always fits).
+    auto tile_col = [&](int t) { return t >= c.n_ftiles ? F : (t / c.sub_per_tile) * c.tile_w + (t % c.sub_per_tile) * ft; };
+    const int64_t max_cols = (fixed_partial && pl->max_slots_in_partition > 0)
+                                 ? (int64_t)(fixed_partial_floats / (size_t)pl->max_slots_in_partition) : F;
+    for (int p = 0; p < P && !pass_buf; ++p)
+    for (int cb = 0, ce; cb < c.n_ftiles; cb = ce) {
+        ce = cb + 1;
+        while (ce < c.n_ftiles && tile_col(ce + 1) - tile_col(cb) <= max_cols) ++ce;
+        const int f0 = tile_col(cb), piece_ld = tile_col(ce) - f0;
         const int64_t i0 = pl->item_off[p], i1 = pl->item_off[p + 1];
         if (i1 > i0) {
             SpmmArgs a;
@@ -1129,7 +1142,7 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
             a.x = tiled ? pl->tiled_dev + (int64_t)p * width * ft : x + (int64_t)p * width * F;
             a.x_row_bytes = (uint32_t)(tiled ? ft : F) * 4u;
             a.x_tile_bytes = tiled ? (uint32_t)((uint64_t)pl->n_src * ft * 4u) : 0u;
-            a.out = out; a.partial = partial;
+            a.out = out; a.partial = partial; a.partial_ld = piece_ld; a.partial_f0 = f0;
             a.F = F; a.tile_w = c.tile_w; a.sub_per_tile = c.sub_per_tile;
             a.heads = heads; a.head_len = F / heads;
             a.vstride = head_major ? 1 : heads; a.head_stride = head_major ? pl->nnz : 1;
@@ -1137,8 +1150,8 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
             // More than 8 tiles: 8 at a time (one per XCD), so that an XCD's L2 serves one tile's
             // slice of this partition per launch; the partition's index arrays stay in the
             // memory-side cache between the launches.
-            for (int tb = 0, per_launch; tb < c.n_ftiles; tb += per_launch) {
-                per_launch = tiles_this_launch(c.n_ftiles - tb);
+            for (int tb = cb, per_launch; tb < ce; tb += per_launch) {
+                per_launch = tiles_this_launch(ce - tb);
                 a.n_ftiles = per_launch; a.tile_base = tb;
                 const int64_t blocks = ((i1 - i0 + kWavesPerBlock - 1) / kWavesPerBlock) * per_launch;
                 if (blocks > 0x7fffffffLL) return fail(FG_ERR_SHAPE, "grid of %lld workgroups is too large", (long long)blocks);
@@ -1151,14 +1164,14 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
         }
         const int64_t x0 = pl->fixup_off[p], x1 = pl->fixup_off[p + 1];
         if (x1 > x0) {
-            const int fv = (aligned16 && F % 4 == 0) ? 4 : 1;
-            const int64_t threads = (x1 - x0) * (F / fv);
+            const int fv = (aligned16 && F % 4 == 0 && f0 % 4 == 0 && piece_ld % 4 == 0) ? 4 : 1;
+            const int64_t threads = (x1 - x0) * (piece_ld / fv);
             const unsigned blocks = (unsigned)((threads + 255) / 256);
             const Fixup *fx = pl->fixups_dev + x0;
             if (reduce == FG_REDUCE_SUM) {
                 const int add = p > 0 ? 1 : 0;
-                if (fv == 4) hipLaunchKernelGGL(spmm_fixup_kernel<4>, dim3(blocks), dim3(256), 0, st, fx, x1 - x0, partial, out, F, add, (int64_t)0, (int64_t)0);
-                else hipLaunchKernelGGL(spmm_fixup_kernel<1>, dim3(blocks), dim3(256), 0, st, fx, x1 - x0, partial, out, F, add, (int64_t)0, (int64_t)0);
+                if (fv == 4) hipLaunchKernelGGL(spmm_fixup_kernel<4>, dim3(blocks), dim3(256), 0, st, fx, x1 - x0, partial, piece_ld, out, F, f0, piece_ld, add, (int64_t)0, (int64_t)0);
+                else hipLaunchKernelGGL(spmm_fixup_kernel<1>, dim3(blocks), dim3(256), 0, st, fx, x1 - x0, partial, piece_ld, out, F, f0, piece_ld, add, (int64_t)0, (int64_t)0);
             } else if (reduce == FG_REDUCE_MAX) {
                 if (fv == 4) hipLaunchKernelGGL((gspmm_extreme_fixup_kernel<4, true>), dim3(blocks), dim3(256), 0, st, fx, x1 - x0, partial, out, F);
                 else hipLaunchKernelGGL((gspmm_extreme_fixup_kernel<1, true>), dim3(blocks), dim3(256), 0, st, fx, x1 - x0, partial, out, F);
@@ -1177,7 +1190,7 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
         // second sweep over the same items: which element equals the extreme that was just written
         SpmmArgs a;
         a.items = pl->items_dev; a.n_items = pl->n_items; a.pos = pos; a.indices = idx; a.vals = vals;
-        a.x = x; a.out = out; a.partial = nullptr; a.arg = arg_out;
+        a.x = x; a.out = out; a.partial = nullptr; a.partial_ld = F; a.arg = arg_out;
         a.F = F; a.tile_w = c.tile_w; a.sub_per_tile = c.sub_per_tile; a.n_ftiles = c.n_ftiles; a.tile_base = 0;
         a.accumulate = 0; a.heads = heads; a.head_len = F / heads;
         a.vstride = head_major ? 1 : heads; a.head_stride = head_major ? pl->nnz : 1;

@@ -76,9 +76,11 @@ int fg_check_csr_host(int64_t n_rows, int64_t n_cols, const int32_t *indptr_host
 typedef struct fg_spmm_plan fg_spmm_plan;
 
 typedef struct {
-    int32_t split_threshold; /* rows longer than this are split over wavefronts; 0 = default */
+    int32_t split_threshold; /* rows longer than this are split over wavefronts; 0 = default: 128 elements on graphs
+                                of fewer than 2^20 elements, 256 below 2^23, 512 below 2^25, else 1024 */
     int32_t item_edges;      /* short rows are packed into items of at most this many elements
-                                (and at most 64 rows); 0 = default, 1 = one row per item      */
+                                (and at most 64 rows); 0 = default: 256, fewer (16 .. 128, about nnz / 4096) on graphs
+                                of fewer than 2^20 elements; 1 = one row per item */
     int32_t wide_offsets;    /* non-zero: address feature rows with 64-bit offsets even when the matrix
                                 is smaller than 4 GiB (the path larger matrices take; for testing it) */
     int32_t tile_major;      /* SpMM / tiled SDDMM gather from a copy of the source features stored tile by
@@ -185,8 +187,9 @@ int fg_spmm_csr_f32(fg_spmm_plan *plan, const int32_t *indptr_dev,
  * the partial sums of split rows go to a 16 MiB array that is part of the library's device image
  * instead of plan-owned memory, X is always gathered from the caller's row-major matrix, and the call
  * itself performs no hipMalloc / hipFree; the plan is not modified.
- * Limit: (largest number of split-row pieces in the plan) * F <= 4,194,304 floats, else FG_ERR_SHAPE
- * (the 232,965-node benchmark graph needs 2.7 M floats at F = 512).
+ * Limit: (pieces of 1024 elements that the plan's longer rows make) * F <= 4,194,304 floats, else FG_ERR_SHAPE
+ * (the 232,965-node benchmark graph needs 2.7 M floats at F = 512); a plan whose rows are cut finer than that
+ * fills the array a range of columns at a time.
  * Each GPU holds one such array for the life of the process and every call on that GPU uses it: calls
  * that overlap on one GPU (two streams, two threads) race on it and must be ordered by the caller.
  * Nothing in it needs clearing between calls (every piece's row is written before it is read).
