@@ -128,14 +128,35 @@ class Graph(object):
             self._mods[key] = m
         return self._mods[key]
 
-    def _mean_weights(self, device):
-        if getattr(self, "_inv_deg", None) is None or self._inv_deg.device != device:
-            deg = np.diff(self._csr.indptr).astype(np.float32)
-            inv = np.where(deg > 0, 1.0 / np.maximum(deg, 1), 0).astype(np.float32)
-            self._inv_deg = torch.from_numpy(np.repeat(inv, np.diff(self._csr.indptr))).to(device)
-            self._ones = torch.ones(self.nnz, device=device)
-            self._cols = torch.from_numpy(self._csr.indices.astype(np.int64)).to(device)
-        return self._inv_deg
+    def _cols(self, device):
+        """Column of every stored edge (CSR order), int32."""
+        if getattr(self, "_cols_dev", None) is None or self._cols_dev.device != device:
+            self._cols_dev = torch.from_numpy(np.ascontiguousarray(self._csr.indices, dtype=np.int32)).to(device)
+        return self._cols_dev
+
+    def _degrees(self, device):
+        """Edges into every destination, at least 1, float32."""
+        if getattr(self, "_deg_dev", None) is None or self._deg_dev.device != device:
+            self._deg_dev = torch.from_numpy(np.maximum(np.diff(self._csr.indptr), 1).astype(np.float32)).to(device)
+        return self._deg_dev
+
+    def _aggregate_grad_mod(self, feat_len, reduce):
+        """The sum over every source's out-edges, with weight 1 (sum) or 1 / degree of the destination (mean) laid out
+        once in the transposed layout's order."""
+        key = ('aggregate_grad', feat_len, reduce)
+        if key not in self._mods:
+            m = self._gspmm_module(True)
+            x_ph = placeholder((self.shape[0], feat_len))
+            if reduce == 'sum':
+                m.build([x_ph], {'msg': 'copy_u'}, {})
+            else:
+                m.build([x_ph, placeholder((self.nnz,))], {}, {})
+                m.set_weight_order(self._tr_pos_host)
+                deg = np.diff(self._csr.indptr)
+                inv = np.where(deg > 0, 1.0 / np.maximum(deg, 1), 0).astype(np.float32)
+                m.fix_weights(torch.from_numpy(np.repeat(inv, deg)).to(m.ctx))
+            self._mods[key] = m
+        return self._mods[key]
 
     def attention(self, q, k, v, scale=None):
         """out[r, h, :] = sum over the edges e into r of softmax_r(scale * <k[col e, h, :], q[r, h, :]>) * v[col e, h, :];
@@ -205,6 +226,16 @@ class Graph(object):
         way (over the transpose the kernel addresses them through the transposed edges' CSR positions);
         return_arg (max / min): also the CSR position of the selected edge per output, as a tensor of the caller's own."""
         arrays = [a.contiguous() for a in arrays]
+        mod = self._bcast_spmm_mod(msg, arrays, reduce, transposed, return_arg)
+        if return_arg:
+            arg = mod.arg_tvm = torch.empty(mod._fresh_like[0] if getattr(mod, '_fresh_like', None) else mod.out_tvm.shape,
+                                            dtype=torch.int32, device=mod._ctx)
+            out = _fresh_run(mod, arrays)
+            mod.arg_tvm = None
+            return out, arg
+        return _fresh_run(mod, arrays)
+
+    def _bcast_spmm_mod(self, msg, arrays, reduce, transposed, return_arg):
         key = ('gspmm', msg, reduce, transposed, return_arg) + tuple(tuple(a.shape) for a in arrays)
         if key not in self._mods:
             m = self._gspmm_module(transposed)
@@ -215,12 +246,11 @@ class Graph(object):
             if transposed:
                 m.set_weight_order(self._tr_pos_host)
             self._mods[key] = m
-        mod = self._mods[key]
-        if return_arg:
-            mod.arg_tvm = torch.empty(mod._fresh_like[0] if getattr(mod, '_fresh_like', None) else mod.out_tvm.shape,
-                                      dtype=torch.int32, device=mod._ctx)
-            return _fresh_run(mod, arrays), mod.arg_tvm
-        return _fresh_run(mod, arrays)
+        return self._mods[key]
+
+    def _bcast_spmm_message(self, msg, arrays, reduce, return_arg):
+        """The resolved message (operand lengths, broadcast offsets) of a forward call."""
+        return self._bcast_spmm_mod(msg, arrays, reduce, False, return_arg)._bop
 
     def _bcast_sddmm_raw(self, op, lt, rt, arrays):
         arrays = [a.contiguous() for a in arrays]
@@ -391,8 +421,7 @@ class _GSpMM(torch.autograd.Function):
         arrays = ctx.saved_tensors
         dout = dout.contiguous()
         if ctx.reduce == "mean":
-            deg = torch.from_numpy(np.maximum(np.diff(g._csr.indptr), 1).astype(np.float32)).to(dout.device)
-            dout = dout / deg.reshape((-1,) + (1,) * (dout.dim() - 1))
+            dout = dout / g._degrees(dout.device).reshape((-1,) + (1,) * (dout.dim() - 1))
         grads = []
         targets = [lt] if rt is None else [lt, rt]
         for i, (p, tp) in enumerate(zip(arrays, targets)):
@@ -431,51 +460,24 @@ class _GSpMMExtreme(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, g, msg, reduce, lhs, rhs=None):
-        arrays = [lhs] if rhs is None else [lhs, rhs]
+        arrays = [a.contiguous() for a in ((lhs,) if rhs is None else (lhs, rhs))]
         out, arg = g._bcast_spmm_raw(msg, arrays, reduce, return_arg=True)
-        ctx.g, ctx.msg = g, msg
+        ctx.g, ctx.message = g, g._bcast_spmm_message(msg, arrays, reduce, return_arg=True)
         ctx.save_for_backward(arg, *arrays)
-        ctx.mark_non_differentiable(arg)
         return out
 
     @staticmethod
     def backward(ctx, dout):
-        g = ctx.g
-        op, lt, rt = parse_message(ctx.msg)
         arg, *arrays = ctx.saved_tensors
-        targets = [lt] if rt is None else [lt, rt]
-        n_dst, out_shape = dout.shape[0], tuple(dout.shape[1:])
-        n_out = int(np.prod(out_shape)) if out_shape else 1
-        g._mean_weights(dout.device)                                   # makes g._cols
-        e = arg.reshape(n_dst, n_out).long()
-        valid = e >= 0
-        e = e.clamp(min=0)
-        rows_of = {"u": g._cols[e], "e": e}                            # operand row per output element
+        return (None, None, None) + _selected_grads(ctx.g, ctx.message, arg, arrays, dout, ctx.needs_input_grad[3:])
 
-        def spread(x):      # (rows, *feat) -> (rows, n_out): the operand feature every output feature reads
-            return _align_features(x, dout).expand((x.shape[0],) + out_shape).reshape(x.shape[0], n_out)
 
-        picked = [spread(x).gather(0, rows_of[t]) for x, t in zip(arrays, targets)]
-        d = dout.reshape(n_dst, n_out) * valid
-        grads = []
-        for i, (p, tp) in enumerate(zip(arrays, targets)):
-            if not ctx.needs_input_grad[3 + i]:
-                grads.append(None)
-                continue
-            if op in ("add", "copy_lhs") or (op == "sub" and i == 0):
-                c = d
-            elif op == "sub":
-                c = -d
-            elif op == "mul":
-                c = d * picked[1 - i]
-            elif i == 0:                                               # div, numerator
-                c = d / picked[1]
-            else:                                                      # div, denominator
-                c = -d * picked[0] / picked[1] ** 2
-            c = torch.where(valid, c, torch.zeros_like(c))
-            full = torch.zeros((p.shape[0], n_out), dtype=dout.dtype, device=dout.device).scatter_add_(0, rows_of[tp], c)
-            grads.append(_reduce_to(full.reshape((p.shape[0],) + out_shape), p.shape))
-        return (None, None, None) + tuple(grads)
+def _selected_grads(g, message, arg, arrays, dout, needed):
+    """Gradients of a max / min aggregation for the operands `arrays`, None where not needed."""
+    grads = [torch.zeros_like(p) if need else None for p, need in zip(arrays, needed)]
+    lhs, rhs = arrays[0], arrays[1] if len(arrays) > 1 else None
+    message.select_backward(arg, g._cols(dout.device), g.nnz, lhs, rhs, dout.contiguous(), grads[0], grads[1] if rhs is not None else None)
+    return tuple(grads)
 
 
 def _sum_over_out_edges(g, d):
@@ -524,25 +526,20 @@ class _Aggregate(torch.autograd.Function):
         ctx.g, ctx.reduce = g, reduce
         x = x.contiguous()
         mod = g._aggregate_mod(x.shape[1], reduce)
-        y = mod.run([x]).clone()
         if reduce in ("max", "min"):
-            ctx.save_for_backward(mod.arg_tvm.clone())
-        ctx.x_shape = tuple(x.shape)
-        return y
+            mod.arg_tvm = torch.empty((g.shape[0], x.shape[1]), dtype=torch.int32, device=mod.ctx)
+            y = _fresh_run(mod, [x])
+            ctx.save_for_backward(mod.arg_tvm, x)
+            mod.arg_tvm = None
+            return y
+        return _fresh_run(mod, [x])
 
     @staticmethod
     def backward(ctx, dy):
         g, reduce = ctx.g, ctx.reduce
         dy = dy.contiguous()
         if reduce in ("sum", "mean"):
-            w = g._mean_weights(dy.device)
-            return None, g._spmm_raw(dy, w if reduce == "mean" else g._ones, transposed=True), None
-        (arg,) = ctx.saved_tensors
-        g._mean_weights(dy.device)
-        n_src, F = ctx.x_shape
-        valid = arg >= 0
-        src = g._cols[arg.clamp(min=0).long()]                               # source vertex of the selected edge
-        flat = (src * F + torch.arange(F, device=dy.device)[None, :])[valid]
-        dx = torch.zeros(n_src * F, dtype=dy.dtype, device=dy.device)
-        dx.index_add_(0, flat, dy[valid])
-        return None, dx.view(n_src, F), None
+            return None, _fresh_run(g._aggregate_grad_mod(dy.shape[1], reduce), [dy]), None
+        arg, x = ctx.saved_tensors
+        (dx,) = _selected_grads(g, g._aggregate_mod(dy.shape[1], reduce)._bop, arg, [x], dy, (True,))
+        return None, dx, None

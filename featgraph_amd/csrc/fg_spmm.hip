@@ -484,8 +484,11 @@ __global__ __launch_bounds__(kBlock) void spmm_items_wide_kernel(const SpmmArgs 
 // each row in turn and a lane without an element in the last batch keeps its running extreme.
 
 template <bool IS_MAX> __device__ __forceinline__ float ext_identity() { return IS_MAX ? -INFINITY : INFINITY; }
-// a NaN message beats every number (it reaches the result, as through a sum); once the running extreme is a NaN it stays
-template <bool IS_MAX> __device__ __forceinline__ float ext_op(float a, float b) { return ((IS_MAX ? b > a : b < a) || b != b) ? b : a; }
+// a NaN message beats every number (it reaches the result, as through a sum); once the running extreme is a NaN it stays:
+// one v_maximum3_f32 / v_minimum3_f32
+template <bool IS_MAX> __device__ __forceinline__ float ext_op(float a, float b) {
+    return IS_MAX ? __builtin_elementwise_maximum(a, b) : __builtin_elementwise_minimum(a, b);
+}
 template <bool IS_MAX> __device__ __forceinline__ void vext(float4 &a, const float4 &b) {
     a.x = ext_op<IS_MAX>(a.x, b.x); a.y = ext_op<IS_MAX>(a.y, b.y);
     a.z = ext_op<IS_MAX>(a.z, b.z); a.w = ext_op<IS_MAX>(a.w, b.w);

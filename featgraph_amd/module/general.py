@@ -129,18 +129,28 @@ class BroadcastOp(object):
         """Feature length of the operand that is gathered from the source nodes (0: none is)."""
         return max(self.lhs_len if self.lhs_target == 'u' else 0, self.rhs_len if self.rhs_target == 'u' else 0)
 
-    def run_spmm(self, plan, pos_dev, idx_dev, reduce, lhs, rhs, row_scale, out, arg, edge_pos_dev=None):
+    def run_spmm(self, plan, pos_dev, idx_dev, reduce, lhs, rhs, row_scale, out, arg, edge_pos_dev=None, ascend=False):
         """pos_dev / idx_dev: indptr / indices, or the arrays of a source-partitioned layout; edge_pos_dev: where each
-        of their elements lies in the edge operands (required with partitions; None: at its own position)."""
+        of their elements lies in the edge operands (required with partitions; None: at its own position); ascend: those
+        positions ascend along every row segment (FG_BCAST_EDGES_ASCEND)."""
         operands = (BINARY[self.op], reduce,
                     _lib.dev_ptr(lhs), TARGET[self.lhs_target or 'u'], self.lhs_len, _lib.dev_ptr(self.lhs_off),
-                    _lib.dev_ptr(rhs), TARGET[self.rhs_target or 'e'], self.rhs_len, _lib.dev_ptr(self.rhs_off), self.flags,
+                    _lib.dev_ptr(rhs), TARGET[self.rhs_target or 'e'], self.rhs_len, _lib.dev_ptr(self.rhs_off), self.flags | (16 if ascend else 0),
                     _lib.dev_ptr(row_scale), _lib.dev_ptr(out), _lib.dev_ptr(arg), self.out_len, common.stream_ptr())
         if edge_pos_dev is None:
             _lib.check(_lib.lib().fg_gspmm_bcast_f32(plan, _lib.dev_ptr(pos_dev), _lib.dev_ptr(idx_dev), *operands))
         else:
             _lib.check(_lib.lib().fg_gspmm_bcast_dds_f32(plan, _lib.dev_ptr(pos_dev), _lib.dev_ptr(idx_dev),
                                                          _lib.dev_ptr(edge_pos_dev), *operands))
+
+    def select_backward(self, arg, col_dev, n_edges, lhs, rhs, dout, dlhs, drhs):
+        """Adds a max / min aggregation's gradient (dout, per result) to dlhs / drhs (None: not wanted), given the
+        positions `arg` that the forward launch reported."""
+        _lib.check(_lib.lib().fg_gspmm_select_backward_f32(
+            _lib.dev_ptr(arg), _lib.dev_ptr(col_dev), arg.shape[0], n_edges, BINARY[self.op],
+            _lib.dev_ptr(lhs), TARGET[self.lhs_target or 'u'], self.lhs_len, _lib.dev_ptr(self.lhs_off),
+            _lib.dev_ptr(rhs), TARGET[self.rhs_target or 'e'], self.rhs_len, _lib.dev_ptr(self.rhs_off),
+            _lib.dev_ptr(dout), self.out_len, _lib.dev_ptr(dlhs), _lib.dev_ptr(drhs), common.stream_ptr()))
 
     def run_sddmm(self, row_dev, col_dev, n_edges, lhs, rhs, out):
         _lib.check(_lib.lib().fg_gsddmm_bcast_f32(

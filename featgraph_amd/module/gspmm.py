@@ -214,8 +214,9 @@ class GSpMMhip(VanillaSpMMhip):
         # values are in CSR order whatever order was announced for operands given to run()
         own = len(inputs) == 1 and self._static_rhs is not None
         pos = (lay['edge_pos32'] if lay['P'] > 1 else None) if own else self._given_pos(lay)
+        ascend = own or getattr(self, '_weight_perm', None) is None
         self._bop.run_spmm(lay['plan'], lay['pos'], lay['idx'], _REDUCE[self._reduce], lhs, rhs, self._row_scale,
-                           self.out_tvm, self.arg_tvm, edge_pos_dev=pos)
+                           self.out_tvm, self.arg_tvm, edge_pos_dev=pos, ascend=ascend)
 
     def lower_to_ir(self, input_placeholders, compute_args, schedule_args):
         compute_args = dict(compute_args)
@@ -280,6 +281,17 @@ class GSpMMhip(VanillaSpMMhip):
                 self._w_head_major = None          # kept; weights given to later runs get a buffer of their own
             return self._w_static
         return self._weights_in_layout(w, lay, given=True)
+
+    def fix_weights(self, weights):
+        """Lays edge weights (as run() would take them) out once: later run() calls take SrcFeat alone and reuse them."""
+        if self._func is None or self._bop is not None or not self._weights_at_run:
+            raise RuntimeError("fix_weights needs a built weighted sum whose weights are given to run()")
+        self._w_static = None
+        self._w_head_major = None
+        self._w_static = self._weights(weights)
+        self._w_head_major = None
+        self._weights_at_run = False
+        self._placeholders = self._placeholders[:1]
 
     def set_weight_order(self, position_of_edge):
         """Weights and edge operands given to run() are stored in another edge order: position_of_edge[i] is

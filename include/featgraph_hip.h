@@ -338,8 +338,10 @@ typedef enum { FG_TARGET_U = 0, FG_TARGET_E = 1, FG_TARGET_V = 2 } fg_target;
 /* flags: what the caller knows about an offset array, which lets the kernels use 128-bit accesses when out_len
  * is a multiple of 4 and the arrays are 16-byte aligned (0 is always valid; an operand without an offset array
  * needs no flag).  _VEC4: every aligned group of 4 output features reads 4 consecutive operand features that
- * start at a multiple of 4.  _SPLAT4: every such group reads one operand feature 4 times. */
-enum { FG_BCAST_LHS_VEC4 = 1, FG_BCAST_LHS_SPLAT4 = 2, FG_BCAST_RHS_VEC4 = 4, FG_BCAST_RHS_SPLAT4 = 8 };
+ * start at a multiple of 4.  _SPLAT4: every such group reads one operand feature 4 times.
+ * FG_BCAST_EDGES_ASCEND: edge_pos ascends along every row segment of the layout (it does for the positions that
+ * fg_csr_to_dds gives), which lets max / min with positions skip comparing positions on ties. */
+enum { FG_BCAST_LHS_VEC4 = 1, FG_BCAST_LHS_SPLAT4 = 2, FG_BCAST_RHS_VEC4 = 4, FG_BCAST_RHS_SPLAT4 = 8, FG_BCAST_EDGES_ASCEND = 16 };
 int fg_gspmm_bcast_f32(fg_spmm_plan *plan, const int32_t *indptr_dev, const int32_t *indices_dev, int op,
                        int reduce, const float *lhs_dev, int lhs_target, int lhs_len,
                        const int32_t *lhs_off_dev, const float *rhs_dev, int rhs_target, int rhs_len,
@@ -350,6 +352,17 @@ int fg_gspmm_bcast_dds_f32(fg_spmm_plan *plan, const int32_t *s1_pos_dev, const 
                            int lhs_len, const int32_t *lhs_off_dev, const float *rhs_dev, int rhs_target, int rhs_len,
                            const int32_t *rhs_off_dev, int flags, const float *row_scale_dev, float *out_dev,
                            int32_t *arg_dev, int out_len, void *stream);
+/*
+ * Gradient of a max / min aggregation: dlhs / drhs (either may be NULL; both are added to, so clear them first) receive
+ * d(out[v, f]) / d(operand) * dout[v, f] at the operands of the element arg[v, f] that fg_gspmm_bcast_f32 reported
+ * (-1: nothing).  op: FG_BIN_ADD .. FG_BIN_COPY_LHS; operands on FG_TARGET_U or FG_TARGET_E with the offset arrays of
+ * the forward call; lhs_dev / rhs_dev are read for FG_BIN_MUL / FG_BIN_DIV only; col_dev [n_edges] holds every stored
+ * element's column.  Additions are atomic, in no fixed order.
+ */
+int fg_gspmm_select_backward_f32(const int32_t *arg_dev, const int32_t *col_dev, int64_t n_dst, int64_t n_edges, int op,
+                                 const float *lhs_dev, int lhs_target, int lhs_len, const int32_t *lhs_off_dev,
+                                 const float *rhs_dev, int rhs_target, int rhs_len, const int32_t *rhs_off_dev,
+                                 const float *dout_dev, int out_len, float *dlhs_dev, float *drhs_dev, void *stream);
 int fg_gsddmm_bcast_f32(const int32_t *row_dev, const int32_t *col_dev, int64_t n_edges, int op,
                         const float *lhs_dev, int lhs_target, int lhs_len, const int32_t *lhs_off_dev,
                         const float *rhs_dev, int rhs_target, int rhs_len, const int32_t *rhs_off_dev,

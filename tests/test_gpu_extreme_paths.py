@@ -1,0 +1,81 @@
+"""max / min with positions: the kernel finds them by one comparison per message and falls back to the full rule (first
+of the best, NaN above everything, the first message always enters) where that may differ -- NaN messages, rows of -inf,
+edge positions in another order.  Values and positions exactly as the oracle's, with ties, signed zeros and split rows,
+at feature lengths with one to sixteen lane groups per wavefront; and the gradient that follows the positions."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+pytestmark = pytest.mark.gpu
+
+
+def _graph(rng, lens, n_src=700):
+    cols = [np.sort(rng.choice(n_src, size=l, replace=False)) for l in lens]
+    indptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    return sp.csr_matrix((np.ones(indptr[-1], np.float32), np.concatenate(cols).astype(np.int32), indptr), shape=(len(lens), n_src))
+
+
+LENS = [1, 2, 3, 0, 17, 64, 65, 127, 128, 129, 300, 600] + [2] * 70 + [40] * 6
+
+
+@pytest.mark.parametrize("special", ["ties", "nan", "minus_inf"])
+@pytest.mark.parametrize("reduce", ["max", "min"])
+@pytest.mark.parametrize("feat_len", [7, 16, 36, 100, 260])
+def test_positions_match_the_oracle(oracle, special, reduce, feat_len):
+    import torch
+    from featgraph_amd.module import GSpMMhip, placeholder
+    rng = np.random.default_rng(feat_len)
+    adj = _graph(rng, LENS)
+    x = rng.integers(-1, 2, size=(700, feat_len)).astype(np.float32)         # -1, 0, 1: ties everywhere
+    x[x == 0] *= np.where(rng.random((x == 0).sum()) < 0.5, -1, 1)           # zeros of both signs tie as well
+    if special == "nan":
+        x[rng.random(x.shape) < 0.01] = np.nan
+    if special == "minus_inf":
+        x[rng.random(x.shape) < 0.7] = -np.inf if reduce == "max" else np.inf
+    e = np.zeros((adj.nnz, 1), np.float32)
+    for msg, arrays, o in (("copy_u", [x], ("copy_lhs", x, None, "u", "e")), ("u_add_e", [x, e], ("add", x, e, "u", "e"))):
+        ref, ref_arg = oracle.gspmm_bcast(adj.indptr, adj.indices, o[0], reduce, o[1], o[2], o[3], o[4])
+        for P in (None, 3):
+            m = GSpMMhip(adj)
+            m.build([placeholder(a.shape) for a in arrays], {'msg': msg, 'reduce': reduce, 'return_arg': True, 'broadcast': True},
+                    {'num_src_partitions': P})
+            out = m.run([torch.from_numpy(a).cuda() for a in arrays]).cpu().numpy()
+            assert np.array_equal(out, ref, equal_nan=True), (msg, P)
+            assert np.array_equal(m.arg_tvm.cpu().numpy(), ref_arg), (msg, P)
+    # edge operands in another order: the first of a tie is the first in that order
+    where = rng.permutation(adj.nnz).astype(np.int32)
+    m = GSpMMhip(adj)
+    m.build([placeholder(x.shape), placeholder(e.shape)], {'msg': 'u_add_e', 'reduce': reduce, 'return_arg': True, 'broadcast': True}, {})
+    m.set_weight_order(where)
+    out = m.run([torch.from_numpy(x).cuda(), torch.from_numpy(e).cuda()]).cpu().numpy()
+    assert np.array_equal(out, ref, equal_nan=True)
+    arg = m.arg_tvm.cpu().numpy()
+    for v in np.flatnonzero(np.diff(adj.indptr)):
+        a, b = adj.indptr[v], adj.indptr[v + 1]
+        seg = x[adj.indices[a:b]]
+        best = (seg == ref[v]) | (np.isnan(seg) & np.isnan(ref[v]))
+        want = np.where(best, where[a:b, None], np.iinfo(np.int32).max).min(0)
+        assert np.array_equal(arg[v], want), v
+
+
+@pytest.mark.parametrize("op,e_len", [("add", 1), ("sub", 5), ("mul", 5), ("mul", 1), ("div", 5)])
+def test_gradient_goes_to_the_selected_edge(op, e_len):
+    import torch
+    from featgraph_amd import ops
+    from featgraph_amd.autograd import Graph
+    rng = np.random.default_rng(3)
+    adj = _graph(rng, LENS)
+    g = Graph(adj)
+    x = torch.from_numpy(rng.standard_normal((700, 5)).astype(np.float32)).cuda().requires_grad_()
+    e = torch.from_numpy((rng.random((adj.nnz, e_len)) + 0.5).astype(np.float32)).cuda().requires_grad_()
+    dout = torch.from_numpy(rng.standard_normal((len(LENS), 5)).astype(np.float32)).cuda()
+    got = torch.autograd.grad(ops.gspmm(g, op, "max", x, e), [x, e], dout)
+    x64, e64 = x.detach().double().requires_grad_(), e.detach().double().requires_grad_()
+    row = torch.repeat_interleave(torch.arange(len(LENS)), torch.from_numpy(np.diff(adj.indptr)).long()).cuda()
+    xs = x64[torch.from_numpy(adj.indices).cuda().long()]
+    m = xs + e64 if op == "add" else xs - e64 if op == "sub" else xs * e64 if op == "mul" else xs / e64
+    out = torch.zeros((len(LENS), 5), dtype=torch.float64, device="cuda").scatter_reduce(
+        0, row[:, None].expand_as(m), m, "amax", include_self=False)
+    for a, b in zip(got, torch.autograd.grad(out, [x64, e64], dout.double())):
+        # one product of three fp32 factors per term, at most 5 * 83 terms per sum
+        assert ((a.double() - b).abs() <= 1e-5 + 1e-4 * b.abs()).all()
