@@ -460,24 +460,74 @@ class _GSpMMExtreme(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, g, msg, reduce, lhs, rhs=None):
-        arrays = [a.contiguous() for a in ((lhs,) if rhs is None else (lhs, rhs))]
+        arrays = [lhs] if rhs is None else [lhs, rhs]
         out, arg = g._bcast_spmm_raw(msg, arrays, reduce, return_arg=True)
-        ctx.g, ctx.message = g, g._bcast_spmm_message(msg, arrays, reduce, return_arg=True)
+        ctx.g, ctx.msg, ctx.message = g, msg, g._bcast_spmm_message(msg, arrays, reduce, return_arg=True)
         ctx.save_for_backward(arg, *arrays)
         return out
 
     @staticmethod
     def backward(ctx, dout):
         arg, *arrays = ctx.saved_tensors
-        return (None, None, None) + _selected_grads(ctx.g, ctx.message, arg, arrays, dout, ctx.needs_input_grad[3:])
+        needed = ctx.needs_input_grad[3:]
+        if _wants_torch_grads():
+            grads = _selected_grads_torch(ctx.g, ctx.msg, arg, arrays, dout, needed)
+        else:
+            grads = _selected_grads(ctx.g, ctx.message, arg, arrays, [p.shape for p in arrays], dout, needed)
+        return (None, None, None) + tuple(grads)
 
 
-def _selected_grads(g, message, arg, arrays, dout, needed):
-    """Gradients of a max / min aggregation for the operands `arrays`, None where not needed."""
-    grads = [torch.zeros_like(p) if need else None for p, need in zip(arrays, needed)]
-    lhs, rhs = arrays[0], arrays[1] if len(arrays) > 1 else None
-    message.select_backward(arg, g._cols(dout.device), g.nnz, lhs, rhs, dout.contiguous(), grads[0], grads[1] if rhs is not None else None)
-    return tuple(grads)
+def _wants_torch_grads():
+    """Whether a max / min gradient has to come from torch's operators: it is differentiated again (create_graph) or must
+    add in a fixed order; one kernel with float atomics gives neither."""
+    return torch.is_grad_enabled() or torch.are_deterministic_algorithms_enabled()
+
+
+def _selected_grads(g, message, arg, arrays, shapes, dout, needed):
+    """Gradients of a max / min aggregation for operands of `shapes`, None where not needed; `arrays` are the operands' values
+    (None: the message copies its one operand)."""
+    grads = [torch.zeros(s, dtype=dout.dtype, device=dout.device) if need else None for s, need in zip(shapes, needed)]
+    values = [None, None] if arrays is None else [a.contiguous() for a in arrays] + [None]
+    message.select_backward(arg, g._cols(dout.device), g.nnz, values[0], values[1], dout.contiguous(),
+                            grads[0], grads[1] if len(grads) > 1 else None)
+    return grads
+
+
+def _selected_grads_torch(g, msg, arg, arrays, dout, needed):
+    """The same in torch's operators."""
+    op, lt, rt = parse_message(msg)
+    targets = [lt] if rt is None else [lt, rt]
+    n_dst, out_shape = dout.shape[0], tuple(dout.shape[1:])
+    n_out = int(np.prod(out_shape)) if out_shape else 1
+    e = arg.reshape(n_dst, n_out).long()
+    valid = e >= 0
+    e = e.clamp(min=0)
+    rows_of = {"u": g._cols(dout.device).long()[e], "e": e}         # operand row per output element
+
+    def spread(x):      # (rows, *feat) -> (rows, n_out): the operand feature every output feature reads
+        return _align_features(x, dout).expand((x.shape[0],) + out_shape).reshape(x.shape[0], n_out)
+
+    picked = [spread(x).gather(0, rows_of[t]) for x, t in zip(arrays, targets)]
+    d = dout.reshape(n_dst, n_out) * valid
+    grads = []
+    for i, (p, tp, need) in enumerate(zip(arrays, targets, needed)):
+        if not need:
+            grads.append(None)
+            continue
+        if op in ("add", "copy_lhs") or (op == "sub" and i == 0):
+            c = d
+        elif op == "sub":
+            c = -d
+        elif op == "mul":
+            c = d * picked[1 - i]
+        elif i == 0:                                               # div, numerator
+            c = d / picked[1]
+        else:                                                      # div, denominator
+            c = -d * picked[0] / picked[1] ** 2
+        c = torch.where(valid, c, torch.zeros_like(c))
+        full = torch.zeros((p.shape[0], n_out), dtype=dout.dtype, device=dout.device).scatter_add(0, rows_of[tp], c)
+        grads.append(_reduce_to(full.reshape((p.shape[0],) + out_shape), p.shape))
+    return grads
 
 
 def _sum_over_out_edges(g, d):
@@ -529,7 +579,8 @@ class _Aggregate(torch.autograd.Function):
         if reduce in ("max", "min"):
             mod.arg_tvm = torch.empty((g.shape[0], x.shape[1]), dtype=torch.int32, device=mod.ctx)
             y = _fresh_run(mod, [x])
-            ctx.save_for_backward(mod.arg_tvm, x)
+            ctx.save_for_backward(mod.arg_tvm)
+            ctx.x_shape = tuple(x.shape)
             mod.arg_tvm = None
             return y
         return _fresh_run(mod, [x])
@@ -540,6 +591,11 @@ class _Aggregate(torch.autograd.Function):
         dy = dy.contiguous()
         if reduce in ("sum", "mean"):
             return None, _fresh_run(g._aggregate_grad_mod(dy.shape[1], reduce), [dy]), None
-        arg, x = ctx.saved_tensors
-        (dx,) = _selected_grads(g, g._aggregate_mod(dy.shape[1], reduce)._bop, arg, [x], dy, (True,))
+        (arg,) = ctx.saved_tensors
+        if _wants_torch_grads():
+            valid = arg >= 0
+            flat = g._cols(dy.device)[arg.clamp(min=0).long()].long() * dy.shape[1] + torch.arange(dy.shape[1], device=dy.device)
+            dx = torch.zeros(ctx.x_shape[0] * dy.shape[1], dtype=dy.dtype, device=dy.device)
+            return None, dx.index_add(0, flat[valid], dy[valid]).view(ctx.x_shape), None
+        (dx,) = _selected_grads(g, g._aggregate_mod(dy.shape[1], reduce)._bop, arg, None, [ctx.x_shape], dy, (True,))
         return None, dx, None

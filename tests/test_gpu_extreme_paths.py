@@ -79,3 +79,47 @@ def test_gradient_goes_to_the_selected_edge(op, e_len):
     for a, b in zip(got, torch.autograd.grad(out, [x64, e64], dout.double())):
         # one product of three fp32 factors per term, at most 5 * 83 terms per sum
         assert ((a.double() - b).abs() <= 1e-5 + 1e-4 * b.abs()).all()
+
+
+@pytest.mark.parametrize("msg", ["copy", "mul"])
+def test_gradient_can_be_differentiated_again(msg):
+    """create_graph: d/d(dout) and d/d(operand) of a max gradient, against the same chain in float64."""
+    import torch
+    from featgraph_amd import ops
+    from featgraph_amd.autograd import Graph
+    rng = np.random.default_rng(5)
+    adj = _graph(rng, LENS)
+    g = Graph(adj)
+    x = torch.from_numpy(rng.standard_normal((5, 700)).astype(np.float32)).cuda().t().requires_grad_()      # not contiguous
+    e = torch.from_numpy((rng.random((adj.nnz, 5)) + 0.5).astype(np.float32)).cuda().requires_grad_()
+    dout = torch.from_numpy(rng.standard_normal((len(LENS), 5)).astype(np.float32)).cuda().requires_grad_()
+    row = torch.repeat_interleave(torch.arange(len(LENS)), torch.from_numpy(np.diff(adj.indptr)).long()).cuda()
+    col = torch.from_numpy(adj.indices).cuda().long()
+
+    def second(forward, x, e, dout):
+        dx = torch.autograd.grad(forward(x, e), x, dout, create_graph=True)[0]
+        return torch.autograd.grad((dx * dx).sum(), [dout, e] if msg == "mul" else [dout])
+
+    def wide(x, e):
+        m = x[col] * e if msg == "mul" else x[col]
+        return torch.zeros((len(LENS), 5), dtype=torch.float64, device="cuda").scatter_reduce(
+            0, row[:, None].expand_as(m), m, "amax", include_self=False)
+
+    got = second((lambda x, e: ops.gspmm(g, "mul", "max", x, e)) if msg == "mul" else (lambda x, e: g.aggregate(x, "max")), x, e, dout)
+    want = second(wide, *[t.detach().double().requires_grad_() for t in (x, e, dout)])
+    for a, b in zip(got, want):      # as above: products of a few fp32 factors, at most 5 * 83 terms per sum
+        assert ((a.double() - b).abs() <= 1e-5 + 1e-4 * b.abs()).all()
+
+
+def test_input_may_change_before_the_gradient():
+    """A max aggregation's gradient needs the positions alone: overwriting its input in between is allowed."""
+    import torch
+    from featgraph_amd.autograd import Graph
+    rng = np.random.default_rng(6)
+    g = Graph(_graph(rng, LENS))
+    leaf = torch.from_numpy(rng.standard_normal((700, 5)).astype(np.float32)).cuda().requires_grad_()
+    x = leaf * 1
+    out = g.aggregate(x, "max")
+    before = torch.autograd.grad(out.sum(), leaf, retain_graph=True)[0]
+    x.mul_(2)
+    assert torch.equal(before, torch.autograd.grad(out.sum(), leaf)[0])
