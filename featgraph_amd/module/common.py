@@ -1,4 +1,6 @@
 """Pieces shared by the SpMM and SDDMM module classes."""
+import ctypes
+
 import numpy as np
 import torch
 
@@ -45,8 +47,9 @@ def to_device_f32(a, dev):
 
 
 def stream_ptr():
-    import ctypes
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    # (the Stream object that torch.cuda.current_stream() makes first costs 8 us a call, of which a step has ten and more:
+    # an attention layer of single operators with gradients on 10,500 edges is bound by such host work)
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
 
 
 def check_inputs(tensors, placeholders, dev):
