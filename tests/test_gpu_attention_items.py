@@ -37,4 +37,25 @@ def test_attention_matches_float64(kind, heads, head_len, repeat):
     ref = torch.zeros((n, heads, head_len), dtype=torch.float64, device="cuda").index_add(0, row, p[..., None] * v64[col])
     for x, y in zip(got, (ref,) + torch.autograd.grad(ref, [a64, b64, v64], dout.double())):
         # sums of up to 900 (gradients: 60 * repeat * a few) fp32 products, and an exponential good to 2 ulp of its argument
-        assert float((x.double() - y).norm() / y.norm()) <= 1e-5
+        assert float((x.detach().double() - y.detach()).norm() / y.detach().norm()) <= 1e-5
+
+
+@pytest.mark.parametrize("degree", [1, 23, 24])
+def test_head_by_head_copy_changes_no_bit(monkeypatch, degree):
+    """On both sides of the line from which the gathered operands are copied (24 elements per source, 64 MB)."""
+    import torch
+    from featgraph_amd import _lib
+    from featgraph_amd.autograd import Graph
+    n, heads, head_len = 33000, 8, 64
+    cols = np.sort((np.arange(n)[:, None] * 7 + np.arange(degree)[None, :] * 613) % n, axis=1)
+    adj = sp.csr_matrix((np.ones(n * degree, np.float32), cols.ravel().astype(np.int32),
+                         (np.arange(n + 1) * degree).astype(np.int32)), shape=(n, n))
+    gen = torch.Generator(device="cuda").manual_seed(degree)
+    q, k, v, dout = (torch.randn(n, heads, head_len, generator=gen, device="cuda").requires_grad_() for _ in range(4))
+    results = []
+    for tile_major in (0, 1, 2):
+        monkeypatch.setattr(_lib, "plan_opts", _lib.FgPlanOpts(tile_major=tile_major) if tile_major else None)
+        out = Graph(adj).attention(q, k, v)
+        results.append((out.detach(),) + torch.autograd.grad(out, [q, k, v], dout.detach()))
+    for other in results[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(results[0], other))
