@@ -165,7 +165,8 @@ __device__ __forceinline__ void run_together(const SoftmaxArgs &a, int64_t e0, i
                 }
             }
             const float mw = lanes_reduce<true, LANEHEAD>(m, H, W, lane);
-            s = (m == -INFINITY) ? 0.f : s * __expf(m - mw);
+            // a lane that met no number has s = 0 (nothing, or -inf only) or NaN (a NaN among them): either stays
+            s = (m == -INFINITY) ? s : s * __expf(m - mw);
             m = mw;
             s = lanes_reduce<false, LANEHEAD>(s, H, W, lane);
         } else {
@@ -434,7 +435,7 @@ __device__ __forceinline__ void sweep_stats(const float *x, const float *g, int 
         for (int c = 0; c < A; ++c) own[c] = m[c];
         fold<true, A, PER, THREADS>(m, G, THREADS == 64 ? nullptr : red[0]);
 #pragma unroll
-        for (int c = 0; c < A; ++c) s[c] = own[c] == -INFINITY ? 0.f : s[c] * __expf(own[c] - m[c]);
+        for (int c = 0; c < A; ++c) s[c] = own[c] == -INFINITY ? s[c] : s[c] * __expf(own[c] - m[c]);     // 0, or NaN where one was met
         fold<false, A, PER, THREADS>(s, G, THREADS == 64 ? nullptr : red[1]);
     }
 }

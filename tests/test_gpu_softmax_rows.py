@@ -89,3 +89,31 @@ def test_special_values_stay_in_their_row(H):
             else:
                 assert bool(inside.all())
             assert int(bad.sum()) == int(inside.sum())
+
+
+@pytest.mark.parametrize("H", [1, 2, 3, 4, 5, 8, 12, 64])
+def test_nan_anywhere_reaches_its_whole_row(H):
+    """A NaN score at the first, a middle or the last element of a row, alone or among scores of -inf, makes the row's every
+    value NaN, also where a lane sees nothing but that NaN: short last pieces (1, 5 and 64 elements) of rows that are
+    swept in pieces, and a row longer than a workgroup takes at every head count."""
+    import torch
+    from featgraph_amd.module import EdgeSoftmaxhip, placeholder
+    lens = np.array([3, 700, 5, 2565, 20, 1025, 40_000, 8, 33, 140_000, 4, 33])
+    indptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    nnz = int(indptr[-1])
+    indices = np.concatenate([np.arange(n) for n in lens]).astype(np.int32)
+    m = EdgeSoftmaxhip(sp.csr_matrix((np.ones(nnz, np.float32), indices, indptr), shape=(len(lens), max(lens))))
+    m.build([placeholder((nnz, H))])
+    x0 = torch.randn(nnz, H, generator=torch.Generator(device="cuda").manual_seed(H), device="cuda")
+    for r in range(len(lens)):
+        b, e = int(indptr[r]), int(indptr[r + 1])
+        for at in sorted({b, (b + e) // 2, e - 1}):
+            for masked in (False, True):
+                x = x0.clone()
+                if masked:
+                    x[b:e, 0] = -float("inf")
+                    x[b if at != b else e - 1, 0] = 0.5         # the row's one number
+                x[at, 0] = float("nan")
+                bad = torch.isnan(m.run([x]))
+                assert bool(bad[b:e, 0].all()), (r, at - b, masked)
+                assert int(bad.sum()) == e - b
