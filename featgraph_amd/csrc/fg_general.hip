@@ -133,6 +133,8 @@ template <int RED> __device__ __forceinline__ bool replaces(float m, int em, flo
     return em != INT_MAX && (ea == INT_MAX || better || (same && em < ea));
 }
 
+enum { kFirst, kFull, kNaNs };      // how a walk finds positions, see batch() below
+
 // LC / RC (V == 4 only): the operand's 4 features are consecutive (one 128-bit load), else one value 4 times.
 // No branch stands between the loads of a step: one around a load would make the wavefront wait for everything
 // issued before it.
@@ -207,13 +209,14 @@ __global__ __launch_bounds__(kBlock) void gspmm_bcast_kernel(const GenArgs a) {
             int at[V];
             // One step of U elements (staged slots tb, tb + step, ...) into acc / at.  ALL: every slot lies below t1; else
             // a slot beyond re-reads the group's element tb, which a maximum does not notice and a sum discards by a select.
-            // CAREFUL: positions by the full rule of replaces(); otherwise by "larger than all before" -- one comparison,
+            // Positions (FIND): kFull, by the full rule of replaces(); kFirst, by "larger than all before" -- one comparison,
             // one maximum and one select per message where the rule takes a dozen instructions -- which agrees with it when
-            // positions ascend along the walk and no NaN and not only -inf was met (the caller checks).  copy_u max with
-            // positions, 12.5M edges, F=100: 1130 us with the rule on every message, 441 us so (11 TB/s of gathered rows);
-            // 114.8M edges, F=64: 4.1 -> 2.56 ms.
-            auto batch = [&](auto all_tag, auto careful_tag, int tb, int t1) {
-                constexpr bool ALL = decltype(all_tag)::value, CAREFUL = decltype(careful_tag)::value;
+            // positions ascend along the walk, except for features with a NaN or with nothing above -inf (the caller
+            // mends them); kNaNs, the earliest NaN's position only.  copy_u max with positions, 12.5M edges, F=100: 1130 us with
+            // the rule on every message, 441 us by kFirst (11 TB/s of gathered rows); 114.8M edges, F=64: 4.1 -> 2.56 ms.
+            auto batch = [&](auto all_tag, auto find_tag, int tb, int t1) {
+                constexpr bool ALL = decltype(all_tag)::value;
+                constexpr int FIND = decltype(find_tag)::value;
                 float m[U][V];
                 int stored[U];          // the element's position in the caller's edge order
 #pragma unroll
@@ -236,7 +239,9 @@ __global__ __launch_bounds__(kBlock) void gspmm_bcast_kernel(const GenArgs a) {
                     for (int i = 0; i < V; ++i) {
                         if (RED == FG_REDUCE_SUM) {
                             acc[i] += (ALL || tb + k * step < t1) ? m[k][i] : 0.f;
-                        } else if (ARG && CAREFUL) {
+                        } else if (ARG && FIND == kNaNs) {
+                            at[i] = m[k][i] != m[k][i] ? min(at[i], stored[k]) : at[i];
+                        } else if (ARG && FIND == kFull) {
                             if (replaces<RED>(m[k][i], stored[k], acc[i], at[i])) { acc[i] = m[k][i]; at[i] = stored[k]; }
                         } else if (ARG) {
                             at[i] = !(m[k][i] <= acc[i]) ? stored[k] : at[i];
@@ -247,9 +252,11 @@ __global__ __launch_bounds__(kBlock) void gspmm_bcast_kernel(const GenArgs a) {
                     }
                 }
             };
-            auto walk = [&](auto careful_tag) {
+            auto walk = [&](auto find_tag) {
+                if (decltype(find_tag)::value != kNaNs) {
 #pragma unroll
-                for (int i = 0; i < V; ++i) { acc[i] = identity<RED>(); at[i] = INT_MAX; }
+                    for (int i = 0; i < V; ++i) { acc[i] = identity<RED>(); at[i] = INT_MAX; }
+                }
                 for (int64_t c0 = e0; c0 < e1; c0 += kStage) {
                     const int64_t c1 = min(c0 + kStage, e1);
                     int64_t base = staged_at;
@@ -260,24 +267,41 @@ __global__ __launch_bounds__(kBlock) void gspmm_bcast_kernel(const GenArgs a) {
                     }
                     const int t1 = (int)(c1 - base);       // positions in the staged window
                     int tb = (int)(c0 - base) + first;
-                    for (; tb + (U - 1) * step < t1; tb += step * U) batch(std::true_type{}, careful_tag, tb, t1);
-                    if (tb < t1) batch(std::false_type{}, careful_tag, tb, t1);
+                    for (; tb + (U - 1) * step < t1; tb += step * U) batch(std::true_type{}, find_tag, tb, t1);
+                    if (tb < t1) batch(std::false_type{}, find_tag, tb, t1);
                 }
             };
-            bool again = ARG && !a.ordered;
+            bool full_rule = ARG && !a.ordered;      // whether the groups' results need it as well
             if constexpr (ARG) {
-                if (a.ordered) {
-                    walk(std::false_type{});
+                if (full_rule) {
+                    walk(std::integral_constant<int, kFull>{});
+                } else {
+                    walk(std::integral_constant<int, kFirst>{});
+                    // Nothing above -inf though the group had elements: the first of them.  12.5M edges, F=64 / 100 / 256, 97 %
+                    // of the messages -inf: 823 / 1277 / 2152 us with such rows walked again by the full rule, 281 / 451 /
+                    // 1040 so (no -inf: 285 / 454 / 1032).
+                    bool none = false, nan = false;
 #pragma unroll
-                    for (int i = 0; i < V; ++i)      // a NaN, or nothing above -inf though the group had elements
-                        again = again || acc[i] != acc[i] || (at[i] == INT_MAX && e0 + first < e1);
+                    for (int i = 0; i < V; ++i) { none = none || at[i] == INT_MAX; nan = nan || acc[i] != acc[i]; }
+                    if (none && e0 + first < e1) {
+                        const int head = PART ? a.edge_pos[e0 + first] : (int)(e0 + first);
+#pragma unroll
+                        for (int i = 0; i < V; ++i) at[i] = at[i] == INT_MAX ? head : at[i];
+                    }
+                    // A NaN: its features' positions by a second walk.  1 % of the messages NaN, so that nearly every row has
+                    // one: 826 / 1516 / 2814 us with the full rule, 460 / 806 / 1800 so (the full rule alone, as the only
+                    // walk: 682 / 1296 / 2419; 1M edges on 200,000 nodes, F=256: 425, 327, 278).
+                    full_rule = __any(nan);              // uniform over the wavefront
+                    if (full_rule) {
+#pragma unroll
+                        for (int i = 0; i < V; ++i) at[i] = acc[i] != acc[i] ? INT_MAX : at[i];
+                        walk(std::integral_constant<int, kNaNs>{});
+                    }
                 }
-                again = __any(again);                // uniform over the wavefront from here on
-                if (again) walk(std::true_type{});
             } else {
-                walk(std::false_type{});
+                walk(std::integral_constant<int, kFirst>{});
             }
-            if (ARG && !OWN && !again) {
+            if (ARG && !OWN && !full_rule) {
                 // no NaN anywhere: the groups' largest value first, then the earliest position that has it
                 float best[V];
 #pragma unroll
