@@ -214,7 +214,8 @@ __device__ __forceinline__ void run_together(const SoftmaxArgs &a, int64_t e0, i
             m = -INFINITY;
             for (int j = lane; j < len; j += 64) m = fmaxf(m, x[(int64_t)j * H + h]);
             m = head_reduce<true>(m, 1);
-            for (int j = lane; j < len; j += 64) s += __expf(x[(int64_t)j * H + h] - m);
+            // -inf adds nothing, also where the run (a piece of a row) holds nothing else and m is -inf
+            for (int j = lane; j < len; j += 64) { const float v = x[(int64_t)j * H + h]; s += v == -INFINITY ? 0.f : __expf(v - m); }
             s = head_reduce<false>(s, 1);
         } else {
             for (int j = lane; j < len; j += 64) m += x[(int64_t)j * H + h] * g[(int64_t)j * H + h];

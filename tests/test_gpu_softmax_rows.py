@@ -117,3 +117,30 @@ def test_nan_anywhere_reaches_its_whole_row(H):
                 bad = torch.isnan(m.run([x]))
                 assert bool(bad[b:e, 0].all()), (r, at - b, masked)
                 assert int(bad.sum()) == e - b
+
+
+@pytest.mark.parametrize("H", [1, 3, 4, 5, 12, 64, 65, 100])
+def test_a_piece_of_masked_scores_leaves_its_row_finite(H):
+    """Scores of -inf throughout the first, a middle or the last piece of a row that is swept in pieces (128 elements each
+    here): zeros there, and the softmax of the rest elsewhere, against float64."""
+    import torch
+    from featgraph_amd.module import EdgeSoftmaxhip, placeholder
+    lens = np.array([300, 3, 700, 129, 20, 2100])
+    indptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    nnz = int(indptr[-1])
+    indices = np.concatenate([np.arange(n) for n in lens]).astype(np.int32)
+    m = EdgeSoftmaxhip(sp.csr_matrix((np.ones(nnz, np.float32), indices, indptr), shape=(len(lens), max(lens))))
+    m.build([placeholder((nnz, H))])
+    x = torch.randn(nnz, H, generator=torch.Generator(device="cuda").manual_seed(H), device="cuda")
+    for b, e in zip(indptr[:-1].tolist(), indptr[1:].tolist()):
+        if e - b == 700:
+            x[b + 120:b + 400, ::2] = -float("inf")
+        elif e - b == 2100:
+            x[b + 1000:e, 1::2] = -float("inf")
+        else:
+            x[b:b + (e - b) // 2 + 1, :] = -float("inf")
+    got = m.run([x]).double()
+    for b, e in zip(indptr[:-1].tolist(), indptr[1:].tolist()):
+        ref = torch.softmax(x[b:e].double(), 0)
+        # as in test_every_row_length_class, with differences of at most 10 between finite scores of a row
+        assert bool(((got[b:e] - ref).abs() <= ref * EPS * (16 + 4 * 10)).all()), (b, e)
