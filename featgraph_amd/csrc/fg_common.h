@@ -36,6 +36,9 @@ struct Item {
 constexpr int kItemEdges = 256;   // elements staged in LDS per wavefront at a time
 constexpr int kItemRows = 64;     // most rows one multi-row item may hold
 constexpr int kMaxPieces = 8192;  // most pieces (per partition) for which a plan cuts rows finer than on a large graph
+constexpr int kMaxTileFloats = 512;                          // widest feature tile of the SpMM kernels
+constexpr size_t kFixedScratchFloats = (size_t)4 << 20;      // fg_spmm_csr_noalloc_f32's array, 16 MiB
+static_assert((size_t)kMaxPieces * kMaxTileFloats <= kFixedScratchFloats, "one tile of a finely cut plan's pieces fits the array");
 
 // A row segment that was split: pieces partial[slot0 .. slot0 + n_pieces) add up to it.
 struct Fixup {

@@ -868,6 +868,7 @@ int choose_config(int F, int T, bool aligned16, SpmmConfig *c) {
     if (lanes <= 64) { c->L = pow2_ceil(lanes) < 4 ? 4 : pow2_ceil(lanes); c->K = 1; }
     else { c->L = 64; c->K = (lanes >= 256 && c->V == 1) ? 4 : 2; }
     const int ft = c->V * c->L * c->K;
+    if (ft > fg::kMaxTileFloats) return fail(FG_ERR_SHAPE, "feature tile of %d floats", ft);
     c->tile_w = Fp;
     c->sub_per_tile = (Fp + ft - 1) / ft;
     c->n_ftiles = T * c->sub_per_tile;
@@ -1127,10 +1128,13 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
         else hipLaunchKernelGGL(spmm_fixup_kernel<1>, dim3(blocks), dim3(256), 0, st, pl->fixups_dev, pl->n_fixups, partial, F, pass_buf, F, 0, F, 0, (int64_t)piece, (int64_t)pass_stride);
     }
     // Kernel tiles [cb, ce) at a time: all of them, unless the pieces' columns have to fit an array of fixed size (a plan
-    // cut finer than 1024 elements per piece has at most kMaxPieces pieces, so one kernel tile always fits).
+    // cut finer than 1024 elements per piece has at most kMaxPieces pieces of at most kMaxTileFloats columns).
     auto tile_col = [&](int t) { return t >= c.n_ftiles ? F : (t / c.sub_per_tile) * c.tile_w + (t % c.sub_per_tile) * ft; };
     const int64_t max_cols = (fixed_partial && pl->max_slots_in_partition > 0)
                                  ? (int64_t)(fixed_partial_floats / (size_t)pl->max_slots_in_partition) : F;
+    if (std::min(ft, c.tile_w) > max_cols)
+        return fail(FG_ERR_SHAPE, "%lld pieces of %d columns exceed the fixed buffer of this entry point",
+                    (long long)pl->max_slots_in_partition, std::min(ft, c.tile_w));
     for (int p = 0; p < P && !pass_buf; ++p)
     for (int cb = 0, ce; cb < c.n_ftiles; cb = ce) {
         ce = cb + 1;
@@ -1262,7 +1266,7 @@ extern "C" int fg_spmm_csr_f32(fg_spmm_plan *plan, const int32_t *indptr_dev,
 // instead of plan-owned memory.  Every device the library runs on holds its own copy of the array
 // until the process ends; its address on a device is looked up once, with that device current.
 namespace {
-constexpr size_t kFixedScratchFloats = (size_t)4 << 20;          // 16 MiB
+using fg::kFixedScratchFloats;
 static __device__ __align__(256) float scratch[kFixedScratchFloats];
 
 constexpr int kMaxDevices = 64;

@@ -78,3 +78,43 @@ def test_fixed_scratch_takes_a_finer_cut_in_column_ranges(feat_len, tiles):
         assert torch.isfinite(ref).all() and torch.equal(ref, got)
     finally:
         L.fg_spmm_plan_destroy(plan)
+
+
+def _plan(indptr, n_src):
+    from featgraph_amd import _lib
+    L, plan = _lib.lib(), ctypes.c_void_p()
+    assert L.fg_spmm_plan_create(_lib.host_ptr(indptr), len(indptr) - 1, n_src, 1, None, ctypes.byref(plan)) == 0
+    return plan
+
+
+@pytest.mark.parametrize("rows", [4096, 4097])
+def test_as_many_pieces_as_a_finer_cut_may_make(rows):
+    """Rows of 129 elements, two pieces each: 8192 pieces are the most that a finer cut makes and with tiles of 512
+    columns fill the fixed array to its last float; one row more and the plan cuts at 256, which leaves every row whole.
+    (The 4,096 hold one row of 1200, ten pieces.)"""
+    import torch
+    from featgraph_amd import _lib
+    L, n_src, F = _lib.lib(), 1200, 1024
+    lens = np.full(rows, 129) if rows > 4096 else np.concatenate([np.full(4091, 129), [1200]])      # 8182 + 10 pieces
+    indptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    rng = np.random.default_rng(rows)
+    nnz = int(indptr[-1])
+    start = rng.integers(0, n_src, size=len(lens))
+    cols = ((np.arange(nnz) - np.repeat(indptr[:-1], lens) + np.repeat(start, lens)) % n_src).astype(np.int32)
+    vals = torch.from_numpy(rng.standard_normal(nnz).astype("float32")).cuda()
+    x = torch.from_numpy(rng.standard_normal((n_src, F)).astype("float32")).cuda()
+    ip, ix = torch.from_numpy(indptr).cuda(), torch.from_numpy(cols).cuda()
+    plan = _plan(indptr, n_src)
+    try:
+        p, s = _lib.dev_ptr, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        ref, got = (torch.full((len(lens), F), float("nan"), device="cuda") for _ in range(2))
+        assert L.fg_spmm_csr_f32(plan, p(ip), p(ix), p(vals), p(x), p(ref), F, 0, s) == 0
+        assert L.fg_spmm_csr_noalloc_f32(plan, p(ip), p(ix), p(vals), p(x), p(got), F, 0, s) == 0
+        torch.cuda.synchronize()
+        assert torch.isfinite(ref).all() and torch.equal(ref, got)
+        row = torch.repeat_interleave(torch.arange(len(lens)), torch.from_numpy(lens)).cuda()
+        want = torch.zeros((len(lens), 8), dtype=torch.float64, device="cuda").index_add(0, row, (vals[:, None] * x[:, -8:][ix.long()].double()))
+        mass = torch.zeros_like(want).index_add(0, row, (vals[:, None] * x[:, -8:][ix.long()].double()).abs())
+        assert bool(((got[:, -8:] - want).abs() <= 64 * 6e-8 * mass).all())
+    finally:
+        L.fg_spmm_plan_destroy(plan)
