@@ -70,4 +70,20 @@ __device__ __forceinline__ float group_sum(float v) {
     return v;
 }
 
+// use(p, load(p)) for p in [first, n), in order, eight loads in flight: a row's pieces added up one load at a time take
+// about 0.3 us each.  3 M elements with rows of up to 60,000 (240 pieces), whole calls: F=16 weighted sum 84 -> 51 us,
+// maximum 176 -> 121; 100 rows of 5,000, F=16 maximum 32 -> 18; the results are the same bits.
+template <typename Load, typename Use>
+__device__ __forceinline__ void each_piece(int first, int n, Load load, Use use) {
+    constexpr int U = 8;
+    for (int p0 = first; p0 < n; p0 += U) {
+        decltype(load(0)) v[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) v[k] = load(min(p0 + k, n - 1));
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+            if (p0 + k < n) use(p0 + k, v[k]);
+    }
+}
+
 }  // namespace fg

@@ -388,14 +388,14 @@ __global__ __launch_bounds__(256) void gspmm_bcast_fixup_kernel(const Fixup *fix
     const int64_t from = fx.part * partial_stride, to = fx.part * out_stride;
     float acc = identity<RED>();
     int at = INT_MAX;
-    for (int p = 0; p < fx.n_pieces; ++p) {
-        const float m = partial[from + (int64_t)(fx.slot0 + p) * F + f];
-        if (RED == FG_REDUCE_SUM) acc = p == 0 ? m : acc + m;
-        else if (ARG) {
-            const int am = partial_arg[from + (int64_t)(fx.slot0 + p) * F + f];
-            if (am >= 0 && replaces<RED>(m, am, acc, at)) { acc = m; at = am; }
-        } else acc = extreme<RED>(acc, m);
-    }
+    const int64_t first = from + (int64_t)fx.slot0 * F + f;
+    struct Piece { float m; int at; };
+    fg::each_piece(0, fx.n_pieces, [&](int p) { return Piece{partial[first + (int64_t)p * F], ARG ? partial_arg[first + (int64_t)p * F] : 0}; },
+                   [&](int p, const Piece &c) {
+        if (RED == FG_REDUCE_SUM) acc = p == 0 ? c.m : acc + c.m;
+        else if (ARG) { if (c.at >= 0 && replaces<RED>(c.m, c.at, acc, at)) { acc = c.m; at = c.at; } }
+        else acc = extreme<RED>(acc, c.m);
+    });
     if (row_scale) acc *= row_scale[fx.row];
     out[to + (int64_t)fx.row * F + f] = acc;
     if (ARG) arg[to + (int64_t)fx.row * F + f] = (at == INT_MAX) ? -1 : at;

@@ -815,13 +815,14 @@ __global__ __launch_bounds__(256) void edge_softmax_merge_kernel(const Fixup *fi
     const int h = (int)(t % H);
     float2 *s = stats + (int64_t)fx.slot0 * H + h;
     float m, sum = 0.f;
+    auto load = [&](int p) { return s[(int64_t)p * H]; };
     if (!BWD) {
         m = s[0].x;
-        for (int p = 1; p < fx.n_pieces; ++p) m = fmaxf(m, s[(int64_t)p * H].x);
-        for (int p = 0; p < fx.n_pieces; ++p) sum += s[(int64_t)p * H].y * __expf(s[(int64_t)p * H].x - m);
+        fg::each_piece(1, fx.n_pieces, load, [&](int, const float2 &c) { m = fmaxf(m, c.x); });
+        fg::each_piece(0, fx.n_pieces, load, [&](int, const float2 &c) { sum += c.y * __expf(c.x - m); });
     } else {
         m = 0.f;
-        for (int p = 0; p < fx.n_pieces; ++p) m += s[(int64_t)p * H].x;
+        fg::each_piece(0, fx.n_pieces, load, [&](int, const float2 &c) { m += c.x; });
     }
     for (int p = 0; p < fx.n_pieces; ++p) s[(int64_t)p * H] = make_float2(m, sum);
 }
@@ -864,8 +865,9 @@ __global__ __launch_bounds__(256) void edge_softmax_stats_merge_kernel(const Fix
     const int h = (int)(t % H);
     const float2 *s = stats + (int64_t)fx.slot0 * H + h;
     float m = s[0].x, sum = 0.f;
-    for (int p = 1; p < fx.n_pieces; ++p) m = fmaxf(m, s[(int64_t)p * H].x);
-    for (int p = 0; p < fx.n_pieces; ++p) sum += s[(int64_t)p * H].y * __expf(s[(int64_t)p * H].x - m);
+    auto load = [&](int p) { return s[(int64_t)p * H]; };
+    fg::each_piece(1, fx.n_pieces, load, [&](int, const float2 &c) { m = fmaxf(m, c.x); });
+    fg::each_piece(0, fx.n_pieces, load, [&](int, const float2 &c) { sum += c.y * __expf(c.x - m); });
     row_stats[(int64_t)fx.row * H + h] = make_float2(m, sum);
 }
 

@@ -622,8 +622,8 @@ __global__ __launch_bounds__(256) void gspmm_extreme_fixup_kernel(const Fixup *f
     const Fixup fx = fixups[t / per_row];
     const int f = (int)(t % per_row) * V;
     vec m = *reinterpret_cast<const vec *>(partial + (int64_t)fx.slot0 * F + f);
-    for (int p = 1; p < fx.n_pieces; ++p)
-        vext<IS_MAX>(m, *reinterpret_cast<const vec *>(partial + (int64_t)(fx.slot0 + p) * F + f));
+    fg::each_piece(1, fx.n_pieces, [&](int p) { return *reinterpret_cast<const vec *>(partial + (int64_t)(fx.slot0 + p) * F + f); },
+                   [&](int, const vec &v) { vext<IS_MAX>(m, v); });
     *reinterpret_cast<vec *>(out + (int64_t)fx.row * F + f) = m;
 }
 
@@ -825,8 +825,8 @@ __global__ __launch_bounds__(256) void spmm_fixup_kernel(const Fixup *fixups, in
     partial += fx.part * part_stride;
     out += fx.part * out_stride;
     vec sum = *reinterpret_cast<const vec *>(partial + (int64_t)fx.slot0 * partial_ld + f);
-    for (int p = 1; p < fx.n_pieces; ++p)
-        vadd(sum, *reinterpret_cast<const vec *>(partial + (int64_t)(fx.slot0 + p) * partial_ld + f));
+    fg::each_piece(1, fx.n_pieces, [&](int p) { return *reinterpret_cast<const vec *>(partial + (int64_t)(fx.slot0 + p) * partial_ld + f); },
+                   [&](int, const vec &v) { vadd(sum, v); });
     vec *o = reinterpret_cast<vec *>(out + (int64_t)fx.row * F + f0 + f);
     if (accumulate) vadd(sum, *o);
     *o = sum;
