@@ -17,21 +17,27 @@ using fg::Item;
 namespace {
 constexpr int kDefaultSplit = 1024;   // elements per wavefront piece of a long row, on a large graph
 
-// How finely a plan of `nnz` elements is cut when the caller leaves it open.  A wavefront works through its item serially,
-// so on a graph that does not fill the chip (8,192 wavefront slots) the longest item is what a launch takes, and on
-// any graph a long row's last piece is what a launch ends with.  Row pieces of 128 elements below 2^20 elements, 256
-// below 2^23, 512 below 2^25 (unless the caller sets the piece length); several rows share an item up to about nnz / 4096 elements (a power of two of 16 .. 256).
-// Measured, operator pairs and training steps, microseconds of kernel time at (1024, 256) -> at the rule's
-// (split, item): 10,500 edges (128, 16) weighted sum F=64 with gradients 47 -> 30, edge softmax H=4 33 -> 8;
-// 169,867 edges (128, 32) 53 -> 39 and 17 -> 16; 400,000 edges (128, 64) 89 -> 60 and 68 -> 41; 2 M edges (256, 256)
-// 154 -> 132; 6 M (256, 256) 367 -> 343, max F=64 822 -> 734; 12.5 M (512, 256) 692 -> 664, 1243 -> 1159.  Smaller items
-// than the rule's lose the one-lane-group-per-row walk of many short rows: 1.5 M edges of degree 15, F=64, 156 at 256,
-// 200 at 64.
-void default_cut(int64_t nnz, int *split, int *item_edges) {
-    *split = nnz < (1 << 20) ? 128 : nnz < (1 << 23) ? 256 : nnz < (1 << 25) ? 512 : kDefaultSplit;
+// How finely a plan is cut when the caller leaves it open.  A wavefront works through its item serially, so on a graph that
+// does not fill the chip (8,192 wavefront slots) the longest item is what a launch takes, and on any graph a long row's last
+// piece is what a launch ends with.  Row pieces of 128 elements below 2^20 elements, 256 below 2^23, 512 below 2^25.  The
+// launch that adds pieces up costs 3 us: none finer than 1024 where no row is longer than 256, or than 512 with 1,700 times
+// that much other work to hide it.  us of a call cut at 128 / 256 / 512 -> whole: 2,000 rows of 500 elements, 8 heads of 8
+// floats 41 / 34 / 30 -> 30, F=64 weighted sum 20 / 18 / 18 -> 18, F=256 111 / 129 / 127 -> 127; longest row 170 of 7,900
+// elements, F=64 17 -> 14, F=256 u_mul_e 20 -> 29.  Rows of 1000 (300 of them), F=8 17 -> 15, F=64 17 -> 30, F=256 49 -> 106.
+// Several rows share an item of up to 256 elements, a power of two of 16 .. 128 on graphs that would have fewer than about
+// 1,700 such items (10,000 rows of 17: F=256 maximum at 16 / 64 / 256 elements 26 / 24 / 52 us, 8 heads of 8 28 / 19 / 19;
+// 30,000 of 8, 16 / 128 / 256: F=8 maximum 25 / 35 / 61, 8 heads of 8 43 / 19 / 19).  Rows of up to 4 elements on average
+// are walked one per lane group where an item holds enough of them (64 fit): whole items of 256 there, or on fewer than
+// 2^17 elements the smallest, nothing between (100,000 rows of 3, F=16 u_mul_e at 16 / 64 / 256: 64 / 90 / 14 us; 20,000 of 3,
+// F=8: 15 / 32 / 36, F=256 24 / 45 / 121).
+void default_cut(int64_t nnz, int64_t rows, int64_t longest, int *split, int *item_edges) {
+    constexpr int kItems = 1700;
+    const bool whole = longest <= std::max<int64_t>(256, std::min<int64_t>(512, nnz / kItems));
+    *split = whole ? kDefaultSplit : nnz < (1 << 20) ? 128 : nnz < (1 << 23) ? 256 : nnz < (1 << 25) ? 512 : kDefaultSplit;
     int item = 16;
-    while (item < fg::kItemEdges && (int64_t)item * 2 * 4096 <= nnz) item *= 2;
-    *item_edges = nnz < (1 << 20) ? item : fg::kItemEdges;
+    if (nnz <= 4 * rows) item = nnz < (1 << 17) ? 16 : fg::kItemEdges;
+    else while (item < fg::kItemEdges && (int64_t)item * 2 * kItems <= nnz) item *= 2;
+    *item_edges = item;
 }
 
 // Pieces of all rows longer than `split` in the partition that has most of them.
@@ -60,18 +66,19 @@ extern "C" int fg_spmm_plan_create(const int32_t *pos, int64_t n_dst, int64_t n_
     const int64_t d2 = n_dst + 1;
 
     // structure check: one non-decreasing run of positions across all partitions
-    int64_t prev = 0;
+    int64_t prev = 0, longest = 0;
     for (int p = 0; p < P; ++p)
         for (int64_t r = 0; r <= n_dst; ++r) {
             const int64_t v = pos[p * d2 + r];
             if ((p == 0 && r == 0 && v != 0) || v < prev || (r == 0 && v != prev))
                 return fail(FG_ERR_GRAPH, "position array is not a monotone run at partition %d row %lld",
                             p, (long long)r);
+            if (r > 0) longest = std::max(longest, v - prev);
             prev = v;
         }
 
     int split, item_edges;
-    default_cut(prev, &split, &item_edges);
+    default_cut(prev, n_dst * P, longest, &split, &item_edges);
     if (opts && opts->split_threshold > 0) split = opts->split_threshold;
     else {
         // (kMaxPieces bounds the scratch and what fg_spmm_csr_noalloc_f32 has to fit into its fixed array)

@@ -77,10 +77,12 @@ typedef struct fg_spmm_plan fg_spmm_plan;
 
 typedef struct {
     int32_t split_threshold; /* rows longer than this are split over wavefronts; 0 = default: 128 elements on graphs
-                                of fewer than 2^20 elements, 256 below 2^23, 512 below 2^25, else 1024 */
+                                of fewer than 2^20 elements, 256 below 2^23, 512 below 2^25, doubled up to 1024 while a
+                                partition's split rows would make more than 8192 pieces; 1024 on larger graphs and
+                                where no row is longer than 256 (512, if the graph has 1,700 times as many elements) */
     int32_t item_edges;      /* short rows are packed into items of at most this many elements
-                                (and at most 64 rows); 0 = default: 256, fewer (16 .. 128, about nnz / 4096) on graphs
-                                of fewer than 2^20 elements; 1 = one row per item */
+                                (and at most 64 rows); 0 = default: 256, or 16 .. 128 on graphs that would have fewer
+                                than about 1,700 such items; 1 = one row per item */
     int32_t wide_offsets;    /* non-zero: address feature rows with 64-bit offsets even when the matrix
                                 is smaller than 4 GiB (the path larger matrices take; for testing it) */
     int32_t tile_major;      /* SpMM / tiled SDDMM gather from a copy of the source features stored tile by

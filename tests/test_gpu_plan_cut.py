@@ -1,6 +1,6 @@
 """How finely a plan cuts its rows follows the graph's size (fg_spmm_plan_create): pieces of 128, 256, 512 or 1024
-elements and items of 16 to 256.  Graphs on both sides of every line, with rows one element below, at and above the piece
-lengths, against float64; and the entry point with a fixed scratch array on a plan cut finer than its limit counts."""
+elements and items of 16 to 256.  Graphs on both sides of every line but the last (2^25), with rows one element below, at and
+above the piece lengths, against float64; the plan's own account of its cut on both sides of all of them; and the entry point with a fixed scratch array on a plan cut finer than its limit counts."""
 import ctypes
 
 import numpy as np
@@ -87,17 +87,15 @@ def _plan(indptr, n_src):
     return plan
 
 
-@pytest.mark.parametrize("rows", [4096, 4097])
-def test_as_many_pieces_as_a_finer_cut_may_make(rows):
-    """Rows of 129 elements, two pieces each: 8192 pieces are the most that a finer cut makes and with tiles of 512
-    columns fill the fixed array to its last float; one row more and the plan cuts at 256, which leaves every row whole.
-    (The 4,096 hold one row of 1200, ten pieces.)"""
+def test_as_many_pieces_as_a_finer_cut_may_make():
+    """4,091 rows of 129 elements, two pieces each, and one of 1200, ten: 8192 pieces are the most that a finer cut makes and
+    with tiles of 512 columns fill the fixed array to its last float."""
     import torch
     from featgraph_amd import _lib
     L, n_src, F = _lib.lib(), 1200, 1024
-    lens = np.full(rows, 129) if rows > 4096 else np.concatenate([np.full(4091, 129), [1200]])      # 8182 + 10 pieces
+    lens = np.concatenate([np.full(4091, 129), [1200]])
     indptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
-    rng = np.random.default_rng(rows)
+    rng = np.random.default_rng(7)
     nnz = int(indptr[-1])
     start = rng.integers(0, n_src, size=len(lens))
     cols = ((np.arange(nnz) - np.repeat(indptr[:-1], lens) + np.repeat(start, lens)) % n_src).astype(np.int32)
@@ -118,3 +116,30 @@ def test_as_many_pieces_as_a_finer_cut_may_make(rows):
         assert bool(((got[:, -8:] - want).abs() <= 64 * 6e-8 * mass).all())
     finally:
         L.fg_spmm_plan_destroy(plan)
+
+
+def _cut(lens):
+    """A default plan's description."""
+    from featgraph_amd import _lib
+    plan = _plan(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32), int(max(lens)))
+    try:
+        text = ctypes.create_string_buffer(4096)
+        assert _lib.lib().fg_spmm_plan_describe(plan, 0, 0, text, 4096) >= 0
+        return text.value.decode()
+    finally:
+        _lib.lib().fg_spmm_plan_destroy(plan)
+
+
+@pytest.mark.parametrize("lens,split,item", [
+    ([256] * 4, 1024, 16), ([257] * 4, 128, 16),                                    # rows left whole up to 256
+    ([512] * 1700, 1024, 256), ([512] * 1699, 128, 128), ([513] * 1700, 256, 256),  # ... up to 512 with 1,700 times as much
+    ([4] * 32767, 1024, 16), ([4] * 32768, 1024, 256),                              # 4 elements per row on average
+    ([5] * 10879, 1024, 16), ([5] * 10880, 1024, 32),                               # 16 * 2 * 1700 elements
+    ([2000] + [16] * 65410, 128, 128), ([2000] + [16] * 65411, 256, 256),           # 2^20
+    ([2000] + [16] * 524162, 256, 256), ([2000] + [16] * 524163, 512, 256),         # 2^23
+    ([3000] + [64] * 524241, 512, 256), ([3000] + [64] * 524242, 1024, 256),        # 2^25
+    ([600] * 1638, 128, 128), ([600] * 1639, 256, 256),                             # 8192 pieces: five of a row
+])
+def test_where_the_cut_changes(lens, split, item):
+    text = _cut(lens)
+    assert "split threshold  : %d elements" % split in text and "(<= %d elements)" % item in text, text
