@@ -553,7 +553,15 @@ constexpr size_t kMaxBufferBytes = (size_t)8 << 30;     // all partitions' resul
 // by another address goes to memory at once.  Few features and many rows, because equal addresses share their feature.
 // 58,000 nodes, F=100, normal features, 12.5M / 0.6M edges: 331 / 300 us with every result added to memory directly,
 // 268 / 250 us with 16 features x 256 rows, 128 / 240 us with 4 x 8192 (2 x 8192: 152 / 246).
+//
+// Without the table (TABLE false: neighbouring lanes take neighbouring features of a row, and nothing is combined) where few
+// results can meet: rows of up to kSelFewEdges elements on average with operands
+// that are not broadcast, or UNIQUE, an operand on the edges without an offset array,
+// whose every feature is one row's and is added to without atomics; a broadcast operand of such rows keeps the table, by whole
+// rows.  Both gradients, with 4 x 8192 always -> now: 500,000 rows of 2, F=64 u_add_e 2116 -> 415 us, u_mul_e with 4 weights
+// per edge 2105 -> 548; maximum of the sources alone 1065 -> 224 (5 elements per row, with the table 274).
 constexpr int kSelWidth = 4, kSelRows = 8192, kSelLogSlots = 13, kSelSlots = 1 << kSelLogSlots, kSelThreads = 1024, kSelUnroll = 4;
+constexpr int kSelFewEdges = 4;
 enum { FG_SEL_PLUS, FG_SEL_MINUS, FG_SEL_TIMES_OTHER, FG_SEL_OVER_OTHER, FG_SEL_DENOMINATOR };
 struct SelectArgs {
     const int32_t *arg, *col;
@@ -566,17 +574,20 @@ struct SelectArgs {
     int F, kind;
     int width, rows;                        // features and rows per workgroup
 };
+template <bool TABLE, bool UNIQUE>
 __global__ __launch_bounds__(kSelThreads) void gspmm_select_backward_kernel(const SelectArgs a) {
-    __shared__ uint32_t s_key[kSelSlots];   // operand feature + 1; 0: free
-    __shared__ float s_sum[kSelSlots];
-    for (int i = threadIdx.x; i < kSelSlots; i += kSelThreads) { s_key[i] = 0; s_sum[i] = 0.f; }
-    __syncthreads();
+    __shared__ uint32_t s_key[TABLE ? kSelSlots : 1];   // operand feature + 1; 0: free
+    __shared__ float s_sum[TABLE ? kSelSlots : 1];
+    if constexpr (TABLE) {
+        for (int i = threadIdx.x; i < kSelSlots; i += kSelThreads) { s_key[i] = 0; s_sum[i] = 0.f; }
+        __syncthreads();
+    }
     const int f_tiles = (a.F + a.width - 1) / a.width;
     const int f = (int)(blockIdx.x % (unsigned)f_tiles) * a.width + (int)(threadIdx.x % (unsigned)a.width);
     const int64_t v0 = (int64_t)(blockIdx.x / (unsigned)f_tiles) * a.rows;
     const int64_t v1 = min(v0 + a.rows, a.n_dst);
     const int rows = kSelThreads / a.width;         // rows per step of the workgroup
-    const bool on = f < a.F;
+    const bool on = f < a.F && (int)(threadIdx.x / (unsigned)a.width) < rows;
     const int fo = on ? (a.own_off ? a.own_off[f] : f) : 0;
     const int fx = on ? (a.other_off ? a.other_off[f] : f) : 0;
     const bool reads_other = a.kind >= FG_SEL_TIMES_OTHER;
@@ -605,7 +616,8 @@ __global__ __launch_bounds__(kSelThreads) void gspmm_select_backward_kernel(cons
                 else if (a.kind == FG_SEL_OVER_OTHER) g = d[k] / x;
                 else { const float r = a.own[to]; g = -d[k] * x / (r * r); }
             }
-            if ((uint64_t)to >= 0xffffffffull) { unsafeAtomicAdd(a.grad + to, g); continue; }
+            if (UNIQUE) { a.grad[to] += g; continue; }
+            if (!TABLE || (uint64_t)to >= 0xffffffffull) { unsafeAtomicAdd(a.grad + to, g); continue; }
             const uint32_t key = (uint32_t)to + 1u;
             const uint32_t slot = (key * 2654435761u) >> (32 - kSelLogSlots);
             const uint32_t was = atomicCAS(&s_key[slot], 0u, key);
@@ -613,9 +625,11 @@ __global__ __launch_bounds__(kSelThreads) void gspmm_select_backward_kernel(cons
             else unsafeAtomicAdd(a.grad + to, g);
         }
     }
-    __syncthreads();
-    for (int i = threadIdx.x; i < kSelSlots; i += kSelThreads)
-        if (s_key[i]) unsafeAtomicAdd(a.grad + (s_key[i] - 1u), s_sum[i]);
+    if constexpr (TABLE) {
+        __syncthreads();
+        for (int i = threadIdx.x; i < kSelSlots; i += kSelThreads)
+            if (s_key[i]) unsafeAtomicAdd(a.grad + (s_key[i] - 1u), s_sum[i]);
+    }
 }
 
 // ---- SDDMM ------------------------------------------------------------------------------------------
@@ -928,12 +942,6 @@ extern "C" int fg_gspmm_select_backward_f32(const int32_t *arg_dev, const int32_
     if (!arg_dev || !col_dev || !dout_dev || (values && (!lhs_dev || !rhs_dev))) return fail(FG_ERR_ARG, "null device pointer");
     SelectArgs a;
     a.arg = arg_dev; a.col = col_dev; a.n_dst = n_dst; a.dout = dout_dev; a.F = out_len;
-    a.width = out_len >= kSelWidth ? kSelWidth : out_len == 1 ? 1 : 2;
-    // fewer rows per workgroup where the launch would leave compute units without one
-    a.rows = kSelRows;
-    int64_t blocks;
-    while ((blocks = ((n_dst + a.rows - 1) / a.rows) * ((out_len + a.width - 1) / a.width)) < 192 && a.rows > 512) a.rows /= 2;
-    if (blocks > 0x7fffffffLL) return fail(FG_ERR_SHAPE, "grid of %lld workgroups is too large", (long long)blocks);
     for (int side = 0; side < 2; ++side) {
         if (!(side ? drhs_dev : dlhs_dev)) continue;
         a.grad = side ? drhs_dev : dlhs_dev;
@@ -943,7 +951,21 @@ extern "C" int fg_gspmm_select_backward_f32(const int32_t *arg_dev, const int32_
         a.own_target = side ? rhs_target : lhs_target; a.other_target = side ? lhs_target : rhs_target;
         a.kind = op == FG_BIN_MUL ? FG_SEL_TIMES_OTHER : op == FG_BIN_DIV ? (side ? FG_SEL_DENOMINATOR : FG_SEL_OVER_OTHER)
                : (op == FG_BIN_SUB && side) ? FG_SEL_MINUS : FG_SEL_PLUS;
-        hipLaunchKernelGGL(gspmm_select_backward_kernel, dim3((unsigned)blocks), dim3(kSelThreads), 0, (hipStream_t)stream, a);
+        const bool unique = a.own_target == FG_TARGET_E && !a.own_off, few = n_edges <= kSelFewEdges * n_dst;
+        const bool table = !unique && (!few || a.own_off);
+        // few features where rows meet; else as many as make whole lines, in tiles of one size
+        a.width = !table || few ? (out_len + (out_len + 255) / 256 - 1) / ((out_len + 255) / 256)
+                : out_len >= kSelWidth ? kSelWidth : out_len == 1 ? 1 : 2;
+        // fewer rows per workgroup where the launch would leave compute units without one
+        a.rows = table && !few ? kSelRows : 2 * kSelUnroll * (kSelThreads / a.width);
+        int64_t blocks;
+        while ((blocks = ((n_dst + a.rows - 1) / a.rows) * ((out_len + a.width - 1) / a.width)) < 192 && a.rows > 512) a.rows /= 2;
+        if (blocks > 0x7fffffffLL) return fail(FG_ERR_SHAPE, "grid of %lld workgroups is too large", (long long)blocks);
+        const dim3 grid((unsigned)blocks), threads(kSelThreads);
+        hipStream_t st = (hipStream_t)stream;
+        if (unique) hipLaunchKernelGGL((gspmm_select_backward_kernel<false, true>), grid, threads, 0, st, a);
+        else if (table) hipLaunchKernelGGL((gspmm_select_backward_kernel<true, false>), grid, threads, 0, st, a);
+        else hipLaunchKernelGGL((gspmm_select_backward_kernel<false, false>), grid, threads, 0, st, a);
     }
     FG_HIP_TRY(hipGetLastError());
     return FG_OK;
