@@ -653,7 +653,7 @@ struct EdgeArgs {
 //          F; a lane finds its edge by one high multiplication (64 * (F / V)^2 < 2^32).
 //   else : a group of L lanes (the power of two not below F / V, at most 64) takes an edge.
 // u_mul_v on 12.5 M edges, F = 64, within a step of 3 such sweeps: 951 -> 741 us (3.2 GB written, 4.3 TB/s).
-template <int OP, int V, bool LC, bool RC, bool FLAT>
+template <int OP, int V, bool LC, bool RC, bool FLAT, int U>
 __global__ __launch_bounds__(kBlock) void gsddmm_bcast_kernel(const EdgeArgs a) {
     const int lane = threadIdx.x & 63;
     const int64_t wave_id = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -664,7 +664,6 @@ __global__ __launch_bounds__(kBlock) void gsddmm_bcast_kernel(const EdgeArgs a) 
     const int n = (int)min((int64_t)64, a.n_edges - e0);
     const bool l_on_e = a.lhs_target == FG_TARGET_E, r_on_e = a.rhs_target == FG_TARGET_E;
     const int il_all = kUsesLhs<OP> ? a.lhs_index[e0 + min(lane, n - 1)] : 0, ir_all = kUsesRhs<OP> ? a.rhs_index[e0 + min(lane, n - 1)] : 0;
-    constexpr int U = V == 4 ? 8 : 4;
     // U edges t[] (valid where ok[]) at the lane's output features fc[], operand features fl[] and fr[]
     auto step = [&](const int (&t)[U], const bool (&ok)[U], const int (&fc)[U], const int (&fl)[U], const int (&fr)[U]) {
         float m[U][V];
@@ -780,12 +779,20 @@ void launch_sddmm(int vec, dim3 grid, hipStream_t st, EdgeArgs a) {
     const int FV = vec ? a.F / 4 : a.F;
     a.vec_magic = FV > 1 ? (uint32_t)((0x100000000ull + FV - 1) / FV) : 0;
     const bool flat = !(kUsesLhs<OP> && a.lhs_off) && !(kUsesRhs<OP> && a.rhs_off) && FV < 8192;
-    if (vec == 1 && flat) hipLaunchKernelGGL((gsddmm_bcast_kernel<OP, 4, true, true, true>), grid, dim3(kBlock), 0, st, a);
-    else if (vec == 1) hipLaunchKernelGGL((gsddmm_bcast_kernel<OP, 4, true, true, false>), grid, dim3(kBlock), 0, st, a);
-    else if (vec == 2) hipLaunchKernelGGL((gsddmm_bcast_kernel<OP, 4, true, false, false>), grid, dim3(kBlock), 0, st, a);
-    else if (vec == 3) hipLaunchKernelGGL((gsddmm_bcast_kernel<OP, 4, false, true, false>), grid, dim3(kBlock), 0, st, a);
-    else if (flat) hipLaunchKernelGGL((gsddmm_bcast_kernel<OP, 1, true, true, true>), grid, dim3(kBlock), 0, st, a);
-    else hipLaunchKernelGGL((gsddmm_bcast_kernel<OP, 1, true, true, false>), grid, dim3(kBlock), 0, st, a);
+    // a wavefront's 64 edges fill eight steps; 3 M edges, u_add_v with eight / four: F=4 35 / 25 us, F=8 38 / 29, F=16 49 / 43
+    const bool wide = FV > 4;
+#define FG_GO(V, LC, RC, FLAT) \
+    do { \
+        if (wide) hipLaunchKernelGGL((gsddmm_bcast_kernel<OP, V, LC, RC, FLAT, 8>), grid, dim3(kBlock), 0, st, a); \
+        else hipLaunchKernelGGL((gsddmm_bcast_kernel<OP, V, LC, RC, FLAT, 4>), grid, dim3(kBlock), 0, st, a); \
+    } while (0)
+    if (vec == 1 && flat) FG_GO(4, true, true, true);
+    else if (vec == 1) FG_GO(4, true, true, false);
+    else if (vec == 2) FG_GO(4, true, false, false);
+    else if (vec == 3) FG_GO(4, false, true, false);
+    else if (flat) FG_GO(1, true, true, true);
+    else hipLaunchKernelGGL((gsddmm_bcast_kernel<OP, 1, true, true, false, 4>), grid, dim3(kBlock), 0, st, a);
+#undef FG_GO
 }
 
 }  // namespace
@@ -1020,7 +1027,7 @@ extern "C" int fg_gsddmm_bcast_f32(const int32_t *row_dev, const int32_t *col_de
         case FG_BIN_COPY_RHS: launch_sddmm<FG_BIN_COPY_RHS>(vec, grid, st, a); break;
         default: {
             const bool wide = R % 4 == 0 && lhs_len % 4 == 0 && rhs_len % 4 == 0 && (((uintptr_t)lhs_dev | (uintptr_t)rhs_dev) & 15) == 0;
-            if (!wide) hipLaunchKernelGGL((gsddmm_bcast_kernel<FG_BIN_DOT, 1, true, true, false>), grid, dim3(kBlock), 0, st, a);
+            if (!wide) hipLaunchKernelGGL((gsddmm_bcast_kernel<FG_BIN_DOT, 1, true, true, false, 4>), grid, dim3(kBlock), 0, st, a);
             else if (R <= 16) hipLaunchKernelGGL(gsddmm_dot_kernel<4>, grid, dim3(kBlock), 0, st, a);
             else if (R <= 32) hipLaunchKernelGGL(gsddmm_dot_kernel<8>, grid, dim3(kBlock), 0, st, a);
             else if (R <= 64) hipLaunchKernelGGL(gsddmm_dot_kernel<16>, grid, dim3(kBlock), 0, st, a);
