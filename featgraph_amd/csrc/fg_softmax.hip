@@ -8,16 +8,18 @@
 // counts is that every value is read once and that enough 128-bit loads are in flight.  The work is cut by the plan's
 // items (one wavefront per run of short rows, per row, or per piece of a long row) and by its list of split rows:
 //   a run of short rows   staged in LDS, several lanes per (row, head);
-//   a row that fits the registers of one wavefront (16 KB of scores; 8 KB each of a and g)   finished there;
-//   a row that fits those of a workgroup (64 KB; 32 KB each)   finished by four wavefronts, split or not;
+//   a row that fits the registers of one wavefront (Chunks::capacity; 4 heads: 8 KB of scores, 4 KB each of a and g)   finished there;
+//   a row that fits those of a workgroup (four times that)   finished by four wavefronts, split or not; up to group_floats() in two
+//                         sweeps by them;
 //   a longer row          by its pieces: (max, sum) per head, a small kernel that merges them, a second sweep.
-// That is for 1, 2, 3, 4, 6, 8, 16, 32 and 64 heads (edge_softmax_rows_kernel); any other number goes through 32-bit loads, with
+// That is for the head counts that are measured to gain by it, 1, 2, 3, 4, 6, 8, 16, 32 and 64 (edge_softmax_rows_kernel); any other number goes through 32-bit loads, with
 // every split row in two sweeps (edge_softmax_kernel).
 // Forward + backward on 232,965 nodes / 114.8 M edges against that general form: 4 heads 2529 -> 2067 us (9.2 GB that
 // have to move, 4.45 TB/s; a copy of arrays this large reaches 4.8, a sum of two 5.9), 1 head 788 -> 611 us, 8 heads
 // 5025 -> 4330 us; 30,000 edges, 4 heads 45 -> 19 us (one launch each way instead of three).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 
 #include "fg_common.h"
@@ -33,7 +35,14 @@ namespace {
 constexpr int kWavesPerBlock = 4;
 constexpr int kBlock = 64 * kWavesPerBlock;
 constexpr int kStage = 1024;          // floats of a multi-row item staged in LDS per wavefront
-constexpr int kGroupFloats = 1 << 17; // longest row that one workgroup takes: about 70 us of it; longer ones are spread by their pieces
+// Longest row that one workgroup takes: 2^15 floats, about 13 us of it, up to 2^17 where all rows together hold 128 times as much
+// (there are 256 compute units); longer ones are spread by their pieces.  us forward + backward with 2^15 / 2^16 / 2^17: one row of
+// 64,000 floats among short ones 24 / 45 / 46, of 128,000 26 / 26 / 84; 500 rows of 40,000 111 / 95 / 95, 128 of 48,000 52 / 44 / 44.
+constexpr int64_t kGroupFloats = 1 << 15, kGroupFloatsMost = 1 << 17;
+// (A caller's own longer pieces are not worth spreading a row for: 2^17.)
+int group_floats(const fg_spmm_plan *pl, int H) {
+    return (int)(pl->split_threshold > 1024 ? kGroupFloatsMost : std::min(std::max(kGroupFloats, pl->nnz * H / 128), kGroupFloatsMost));
+}
 
 struct SoftmaxArgs {
     const Item *items;
@@ -45,6 +54,7 @@ struct SoftmaxArgs {
     const float *g;       // backward: dL/da
     float *y;
     float2 *stats;        // per (piece, head): forward (max, sum of exp); backward (sum of a * g, 0)
+    int group_floats;     // rows of more floats are left to their pieces
     int H;
     int W;                // lanes of a wavefront in use when lanes are tied to heads: the largest multiple of H <= 64
 };
@@ -478,7 +488,6 @@ __device__ __forceinline__ void wave_row(const SoftmaxArgs &a, int64_t e0, int l
     if (n <= 64 * CH) { chunk_row<BWD, Q, A, PER, 64, 1>(x, g, y, n, G, nullptr); return; }
     if constexpr (RM > 2) { if (n <= 64 * CH * 2) { chunk_row<BWD, Q, A, PER, 64, 2>(x, g, y, n, G, nullptr); return; } }
     if constexpr (RM > 4) { if (n <= 64 * CH * 4) { chunk_row<BWD, Q, A, PER, 64, 4>(x, g, y, n, G, nullptr); return; } }
-    if constexpr (RM > 8) { if (n <= 64 * CH * 8) { chunk_row<BWD, Q, A, PER, 64, 8>(x, g, y, n, G, nullptr); return; } }
     if (n <= 64 * CH * RM) { chunk_row<BWD, Q, A, PER, 64, RM>(x, g, y, n, G, nullptr); return; }
     float m[A], s[A];
     sweep_stats<BWD, Q, A, PER, 64>(x, g, n, G, nullptr, m, s);
@@ -634,7 +643,7 @@ __device__ __forceinline__ void rows_body(const SoftmaxArgs &a) {
         const int row = a.fixups[blockIdx.x].row;
         const int b = a.indptr[row], len = a.indptr[row + 1] - b;
         const int64_t n = (int64_t)len * H;
-        if (n > kGroupFloats) return;
+        if (n > a.group_floats) return;
         if (n <= wave_cap) { if (wave == 0) wave_row<BWD, Q, A, PER>(a, b, len, lane, G); }
         else group_row<BWD, Q, A, PER>(a, b, len, G, red);
         return;
@@ -647,7 +656,7 @@ __device__ __forceinline__ void rows_body(const SoftmaxArgs &a) {
         if (it.len == 0 || shared_row(it)) {
         } else if (it.info >= 0) {
             const int len = a.indptr[it.row + 1] - a.indptr[it.row];
-            if ((int64_t)len * H > kGroupFloats) piece<BWD, Q, A, PER, true>(a, it, lane, G);
+            if ((int64_t)len * H > a.group_floats) piece<BWD, Q, A, PER, true>(a, it, lane, G);
         } else if (it.info == -1) {
             wave_row<BWD, Q, A, PER>(a, it.start, it.len, lane, G);
         } else {
@@ -675,7 +684,7 @@ __global__ __launch_bounds__(kBlock) void edge_softmax_pieces_kernel(const Softm
     if (item_id >= a.n_items) return;         // uniform per wavefront; no workgroup barriers below
     const Item it = a.items[item_id];
     if (it.info < 0) return;
-    if ((int64_t)(a.indptr[it.row + 1] - a.indptr[it.row]) * a.H > kGroupFloats) piece<BWD, Q, A, PER, false>(a, it, lane, PER ? a.H / 4 : 1);
+    if ((int64_t)(a.indptr[it.row + 1] - a.indptr[it.row]) * a.H > a.group_floats) piece<BWD, Q, A, PER, false>(a, it, lane, PER ? a.H / 4 : 1);
 }
 
 // PIECES == false: rows held whole by an item are finished, pieces write their statistics.
@@ -804,27 +813,39 @@ __global__ __launch_bounds__(kBlock) void edge_softmax_backward_kernel(const Sof
     edge_softmax_body<true, LANEHEAD, PIECES>(a);
 }
 
-// Merges the pieces' statistics of every split row, in piece order, and writes the row's
-// statistics back to each of its pieces.  One lane per (split row, head).
+// Merges the pieces' statistics of every split row of more than `above` floats and writes the row's statistics back to each of
+// its pieces.  kMergeLanes lanes per (split row, head): a row of 24,000 elements is 190 pieces on a small graph, which one lane
+// takes longer over than the two sweeps around this launch (4 heads, whole call: 32 us, 20 with pieces of 1024).
+constexpr int kMergeLanes = 16;
+template <bool IS_MAX>
+__device__ __forceinline__ float merge_lanes(float v) {
+    for (int off = 1; off < kMergeLanes; off <<= 1) { const float o = __shfl_xor(v, off); v = IS_MAX ? fmaxf(v, o) : v + o; }
+    return v;
+}
 template <bool BWD>
-__global__ __launch_bounds__(256) void edge_softmax_merge_kernel(const Fixup *fixups, int64_t n_fixups,
-                                                                 float2 *stats, int H) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ float2 merged_stats(const float2 *s, int n, int H, int lane) {
+    auto load = [&](int q) { return s[(int64_t)(lane + q * kMergeLanes) * H]; };
+    const int mine = lane < n ? (n - lane + kMergeLanes - 1) / kMergeLanes : 0;
+    float m = BWD ? 0.f : -INFINITY, sum = 0.f;
+    fg::each_piece(0, mine, load, [&](int, const float2 &c) { m = BWD ? m + c.x : fmaxf(m, c.x); });
+    m = merge_lanes<!BWD>(m);
+    if (!BWD) {
+        fg::each_piece(0, mine, load, [&](int, const float2 &c) { sum += c.y * __expf(c.x - m); });
+        sum = merge_lanes<false>(sum);
+    }
+    return make_float2(m, sum);
+}
+template <bool BWD>
+__global__ __launch_bounds__(256) void edge_softmax_merge_kernel(const Fixup *fixups, int64_t n_fixups, const int32_t *indptr,
+                                                                 int above, float2 *stats, int H) {
+    const int64_t t = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kMergeLanes;
     if (t >= n_fixups * H) return;
     const Fixup fx = fixups[t / H];
-    const int h = (int)(t % H);
-    float2 *s = stats + (int64_t)fx.slot0 * H + h;
-    float m, sum = 0.f;
-    auto load = [&](int p) { return s[(int64_t)p * H]; };
-    if (!BWD) {
-        m = s[0].x;
-        fg::each_piece(1, fx.n_pieces, load, [&](int, const float2 &c) { m = fmaxf(m, c.x); });
-        fg::each_piece(0, fx.n_pieces, load, [&](int, const float2 &c) { sum += c.y * __expf(c.x - m); });
-    } else {
-        m = 0.f;
-        fg::each_piece(0, fx.n_pieces, load, [&](int, const float2 &c) { m += c.x; });
-    }
-    for (int p = 0; p < fx.n_pieces; ++p) s[(int64_t)p * H] = make_float2(m, sum);
+    if ((int64_t)(indptr[fx.row + 1] - indptr[fx.row]) * H <= above) return;
+    const int lane = threadIdx.x % kMergeLanes;
+    float2 *s = stats + (int64_t)fx.slot0 * H + (int)(t % H);
+    const float2 row = merged_stats<BWD>(s, fx.n_pieces, H, lane);
+    for (int p = lane; p < fx.n_pieces; p += kMergeLanes) s[(int64_t)p * H] = row;
 }
 
 // ---- statistics only, and the fused normalise-and-relayout step ------------------------------------
@@ -859,16 +880,12 @@ __global__ __launch_bounds__(kBlock) void edge_softmax_stats_kernel(const Softma
 // Merges the pieces of every split row and writes the row's entry of row_stats.
 __global__ __launch_bounds__(256) void edge_softmax_stats_merge_kernel(const Fixup *fixups, int64_t n_fixups,
                                                                        const float2 *stats, float2 *row_stats, int H) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t t = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kMergeLanes;
     if (t >= n_fixups * H) return;
     const Fixup fx = fixups[t / H];
-    const int h = (int)(t % H);
-    const float2 *s = stats + (int64_t)fx.slot0 * H + h;
-    float m = s[0].x, sum = 0.f;
-    auto load = [&](int p) { return s[(int64_t)p * H]; };
-    fg::each_piece(1, fx.n_pieces, load, [&](int, const float2 &c) { m = fmaxf(m, c.x); });
-    fg::each_piece(0, fx.n_pieces, load, [&](int, const float2 &c) { sum += c.y * __expf(c.x - m); });
-    row_stats[(int64_t)fx.row * H + h] = make_float2(m, sum);
+    const int h = (int)(t % H), lane = threadIdx.x % kMergeLanes;
+    const float2 row = merged_stats<false>(stats + (int64_t)fx.slot0 * H + h, fx.n_pieces, H, lane);
+    if (lane == 0) row_stats[(int64_t)fx.row * H + h] = row;
 }
 
 // dst[h, e'] = exp(x[pos[e'], h] - max) / sum with the statistics of the row of stored element pos[e'].
@@ -921,15 +938,20 @@ __global__ __launch_bounds__(256) void edge_softmax_head_major_vec_kernel(const 
     }
 }
 
+template <bool BWD>
+void launch_merge(const fg_spmm_plan *pl, const SoftmaxArgs &a, int above, hipStream_t st) {
+    const int64_t threads = pl->n_fixups * a.H * kMergeLanes;
+    hipLaunchKernelGGL(edge_softmax_merge_kernel<BWD>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st,
+                       pl->fixups_dev, pl->n_fixups, a.indptr, above, a.stats, a.H);
+}
+
 template <bool BWD, int LANEHEAD>
 void launch_both(const fg_spmm_plan *pl, const SoftmaxArgs &a, hipStream_t st) {
     const dim3 grid((unsigned)((pl->n_items + kWavesPerBlock - 1) / kWavesPerBlock));
     if (BWD) hipLaunchKernelGGL((edge_softmax_backward_kernel<LANEHEAD, false>), grid, dim3(kBlock), 0, st, a);
     else hipLaunchKernelGGL((edge_softmax_kernel<LANEHEAD, false>), grid, dim3(kBlock), 0, st, a);
     if (pl->n_fixups > 0) {
-        const int64_t threads = pl->n_fixups * a.H;
-        hipLaunchKernelGGL(edge_softmax_merge_kernel<BWD>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st,
-                           pl->fixups_dev, pl->n_fixups, a.stats, a.H);
+        launch_merge<BWD>(pl, a, 0, st);
         if (BWD) hipLaunchKernelGGL((edge_softmax_backward_kernel<LANEHEAD, true>), grid, dim3(kBlock), 0, st, a);
         else hipLaunchKernelGGL((edge_softmax_kernel<LANEHEAD, true>), grid, dim3(kBlock), 0, st, a);
     }
@@ -941,10 +963,8 @@ void launch_rows(const fg_spmm_plan *pl, const SoftmaxArgs &a, hipStream_t st) {
     const dim3 grid((unsigned)(item_blocks + pl->n_fixups));
     if (BWD) hipLaunchKernelGGL((edge_softmax_rows_backward_kernel<Q, A, PER>), grid, dim3(kBlock), 0, st, a);
     else hipLaunchKernelGGL((edge_softmax_rows_kernel<Q, A, PER>), grid, dim3(kBlock), 0, st, a);
-    if (pl->n_fixups == 0 || pl->max_len * a.H <= kGroupFloats) return;
-    const int64_t threads = pl->n_fixups * a.H;
-    hipLaunchKernelGGL(edge_softmax_merge_kernel<BWD>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st,
-                       pl->fixups_dev, pl->n_fixups, a.stats, a.H);
+    if (pl->n_fixups == 0 || pl->max_len * a.H <= a.group_floats) return;
+    launch_merge<BWD>(pl, a, a.group_floats, st);
     hipLaunchKernelGGL((edge_softmax_pieces_kernel<BWD, Q, A, PER>), dim3((unsigned)item_blocks), dim3(kBlock), 0, st, a);
 }
 
@@ -985,6 +1005,7 @@ int softmax_run(fg_spmm_plan *pl, const int32_t *indptr, const float *x, const f
     a.items = pl->items_dev; a.n_items = pl->n_items; a.indptr = indptr;
     a.fixups = pl->fixups_dev; a.n_fixups = pl->n_fixups;
     a.x = x; a.g = g; a.y = y; a.stats = reinterpret_cast<float2 *>(pl->partial_dev); a.H = H;
+    a.group_floats = group_floats(pl, H);
     hipStream_t st = (hipStream_t)stream;
     const int mode = lane_mode(H);
     a.W = H <= 64 ? 64 / H * H : 64;
@@ -1037,7 +1058,7 @@ extern "C" int fg_edge_softmax_stats_f32(fg_spmm_plan *pl, const int32_t *indptr
     else if (mode == 2) hipLaunchKernelGGL(edge_softmax_stats_kernel<2>, grid, dim3(kBlock), 0, st, a, row_stats);
     else hipLaunchKernelGGL(edge_softmax_stats_kernel<0>, grid, dim3(kBlock), 0, st, a, row_stats);
     if (pl->n_fixups > 0) {
-        const int64_t threads = pl->n_fixups * heads;
+        const int64_t threads = pl->n_fixups * heads * kMergeLanes;
         hipLaunchKernelGGL(edge_softmax_stats_merge_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st,
                            pl->fixups_dev, pl->n_fixups, a.stats, row_stats, heads);
     }

@@ -144,3 +144,31 @@ def test_a_piece_of_masked_scores_leaves_its_row_finite(H):
         ref = torch.softmax(x[b:e].double(), 0)
         # as in test_every_row_length_class, with differences of at most 10 between finite scores of a row
         assert bool(((got[b:e] - ref).abs() <= ref * EPS * (16 + 4 * 10)).all()), (b, e)
+
+
+@pytest.mark.parametrize("many", [False, True])
+@pytest.mark.parametrize("H", [1, 3, 4, 16])
+def test_longest_row_of_a_workgroup(H, many):
+    """Rows around the most floats that one workgroup takes: 2^15, or a 128th of all there are (many: 160 rows of 40,000 and
+    more, which workgroups take there and pieces take on the small graph); the merge of many pieces' statistics."""
+    import torch
+    from featgraph_amd.module import EdgeSoftmaxhip, placeholder
+    at = (1 << 15) // H
+    lens = np.array([at - 1, 7, at, at + 1, 3, 40_000 // H, 60_000 // H] + [40_000 // H] * (160 if many else 0) + [140_000 // H])
+    indptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    nnz = int(indptr[-1])
+    indices = np.concatenate([np.arange(n) for n in lens]).astype(np.int32)
+    m = EdgeSoftmaxhip(sp.csr_matrix((np.ones(nnz, np.float32), indices, indptr), shape=(len(lens), max(lens))))
+    m.build([placeholder((nnz, H))])
+    gen = torch.Generator(device="cuda").manual_seed(H)
+    x, g = torch.randn(nnz, H, generator=gen, device="cuda"), torch.randn(nnz, H, generator=gen, device="cuda")
+    a = m.run([x]).clone()
+    dx = m.backward(a, g)
+    for b, e in zip(indptr[:8].tolist() + [int(indptr[-2])], indptr[1:9].tolist() + [nnz]):
+        ref = torch.softmax(x[b:e].double(), 0)
+        # the exponent's rounding (differences of at most 10) and up to 128 terms per lane, added up with few roundings to one side
+        assert bool(((a[b:e].double() - ref).abs() <= ref * EPS * (64 + 4 * 10)).all()), (b, e)
+        ag = a[b:e].double() * g[b:e].double()
+        ref = ag - a[b:e].double() * ag.sum(0)
+        mass = ag.abs() + a[b:e].double() * ag.abs().sum(0)
+        assert bool(((dx[b:e].double() - ref).abs() <= 64 * EPS * mass).all()), (b, e)
