@@ -558,10 +558,11 @@ int attention_scratch_need(const fg_spmm_plan *pl, int heads, int head_len, bool
         need->partial = ((need->partial + 3) & ~(size_t)3) +
                         (size_t)pl->num_col_partitions * ((size_t)pl->n_dst * F + (size_t)pl->n_dst * heads * 2);
     need->tiled = 0;
-    // A copy costs its 8 bytes per float whatever the graph, and pays per gathered row: from 24 elements per source on.
-    // Whole steps with gradients, 200,000 nodes, with -> without, 8 x 64 dot / 8 x 32 additive: degree 5 4227 -> 3593 /
-    // 1200 -> 1114 us, degree 16 8215 -> 7882 / 2169 -> 2107, degree 32 13586 -> 13803 / 3460 -> 3611.
-    const bool pays = pl->tile_major == 1 || pl->nnz >= 24 * pl->n_src;
+    // A copy costs its 8 bytes per float whatever the graph, and pays per gathered row, the more the shorter the rows it
+    // packs: from 12 / 20 / 24 elements per source on with heads of 16 / 32 / 64 floats.  Whole steps with gradients, 200,000
+    // nodes, with -> without: 8 x 16 dot degree 10 2236 -> 2244 us, 16 3045 -> 3269, 23 4066 -> 4553; 8 x 32 dot 10 2752 -> 2635,
+    // 16 3659 -> 3717, 23 4780 -> 5001 (additive 16 2135 -> 2060, 23 2656 -> 2713); 8 x 64 dot 16 8215 -> 7882, 32 13586 -> 13803.
+    const bool pays = pl->tile_major == 1 || pl->nnz >= (head_len == 16 ? 12 : head_len == 32 ? 20 : 24) * pl->n_src;
     if (pays && pl->nnz > 0 && wants_tile_major(pl, heads, (uint64_t)pl->n_src * F * 4u))
         need->tiled = (size_t)pl->n_src * F * (additive ? 1 : 2);
     return FG_OK;

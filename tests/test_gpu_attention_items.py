@@ -40,13 +40,13 @@ def test_attention_matches_float64(kind, heads, head_len, repeat):
         assert float((x.detach().double() - y.detach()).norm() / y.detach().norm()) <= 1e-5
 
 
-@pytest.mark.parametrize("degree", [1, 23, 24])
-def test_head_by_head_copy_changes_no_bit(monkeypatch, degree):
-    """On both sides of the line from which the gathered operands are copied (24 elements per source, 64 MB)."""
+@pytest.mark.parametrize("head_len,degree", [(64, 1), (64, 23), (64, 24), (32, 19), (32, 20), (16, 11), (16, 12)])
+def test_head_by_head_copy_changes_no_bit(monkeypatch, head_len, degree):
+    """On both sides of the line from which the gathered operands are copied (24, 20 or 12 elements per source, 64 MB)."""
     import torch
     from featgraph_amd import _lib
     from featgraph_amd.autograd import Graph
-    n, heads, head_len = 33000, 8, 64
+    n, heads = 33000, 512 // head_len
     cols = np.sort((np.arange(n)[:, None] * 7 + np.arange(degree)[None, :] * 613) % n, axis=1)
     adj = sp.csr_matrix((np.ones(n * degree, np.float32), cols.ravel().astype(np.int32),
                          (np.arange(n + 1) * degree).astype(np.int32)), shape=(n, n))
