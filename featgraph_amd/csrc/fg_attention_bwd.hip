@@ -282,7 +282,10 @@ __global__ __launch_bounds__(kBlock) void attention_backward_kernel(const BwdArg
             // LDS), walks the row's elements KU at a time and stores the row itself: G rows in flight per wavefront,
             // nothing crosses lane groups.  Whole step, against every row shared by the wavefront: 200,000 nodes of degree
             // 7.5 on average, 4 x 32 additive 790 -> 710 us, 50,000 of degree 12, 2 x 32 dot 164 -> 151; where the gathers
-            // come from HBM (200,000 nodes, 8 x 64 dot) no difference.
+            // come from HBM (200,000 nodes, 8 x 64 dot) no difference to 2 % more.  The mean alone decides: an item with one long row
+            // occupies one lane group beyond the rest, yet sharing such items costs more over a launch.  200,000 nodes, 4 x 32
+            // additive, one row of 190 in 60 (of 40 in 20) and the rest of 1 or 2: every row shared 560 (552) us, items with a row
+            // above 32 shared 411 (497), none 411 (431); degrees by a power law of exponent 2.1: 643, 566, 525.
             int r = 0, j = 0, e = 0;
             bool live = false;
             float4 accA = zero4(), accB = zero4();
