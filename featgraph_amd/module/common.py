@@ -46,10 +46,15 @@ def to_device_f32(a, dev):
     return torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32)).to(dev)
 
 
+# The current stream's handle without the Stream object that torch.cuda.current_stream() makes first, where torch has the
+# function that its own compiled code uses; what it saves is host time, within the spread of host-bound steps.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_ptr():
-    # (the Stream object that torch.cuda.current_stream() makes first costs 6 us a call, of which a step has ten and more:
-    # an attention layer of single operators with gradients on 10,500 edges, bound by host work, 370 -> 305 us)
-    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+    if _raw_stream is None:
+        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(_raw_stream(torch.cuda.current_device()))
 
 
 def check_inputs(tensors, placeholders, dev):
