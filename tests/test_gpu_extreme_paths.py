@@ -173,3 +173,68 @@ def test_masked_messages_cost_no_second_walk(feat_len):
             torch.cuda.synchronize()
             best[name] = min(best.get(name, 1e9), a.elapsed_time(b))
     assert best["masked"] < 1.6 * best["plain"], best
+
+
+@pytest.mark.parametrize("what", ["aggregate", "gspmm"])
+def test_fixed_order_on_request(monkeypatch, what):
+    """Under use_deterministic_algorithms the gradient comes from torch's operators: the same bits twice, close to float64, and
+    without the kernel that adds by atomics."""
+    import torch
+    from featgraph_amd.autograd import Graph
+    from featgraph_amd.module.general import BroadcastOp
+    rng = np.random.default_rng(11)
+    adj = _graph(rng, LENS)
+    g = Graph(adj)
+    t = lambda *s: torch.from_numpy(rng.standard_normal(s).astype(np.float32)).cuda().requires_grad_()
+    x, e, d = t(700, 36), t(adj.nnz, 36), t(adj.shape[0], 36).detach()
+    operands = [x] if what == "aggregate" else [x, e]
+    step = lambda: torch.autograd.grad(g.aggregate(x, "max") if what == "aggregate" else g.gspmm("u_mul_e", x, e, "max"), operands, d)
+    free = step()
+
+    def never(*args, **kwargs):
+        raise AssertionError("the kernel with atomics was called")
+    monkeypatch.setattr(BroadcastOp, "select_backward", never)
+    before = torch.are_deterministic_algorithms_enabled()
+    torch.use_deterministic_algorithms(True)
+    try:
+        first, second = step(), step()
+    finally:
+        torch.use_deterministic_algorithms(before)
+    assert all(torch.equal(a, b) for a, b in zip(first, second))
+    # float64 by the selected elements: a row's messages, the first largest
+    x64, e64 = x.detach().cpu().double().numpy(), e.detach().cpu().double().numpy()
+    ref = [np.zeros_like(x64), np.zeros_like(e64)]
+    for v in np.flatnonzero(np.diff(adj.indptr)):
+        a, b = adj.indptr[v], adj.indptr[v + 1]
+        u = adj.indices[a:b]
+        m = x64[u] if what == "aggregate" else (x.detach().cpu().numpy()[u] * e.detach().cpu().numpy()[a:b])
+        at, f, dv = m.argmax(0), np.arange(36), d[v].cpu().double().numpy()
+        np.add.at(ref[0], (u[at], f), dv if what == "aggregate" else dv * e64[a + at, f])
+        ref[1][a + at, f] += dv * x64[u[at], f]
+    for got in (first, free):
+        for i, r in enumerate(got):
+            # sums of up to about 100 fp32 products
+            assert np.linalg.norm(r.cpu().double().numpy() - ref[i]) <= 1e-6 * np.linalg.norm(ref[i])
+
+
+@pytest.mark.parametrize("feat_len", [1, 3, 36, 257])
+@pytest.mark.parametrize("degree", [1, 4, 5])
+def test_gradients_of_rows_of_a_few_elements(feat_len, degree):
+    """Both sides of the line from which results that meet are combined first, with operands that broadcast and that do not."""
+    import torch
+    from featgraph_amd.autograd import Graph
+    n, rng = 700, np.random.default_rng(degree)
+    adj = _graph(rng, [degree] * n)
+    g = Graph(adj)
+    t = lambda *s: torch.from_numpy(rng.standard_normal(s).astype(np.float32)).cuda().requires_grad_()
+    x, d = t(n, 2, feat_len), t(n, 2, feat_len).detach()
+    for e in (t(adj.nnz, 2, feat_len), t(adj.nnz, 2, 1)):
+        for msg in ("u_mul_e", "u_sub_e"):
+            got = torch.autograd.grad(g.gspmm(msg, x, e, "max"), [x, e], d)
+            xs, es = x.detach().double().requires_grad_(), e.detach().double().requires_grad_()
+            gathered = xs[torch.from_numpy(adj.indices).cuda().long()]
+            m = gathered * es if msg == "u_mul_e" else gathered - es
+            ref = torch.autograd.grad(m.view(n, degree, 2, feat_len).amax(1), [xs, es], d.double())
+            for a, b in zip(got, ref):
+                # sums of at most a few hundred fp32 products
+                assert float((a.double() - b).norm()) <= 1e-5 * float(b.norm())
