@@ -855,8 +855,8 @@ int gspmm_bcast_run(fg_spmm_plan *pl, const int32_t *pos_dev, const int32_t *idx
     a.partial = values; a.partial_arg = positions;
     // Feature tiles of 64 floats over the workgroups (as for the weighted sum) when an operand is gathered from the
     // source nodes and the 128-bit paths apply: a partition's slice of a tile is what an L2 has to hold.
-    // (Not with the positions of the selected elements, whose kernels hold too many registers to gain from it --
-    // F=256: 17.1 ms tiled against 14.7 ms -- nor with an operand streamed from the edges, which sets the time.)
+    // (Not with the positions of the selected elements, whose kernels held too many registers to gain from it
+    // when each message went by the full rule, F=256 17.1 ms tiled against 14.7 ms, not measured since -- nor with an operand streamed from the edges, which sets the time.)
     const bool gathers = (uses_l && lhs_target == FG_TARGET_U) || (uses_r && rhs_target == FG_TARGET_U);
     const bool streams = (uses_l && lhs_target == FG_TARGET_E && lmode == 1) || (uses_r && rhs_target == FG_TARGET_E && rmode == 1);
     const int T = (V == 4 && gathers && !streams && !arg_dev && out_len >= 128 && out_len % 64 == 0) ? out_len / 64 : 1;
