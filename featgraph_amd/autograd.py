@@ -173,8 +173,8 @@ class Graph(object):
     def gat_attention(self, er, el, v, negative_slope=0.2):
         """The attention of a GAT layer: out[r, h, :] = sum over the edges e into r of
         softmax_r(leaky_relu(el[col e, h] + er[r, h])) * v[col e, h, :]; er (num_rows, H), el (num_cols, H),
-        v (num_cols, H, D) with D in {16, 32, 64}.  One operator forward, two sweeps backward; no per-edge
-        array is stored."""
+        v (num_cols, H, D) with D in {16, 32, 64}.  One operator forward, one sweep backward; no per-edge
+        array is stored (with gradients the forward pass keeps a second array of the output's size)."""
         return _GatAttention.apply(self, er, el, v, float(negative_slope))
 
     def _gat_mod(self, er, el, v, slope):
@@ -302,13 +302,19 @@ def _fresh_run(mod, inputs):
     """run() into a tensor of the caller's own: the module's output buffer (every element of which a run
     overwrites) is replaced first, so nothing has to be copied out of it, and the module lets go of it
     afterwards -- autograd takes a gradient it alone refers to as it is, and clones one that is shared."""
-    like = getattr(mod, '_fresh_like', None)
-    if like is None:
-        like = mod._fresh_like = (tuple(mod.out_tvm.shape), mod.out_tvm.dtype, mod.out_tvm.device)
+    like = _let_go(mod)
     mod.out_tvm = torch.empty(like[0], dtype=like[1], device=like[2])
     out = mod.run(inputs)
     mod.out_tvm = None
     return out
+
+
+def _let_go(mod):
+    """Drops the module's output buffer, for callers that bring their own; (shape, dtype, device) of it."""
+    if getattr(mod, '_fresh_like', None) is None:
+        mod._fresh_like = (tuple(mod.out_tvm.shape), mod.out_tvm.dtype, mod.out_tvm.device)
+    mod.out_tvm = None
+    return mod._fresh_like
 
 
 class _SpMM(torch.autograd.Function):
@@ -366,16 +372,18 @@ class _GatAttention(torch.autograd.Function):
     def forward(ctx, g, er, el, v, slope):
         er, el, v = er.contiguous(), el.contiguous(), v.contiguous()
         mod = g._gat_mod(er, el, v, slope)
-        mod.state_tvm = torch.empty_like(mod.state_tvm)
-        out = _fresh_run(mod, [er, el, v])
+        if not any(ctx.needs_input_grad):
+            return _fresh_run(mod, [er, el, v])
+        _let_go(mod)
+        out, saved = mod.train_forward(er, el, v)
         ctx.g, ctx.slope = g, slope
-        ctx.save_for_backward(er, el, v, out, mod.state_tvm)
+        ctx.save_for_backward(er, el, v, out, *saved)
         return out
 
     @staticmethod
     def backward(ctx, dout):
-        er, el, v, out, state = ctx.saved_tensors
-        der, del_, dv = ctx.g._gat_mod(er, el, v, ctx.slope).backward(er, el, v, out, state, dout.contiguous())
+        er, el, v, out, *saved = ctx.saved_tensors
+        der, del_, dv = ctx.g._gat_mod(er, el, v, ctx.slope).train_backward(er, el, v, out, saved, dout.contiguous())
         return None, der, del_, dv, None
 
 

@@ -47,16 +47,12 @@ struct AttnArgs {
     int F, H;
     int n_heads, head_base;   // heads of this launch
     float scale;
-    // additive scores: q = er [H, n_dst] and k = el [H, n_src] (k offset to the partition's first source), one
-    // scalar per vertex and head; floats from one head's block to the next; negative slope of the leaky ReLU
-    int64_t q_head_floats, k_head_floats;
-    float slope;
     // One launch over the items of all source partitions, every partition into buffers of its own (FIRST in every
     // pass): the plan's item_off on the device (n_parts + 1 entries; null: one partition's items, strides unused) and
     // the distance from one partition's pos / k / v / out / state to the next, in elements.
     const int64_t *item_off = nullptr;
     int n_parts = 1;
-    int64_t pos_stride = 0, k_stride = 0, v_stride = 0, out_stride = 0, state_stride = 0;
+    int64_t pos_stride = 0, kv_stride = 0, out_stride = 0, state_stride = 0;
 };
 
 // Running softmax-weighted sum of one lane group: maximum, sum of exponentials, weighted sum.
@@ -78,43 +74,24 @@ __device__ __forceinline__ void running_merge(Running &r, const Running &s) {
     r.m = m;
 }
 
-// What is staged per element: the byte offset of its row in K / V, and, for additive scores, its scalar
-// el[col, h] as well (gathered once per item, 64 elements per load, instead of once per step).
-template <bool ADD> struct Staged;
-template <> struct Staged<false> { using type = int32_t; };
-template <> struct Staged<true> { using type = int2; };
-__device__ __forceinline__ uint32_t slice_off(int32_t c) { return (uint32_t)c; }
-__device__ __forceinline__ uint32_t slice_off(const int2 &c) { return (uint32_t)c.x; }
-__device__ __forceinline__ float staged_scalar(int32_t) { return 0.f; }
-__device__ __forceinline__ float staged_scalar(const int2 &c) { return __int_as_float(c.y); }
-
 // NU elements of one row, those with valid[u] counted: all gathers are issued before the first is used,
 // then the scores and the running update.
-//   ADD == false: score = scale * <K[c, h, :], q>  (k: the K slices, this lane's 16 bytes at lane_bytes);
-//   ADD == true : score = leaky_relu(el + q.x) with negative slope `scale`  (el: the element's staged scalar).
-template <int L, int NU, bool ADD, typename S>
-__device__ __forceinline__ void update(const S (&c)[NU], const bool (&valid)[NU], const float *k, const float *v,
+// score = scale * <K[c, h, :], q>  (k: the K slices, this lane's 16 bytes at lane_bytes).
+template <int L, int NU>
+__device__ __forceinline__ void update(const int32_t (&c)[NU], const bool (&valid)[NU], const float *k, const float *v,
                                        uint32_t lane_bytes, const float4 &q, float scale, Running &r) {
     float4 kk[NU], vv[NU];
-    float ev[NU];
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
-        if constexpr (ADD) ev[u] = staged_scalar(c[u]);
-        else kk[u] = *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(k) + (slice_off(c[u]) + lane_bytes));
-        vv[u] = *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(v) + (slice_off(c[u]) + lane_bytes));
+        kk[u] = *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(k) + ((uint32_t)c[u] + lane_bytes));
+        vv[u] = *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(v) + ((uint32_t)c[u] + lane_bytes));
     }
     float s[NU];
     float m = r.m;
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
-        float t;
-        if constexpr (ADD) {
-            const float z = ev[u] + q.x;
-            t = z > 0.f ? z : z * scale;
-        } else {
-            const float d = kk[u].x * q.x + kk[u].y * q.y + kk[u].z * q.z + kk[u].w * q.w;
-            t = group_sum<L>(d) * scale;                // every lane takes part in the cross-lane sum
-        }
+        const float d = kk[u].x * q.x + kk[u].y * q.y + kk[u].z * q.z + kk[u].w * q.w;
+        const float t = group_sum<L>(d) * scale;                // every lane takes part in the cross-lane sum
         s[u] = valid[u] ? t : -INFINITY;
         m = fmaxf(m, s[u]);
     }
@@ -137,51 +114,51 @@ __device__ __forceinline__ void update(const S (&c)[NU], const bool (&valid)[NU]
 // NU steps of one row for this lane group: staged elements s0 + g, s0 + g + G, ...; every step but the
 // last lies wholly below e, and in the last one (unless ALLVALID) a group whose element would be e or
 // beyond re-reads element e - 1 and gives it no weight.
-template <int L, int NU, bool ALLVALID, bool ADD, typename S>
-__device__ __forceinline__ void walk_batch(const S *cols, int s0, int e, int g, const float *k, const float *v,
+template <int L, int NU, bool ALLVALID>
+__device__ __forceinline__ void walk_batch(const int32_t *cols, int s0, int e, int g, const float *k, const float *v,
                                            uint32_t lane_bytes, const float4 &q, float scale, Running &r) {
     constexpr int G = 64 / L;
     const bool last_valid = ALLVALID || s0 + (NU - 1) * G + g < e;
-    S c[NU];
+    int32_t c[NU];
     bool valid[NU];
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
         valid[u] = u < NU - 1 || last_valid;
         c[u] = cols[valid[u] ? s0 + u * G + g : e - 1];
     }
-    update<L, NU, ADD>(c, valid, k, v, lane_bytes, q, scale, r);
+    update<L, NU>(c, valid, k, v, lane_bytes, q, scale, r);
 }
 
 // Staged elements [b, e) of one row, shared by the G lane groups; the last batch is issued with exactly
 // the steps it has left.
-template <int L, bool ADD, typename S>
-__device__ __forceinline__ void walk(const S *cols, int b, int e, int g, const float *k, const float *v,
+template <int L>
+__device__ __forceinline__ void walk(const int32_t *cols, int b, int e, int g, const float *k, const float *v,
                                      uint32_t lane_bytes, const float4 &q, float scale, Running &r) {
     constexpr int G = 64 / L;
     int s0 = b;
-    for (; s0 + G * kU <= e; s0 += G * kU) walk_batch<L, kU, true, ADD>(cols, s0, e, g, k, v, lane_bytes, q, scale, r);
+    for (; s0 + G * kU <= e; s0 += G * kU) walk_batch<L, kU, true>(cols, s0, e, g, k, v, lane_bytes, q, scale, r);
     if (s0 >= e) return;
     const int nu = (e - s0 + G - 1) / G;    // uniform: 1 .. kU
     static_assert(kU == 4, "the tail below lists the step counts");
-    if (nu == 1) walk_batch<L, 1, false, ADD>(cols, s0, e, g, k, v, lane_bytes, q, scale, r);
-    else if (nu == 2) walk_batch<L, 2, false, ADD>(cols, s0, e, g, k, v, lane_bytes, q, scale, r);
-    else if (nu == 3) walk_batch<L, 3, false, ADD>(cols, s0, e, g, k, v, lane_bytes, q, scale, r);
-    else walk_batch<L, 4, false, ADD>(cols, s0, e, g, k, v, lane_bytes, q, scale, r);
+    if (nu == 1) walk_batch<L, 1, false>(cols, s0, e, g, k, v, lane_bytes, q, scale, r);
+    else if (nu == 2) walk_batch<L, 2, false>(cols, s0, e, g, k, v, lane_bytes, q, scale, r);
+    else if (nu == 3) walk_batch<L, 3, false>(cols, s0, e, g, k, v, lane_bytes, q, scale, r);
+    else walk_batch<L, 4, false>(cols, s0, e, g, k, v, lane_bytes, q, scale, r);
 }
 
 // kU consecutive staged elements j .. j + kU - 1 of this lane group's own row (those below e count; the
 // slots behind them hold later rows' elements or the padding: loadable, given no weight).
-template <int L, bool ADD, typename S>
-__device__ __forceinline__ void own_batch(const S *cols, int j, int e, const float *k, const float *v,
+template <int L>
+__device__ __forceinline__ void own_batch(const int32_t *cols, int j, int e, const float *k, const float *v,
                                           uint32_t lane_bytes, const float4 &q, float scale, Running &r) {
-    S c[kU];
+    int32_t c[kU];
     bool valid[kU];
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
         c[u] = cols[j + u];
         valid[u] = j + u < e;
     }
-    update<L, kU, ADD>(c, valid, k, v, lane_bytes, q, scale, r);
+    update<L, kU>(c, valid, k, v, lane_bytes, q, scale, r);
 }
 
 // What the earlier partitions left for a row (read before the row's gathers are issued).
@@ -222,13 +199,10 @@ __device__ __forceinline__ void finish_row(Running r, const Running &old, int g,
 // L lanes x 128 bits cover one head.  FIRST: the pass writes every row's state -- the first partition's pass, or
 // every partition's when each has buffers of its own (one launch over all partitions, merged afterwards);
 // otherwise later passes merge into the stored state and skip rows without elements in their partition.
-// ADD: scores are leaky_relu(el[col e, h] + er[row e, h]) (a.k = el and a.q = er, one scalar per vertex and head,
-// head by head) instead of scaled dot products of K and Q slices.
-template <int L, bool FIRST, bool ADD>
+template <int L, bool FIRST>
 __global__ __launch_bounds__(kBlock) void attention_items_kernel(const AttnArgs a) {
     constexpr int G = 64 / L, D = 4 * L;
-    using S = typename Staged<ADD>::type;
-    __shared__ __align__(16) S s_col[kWavesPerBlock][fg::kItemEdges + kPad];
+    __shared__ __align__(16) int32_t s_col[kWavesPerBlock][fg::kItemEdges + kPad];
     __shared__ int32_t s_end[kWavesPerBlock][fg::kItemRows];
     __shared__ int32_t s_next[kWavesPerBlock];
 
@@ -245,19 +219,15 @@ __global__ __launch_bounds__(kBlock) void attention_items_kernel(const AttnArgs 
         while (part + 1 < a.n_parts && id >= a.item_off[part + 1]) ++part;
     }
     const int32_t *const pos_p = a.pos + part * a.pos_stride;
-    const float *const k_p = a.k + part * a.k_stride;
-    const float *const v_p = a.v + part * a.v_stride;
+    const float *const k_p = a.k + part * a.kv_stride;
+    const float *const v_p = a.v + part * a.kv_stride;
     float *const out_p = a.out + part * a.out_stride;
     float *const state_p = a.state + part * a.state_stride;
     const int g = lane / L, li = lane % L;
     const int f_lo = head * D + li * 4;
     const uint32_t lane_bytes = a.kv_tile_bytes ? (uint32_t)head * a.kv_tile_bytes + (uint32_t)li * 16u : (uint32_t)f_lo * 4u;
     const int64_t F = a.F;
-    S *cols = s_col[wave];
-    // ADD: this head's scalars; the score's second parameter is the negative slope
-    const float *kptr = ADD ? k_p + (int64_t)head * a.k_head_floats : k_p;
-    const float *q_head = a.q + (int64_t)head * a.q_head_floats;
-    const float sparam = ADD ? a.slope : a.scale;
+    int32_t *cols = s_col[wave];
 
     auto stage = [&](int64_t base, int n) {
         int32_t c[4];
@@ -265,24 +235,10 @@ __global__ __launch_bounds__(kBlock) void attention_items_kernel(const AttnArgs 
         uint32_t b[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) b[i] = (uint32_t)c[i] * a.kv_row_bytes;
-        if constexpr (ADD) {
-            int ev[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) ev[i] = __float_as_int(kptr[c[i]]);
-            int4 *c4 = reinterpret_cast<int4 *>(cols);
-            c4[2 * lane] = make_int4((int)b[0], ev[0], (int)b[1], ev[1]);
-            c4[2 * lane + 1] = make_int4((int)b[2], ev[2], (int)b[3], ev[3]);
-            if (lane < kPad) cols[fg::kItemEdges + lane] = make_int2((int)b[3], ev[3]);
-        } else {
-            *reinterpret_cast<int4 *>(cols + 4 * lane) = make_int4((int)b[0], (int)b[1], (int)b[2], (int)b[3]);
-            if (lane < kPad) cols[fg::kItemEdges + lane] = (int)b[3];
-        }
+        *reinterpret_cast<int4 *>(cols + 4 * lane) = make_int4((int)b[0], (int)b[1], (int)b[2], (int)b[3]);
+        if (lane < kPad) cols[fg::kItemEdges + lane] = (int)b[3];
     };
-    // the row's own operand: its slice of Q, or (ADD) its scalar in .x
-    auto own_q = [&](int64_t row) {
-        if constexpr (ADD) return make_float4(q_head[row], 0.f, 0.f, 0.f);
-        else return *reinterpret_cast<const float4 *>(a.q + row * F + f_lo);
-    };
+    auto own_q = [&](int64_t row) { return *reinterpret_cast<const float4 *>(a.q + row * F + f_lo); };
     auto out_row = [&](int64_t row) { return out_p + row * F + f_lo; };
     auto state_row = [&](int64_t row) { return state_p + (row * a.H + head) * 2; };
 
@@ -299,7 +255,7 @@ __global__ __launch_bounds__(kBlock) void attention_items_kernel(const AttnArgs 
         for (int i = 0; i < 2; ++i) {
             const int t = lane + 64 * i;
             const int64_t at = (int64_t)(it.row + min(t / kLines, nrows - 1)) * F + head * D + min((t % kLines) * 32, D - 1);
-            if (!ADD) touched += a.q[at];
+            touched += a.q[at];
             if (!FIRST) touched += out_p[at];
         }
         if (it.len > 0) stage(it.start, it.len);
@@ -341,7 +297,7 @@ __global__ __launch_bounds__(kBlock) void attention_items_kernel(const AttnArgs 
                 }
                 if (__all(done)) break;
                 if (!done && j < e) {
-                    own_batch<L, ADD>(cols, j, e, kptr, v_p, lane_bytes, q, sparam, run);
+                    own_batch<L>(cols, j, e, k_p, v_p, lane_bytes, q, a.scale, run);
                     j += kU;
                 }
             }
@@ -354,7 +310,7 @@ __global__ __launch_bounds__(kBlock) void attention_items_kernel(const AttnArgs 
                 const float4 q = own_q(it.row + r);
                 const Running old = load_state<FIRST>(out_row(it.row + r), state_row(it.row + r));
                 Running run = running_empty();
-                walk<L, ADD>(cols, b, e, g, kptr, v_p, lane_bytes, q, sparam, run);
+                walk<L>(cols, b, e, g, k_p, v_p, lane_bytes, q, a.scale, run);
                 finish_row<L, FIRST>(run, old, g, li, out_row(it.row + r), state_row(it.row + r));
             }
             b = e;
@@ -370,7 +326,7 @@ __global__ __launch_bounds__(kBlock) void attention_items_kernel(const AttnArgs 
         wave_lds_sync();
         stage((int64_t)it.start + base, n);
         wave_lds_sync();
-        walk<L, ADD>(cols, 0, n, g, kptr, v_p, lane_bytes, q, sparam, run);
+        walk<L>(cols, 0, n, g, k_p, v_p, lane_bytes, q, a.scale, run);
     }
     if (it.len > 0 || FIRST) finish_row<L, FIRST>(run, old, g, li, out_row(it.row), state_row(it.row));
 }
@@ -419,18 +375,16 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(float4 *out, float
     if (w == h * head_words) { state[srow] = run.m; state[srow + 1] = run.l; }
 }
 
-template <int L, bool ADD>
+template <int L>
 void launch(bool first, dim3 grid, hipStream_t st, const AttnArgs &a) {
-    if (first) hipLaunchKernelGGL((attention_items_kernel<L, true, ADD>), grid, dim3(kBlock), 0, st, a);
-    else hipLaunchKernelGGL((attention_items_kernel<L, false, ADD>), grid, dim3(kBlock), 0, st, a);
+    if (first) hipLaunchKernelGGL((attention_items_kernel<L, true>), grid, dim3(kBlock), 0, st, a);
+    else hipLaunchKernelGGL((attention_items_kernel<L, false>), grid, dim3(kBlock), 0, st, a);
 }
 
-// The passes over the source partitions.  ADD == false: q / k are the [n, F] operands of the dot products and
-// `param` their scale; ADD == true: q = er [H, n_dst], k = el [H, n_src] and `param` the leaky ReLU's slope.
-template <bool ADD>
+// The passes over the source partitions.
 int run_forward(fg_spmm_plan *pl, const int32_t *pos_dev, const int32_t *idx_dev, const float *q_dev,
                 const float *k_dev, const float *v_dev, float *out_dev, float *row_state_dev, int heads,
-                int head_len, float param, void *stream) {
+                int head_len, float scale, void *stream) {
     if (!pl) return fail(FG_ERR_ARG, "plan is null");
     if (int drc = fg::check_device(pl)) return drc;
     if (heads < 1 || !(head_len == 16 || head_len == 32 || head_len == 64))
@@ -440,13 +394,13 @@ int run_forward(fg_spmm_plan *pl, const int32_t *pos_dev, const int32_t *idx_dev
     if (pl->n_dst == 0) return FG_OK;
     if (!pos_dev || !q_dev || !out_dev || (pl->nnz > 0 && (!idx_dev || !k_dev || !v_dev)))
         return fail(FG_ERR_ARG, "null device pointer");
-    if ((((uintptr_t)v_dev | (uintptr_t)out_dev | (ADD ? 0 : ((uintptr_t)q_dev | (uintptr_t)k_dev))) & 15) != 0)
+    if ((((uintptr_t)v_dev | (uintptr_t)out_dev | (uintptr_t)q_dev | (uintptr_t)k_dev) & 15) != 0)
         return fail(FG_ERR_ARG, "attention needs 16-byte aligned arrays");
     const int F = heads * head_len;
     if ((uint64_t)pl->n_src * (uint64_t)F * 4u >= (1ull << 32) || (uint64_t)pl->n_dst * (uint64_t)F >= (1ull << 32))
         return fail(FG_ERR_SHAPE, "attention operands of 4 GiB and more are not supported");
     fg::ScratchNeed need;
-    int rc = fg::attention_scratch_need(pl, heads, head_len, ADD, !row_state_dev, &need);
+    int rc = fg::attention_scratch_need(pl, heads, head_len, 2, !row_state_dev, &need);
     if (rc == FG_OK) rc = fg::ensure_scratch(pl, need, stream);
     if (rc != FG_OK) return rc;
     if (!row_state_dev) row_state_dev = pl->partial_dev;
@@ -457,13 +411,10 @@ int run_forward(fg_spmm_plan *pl, const int32_t *pos_dev, const int32_t *idx_dev
     const bool tiled = need.tiled > 0;
     const float *k = k_dev, *v = v_dev;
     if (tiled) {
-        const int slots = ADD ? 1 : 2;
-        if ((rc = fg::make_tile_major(pl, v_dev, pl->n_src, F, head_len, stream, 0, slots)) != FG_OK) return rc;
+        if ((rc = fg::make_tile_major(pl, v_dev, pl->n_src, F, head_len, stream, 0, 2)) != FG_OK) return rc;
+        if ((rc = fg::make_tile_major(pl, k_dev, pl->n_src, F, head_len, stream, 1, 2)) != FG_OK) return rc;
         v = pl->tiled_dev;
-        if (!ADD) {
-            if ((rc = fg::make_tile_major(pl, k_dev, pl->n_src, F, head_len, stream, 1, slots)) != FG_OK) return rc;
-            k = pl->tiled_dev + (size_t)pl->n_src * F;
-        }
+        k = pl->tiled_dev + (size_t)pl->n_src * F;
     }
     const int row_floats = tiled ? head_len : F;
     const size_t own_state = row_state_dev == pl->partial_dev ? (size_t)pl->n_dst * heads * 2 : 0;
@@ -477,23 +428,21 @@ int run_forward(fg_spmm_plan *pl, const int32_t *pos_dev, const int32_t *idx_dev
         a.items = pl->items_dev; a.n_items = pl->n_items; a.item_off = pl->item_off_dev; a.n_parts = P;
         a.pos = pos_dev; a.pos_stride = pl->n_dst + 1;
         a.indices = idx_dev; a.indices16 = fg::narrow_indices(pl, idx_dev); a.q = q_dev;
-        a.k = k; a.k_stride = ADD ? width : width * row_floats;
-        a.v = v; a.v_stride = width * row_floats;
+        a.k = k; a.v = v; a.kv_stride = width * row_floats;
         a.kv_row_bytes = (uint32_t)row_floats * 4u;
         a.kv_tile_bytes = tiled ? (uint32_t)((uint64_t)pl->n_src * head_len * 4u) : 0u;
         a.out = buf_out; a.out_stride = (int64_t)buf_out_floats;
         a.state = buf_state; a.state_stride = (int64_t)buf_state_floats;
-        a.F = F; a.H = heads; a.scale = param; a.slope = param;
-        a.q_head_floats = ADD ? pl->n_dst : 0; a.k_head_floats = ADD ? pl->n_src : 0;
+        a.F = F; a.H = heads; a.scale = scale;
         const int per_launch = (heads > 8 && heads % 8 == 0) ? 8 : heads;
         for (int hb = 0; hb < heads; hb += per_launch) {
             a.n_heads = per_launch; a.head_base = hb;
             const int64_t blocks = ((pl->n_items + kWavesPerBlock - 1) / kWavesPerBlock) * per_launch;
             if (blocks > 0x7fffffffLL) return fail(FG_ERR_SHAPE, "grid of %lld workgroups is too large", (long long)blocks);
             const dim3 grid((unsigned)blocks);
-            if (head_len == 64) launch<16, ADD>(true, grid, st, a);
-            else if (head_len == 32) launch<8, ADD>(true, grid, st, a);
-            else launch<4, ADD>(true, grid, st, a);
+            if (head_len == 64) launch<16>(true, grid, st, a);
+            else if (head_len == 32) launch<8>(true, grid, st, a);
+            else launch<4>(true, grid, st, a);
         }
         const uint32_t n_words = (uint32_t)((uint64_t)pl->n_dst * F / 4);
         hipLaunchKernelGGL(attention_merge_kernel, dim3((n_words + 255u) / 256u), dim3(256), 0, st,
@@ -509,21 +458,20 @@ int run_forward(fg_spmm_plan *pl, const int32_t *pos_dev, const int32_t *idx_dev
         a.items = pl->items_dev + i0; a.n_items = i1 - i0;
         a.pos = pos_dev + (int64_t)p * (pl->n_dst + 1);
         a.indices = idx_dev; a.indices16 = fg::narrow_indices(pl, idx_dev); a.q = q_dev;
-        a.k = ADD ? k + (int64_t)p * width : k + (int64_t)p * width * row_floats;
+        a.k = k + (int64_t)p * width * row_floats;
         a.v = v + (int64_t)p * width * row_floats;
         a.kv_row_bytes = (uint32_t)row_floats * 4u;
         a.kv_tile_bytes = tiled ? (uint32_t)((uint64_t)pl->n_src * head_len * 4u) : 0u;
-        a.out = out_dev; a.state = row_state_dev; a.F = F; a.H = heads; a.scale = param; a.slope = param;
-        a.q_head_floats = ADD ? pl->n_dst : 0; a.k_head_floats = ADD ? pl->n_src : 0;
+        a.out = out_dev; a.state = row_state_dev; a.F = F; a.H = heads; a.scale = scale;
         const int per_launch = (heads > 8 && heads % 8 == 0) ? 8 : heads;
         for (int hb = 0; hb < heads; hb += per_launch) {
             a.n_heads = per_launch; a.head_base = hb;
             const int64_t blocks = ((i1 - i0 + kWavesPerBlock - 1) / kWavesPerBlock) * per_launch;
             if (blocks > 0x7fffffffLL) return fail(FG_ERR_SHAPE, "grid of %lld workgroups is too large", (long long)blocks);
             const dim3 grid((unsigned)blocks);
-            if (head_len == 64) launch<16, ADD>(p == 0, grid, st, a);
-            else if (head_len == 32) launch<8, ADD>(p == 0, grid, st, a);
-            else launch<4, ADD>(p == 0, grid, st, a);
+            if (head_len == 64) launch<16>(p == 0, grid, st, a);
+            else if (head_len == 32) launch<8>(p == 0, grid, st, a);
+            else launch<4>(p == 0, grid, st, a);
         }
     }
     const uint32_t n_words = (uint32_t)((uint64_t)pl->n_dst * F / 4);
@@ -546,9 +494,9 @@ bool attention_pass_buffers(const fg_spmm_plan *pl, int heads, int head_len) {
     const uint64_t floats = (uint64_t)pl->n_dst * heads * (head_len + 2);
     return floats * 4u * (uint64_t)P <= (8ull << 30);
 }
-// The rows' (max, sum) state when the caller passes none, and the head-by-head copies of the gathered
-// operands (V, and K for dot-product scores); the gradient kernels need the same copies and no state.
-int attention_scratch_need(const fg_spmm_plan *pl, int heads, int head_len, bool additive, bool own_row_state,
+// The rows' (max, sum) state when the caller passes none, and the head-by-head copies of the `gathered`
+// operands (K and V; V alone with additive scores); the gradient kernels need the same copies and no state.
+int attention_scratch_need(const fg_spmm_plan *pl, int heads, int head_len, int gathered, bool own_row_state,
                            ScratchNeed *need, bool forward) {
     if (heads < 1 || !(head_len == 16 || head_len == 32 || head_len == 64))
         return fail(FG_ERR_SHAPE, "attention takes heads of 16, 32 or 64 floats, got %d heads of %d", heads, head_len);
@@ -564,7 +512,7 @@ int attention_scratch_need(const fg_spmm_plan *pl, int heads, int head_len, bool
     // 16 3659 -> 3717, 23 4780 -> 5001 (additive 16 2135 -> 2060, 23 2656 -> 2713); 8 x 64 dot 16 8215 -> 7882, 32 13586 -> 13803.
     const bool pays = pl->tile_major == 1 || pl->nnz >= (head_len == 16 ? 12 : head_len == 32 ? 20 : 24) * pl->n_src;
     if (pays && pl->nnz > 0 && wants_tile_major(pl, heads, (uint64_t)pl->n_src * F * 4u))
-        need->tiled = (size_t)pl->n_src * F * (additive ? 1 : 2);
+        need->tiled = (size_t)pl->n_src * F * gathered;
     return FG_OK;
 }
 }  // namespace fg
@@ -572,13 +520,5 @@ int attention_scratch_need(const fg_spmm_plan *pl, int heads, int head_len, bool
 extern "C" int fg_graph_attention_f32(fg_spmm_plan *pl, const int32_t *pos_dev, const int32_t *idx_dev,
                                       const float *q_dev, const float *k_dev, const float *v_dev, float *out_dev,
                                       float *row_state_dev, int heads, int head_len, float scale, void *stream) {
-    return run_forward<false>(pl, pos_dev, idx_dev, q_dev, k_dev, v_dev, out_dev, row_state_dev, heads, head_len, scale, stream);
-}
-
-extern "C" int fg_graph_attention_additive_f32(fg_spmm_plan *pl, const int32_t *pos_dev, const int32_t *idx_dev,
-                                               const float *er_dev, const float *el_dev, const float *v_dev,
-                                               float *out_dev, float *row_state_dev, int heads, int head_len,
-                                               float negative_slope, void *stream) {
-    return run_forward<true>(pl, pos_dev, idx_dev, er_dev, el_dev, v_dev, out_dev, row_state_dev, heads, head_len,
-                             negative_slope, stream);
+    return run_forward(pl, pos_dev, idx_dev, q_dev, k_dev, v_dev, out_dev, row_state_dev, heads, head_len, scale, stream);
 }

@@ -122,6 +122,9 @@ int gspmm_bcast_scratch_need(const fg_spmm_plan *plan, int out_len, bool with_ar
 bool attention_pass_buffers(const fg_spmm_plan *plan, int heads, int head_len);
 // forward: the call is the forward pass (whose partitions may write buffers of their own); the gradient sweeps need
 // only the head-by-head copies of the gathered operands.
-int attention_scratch_need(const fg_spmm_plan *plan, int heads, int head_len, bool additive, bool own_row_state,
+int attention_scratch_need(const fg_spmm_plan *plan, int heads, int head_len, int gathered, bool own_row_state,
                            ScratchNeed *need, bool forward = true);
+// The same for additive scores; plus: the forward pass also keeps the sums over the edges with a positive score.
+int additive_scratch_need(const fg_spmm_plan *plan, int heads, int head_len, bool own_row_state, bool plus, ScratchNeed *need,
+                          bool forward = true);
 }  // namespace fg

@@ -70,6 +70,48 @@ __device__ __forceinline__ float group_sum(float v) {
     return v;
 }
 
+// Lanes l and l + 32 (l < 32) trade: afterwards a holds {a of the lower half, b of the lower half} and b the two upper
+// halves.  a + b is then a's sum over l and l + 32 in the lower half and b's in the upper one: two values reduced by one
+// vector instruction and one add, where ds_bpermute takes a trip through LDS for each.
+__device__ __forceinline__ void swap_halves(float &a, float &b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]); b = __uint_as_float(r[1]);
+}
+// The same between the odd 16-lane rows of a and the even rows of b.
+__device__ __forceinline__ void swap_rows(float &a, float &b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]); b = __uint_as_float(r[1]);
+}
+// Sum (maximum) over lanes l, l ^ 16, l ^ 32, l ^ 48; every lane gets it.
+__device__ __forceinline__ float rows_sum(float v) {
+    float w = v;
+    swap_halves(v, w);
+    v += w; w = v;
+    swap_rows(v, w);
+    return v + w;
+}
+__device__ __forceinline__ float rows_max(float v) {
+    float w = v;
+    swap_halves(v, w);
+    v = fmaxf(v, w); w = v;
+    swap_rows(v, w);
+    return fmaxf(v, w);
+}
+// Sum of v over the 64 / L lane groups of the wavefront (lanes l, l + L, ...): component word_of_row() of it in every
+// lane, i.e. a lane's four words end up in the wavefront's four 16-lane rows.
+template <int L>
+__device__ __forceinline__ float groups_sum(float4 v) {
+    swap_halves(v.x, v.y);
+    swap_halves(v.z, v.w);
+    float a = v.x + v.y, b = v.z + v.w;      // lower half x / z, upper half y / w
+    swap_rows(a, b);
+    a += b;                                  // rows 0 .. 3: x, z, y, w
+    if (L <= 8) a += dpp_move<0x128>(a);     // row_ror:8
+    if (L <= 4) a += dpp_move<0x124>(a);     // row_ror:4
+    return a;
+}
+__device__ __forceinline__ int word_of_row(int lane) { return ((lane >> 5) & 1) | ((lane >> 3) & 2); }
+
 // use(p, load(p)) for p in [first, n), in order, eight loads in flight: a row's pieces added up one load at a time take
 // about 0.3 us each.  3 M elements with rows of up to 60,000 (240 pieces), whole calls: F=16 weighted sum 84 -> 51 us,
 // maximum 176 -> 121; 100 rows of 5,000, F=16 maximum 32 -> 18; the results are the same bits.

@@ -410,8 +410,9 @@ extern "C" int fg_spmm_plan_reserve(fg_spmm_plan *pl, int op, int heads, int hea
         case FG_OP_SPMM_EXTREME: rc = fg::spmm_scratch_need(pl, heads * head_len, heads, FG_REDUCE_MAX, num_feat_partitions, &need); break;
         case FG_OP_SDDMM_DDS: rc = fg::sddmm_dds_scratch_need(pl, heads, head_len, num_feat_partitions, &need); break;
         case FG_OP_EDGE_SOFTMAX: rc = fg::softmax_scratch_need(pl, heads, &need); break;
-        case FG_OP_ATTENTION: rc = fg::attention_scratch_need(pl, heads, head_len, false, true, &need); break;
-        case FG_OP_ATTENTION_ADDITIVE: rc = fg::attention_scratch_need(pl, heads, head_len, true, true, &need); break;
+        case FG_OP_ATTENTION: rc = fg::attention_scratch_need(pl, heads, head_len, 2, true, &need); break;
+        case FG_OP_ATTENTION_ADDITIVE: rc = fg::additive_scratch_need(pl, heads, head_len, true, false, &need); break;
+        case FG_OP_ATTENTION_ADDITIVE_TRAIN: rc = fg::additive_scratch_need(pl, heads, head_len, false, true, &need); break;
         case FG_OP_GSPMM_BCAST: rc = fg::gspmm_bcast_scratch_need(pl, heads * head_len, false, &need); break;
         case FG_OP_GSPMM_BCAST_ARG: rc = fg::gspmm_bcast_scratch_need(pl, heads * head_len, true, &need); break;
         default: return fail(FG_ERR_ARG, "fg_spmm_plan_reserve: unknown operator %d", op);

@@ -52,7 +52,8 @@ class GraphAttentionhip(object):
                'plan': ctypes.c_void_p()}
         base = _lib.plan_opts
         opts = _lib.FgPlanOpts(split_threshold=_INT32_MAX, item_edges=base.item_edges if base is not None else 0,
-                               wide_offsets=0, tile_major=base.tile_major if base is not None else 0)
+                               wide_offsets=0, tile_major=base.tile_major if base is not None else 0,
+                               pass_buffers=base.pass_buffers if base is not None else 0)
         with torch.cuda.device(self._ctx):
             _lib.check(_lib.lib().fg_spmm_plan_create(_lib.host_ptr(np.ascontiguousarray(pos, dtype=np.int32)),
                                                       self._num_rows, self._num_cols, P, ctypes.byref(opts),
@@ -184,7 +185,8 @@ class GraphAttentionhip(object):
                'idx': common.to_device_i32(np.ascontiguousarray(idx, dtype=np.int32), self._ctx), 'plan': ctypes.c_void_p()}
         base = _lib.plan_opts
         opts = _lib.FgPlanOpts(split_threshold=_INT32_MAX, item_edges=base.item_edges if base is not None else 0,
-                               wide_offsets=0, tile_major=base.tile_major if base is not None else 0)
+                               wide_offsets=0, tile_major=base.tile_major if base is not None else 0,
+                               pass_buffers=base.pass_buffers if base is not None else 0)
         with torch.cuda.device(self._ctx):
             _lib.check(_lib.lib().fg_spmm_plan_create(_lib.host_ptr(pos), self._num_cols, self._num_rows, P,
                                                       ctypes.byref(opts), ctypes.byref(lay['plan'])))
@@ -255,6 +257,45 @@ class GraphAttentionhip(object):
             ctypes.c_float(self._slope), s))
         self._coef = coef
         return der_t.t().contiguous(), del_t.t().contiguous(), dv
+
+    def train_forward(self, er, el, v):
+        """Additive scores: (out, saved) as new tensors, `saved` being what train_backward() starts from -- the row state and
+        the sums over the edges with a positive score (as large as `out`), with which dEr takes no sweep of its own."""
+        if self._placeholders is None or not self._additive:
+            raise RuntimeError("build() with additive scores before train_forward()")
+        common.check_inputs([er, el, v], self._placeholders, self._ctx)
+        H, D, lay = self._heads, self._head_len, self._active
+        if not getattr(self, '_train_reserved', False):
+            common.reserve(lay['plan'], common.OP_ATTENTION_ADDITIVE_TRAIN, H, D, 0, self._ctx)
+            self._train_reserved = True
+        new = lambda *shape: torch.empty(shape, dtype=torch.float32, device=self._ctx)
+        n = self._num_rows
+        out, plus, state, share = new(n, H, D), new(n, H, D), new(n, H, 2), new(n, H)
+        el_t = el.t().contiguous()                      # head by head: one head's scalars are what an XCD gathers
+        _lib.check(_lib.lib().fg_graph_attention_additive_train_f32(
+            lay['plan'], _lib.dev_ptr(lay['pos']), _lib.dev_ptr(lay['idx']), _lib.dev_ptr(er), _lib.dev_ptr(el_t),
+            _lib.dev_ptr(v), _lib.dev_ptr(out), _lib.dev_ptr(state), _lib.dev_ptr(plus), _lib.dev_ptr(share), H, D,
+            ctypes.c_float(self._slope), common.stream_ptr()))
+        return out, (state, plus, share)
+
+    def train_backward(self, er, el, v, out, saved, grad_out):
+        """(dEr, dEl, dV) from what train_forward() returned on these inputs."""
+        out_ph = common.placeholder((self._num_rows, self._heads, self._head_len))
+        common.check_inputs([er, el, v], self._placeholders, self._ctx)
+        common.check_inputs([out, grad_out], [out_ph] * 2, self._ctx)
+        L, s = _lib.lib(), common.stream_ptr()
+        H, D = self._heads, self._head_len
+        state, plus, share = saved
+        coef = torch.empty((H, self._num_rows, 4), dtype=torch.float32, device=self._ctx)
+        der, del_, dv = torch.empty_like(er), torch.empty_like(el), torch.empty_like(v)
+        _lib.check(L.fg_graph_attention_additive_train_coef_f32(
+            _lib.dev_ptr(out), _lib.dev_ptr(grad_out), _lib.dev_ptr(state), _lib.dev_ptr(er), _lib.dev_ptr(plus),
+            _lib.dev_ptr(share), _lib.dev_ptr(coef), _lib.dev_ptr(der), self._num_rows, H, D, ctypes.c_float(self._slope), s))
+        lt = self._layout_t(self._dst_partitions(4 * D))
+        _lib.check(L.fg_graph_attention_additive_train_elv_f32(
+            lt['plan'], _lib.dev_ptr(lt['pos']), _lib.dev_ptr(lt['idx']), _lib.dev_ptr(grad_out), _lib.dev_ptr(el),
+            _lib.dev_ptr(v), _lib.dev_ptr(coef), _lib.dev_ptr(del_), _lib.dev_ptr(dv), H, D, ctypes.c_float(self._slope), s))
+        return der, del_, dv
 
     def measure_average_time(self, input_tvm_ndarrays, num_runs):
         if self._placeholders is None:

@@ -132,7 +132,8 @@ typedef enum {
     FG_OP_ATTENTION = 4,          /* fg_graph_attention_f32 and its two gradient calls */
     FG_OP_ATTENTION_ADDITIVE = 5, /* fg_graph_attention_additive_f32 and its two gradient calls */
     FG_OP_GSPMM_BCAST = 6,        /* fg_gspmm_bcast_f32 / _dds_f32 without arg_dev (heads * head_len = out_len) */
-    FG_OP_GSPMM_BCAST_ARG = 7     /* fg_gspmm_bcast_f32 / _dds_f32 with arg_dev */
+    FG_OP_GSPMM_BCAST_ARG = 7,    /* fg_gspmm_bcast_f32 / _dds_f32 with arg_dev */
+    FG_OP_ATTENTION_ADDITIVE_TRAIN = 8 /* fg_graph_attention_additive_train_f32 and _train_elv_f32 */
 } fg_op;
 int fg_spmm_plan_reserve(fg_spmm_plan *plan, int op, int heads, int head_len, int num_feat_partitions);
 
@@ -470,6 +471,28 @@ int fg_graph_attention_additive_backward_elv_f32(fg_spmm_plan *plan_t, const int
                                                  const float *el_dev, const float *v_dev, const float *row_coef_dev,
                                                  float *del_dev, float *dv_dev, int heads, int head_len,
                                                  float negative_slope, void *stream);
+
+/*
+ * The same operator and gradients for a training step, with one sweep each way.  er and el's gradient-side uses are
+ * vertex by vertex here: er_dev [n_dst, heads], der_dev [n_dst, heads], and in _train_elv el_dev / del_dev [n_src, heads]
+ * (the forward call still takes el_dev [heads, n_src], which it gathers).
+ *   _train: also plus[v, h, :] and share[v, h], the sums of a * V and of a over the edges with el + er > 0
+ *     ([n_dst, heads, head_len] and [n_dst, heads]); row_state_dev must be given.
+ *   _train_coef: row_coef as above, and der = (1 - slope) * (<dout, plus> - <dout, out> * share).
+ *   _train_elv: as _backward_elv.
+ */
+int fg_graph_attention_additive_train_f32(fg_spmm_plan *plan, const int32_t *pos_dev, const int32_t *idx_dev,
+                                          const float *er_dev, const float *el_dev, const float *v_dev, float *out_dev,
+                                          float *row_state_dev, float *plus_dev, float *share_dev, int heads,
+                                          int head_len, float negative_slope, void *stream);
+int fg_graph_attention_additive_train_coef_f32(const float *out_dev, const float *dout_dev, const float *row_state_dev,
+                                               const float *er_dev, const float *plus_dev, const float *share_dev,
+                                               float *row_coef_dev, float *der_dev, int64_t n_dst, int heads,
+                                               int head_len, float negative_slope, void *stream);
+int fg_graph_attention_additive_train_elv_f32(fg_spmm_plan *plan_t, const int32_t *pos_t_dev, const int32_t *idx_t_dev,
+                                              const float *dout_dev, const float *el_dev, const float *v_dev,
+                                              const float *row_coef_dev, float *del_dev, float *dv_dev, int heads,
+                                              int head_len, float negative_slope, void *stream);
 
 /* ---- synthetic graphs ---------------------------------------------------------------- */
 
