@@ -97,6 +97,17 @@ class Graph(object):
         mod = self._spmm_mod(transposed, tuple(x.shape[1:]), 0 if w.dim() == 1 else w.shape[1])
         return _fresh_run(mod, [x, w.contiguous()])
 
+    def _spmm_grads_raw(self, x, w, dy):
+        """(A(w)^T dy, <dy[row e], x[col e]> per edge) in one sweep over the transposed graph, which gathers dy once for both,
+        or, where there is no kernel for that, in two."""
+        dy = dy.contiguous()
+        mod = self._spmm_mod(True, tuple(dy.shape[1:]), 0 if w.dim() == 1 else w.shape[1])
+        like = _let_go(mod)
+        mod.out_tvm = torch.empty(like[0], dtype=like[1], device=like[2])
+        both = mod.run_with_dots(dy, w.contiguous(), x.contiguous())
+        mod.out_tvm = None
+        return both if both is not None else (self._spmm_raw(dy, w, transposed=True), self._sddmm_raw(x, dy))
+
     def _sddmm_raw(self, src, dst):
         return _fresh_run(self._sddmm_mod(tuple(src.shape[1:])), [src.contiguous(), dst.contiguous()])
 
@@ -328,6 +339,8 @@ class _SpMM(torch.autograd.Function):
     def backward(ctx, dy):
         g = ctx.g
         x, w = ctx.saved_tensors
+        if ctx.needs_input_grad[1] and ctx.needs_input_grad[2]:
+            return (None,) + g._spmm_grads_raw(x, w, dy)
         dx = g._spmm_raw(dy, w, transposed=True) if ctx.needs_input_grad[1] else None
         dw = g._sddmm_raw(x, dy) if ctx.needs_input_grad[2] else None
         return None, dx, dw

@@ -70,6 +70,17 @@ __device__ __forceinline__ float group_sum(float v) {
     return v;
 }
 
+// The workgroup's place in a one-dimensional grid when every XCD (workgroups are dealt to the 8 of them in turn) is to work
+// on one contiguous share: of n blocks the XCD of block b takes [x * n / 8, (x + 1) * n / 8), x = b mod 8.  For kernels
+// that read or write through a permutation with locality (edges in column order, results in row order): what one XCD
+// touches around the same time shares lines, which its own L2 then fills or reads whole.  58,000 nodes, 12.5 M edges, 64-float
+// rows: step of a weighted sum with both gradients 738 -> 722 us, and 605 once all its results are placed this way.
+__device__ __forceinline__ unsigned xcd_contiguous_block() {
+    const unsigned n = gridDim.x, x = blockIdx.x & 7u, i = blockIdx.x >> 3;
+    const unsigned q = n >> 3, r = n & 7u;             // the first r XCDs hold q + 1 blocks
+    return x * q + (x < r ? x : r) + i;
+}
+
 // Lanes l and l + 32 (l < 32) trade: afterwards a holds {a of the lower half, b of the lower half} and b the two upper
 // halves.  a + b is then a's sum over l and l + 32 in the lower half and b's in the upper one: two values reduced by one
 // vector instruction and one add, where ds_bpermute takes a trip through LDS for each.

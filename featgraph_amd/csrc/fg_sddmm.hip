@@ -588,13 +588,14 @@ __global__ __launch_bounds__(kBlock) void sddmm_tiled_kernel(const SddmmTiledArg
 // and are read as 128-bit non-temporal loads (each word is read once: 13.24 -> 13.16 ms at F=512 on the 232,965-node graph).
 __global__ __launch_bounds__(256) void sddmm_tile_sum_kernel(const float *partial, const int32_t *edge_pos,
                                                              float *out, int64_t n_edges, int64_t stride, int n_tiles) {
-    const int64_t e = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+    const int64_t e = ((int64_t)fg::xcd_contiguous_block() * blockDim.x + threadIdx.x) * 4;
     if (e >= n_edges) return;
     if (e + 4 <= n_edges) {
         typedef float f4 __attribute__((ext_vector_type(4)));
         f4 s = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(partial + e));
         for (int t = 1; t < n_tiles; ++t) s += __builtin_nontemporal_load(reinterpret_cast<const f4 *>(partial + (int64_t)t * stride + e));
-        const int4 at = *reinterpret_cast<const int4 *>(edge_pos + e);
+        typedef int i4 __attribute__((ext_vector_type(4)));
+        const i4 at = __builtin_nontemporal_load(reinterpret_cast<const i4 *>(edge_pos + e));
         out[at.x] = s.x; out[at.y] = s.y; out[at.z] = s.z; out[at.w] = s.w;
         return;
     }
@@ -609,7 +610,7 @@ __global__ __launch_bounds__(256) void sddmm_tile_sum_kernel(const float *partia
 // in traversal order, written as one run of H floats at the edge's stored position.
 __global__ __launch_bounds__(256) void sddmm_tile_heads_kernel(const float *staged, const int32_t *edge_pos,
                                                                float *out, int64_t n_edges, int64_t tile_stride, int n_tiles, int hpt) {
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t e = (int64_t)fg::xcd_contiguous_block() * blockDim.x + threadIdx.x;
     if (e >= n_edges) return;
     float *o = out + (int64_t)edge_pos[e] * n_tiles * hpt;
     for (int t = 0; t < n_tiles; ++t) {
@@ -627,7 +628,7 @@ __global__ __launch_bounds__(256) void sddmm_tile_heads_vec_kernel(const float *
                                                                    float *out, int64_t n_edges, int64_t tile_stride, int H) {
     typedef float f4 __attribute__((ext_vector_type(4)));
     const int per_edge = H / 4;
-    const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t id = (int64_t)fg::xcd_contiguous_block() * blockDim.x + threadIdx.x;
     const int64_t e = id / per_edge;
     if (e >= n_edges) return;
     const int q = (int)(id - e * per_edge);                 // heads 4q .. 4q + 3
@@ -1025,24 +1026,33 @@ extern "C" int fg_sddmm_dds_f32(fg_spmm_plan *pl, const int32_t *s1_pos_dev, con
         }
     }
     if (tile_sum) {
-        const unsigned blocks = (unsigned)((pl->nnz + 1023) / 1024);
-        hipLaunchKernelGGL(sddmm_tile_sum_kernel, dim3(blocks), dim3(256), 0, st, pl->partial_dev, edge_pos_dev,
-                           out_dev, pl->nnz, (pl->nnz + 3) & ~(int64_t)3, T);
+        fg::sum_tiles(pl->partial_dev, edge_pos_dev, out_dev, pl->nnz, (pl->nnz + 3) & ~(int64_t)3, T, stream);
+    } else if (staged && hpt == 1) {
+        fg::gather_heads(pl->partial_dev, edge_pos_dev, out_dev, pl->nnz, staged_stride(pl->nnz, 1), H, stream);
     } else if (staged) {
-        const int64_t blocks_vec = (pl->nnz * (H / 4) + 255) / 256;
-        const int64_t tstride = staged_stride(pl->nnz, hpt);
-        if (H % 4 == 0 && hpt == 1 && (((uintptr_t)out_dev) & 15) == 0 && blocks_vec <= 0x7fffffffLL) {
-            hipLaunchKernelGGL(sddmm_tile_heads_vec_kernel, dim3((unsigned)blocks_vec), dim3(256), 0, st, pl->partial_dev,
-                               edge_pos_dev, out_dev, pl->nnz, tstride, H);
-        } else {
-            const unsigned blocks = (unsigned)((pl->nnz + 255) / 256);
-            hipLaunchKernelGGL(sddmm_tile_heads_kernel, dim3(blocks), dim3(256), 0, st, pl->partial_dev, edge_pos_dev,
-                               out_dev, pl->nnz, tstride, T, hpt);
-        }
+        const unsigned blocks = (unsigned)((pl->nnz + 255) / 256);
+        hipLaunchKernelGGL(sddmm_tile_heads_kernel, dim3(blocks), dim3(256), 0, st, pl->partial_dev, edge_pos_dev,
+                           out_dev, pl->nnz, staged_stride(pl->nnz, hpt), T, hpt);
     }
     FG_HIP_TRY(hipGetLastError());
     return FG_OK;
 }
+
+namespace fg {
+void sum_tiles(const float *partial, const int32_t *edge_pos, float *out, int64_t n_edges, int64_t stride, int n_tiles, void *stream) {
+    hipLaunchKernelGGL(sddmm_tile_sum_kernel, dim3((unsigned)((n_edges + 1023) / 1024)), dim3(256), 0, (hipStream_t)stream, partial,
+                       edge_pos, out, n_edges, stride, n_tiles);
+}
+void gather_heads(const float *staged, const int32_t *edge_pos, float *out, int64_t n_edges, int64_t stride, int H, void *stream) {
+    const int64_t blocks_vec = (n_edges * (H / 4) + 255) / 256;
+    if (H % 4 == 0 && (((uintptr_t)out) & 15) == 0 && blocks_vec <= 0x7fffffffLL)
+        hipLaunchKernelGGL(sddmm_tile_heads_vec_kernel, dim3((unsigned)blocks_vec), dim3(256), 0, (hipStream_t)stream, staged, edge_pos,
+                           out, n_edges, stride, H);
+    else
+        hipLaunchKernelGGL(sddmm_tile_heads_kernel, dim3((unsigned)((n_edges + 255) / 256)), dim3(256), 0, (hipStream_t)stream, staged,
+                           edge_pos, out, n_edges, stride, H, 1);
+}
+}  // namespace fg
 
 // ---- element-wise edge operators ---------------------------------------------------------------
 //

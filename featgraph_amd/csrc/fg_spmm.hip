@@ -84,6 +84,14 @@ struct SpmmArgs {
     const int64_t *item_off = nullptr;
     int n_parts = 1;
     int64_t pos_stride = 0, x_stride = 0, out_stride = 0, partial_stride = 0;
+    // Sum with dots: every element's dot product of its gathered row with its output row's row of `own`, per head or, with
+    // one head, per kernel tile.  Rows of `own` lie own_ld floats apart and hold heads of own_len <= head_len floats (the
+    // kernel's columns beyond own_len meet zeros).  dots[(tile * HPT + head of the tile) * dots_stride + element].
+    const float *own = nullptr;
+    int64_t own_ld = 0;
+    int own_len = 0;
+    float *dots = nullptr;
+    int64_t dots_stride = 0;
 };
 
 
@@ -97,19 +105,53 @@ __device__ __forceinline__ const float *row_ptr(const float *x, uint32_t lane_by
     return reinterpret_cast<const float *>(reinterpret_cast<const char *>(x + (int64_t)staged * F) + lane_bytes);
 }
 
+// Sum over the L (a power of two up to 64) consecutive lanes of a lane group; every lane of the group gets it.
+template <int L>
+__device__ __forceinline__ float lanes_sum(float v) {
+    if constexpr (L == 2) { return v + fg::dpp_move<0xB1>(v); }
+    else {
+        v = fg::group_sum<(L < 16 ? L : 16)>(v);
+        if constexpr (L >= 32) {
+            float w = v;
+            fg::swap_rows(v, w);
+            v += w;
+        }
+        if constexpr (L >= 64) {
+            float w = v;
+            fg::swap_halves(v, w);
+            v += w;
+        }
+        return v;
+    }
+}
+
+// Where the dot products of a sum with dots go: into the staging row, in the place of the element's weight.  RL lanes hold
+// a head's part of a row; ON == false: no dots, nothing is done.
+template <bool ON, int RL>
+struct Dots {
+    float4 own;                     // this lane's four floats of the output row's row of `own`
+    __device__ __forceinline__ void put(int lane, const float4 &x, bool ok, int32_t *slot) const {
+        if constexpr (ON) {
+            const float d = lanes_sum<RL>(x.x * own.x + x.y * own.y + x.z * own.z + x.w * own.w);
+            if (ok && lane % RL == 0) *slot = __float_as_int(d);
+        }
+    }
+    __device__ __forceinline__ void put(int, float, bool, int32_t *) const {}
+};
+
 // The last, partly filled batch of gather_rows: exactly `nu` steps (1 <= nu <= NU, uniform over
 // the wavefront), so that no step is spent re-reading the row's last element; inside the last
 // step a lane without an element still re-reads it (no load under a branch) and replaces what it
 // loaded by zeros -- a select, not a product with weight zero, so that a non-finite source row
 // only ever reaches the rows that reference it.
-template <int V, int L, int K, bool FULL, int NU, bool OFF32, int HPT>
-__device__ __forceinline__ void gather_tail(int nu, const int2 *s_edge, const float *wrow, int s0, int e, int g,
+template <int V, int L, int K, bool FULL, int NU, bool OFF32, int HPT, typename DOTS>
+__device__ __forceinline__ void gather_tail(int nu, int2 *s_edge, float *wrow, int s0, int e, int g,
                                             const float *x, uint32_t lane_bytes, int64_t F, const bool (&on)[K],
-                                            typename Vec<V>::type (&acc)[K]) {
+                                            typename Vec<V>::type (&acc)[K], const DOTS &dots) {
     using vec = typename Vec<V>::type;
     constexpr int G = 64 / L;
     if (nu < NU) {
-        if constexpr (NU > 1) gather_tail<V, L, K, FULL, NU - 1, OFF32, HPT>(nu, s_edge, wrow, s0, e, g, x, lane_bytes, F, on, acc);
+        if constexpr (NU > 1) gather_tail<V, L, K, FULL, NU - 1, OFF32, HPT>(nu, s_edge, wrow, s0, e, g, x, lane_bytes, F, on, acc, dots);
         return;
     }
     int2 cw[NU];
@@ -135,6 +177,9 @@ __device__ __forceinline__ void gather_tail(int nu, const int2 *s_edge, const fl
             if (FULL || on[k]) {
                 if (u == NU - 1) xv[u][k] = vkeep(last_has, xv[u][k]);
                 vfma(acc[k], __int_as_float(cw[u].y), xv[u][k]);
+                const int j = u < NU - 1 || last_has ? s0 + u * G + g : e - 1;
+                dots.put(threadIdx.x & 63, xv[u][k], u < NU - 1 || last_has,
+                         HPT > 1 ? reinterpret_cast<int32_t *>(wrow + j) : &s_edge[j].y);
             }
 }
 
@@ -144,10 +189,11 @@ __device__ __forceinline__ void gather_tail(int nu, const int2 *s_edge, const fl
 // filled batch a lane without an element re-reads the row's last element and discards it.
 // HPT > 1: the kernel tile holds HPT heads and the lane's weight is wrow[slot] (its head's staged
 // weights) instead of the word staged next to the column.
-template <int V, int L, int K, bool FULL, int U, bool OFF32, int HPT>
-__device__ __forceinline__ void gather_rows(const int2 *s_edge, const float *wrow, int b, int e, int g, const float *x,
+// dots: with ON, each element's weight is replaced by its dot product once it has been used.
+template <int V, int L, int K, bool FULL, int U, bool OFF32, int HPT, typename DOTS>
+__device__ __forceinline__ void gather_rows(int2 *s_edge, float *wrow, int b, int e, int g, const float *x,
                                             uint32_t lane_bytes, int64_t F, const bool (&on)[K],
-                                            typename Vec<V>::type (&acc)[K]) {
+                                            typename Vec<V>::type (&acc)[K], const DOTS &dots) {
     using vec = typename Vec<V>::type;
     constexpr int G = 64 / L;
     int s0 = b;
@@ -169,10 +215,14 @@ __device__ __forceinline__ void gather_rows(const int2 *s_edge, const float *wro
         for (int u = 0; u < U; ++u)
 #pragma unroll
             for (int k = 0; k < K; ++k)
-                if (FULL || on[k]) vfma(acc[k], __int_as_float(cw[u].y), xv[u][k]);
+                if (FULL || on[k]) {
+                    vfma(acc[k], __int_as_float(cw[u].y), xv[u][k]);
+                    const int j = s0 + u * G + g;
+                    dots.put(threadIdx.x & 63, xv[u][k], true, HPT > 1 ? reinterpret_cast<int32_t *>(wrow + j) : &s_edge[j].y);
+                }
     }
     if (s0 < e)                            // uniform: fewer than G*U elements left
-        gather_tail<V, L, K, FULL, U, OFF32, HPT>((e - s0 + G - 1) / G, s_edge, wrow, s0, e, g, x, lane_bytes, F, on, acc);
+        gather_tail<V, L, K, FULL, U, OFF32, HPT>((e - s0 + G - 1) / G, s_edge, wrow, s0, e, g, x, lane_bytes, F, on, acc, dots);
 }
 
 // Adds the lane groups' sums (group 0 gets the total) and stores one output row; `old` is what
@@ -252,8 +302,9 @@ __device__ __forceinline__ void stage_store_w(float (*rows)[ROW], int lane, cons
 // V: floats per lane per load; L: lanes per source row; K: loads per lane per source row;
 // FULL: every lane's columns are inside the tile (no masking needed); ACC: add to out;
 // OFF32: X spans less than 4 GiB, rows are addressed by 32-bit byte offsets; HPT: heads (with
-// their own weights) per kernel tile, each covered by L / HPT lanes.
-template <int V, int L, int K, bool FULL, bool ACC, bool OFF32, int HPT = 1>
+// their own weights) per kernel tile, each covered by L / HPT lanes; DOT: each element's dot product with the output
+// row's row of `own` as well.
+template <int V, int L, int K, bool FULL, bool ACC, bool OFF32, int HPT = 1, bool DOT = false>
 __device__ __forceinline__ void spmm_items_body(const SpmmArgs &a) {
     using vec = typename Vec<V>::type;
     static_assert(fg::kItemEdges == 256, "stage_load/stage_store move 4 x 64 elements");
@@ -268,13 +319,18 @@ __device__ __forceinline__ void spmm_items_body(const SpmmArgs &a) {
     constexpr int kWRow = HPT > 1 ? fg::kItemEdges + kPad : 1;
     __shared__ __align__(16) float s_w[kWavesPerBlock][HPT][kWRow];
     static_assert(HPT == 1 || (L % HPT == 0 && K == 1 && FULL), "heads of a tile split its lanes evenly");
+    static_assert(!DOT || (V == 4 && K == 1 && FULL && !ACC), "dots: whole tiles of 128-bit lanes, every pass in its own buffer");
 
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int tile = a.tile_base + (int)(blockIdx.x % (unsigned)a.n_ftiles);
     const int64_t item_id = (int64_t)(blockIdx.x / (unsigned)a.n_ftiles) * kWavesPerBlock + wave;
     if (item_id >= a.n_items) return;      // uniform per wavefront; no workgroup barriers below
-    const Item it = a.items[item_id];
+    Item it = a.items[item_id];
+    if (DOT) {                             // the item's fields as scalars: fewer vector registers, scalar loop bounds
+        it.start = __builtin_amdgcn_readfirstlane(it.start); it.len = __builtin_amdgcn_readfirstlane(it.len);
+        it.row = __builtin_amdgcn_readfirstlane(it.row); it.info = __builtin_amdgcn_readfirstlane(it.info);
+    }
     // the partition this item belongs to (uniform per wavefront): selects its position array, its slice of x,
     // its output buffer and its share of the split rows' scratch
     int part = 0;
@@ -301,11 +357,38 @@ __device__ __forceinline__ void spmm_items_body(const SpmmArgs &a) {
     const int64_t voff = (int64_t)((rt * a.tile_w + st * FT) / a.head_len) * a.head_stride;     // head of this kernel tile
     const int64_t F = a.F;
     int2 *edge = s_edge[wave];
-    const float *wrow = s_w[wave][HPT > 1 ? (lane % L) / (L / HPT) : 0];
+    float *wrow = s_w[wave][HPT > 1 ? (lane % L) / (L / HPT) : 0];
     const float *col_vals = HPT > 1 ? nullptr : a.vals;     // HPT > 1: weights are staged per head instead
     vec acc[K], old[K];
     int2 regs[4];
     float wregs[HPT][4];
+    Dots<DOT, L / HPT> dots;
+    // the lane's floats of a row of `own`, in two halves (the load is far from its use); columns that `own` lacks are 0
+    const int own_head = DOT ? f_lo / a.head_len : 0, own_d = DOT ? f_lo - own_head * a.head_len : 0;
+    auto load_own = [&](int64_t row) {
+        if constexpr (DOT) {
+            const float *p = a.own + row * a.own_ld + (int64_t)own_head * a.own_len + own_d;
+            if (own_d + 4 <= a.own_len) {
+                const fg::Words4<float> w = *reinterpret_cast<const fg::Words4<float> *>(p);
+                dots.own = make_float4(w.v[0], w.v[1], w.v[2], w.v[3]);
+            } else {
+                const int left = a.own_len - own_d;
+                dots.own = make_float4(left > 0 ? p[0] : 0.f, left > 1 ? p[1] : 0.f, left > 2 ? p[2] : 0.f, 0.f);
+            }
+        }
+    };
+    // the staged elements' dot products, [0, n) of the staging row, as runs; `first`: element 0's position in the layout
+    auto flush_dots = [&](int64_t first, int n) {
+        if constexpr (DOT) {
+            wave_lds_sync();
+            for (int j = lane; j < n; j += 64) {
+#pragma unroll
+                for (int h = 0; h < HPT; ++h)
+                    __builtin_nontemporal_store(HPT > 1 ? s_w[wave][h][j] : __int_as_float(edge[j].y),
+                                                a.dots + ((int64_t)tile * HPT + h) * a.dots_stride + first + j);
+            }
+        }
+    };
 
     if (it.info < -1) {
         // Several whole rows: stage all their elements once.
@@ -328,6 +411,18 @@ __device__ __forceinline__ void spmm_items_body(const SpmmArgs &a) {
                 touched[i] = out_p[(int64_t)(it.row + r) * F + f];
             }
         }
+        // (the rows of `own` likewise)
+        constexpr int kOwnTouch = DOT ? (fg::kItemRows * kLines + 63) / 64 : 1;
+        float own_touched[kOwnTouch];
+        if constexpr (DOT) {
+#pragma unroll
+            for (int i = 0; i < kOwnTouch; ++i) {
+                const int t = lane + 64 * i;
+                const int f = rt * a.tile_w + st * FT + (t % kLines) * 32, h = f / a.head_len;
+                own_touched[i] = a.own[(int64_t)(it.row + min(t / kLines, nrows - 1)) * a.own_ld + (int64_t)h * a.own_len +
+                                       min(f - h * a.head_len, a.own_len - 1)];
+            }
+        }
         if (it.len > 0) {
             stage_load(a.indices, a.indices16, col_vals, it.start, it.len, lane, scale, a.vstride, voff, regs);
             if (HPT > 1) stage_load_w<HPT>(a.vals, it.start, it.len, lane, a.vstride, voff, a.head_stride, wregs);
@@ -340,6 +435,10 @@ __device__ __forceinline__ void spmm_items_body(const SpmmArgs &a) {
         if (ACC) {
 #pragma unroll
             for (int i = 0; i < kTouch; ++i) asm volatile("" ::"v"(touched[i]));    // keeps the loads
+        }
+        if constexpr (DOT) {
+#pragma unroll
+            for (int i = 0; i < kOwnTouch; ++i) asm volatile("" ::"v"(own_touched[i]));
         }
         if (nrows < 2 * G) {
             // Few, longer rows: all lane groups share each row in turn.
@@ -355,11 +454,13 @@ __device__ __forceinline__ void spmm_items_body(const SpmmArgs &a) {
                     }
 #pragma unroll
                     for (int k = 0; k < K; ++k) acc[k] = vzero(vec());
-                    gather_rows<V, L, K, FULL, U, OFF32, HPT>(edge, wrow, b, e, g, x_p, lane_bytes, F, on, acc);
+                    load_own(it.row + q);
+                    gather_rows<V, L, K, FULL, U, OFF32, HPT>(edge, wrow, b, e, g, x_p, lane_bytes, F, on, acc, dots);
                     finish_row<V, L, K, FULL, ACC>(acc, old, g, on, dst);
                 }
                 b = e;
             }
+            flush_dots(it.start, it.len);
             return;
         }
         // Many short rows: every lane group takes rows of its own (next free row from a counter
@@ -388,6 +489,7 @@ __device__ __forceinline__ void spmm_items_body(const SpmmArgs &a) {
                     j = q ? s_end[wave][q - 1] : 0;
                     e = s_end[wave][q];
                     nonempty = e > j;
+                    load_own(it.row + q);
 #pragma unroll
                     for (int k = 0; k < K; ++k) acc[k] = vzero(vec());
                     if (ACC && nonempty) {
@@ -424,10 +526,12 @@ __device__ __forceinline__ void spmm_items_body(const SpmmArgs &a) {
                             // u == 0 is always the row's own element (j < e)
                             if (u > 0) xv[u][k] = vkeep(j + u < e, xv[u][k]);
                             vfma(acc[k], __int_as_float(cw[u].y), xv[u][k]);
+                            dots.put(lane, xv[u][k], j + u < e, HPT > 1 ? reinterpret_cast<int32_t *>(wrow + j + u) : &edge[j + u].y);
                         }
                 j += U;
             }
         }
+        flush_dots(it.start, it.len);
         return;
     }
 
@@ -435,6 +539,7 @@ __device__ __forceinline__ void spmm_items_body(const SpmmArgs &a) {
     // while the current ones are used
     float *dst = (it.info < 0 ? out_p + (int64_t)it.row * F : partial_p + (int64_t)it.info * a.partial_ld - a.partial_f0) + f_lo;
     const bool add = ACC && it.info < 0;
+    load_own(it.row);
 #pragma unroll
     for (int k = 0; k < K; ++k) acc[k] = vzero(vec());
     if (it.len > 0) {
@@ -459,7 +564,8 @@ __device__ __forceinline__ void spmm_items_body(const SpmmArgs &a) {
                 stage_load_w<HPT>(a.vals, (int64_t)it.start + base + fg::kItemEdges, it.len - base - fg::kItemEdges,
                                   lane, a.vstride, voff, a.head_stride, wregs);
         }
-        gather_rows<V, L, K, FULL, U, OFF32, HPT>(edge, wrow, 0, n, g, x_p, lane_bytes, F, on, acc);
+        gather_rows<V, L, K, FULL, U, OFF32, HPT>(edge, wrow, 0, n, g, x_p, lane_bytes, F, on, acc, dots);
+        flush_dots((int64_t)it.start + base, n);
     }
     finish_row<V, L, K, FULL, ACC>(acc, old, g, on, dst);
 }
@@ -475,6 +581,17 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) 
 template <int V, int L, int K, bool FULL, bool ACC, bool OFF32, int HPT>
 __global__ __launch_bounds__(kBlock) void spmm_items_wide_kernel(const SpmmArgs a) {
     spmm_items_body<V, L, K, FULL, ACC, OFF32, HPT>(a);
+}
+
+// The sum with dots: one gather of a source row serves the row's weighted sum and its dot product with the output row's
+// own vector, which is what the two gradients of a weighted sum need from the transposed graph (dx = A^T dy and
+// dw[e] = <dy[row e], x[col e]>).  Bound as the plain sum is, by the gathers' L2 misses.  58,000 nodes, 12.5 M elements, rows
+// of 602 floats: 1.80 ms and 0.17 ms to add the tiles' parts up, in the place of a sum of 1.47 ms and an SDDMM of 1.72 (whole
+// step 5194 -> 3850 us); 7 wavefronts per SIMD without spills beat 8 with them (step 4172 against 3990 before the last kernel's
+// own gain).
+template <int L, int HPT>
+__global__ __launch_bounds__(kBlock, HPT == 1 ? 7 : 4) void spmm_dot_kernel(const SpmmArgs a) {
+    spmm_items_body<4, L, 1, true, false, true, HPT, true>(a);
 }
 
 // ---- max / min aggregation ------------------------------------------------------------------------
@@ -934,6 +1051,21 @@ int launch_v(const SpmmConfig &c, dim3 grid, hipStream_t st, const SpmmArgs &a) 
     return fail(FG_ERR_SHAPE, "no SpMM kernel for V=%d L=%d K=%d", V, c.L, c.K);
 }
 
+int launch_dot(const SpmmConfig &c, dim3 grid, hipStream_t st, const SpmmArgs &a) {
+    if (c.hpt == 1) {
+        switch (c.L) {
+            case 4: hipLaunchKernelGGL((spmm_dot_kernel<4, 1>), grid, dim3(kBlock), 0, st, a); return FG_OK;
+            case 8: hipLaunchKernelGGL((spmm_dot_kernel<8, 1>), grid, dim3(kBlock), 0, st, a); return FG_OK;
+            case 16: hipLaunchKernelGGL((spmm_dot_kernel<16, 1>), grid, dim3(kBlock), 0, st, a); return FG_OK;
+            case 32: hipLaunchKernelGGL((spmm_dot_kernel<32, 1>), grid, dim3(kBlock), 0, st, a); return FG_OK;
+            case 64: hipLaunchKernelGGL((spmm_dot_kernel<64, 1>), grid, dim3(kBlock), 0, st, a); return FG_OK;
+        }
+    } else if (c.L == 16 && c.hpt == 2) { hipLaunchKernelGGL((spmm_dot_kernel<16, 2>), grid, dim3(kBlock), 0, st, a); return FG_OK; }
+    else if (c.L == 16 && c.hpt == 4) { hipLaunchKernelGGL((spmm_dot_kernel<16, 4>), grid, dim3(kBlock), 0, st, a); return FG_OK; }
+    else if (c.L == 8 && c.hpt == 4) { hipLaunchKernelGGL((spmm_dot_kernel<8, 4>), grid, dim3(kBlock), 0, st, a); return FG_OK; }
+    return fail(FG_ERR_SHAPE, "no SpMM kernel with dots for %d heads per tile with L=%d K=%d", c.hpt, c.L, c.K);
+}
+
 template <int V, int L, int K, bool IS_MAX>
 void launch_ext_vlk(const SpmmConfig &c, dim3 grid, hipStream_t st, const SpmmArgs &a) {
     if (c.full) {
@@ -1039,6 +1171,32 @@ fg::ScratchNeed scratch_need(const fg_spmm_plan *pl, const SpmmConfig &c, int F,
     return need;
 }
 
+// What a sum with dots is asked for besides the sum (SpmmArgs: own, own_ld, own_len); out[pos[element], head].
+struct DotRequest {
+    const float *own;
+    int64_t own_ld;
+    int own_len;
+    float *out;
+    const int32_t *pos;
+};
+// Whether this configuration takes the kernels with dots: whole tiles of 128-bit lanes, one load per lane, 32-bit offsets,
+// a wavefront's own place for every row of every pass, and no tile that cuts a head of several (its parts would have to be
+// added up).  Tiles of several heads keep few wavefronts in flight (104 registers): below 128 floats per row they lose on
+// large graphs what the second gather costs.  Step with both gradients, separate sweeps -> one: 12.5 M elements 4 x 8
+// 790 -> 874 us, 2 x 32 911 -> 957, 8 x 16 1831 -> 1808; 4 M: 357 -> 364, 602 -> 563, 950 -> 840; 400,000: 161 -> 145, 268 -> 191, 168 -> 152.
+bool takes_dots(const fg_spmm_plan *pl, const SpmmConfig &c, int F, int heads) {
+    return c.V == 4 && c.K == 1 && c.full && c.off32 && c.sub_per_tile == 1 &&
+           !(c.hpt > 1 && (c.L < 8 || (F < 128 && pl->nnz >= (4 << 20)))) &&
+           (pl->num_col_partitions == 1 || uses_pass_buffers(pl, c, F, FG_REDUCE_SUM)) &&
+           (heads == 1 || c.tile_w % (F / heads) == 0);
+}
+// Arrays of nnz dot products, one per head or tile, that the kernel leaves in traversal order (written straight to their
+// places from there, single results of a row meet lines that other XCDs are writing too: 58,000 nodes, 12.5 M elements, one
+// 64-float tile, step 722 against 605 us).
+int dot_arrays(const SpmmConfig &c) { return c.n_ftiles * c.hpt; }
+// Floats between them: a multiple of 4, so that a closing kernel's 128-bit loads of every array are aligned.
+size_t dot_stride(const fg_spmm_plan *pl) { return ((size_t)pl->nnz + 3) & ~(size_t)3; }
+
 // Kernel tiles per launch: 8, 4, 2 or 1 -- counts that divide the 8 XCDs, so that workgroup id % tiles-per-launch
 // always puts a tile on the same XCDs and an L2 serves one tile's slice at a time (10 tiles: 8 + 2; 5: 4 + 1).  With
 // any other count every XCD would see every tile (232,965-node graph, F=640: 27.4 ms with 10 tiles in one launch).
@@ -1051,7 +1209,8 @@ int tiles_this_launch(int remaining) {
 int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const float *vals,
              const float *x, float *out, int F, int T, void *stream, int heads = 1,
              int reduce = FG_REDUCE_SUM, bool allow_no_vals = false, bool head_major = false,
-             int32_t *arg_out = nullptr, float *fixed_partial = nullptr, size_t fixed_partial_floats = 0) {
+             int32_t *arg_out = nullptr, float *fixed_partial = nullptr, size_t fixed_partial_floats = 0,
+             const DotRequest *dot = nullptr) {
     if (!pl) return fail(FG_ERR_ARG, "plan is null");
     if (arg_out && reduce == FG_REDUCE_SUM) return fail(FG_ERR_ARG, "positions of the selected elements exist for max / min only");
     if (int drc = fg::check_device(pl)) return drc;
@@ -1065,6 +1224,12 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
     // fixed_partial: the split rows' partial sums go to this buffer of fixed size instead of the plan's,
     // X is gathered from the caller's matrix (no tile-by-tile copy), and nothing is allocated.
     fg::ScratchNeed need = scratch_need(pl, c, F, reduce);
+    // dots: behind everything else that the call keeps in the plan's scratch
+    const size_t dots_at = (need.partial + 3) & ~(size_t)3;
+    if (dot) {
+        if (!takes_dots(pl, c, F, heads)) return fail(FG_ERR_SHAPE, "no sum with dots for %d heads of %d floats on this plan", heads, F / heads);
+        need.partial = dots_at + (size_t)dot_arrays(c) * dot_stride(pl);
+    }
     if (fixed_partial) {
         // the limit counts pieces of 1024 elements; a plan cut finer than that fills the buffer a range of columns at a time
         need.partial = (((size_t)pl->default_pieces * (size_t)F) + 3) & ~(size_t)3;
@@ -1090,6 +1255,15 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
     // at F=512, 6.8 -> 6.1 ms at F=256, before the 0.25 / 0.13 ms that the copy takes); the sums
     // are the same, in the same order.
     const int ft = c.V * c.L * c.K;
+    auto with_dots = [&](SpmmArgs &a) {
+        if (!dot) return;
+        a.own = dot->own; a.own_ld = dot->own_ld; a.own_len = dot->own_len;
+        a.dots = pl->partial_dev + dots_at;
+        a.dots_stride = (int64_t)dot_stride(pl);
+    };
+    auto launch_sum = [&](dim3 grid, const SpmmArgs &a) {
+        return dot ? launch_dot(c, grid, st, a) : c.V == 4 ? launch_v<4>(c, grid, st, a) : launch_v<1>(c, grid, st, a);
+    };
     const bool tiled = need.tiled > 0;
     if (tiled && (rc = fg::make_tile_major(pl, x, pl->n_src, F, ft, stream)) != FG_OK) return rc;
     if (pass_buf && pl->n_items > 0) {
@@ -1110,12 +1284,13 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
         a.heads = heads; a.head_len = F / heads;
         a.vstride = head_major ? 1 : heads; a.head_stride = head_major ? pl->nnz : 1;
         a.accumulate = 0;
+        with_dots(a);
         for (int tb = 0, per_launch; tb < c.n_ftiles; tb += per_launch) {
             per_launch = tiles_this_launch(c.n_ftiles - tb);
             a.n_ftiles = per_launch; a.tile_base = tb;
             const int64_t blocks = ((pl->n_items + kWavesPerBlock - 1) / kWavesPerBlock) * per_launch;
             if (blocks > 0x7fffffffLL) return fail(FG_ERR_SHAPE, "grid of %lld workgroups is too large", (long long)blocks);
-            rc = (c.V == 4) ? launch_v<4>(c, dim3((unsigned)blocks), st, a) : launch_v<1>(c, dim3((unsigned)blocks), st, a);
+            rc = launch_sum(dim3((unsigned)blocks), a);
             if (rc != FG_OK) return rc;
         }
     }
@@ -1154,6 +1329,7 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
             a.heads = heads; a.head_len = F / heads;
             a.vstride = head_major ? 1 : heads; a.head_stride = head_major ? pl->nnz : 1;
             a.accumulate = p > 0;
+            with_dots(a);
             // More than 8 tiles: 8 at a time (one per XCD), so that an XCD's L2 serves one tile's
             // slice of this partition per launch; the partition's index arrays stay in the
             // memory-side cache between the launches.
@@ -1163,7 +1339,7 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
                 const int64_t blocks = ((i1 - i0 + kWavesPerBlock - 1) / kWavesPerBlock) * per_launch;
                 if (blocks > 0x7fffffffLL) return fail(FG_ERR_SHAPE, "grid of %lld workgroups is too large", (long long)blocks);
                 const dim3 grid((unsigned)blocks);
-                if (reduce == FG_REDUCE_SUM) rc = (c.V == 4) ? launch_v<4>(c, grid, st, a) : launch_v<1>(c, grid, st, a);
+                if (reduce == FG_REDUCE_SUM) rc = launch_sum(grid, a);
                 else if (reduce == FG_REDUCE_MAX) rc = (c.V == 4) ? launch_ext_v<4, true>(c, grid, st, a) : launch_ext_v<1, true>(c, grid, st, a);
                 else rc = (c.V == 4) ? launch_ext_v<4, false>(c, grid, st, a) : launch_ext_v<1, false>(c, grid, st, a);
                 if (rc != FG_OK) return rc;
@@ -1192,6 +1368,10 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
         const size_t words = pass_stride / 4;
         hipLaunchKernelGGL(spmm_pass_sum_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st,
                            reinterpret_cast<const float4 *>(pass_buf), reinterpret_cast<float4 *>(out), words, P);
+    }
+    if (dot && pl->nnz > 0) {
+        if (heads == 1) fg::sum_tiles(pl->partial_dev + dots_at, dot->pos, dot->out, pl->nnz, (int64_t)dot_stride(pl), c.n_ftiles, stream);
+        else fg::gather_heads(pl->partial_dev + dots_at, dot->pos, dot->out, pl->nnz, (int64_t)dot_stride(pl), heads, stream);
     }
     if (arg_out) {
         // second sweep over the same items: which element equals the extreme that was just written
@@ -1326,6 +1506,26 @@ extern "C" int fg_gspmm_f32(fg_spmm_plan *plan, const int32_t *pos_dev, const in
                     reduce, /*allow_no_vals=*/true, vals_head_major != 0);
 }
 
+extern "C" int fg_spmm_dot_takes(const fg_spmm_plan *plan, int F, int heads, int num_feat_partitions) {
+    SpmmConfig c;
+    if (!plan || resolve_config(plan, F, num_feat_partitions, heads, FG_REDUCE_SUM, true, &c) != FG_OK) return 0;
+    return takes_dots(plan, c, F, heads) ? 1 : 0;
+}
+
+extern "C" int fg_spmm_dot_f32(fg_spmm_plan *plan, const int32_t *pos_dev, const int32_t *idx_dev, const float *vals_dev,
+                               const float *x_dev, const float *own_dev, int own_len, float *out_dev,
+                               const int32_t *edge_pos_dev, float *dots_dev, int F, int heads, int vals_head_major,
+                               int num_feat_partitions, void *stream) {
+    if (!plan) return fail(FG_ERR_ARG, "plan is null");
+    if (heads < 1 || F < 1 || F % heads != 0) return fail(FG_ERR_SHAPE, "feature length %d is not divisible by %d heads", F, heads);
+    if (own_len < 1 || own_len > F / heads) return fail(FG_ERR_SHAPE, "heads of %d floats in own, of %d in x", own_len, F / heads);
+    if (plan->n_dst > 0 && plan->nnz > 0 && (!own_dev || !edge_pos_dev || !dots_dev)) return fail(FG_ERR_ARG, "null device pointer");
+    if (((uintptr_t)edge_pos_dev & 15) != 0) return fail(FG_ERR_ARG, "the positions of the dots must be 16-byte aligned");
+    const DotRequest dot = {own_dev, (int64_t)heads * own_len, own_len, dots_dev, edge_pos_dev};
+    return spmm_run(plan, pos_dev, idx_dev, vals_dev, x_dev, out_dev, F, num_feat_partitions, stream, heads, FG_REDUCE_SUM,
+                    /*allow_no_vals=*/false, vals_head_major != 0, nullptr, nullptr, 0, &dot);
+}
+
 extern "C" int fg_gspmm_arg_f32(fg_spmm_plan *plan, const int32_t *indptr_dev, const int32_t *indices_dev,
                                 const float *vals_dev, const float *x_dev, float *out_dev, int32_t *arg_dev, int F,
                                 int heads, int vals_head_major, int reduce, int num_feat_partitions, void *stream) {
@@ -1339,7 +1539,7 @@ namespace {
 // heads are read together and written to the heads' own contiguous arrays.
 __global__ __launch_bounds__(256) void edge_values_head_major_kernel(const float *src, const int32_t *pos,
                                                                      int64_t n, int H, float *dst) {
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t e = (int64_t)fg::xcd_contiguous_block() * blockDim.x + threadIdx.x;
     if (e >= n) return;
     const float *s = src + (pos ? (int64_t)pos[e] : e) * H;
     for (int h = 0; h < H; ++h) dst[(int64_t)h * n + e] = s[h];
@@ -1347,11 +1547,14 @@ __global__ __launch_bounds__(256) void edge_values_head_major_kernel(const float
 // One head, weights in another order: dst[e] = src[pos[e]], four consecutive elements per lane (their positions by one
 // 128-bit load, the results by one 128-bit store; pos and dst 16-byte aligned).
 __global__ __launch_bounds__(256) void edge_values_permute_kernel(const float *src, const int32_t *pos, int64_t n, float *dst) {
-    const int64_t e = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+    const int64_t e = ((int64_t)fg::xcd_contiguous_block() * blockDim.x + threadIdx.x) * 4;
     if (e >= n) return;
     if (e + 4 <= n) {
-        const int4 p = *reinterpret_cast<const int4 *>(pos + e);
-        *reinterpret_cast<float4 *>(dst + e) = make_float4(src[p.x], src[p.y], src[p.z], src[p.w]);
+        typedef int i4 __attribute__((ext_vector_type(4)));
+        typedef float f4 __attribute__((ext_vector_type(4)));
+        const i4 p = __builtin_nontemporal_load(reinterpret_cast<const i4 *>(pos + e));
+        f4 v; v.x = src[p.x]; v.y = src[p.y]; v.z = src[p.z]; v.w = src[p.w];
+        __builtin_nontemporal_store(v, reinterpret_cast<f4 *>(dst + e));
     } else {
         for (int64_t i = e; i < n; ++i) dst[i] = src[pos[i]];
     }
@@ -1362,7 +1565,7 @@ template <int Q>
 __global__ __launch_bounds__(256) void edge_values_head_major_vec_kernel(const float *src, const int32_t *pos,
                                                                          int64_t n, float *dst) {
     constexpr int H = 4 * Q;
-    const int64_t e0 = (int64_t)blockIdx.x * 512 + threadIdx.x;
+    const int64_t e0 = (int64_t)fg::xcd_contiguous_block() * 512 + threadIdx.x;
     float4 v[2][Q];
     bool ok[2];
 #pragma unroll

@@ -354,6 +354,37 @@ class GSpMMhip(VanillaSpMMhip):
         if out is not self.out_tvm:
             self.out_tvm.copy_(out[..., :self._pad_from])
 
+    def run_with_dots(self, src_feat, weights, own):
+        """run([src_feat, weights]) and, in the same sweep, dots[e, h] = <own[row e, h, :], src_feat[col e, h, :]> per edge in
+        the order of the weights given (set_weight_order) -- the two gradients of a weighted sum over the transposed graph.
+        Returns (self.out_tvm, dots), or None where the library has no kernel for both (fg_spmm_dot_takes)."""
+        if self._func is None:
+            raise RuntimeError("call build() before run_with_dots()")
+        if self._bop is not None or not self._weights_at_run or self._reduce != 'sum':
+            return None
+        lay = self._active
+        pos = self._given_pos(lay)
+        if pos is None or any(t.data_ptr() % 16 for t in (src_feat, pos)) \
+                or not _lib.lib().fg_spmm_dot_takes(lay['plan'], self._feat_len, self._heads, self._num_feat_partitions):
+            return None
+        common.ensure_output(self)
+        own_ph = common.placeholder((self._num_rows,) + tuple(src_feat.shape[1:]))
+        common.check_inputs([src_feat, weights, own], self._placeholders + [own_ph], self._ctx)
+        w, head_major = self._weights(weights)
+        self._w_keepalive = w
+        dots = torch.empty_like(weights)
+        out = self.out_tvm
+        if self._pad_from is not None:
+            self._x_pad[..., :self._pad_from].copy_(src_feat)
+            src_feat, out = self._x_pad, self._out_pad
+        _lib.check(_lib.lib().fg_spmm_dot_f32(
+            lay['plan'], _lib.dev_ptr(lay['pos']), _lib.dev_ptr(lay['idx']), _lib.dev_ptr(w), _lib.dev_ptr(src_feat), _lib.dev_ptr(own),
+            own.shape[-1], _lib.dev_ptr(out), _lib.dev_ptr(pos), _lib.dev_ptr(dots), self._feat_len, self._heads, head_major,
+            self._num_feat_partitions, common.stream_ptr()))
+        if out is not self.out_tvm:
+            self.out_tvm.copy_(out[..., :self._pad_from])
+        return self.out_tvm, dots
+
     def run(self, input_tvm_ndarrays):
         """[SrcFeat] or [SrcFeat, edge_weights]; returns self.out_tvm (overwritten in place)."""
         if self._func is None:

@@ -230,6 +230,19 @@ int fg_gspmm_f32(fg_spmm_plan *plan, const int32_t *pos_dev, const int32_t *idx_
                  int vals_head_major, int reduce, int num_feat_partitions, void *stream);
 
 /*
+ * The two gradients of a weighted sum y[r] = sum over e of w[e] * x[col e] in one sweep over the TRANSPOSED adjacency (its
+ * rows are y's sources; no counterpart in the reference): out as fg_gspmm_f32 (sum) with x_dev = dL/dy, and
+ *   dots[edge_pos[t], h] = <own[row of element t, h, :], x[idx[t], h, :]>
+ * for every element t of the layout, own_dev [n_dst, heads, own_len] (own_len <= F / heads; columns of x beyond it count
+ * as zeros of own).  fg_spmm_dot_takes says whether this plan and shape do (arrays 16-byte aligned): whole tiles of 16 to 256
+ * floats, X below 4 GiB, and with several partitions every pass in a buffer of its own.
+ */
+int fg_spmm_dot_takes(const fg_spmm_plan *plan, int F, int heads, int num_feat_partitions);
+int fg_spmm_dot_f32(fg_spmm_plan *plan, const int32_t *pos_dev, const int32_t *idx_dev, const float *vals_dev,
+                    const float *x_dev, const float *own_dev, int own_len, float *out_dev, const int32_t *edge_pos_dev,
+                    float *dots_dev, int F, int heads, int vals_head_major, int num_feat_partitions, void *stream);
+
+/*
  * fg_gspmm_f32 with FG_REDUCE_MAX / FG_REDUCE_MIN that also reports which element was selected (no
  * counterpart in the reference; what the gradient of a max / min aggregation needs):
  * arg_dev[v, f] = position in the CSR element order of the first element of row v whose message
