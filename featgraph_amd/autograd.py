@@ -9,6 +9,8 @@ so `Graph` keeps plans for the adjacency in CSR order and for its transpose, and
 between the two edge orders.  The reference has no autograd layer; this is the consumer-side API
 its README (README.md:13-14, DGL integration) points at.
 """
+import weakref
+
 import numpy as np
 import scipy.sparse
 import torch
@@ -172,8 +174,8 @@ class Graph(object):
     def attention(self, q, k, v, scale=None):
         """out[r, h, :] = sum over the edges e into r of softmax_r(scale * <k[col e, h, :], q[r, h, :]>) * v[col e, h, :];
         q (num_rows, H, D), k and v (num_cols, H, D), scale 1 / sqrt(D) unless given.  With D in {16, 32, 64}
-        this is one operator that stores no scores, and its backward pass forms them again (two sweeps, one
-        of them over the transposed adjacency); otherwise the differentiable chain sddmm -> edge_softmax ->
+        this is one operator that stores no scores, and its backward pass forms them again (a sweep over the transposed
+        adjacency, and a second one or a weighted sum over the adjacency); otherwise the differentiable chain sddmm -> edge_softmax ->
         spmm."""
         if scale is None:
             scale = 1.0 / float(q.shape[-1]) ** 0.5
@@ -203,6 +205,8 @@ class Graph(object):
             m = GraphAttentionhip(self._csr)
             m.build([placeholder(tuple(q.shape)), placeholder(tuple(k.shape)), placeholder(tuple(v.shape))],
                     {'scale': scale}, {})
+            graph = weakref.ref(self)           # no cycle: a Graph's device memory goes when its last user does
+            m._new_sum = lambda: graph()._gspmm_module(False)
             self._mods[key] = m
         return self._mods[key]
 

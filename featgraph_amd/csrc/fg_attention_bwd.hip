@@ -1,4 +1,4 @@
-// Gradients of the graph attention operator (fg_attention.hip), without any [nnz, H] array.
+// Gradients of the graph attention operator (fg_attention.hip).
 //
 // With s[e, h] = scale * <K[c, h, :], Q[r, h, :]>, a[e, h] = exp(s - m[r, h]) / l[r, h] (m, l: the row's
 // maximum and sum of exponentials, kept by the forward pass) and out[r, h, :] = sum_e a * V[c, h, :]:
@@ -10,7 +10,8 @@
 //                                                            traversal of the transposed adjacency)
 //
 // Both kernels form s again from Q and K, read (m + log l, delta) per row and head, and gather two
-// operands per edge, as the forward pass does.  Not in the reference.
+// operands per edge, as the forward pass does.  The kernel by column can leave scale * ds of every edge and head behind:
+// dQ is then a weighted sum that gathers K alone (fg_gspmm_f32), and the kernel by row is not needed.  Not in the reference.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -67,6 +68,8 @@ struct BwdArgs {
     const float *coef;        // [H, n_dst, 2]: (m + log l, delta), head by head; BY_COLUMN: offset to the partition's first far row
     int64_t coef_head_floats; // floats from one head's block of coef to the next (2 * n_dst)
     float *res0, *res1;       // [n_own, F]: dQ, or dK and dV
+    float *ds = nullptr;      // BY_COLUMN: scale * ds of every element, head by head (null: not kept)
+    int64_t ds_head_floats = 0;
     int F, H;
     int n_heads, head_base;
     float scale;
@@ -112,8 +115,27 @@ __global__ __launch_bounds__(kBlock) void attention_backward_kernel(const BwdArg
         if (lane < kPad) far[fg::kItemEdges + lane] = w[3];
     };
 
-    // NU staged elements of one row, those with ok[u] counted: all gathers are issued before the first is used.
-    auto apply = [&](auto nu_tag, const auto &w, const auto &ok, const float4 &o0, const float4 &o1, float c1, float delta,
+    // The element's own slot in LDS, whose last word is free, carries its scale * ds from the lane group that formed it to
+    // flush(), which writes the stage's values as one run per head (as the kernel's registers had them; nothing crosses
+    // wavefronts).
+    auto keep_ds = [&](int slot, float ds) {
+        if constexpr (BY_COLUMN) { if (li == 0) far[slot].w = __float_as_int(ds * a.scale); }
+    };
+    auto flush = [&](int64_t base, int n) {
+        if constexpr (BY_COLUMN) {
+            if (!a.ds) return;
+            wave_lds_sync();
+            float *d = a.ds + (int64_t)head * a.ds_head_floats + base;
+#pragma unroll
+            for (int i = 0; i < fg::kItemEdges / 64; ++i) {
+                const int at = lane + 64 * i;
+                if (at < n) d[at] = __int_as_float(far[at].w);
+            }
+        }
+    };
+
+    // NU staged elements of one row (in slots at[u]), those with ok[u] counted: all gathers are issued before the first is used.
+    auto apply = [&](auto nu_tag, const auto &w, const auto &at, const auto &ok, const float4 &o0, const float4 &o1, float c1, float delta,
                      float4 &accA, float4 &accB) {
         constexpr int NU = decltype(nu_tag)::value;
         float4 f0[NU], f1[NU];
@@ -138,6 +160,7 @@ __global__ __launch_bounds__(kBlock) void attention_backward_kernel(const BwdArg
                 f0[u] = zero4();
                 f1[u] = zero4();
             }
+            if (ok[u]) keep_ds(at[u], ds);
             if (BY_COLUMN) { fma4(accA, ds, f0[u]); fma4(accB, p, f1[u]); }     // dK += ds * Q[r], dV += a * dout[r]
             else fma4(accA, ds, f0[u]);                                         // dQ += ds * K[c]
         }
@@ -150,13 +173,15 @@ __global__ __launch_bounds__(kBlock) void attention_backward_kernel(const BwdArg
         constexpr bool ALLVALID = decltype(allvalid_tag)::value;
         const bool last_valid = ALLVALID || s0 + (NU - 1) * G + g < e;
         W w[NU];
+        int at[NU];
         bool ok[NU];
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
             ok[u] = u < NU - 1 || last_valid;
-            w[u] = far[ok[u] ? s0 + u * G + g : e - 1];
+            at[u] = ok[u] ? s0 + u * G + g : e - 1;
+            w[u] = far[at[u]];
         }
-        apply(nu_tag, w, ok, o0, o1, c1, delta, accA, accB);
+        apply(nu_tag, w, at, ok, o0, o1, c1, delta, accA, accB);
     };
     auto walk = [&](int b, int e, const float4 &o0, const float4 &o1, float c1, float delta, float4 &accA, float4 &accB) {
         using std::integral_constant;
@@ -255,13 +280,15 @@ __global__ __launch_bounds__(kBlock) void attention_backward_kernel(const BwdArg
                 if (j < e) {
                     // slots beyond e hold later rows' elements or the padding: loadable, discarded
                     W w[KU];
+                    int at[KU];
                     bool ok[KU];
 #pragma unroll
-                    for (int u = 0; u < KU; ++u) { w[u] = far[j + u]; ok[u] = j + u < e; }
-                    apply(std::integral_constant<int, KU>(), w, ok, o0, o1, c1, delta, accA, accB);
+                    for (int u = 0; u < KU; ++u) { at[u] = j + u; w[u] = far[at[u]]; ok[u] = j + u < e; }
+                    apply(std::integral_constant<int, KU>(), w, at, ok, o0, o1, c1, delta, accA, accB);
                     j += KU;
                 }
             }
+            flush(it.start, it.len);
             return;
         }
         int b = 0;
@@ -275,6 +302,7 @@ __global__ __launch_bounds__(kBlock) void attention_backward_kernel(const BwdArg
             }
             b = e;
         }
+        flush(it.start, it.len);
         return;
     }
     // one row of any length: 256 elements at a time
@@ -286,6 +314,7 @@ __global__ __launch_bounds__(kBlock) void attention_backward_kernel(const BwdArg
         stage((int64_t)it.start + base, n);
         wave_lds_sync();
         walk(0, n, o0, o1, c1, delta, accA, accB);
+        flush((int64_t)it.start + base, n);
     }
     if (it.len > 0 || !ACC) finish(it.row, accA, accB, oldA, oldB);
 }
@@ -335,7 +364,7 @@ int check_common(const fg_spmm_plan *pl, int heads, int head_len, int64_t n_far_
 template <bool BY_COLUMN>
 int run_backward(fg_spmm_plan *pl, const int32_t *pos_dev, const int32_t *idx_dev, const float *own0,
                  const float *own1, const float *far0_dev, const float *far1_dev, const float *coef_dev,
-                 float *res0, float *res1, int heads, int head_len, float scale, void *stream) {
+                 float *res0, float *res1, int heads, int head_len, float scale, void *stream, float *ds = nullptr) {
     const int F = heads * head_len;
     hipStream_t st = (hipStream_t)stream;
     const int P = pl->num_col_partitions;
@@ -366,6 +395,7 @@ int run_backward(fg_spmm_plan *pl, const int32_t *pos_dev, const int32_t *idx_de
         a.far_tile_bytes = tiled ? (uint32_t)((uint64_t)pl->n_src * head_len * 4u) : 0u;
         a.coef = BY_COLUMN ? coef_dev + (int64_t)p * width * 2 : coef_dev;
         a.coef_head_floats = 2 * (BY_COLUMN ? pl->n_src : pl->n_dst);
+        a.ds = ds; a.ds_head_floats = pl->nnz;
         a.res0 = res0; a.res1 = res1; a.F = F; a.H = heads; a.scale = scale;
         const int per_launch = (heads > 8 && heads % 8 == 0) ? 8 : heads;
         for (int hb = 0; hb < heads; hb += per_launch) {
@@ -424,18 +454,35 @@ extern "C" int fg_graph_attention_backward_q_f32(fg_spmm_plan *pl, const int32_t
                                heads, head_len, scale, stream);
 }
 
-extern "C" int fg_graph_attention_backward_kv_f32(fg_spmm_plan *pl, const int32_t *pos_t_dev, const int32_t *idx_t_dev,
-                                                  const float *q_dev, const float *dout_dev, const float *k_dev,
-                                                  const float *v_dev, const float *row_coef_dev, float *dk_dev,
-                                                  float *dv_dev, int heads, int head_len, float scale, void *stream) {
+static int backward_kv(fg_spmm_plan *pl, const int32_t *pos_t_dev, const int32_t *idx_t_dev, const float *q_dev, const float *dout_dev,
+                       const float *k_dev, const float *v_dev, const float *row_coef_dev, float *dk_dev, float *dv_dev, bool want_ds,
+                       float *ds_dev, int heads, int head_len, float scale, void *stream) {
     if (pl == nullptr) return fail(FG_ERR_ARG, "plan is null");
     if (int rc = check_common(pl, heads, head_len, pl->n_src)) return rc;
     if (pl->n_dst == 0) return FG_OK;
     if (!pos_t_dev || !k_dev || !v_dev || !dk_dev || !dv_dev || (pl->nnz > 0 && (!idx_t_dev || !q_dev || !dout_dev || !row_coef_dev)))
         return fail(FG_ERR_ARG, "null device pointer");
+    if (want_ds && pl->nnz > 0 && !ds_dev) return fail(FG_ERR_ARG, "null device pointer");
     if ((((uintptr_t)q_dev | (uintptr_t)k_dev | (uintptr_t)v_dev | (uintptr_t)dout_dev | (uintptr_t)dk_dev | (uintptr_t)dv_dev) & 15) != 0 ||
         ((uintptr_t)row_coef_dev & 7) != 0)
         return fail(FG_ERR_ARG, "attention needs 16-byte aligned arrays");
     return run_backward<true>(pl, pos_t_dev, idx_t_dev, k_dev, v_dev, q_dev, dout_dev, row_coef_dev, dk_dev, dv_dev,
-                              heads, head_len, scale, stream);
+                              heads, head_len, scale, stream, ds_dev);
+}
+
+extern "C" int fg_graph_attention_backward_kv_f32(fg_spmm_plan *pl, const int32_t *pos_t_dev, const int32_t *idx_t_dev,
+                                                  const float *q_dev, const float *dout_dev, const float *k_dev,
+                                                  const float *v_dev, const float *row_coef_dev, float *dk_dev,
+                                                  float *dv_dev, int heads, int head_len, float scale, void *stream) {
+    return backward_kv(pl, pos_t_dev, idx_t_dev, q_dev, dout_dev, k_dev, v_dev, row_coef_dev, dk_dev, dv_dev, false, nullptr,
+                       heads, head_len, scale, stream);
+}
+
+extern "C" int fg_graph_attention_backward_kv_ds_f32(fg_spmm_plan *pl, const int32_t *pos_t_dev, const int32_t *idx_t_dev,
+                                                     const float *q_dev, const float *dout_dev, const float *k_dev,
+                                                     const float *v_dev, const float *row_coef_dev, float *dk_dev,
+                                                     float *dv_dev, float *ds_dev, int heads, int head_len, float scale,
+                                                     void *stream) {
+    return backward_kv(pl, pos_t_dev, idx_t_dev, q_dev, dout_dev, k_dev, v_dev, row_coef_dev, dk_dev, dv_dev, true, ds_dev,
+                       heads, head_len, scale, stream);
 }

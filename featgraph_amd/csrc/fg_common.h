@@ -109,7 +109,8 @@ int make_tile_major(const fg_spmm_plan *plan, const float *x, int64_t n_rows, in
 // rewritten or replaced at the same address is then read as int32 and the mismatch is left in fg_last_error().
 const uint16_t *narrow_indices(const fg_spmm_plan *plan, const int32_t *idx);
 // out[edge_pos[e]] = sum over the n_tiles arrays `stride` floats apart (a multiple of 4, 16-byte aligned) of array[e], and
-// out[edge_pos[e] * H + h] = array h's [e], for all n_edges elements, on `stream` (edge_pos 16-byte aligned).
+// out[edge_pos[e] * H + h] = array h's [e], for all n_edges elements, on `stream` (edge_pos 16-byte aligned; gather_heads with
+// H % 4 == 0 and a 16-byte aligned out also takes nullptr: out[e * H + h]).
 void sum_tiles(const float *partial, const int32_t *edge_pos, float *out, int64_t n_edges, int64_t stride, int n_tiles, void *stream);
 void gather_heads(const float *staged, const int32_t *edge_pos, float *out, int64_t n_edges, int64_t stride, int H, void *stream);
 // Looks up, once per device, the address of the fixed array that fg_spmm_csr_noalloc_f32 keeps its partial sums in.

@@ -623,7 +623,8 @@ __global__ __launch_bounds__(256) void sddmm_tile_heads_kernel(const float *stag
 // each of their tiles' arrays, and one 128-bit store), and consecutive lanes take an edge's groups of four and then the
 // next edge's, so that a wavefront reads runs of consecutive edges from each tile's array and writes whole runs of H
 // floats per edge.  232,965-node graph, H=8, D=64: 2.3 ms with one thread per edge and scalar stores (3.4 TB/s), 1.5 ms
-// this way (5.2 TB/s); plain loads (non-temporal ones: +0.2 ms), one edge group per lane (four: no change).
+// this way (5.2 TB/s); plain loads (non-temporal ones: +0.2 ms), one edge group per lane (four: no change).  edge_pos == nullptr:
+// every edge at its place in the traversal.
 __global__ __launch_bounds__(256) void sddmm_tile_heads_vec_kernel(const float *staged, const int32_t *edge_pos,
                                                                    float *out, int64_t n_edges, int64_t tile_stride, int H) {
     typedef float f4 __attribute__((ext_vector_type(4)));
@@ -638,7 +639,7 @@ __global__ __launch_bounds__(256) void sddmm_tile_heads_vec_kernel(const float *
     v.y = s[tile_stride];
     v.z = s[2 * tile_stride];
     v.w = s[3 * tile_stride];
-    *reinterpret_cast<f4 *>(out + (int64_t)edge_pos[e] * H + 4 * q) = v;
+    *reinterpret_cast<f4 *>(out + (edge_pos ? (int64_t)edge_pos[e] : e) * H + 4 * q) = v;
 }
 
 template <int L, int K, int RW, int KH, bool SCATTER>

@@ -1,15 +1,18 @@
 """Dot-product attention over a graph's edges in one operator: multi-head SDDMM, edge softmax and per-head
-weighted SpMM without the [nnz, H] scores ever being stored.  The reference has no such operator; the
+weighted SpMM without the [nnz, H] scores being stored (the gradients of larger calls keep the scores' gradients for a
+while: tuning.attention_keeps_score_gradients).  The reference has no such operator; the
 class follows the build()/run() conventions of its modules (python/featgraph/module/spmm.py:81-161)."""
 import ctypes
 
 import numpy as np
+import scipy.sparse
 import torch
 
 from .. import _lib
 from .. import tuning
 from ..util import util_convert_csr_to_dds
 from . import common
+from .gspmm import GSpMMhip
 
 _INT32_MAX = 2 ** 31 - 1
 
@@ -37,6 +40,9 @@ class GraphAttentionhip(object):
                                                 _lib.host_ptr(self._indices)))
         self._csr = csr
         self._layouts = {}
+        self._sum = None
+        # where the weighted sum of backward() comes from (a Graph gives one that shares its layouts)
+        self._new_sum = lambda: GSpMMhip(scipy.sparse.csr_matrix((np.ones(csr.nnz, np.float32), csr.indices, csr.indptr), shape=csr.shape))
         self._placeholders = None
         self.out_tvm = None
 
@@ -104,6 +110,9 @@ class GraphAttentionhip(object):
         # every row's maximum score and sum of exponentials, per head: what backward() starts from
         self.state_tvm = torch.zeros((self._num_rows, heads, 2), dtype=torch.float32, device=self._ctx)
         self._coef = None
+        self._sum = None
+        for lay in self._layouts.values():
+            lay.pop('sum_position', None)
 
     def _partitions(self, schedule_args, slice_row_bytes):
         """Source partitions: one head per XCD, whose L2 holds the head's slices of the gathered operands."""
@@ -174,12 +183,13 @@ class GraphAttentionhip(object):
         key = ('t', P)
         if key in self._layouts:
             return self._layouts[key]
-        tr = self._csr.T.tocsr()
+        nnz = self._indices.shape[0]
+        tr = scipy.sparse.csr_matrix((np.arange(nnz, dtype=np.int32), self._indices, self._indptr), shape=self._csr.shape).T.tocsr()
         tr.sort_indices()
         if P > 1:
-            pos, idx, _ = util_convert_csr_to_dds(tr, P)
+            pos, idx, csr_pos = util_convert_csr_to_dds(tr, P)
         else:
-            pos, idx = tr.indptr, tr.indices
+            pos, idx, csr_pos = tr.indptr, tr.indices, tr.data
         pos = np.ascontiguousarray(pos, dtype=np.int32)
         lay = {'P': P, 'pos': common.to_device_i32(pos, self._ctx),
                'idx': common.to_device_i32(np.ascontiguousarray(idx, dtype=np.int32), self._ctx), 'plan': ctypes.c_void_p()}
@@ -191,14 +201,16 @@ class GraphAttentionhip(object):
             _lib.check(_lib.lib().fg_spmm_plan_create(_lib.host_ptr(pos), self._num_cols, self._num_rows, P,
                                                       ctypes.byref(opts), ctypes.byref(lay['plan'])))
         common.narrow_indices(lay['plan'], lay['idx'], self._num_rows, P, self._ctx)      # the transposed graph gathers from the rows
+        lay['csr_pos_host'] = csr_pos
         self._layouts[key] = lay
         return lay
 
     def backward(self, q, k, v, out, state, grad_out):
         """(dQ, dK, dV) for dL/d(out) = grad_out, given the inputs, the output and the row state
         (out_tvm / state_tvm as they were after run() on these inputs).  The scores are formed again from Q
-        and K; dQ comes from a sweep like the forward pass, dK and dV from the same sweep over the
-        transposed adjacency.  Returns new tensors."""
+        and K; dK and dV come from a sweep like the forward pass over the transposed adjacency, dQ from a weighted sum
+        with the scores' gradients that this sweep leaves (two arrays of nnz * H floats while the call lasts), or, where
+        that does not pay or the arrays would not fit, from a sweep of its own over the adjacency.  Returns new tensors."""
         if self._placeholders is None:
             raise RuntimeError("call build() before backward()")
         common.check_inputs([q, k, v], self._placeholders, self._ctx)
@@ -210,20 +222,56 @@ class GraphAttentionhip(object):
         _lib.check(L.fg_graph_attention_coef_f32(_lib.dev_ptr(out), _lib.dev_ptr(grad_out), _lib.dev_ptr(state),
                                                  _lib.dev_ptr(coef), self._num_rows, self._heads, self._head_len, s))
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-        lay = self._active
-        _lib.check(L.fg_graph_attention_backward_q_f32(lay['plan'], _lib.dev_ptr(lay['pos']), _lib.dev_ptr(lay['idx']),
-                                                       _lib.dev_ptr(q), _lib.dev_ptr(k), _lib.dev_ptr(v),
-                                                       _lib.dev_ptr(grad_out), _lib.dev_ptr(coef), _lib.dev_ptr(dq),
-                                                       self._heads, self._head_len, ctypes.c_float(self._scale), s))
         # partitions over the destinations, sized like the forward pass's over the sources
         lt = self._layout_t(self._dst_partitions(2 * 4 * self._head_len))
-        _lib.check(L.fg_graph_attention_backward_kv_f32(lt['plan'], _lib.dev_ptr(lt['pos']), _lib.dev_ptr(lt['idx']),
-                                                        _lib.dev_ptr(q), _lib.dev_ptr(grad_out), _lib.dev_ptr(k),
-                                                        _lib.dev_ptr(v), _lib.dev_ptr(coef), _lib.dev_ptr(dk),
-                                                        _lib.dev_ptr(dv), self._heads, self._head_len,
-                                                        ctypes.c_float(self._scale), s))
+        kv = (lt['plan'], _lib.dev_ptr(lt['pos']), _lib.dev_ptr(lt['idx']), _lib.dev_ptr(q), _lib.dev_ptr(grad_out),
+              _lib.dev_ptr(k), _lib.dev_ptr(v), _lib.dev_ptr(coef), _lib.dev_ptr(dk), _lib.dev_ptr(dv))
+        tail = (self._heads, self._head_len, ctypes.c_float(self._scale), s)
+        edges = self._edge_buffers()
+        if edges is not None:
+            total, position = self._query_sum(lt)
+            ds, other = edges
+            _lib.check(L.fg_graph_attention_backward_kv_ds_f32(*kv, _lib.dev_ptr(ds), *tail))
+            result = ctypes.c_void_p()
+            _lib.check(L.fg_edge_values_permute_f32(_lib.dev_ptr(ds), _lib.dev_ptr(position), ds.shape[1], self._heads,
+                                                    _lib.dev_ptr(other), ctypes.byref(result), s))
+            flat = total._placeholders[0].shape
+            total.run_laid_out(k.view(flat), ds if result.value == ds.data_ptr() else other, dq.view((self._num_rows,) + flat[1:]))
+        else:
+            lay = self._active
+            _lib.check(L.fg_graph_attention_backward_q_f32(lay['plan'], _lib.dev_ptr(lay['pos']), _lib.dev_ptr(lay['idx']),
+                                                           _lib.dev_ptr(q), _lib.dev_ptr(k), _lib.dev_ptr(v),
+                                                           _lib.dev_ptr(grad_out), _lib.dev_ptr(coef), _lib.dev_ptr(dq), *tail))
+            _lib.check(L.fg_graph_attention_backward_kv_f32(*kv, *tail))
         self._coef = coef
         return dq, dk, dv
+
+    def _edge_buffers(self):
+        """Two (H, nnz) arrays for the scores' gradients, or None where dQ is to come from a sweep of its own."""
+        nnz = self._indices.shape[0]
+        if not tuning.attention_keeps_score_gradients(nnz, self._num_rows, self._heads, self._head_len):
+            return None
+        try:
+            return tuple(torch.empty((2, self._heads, nnz), dtype=torch.float32, device=self._ctx))
+        except torch.cuda.OutOfMemoryError:
+            return None
+
+    def _query_sum(self, lt):
+        """(weighted sum over the adjacency with H heads, position in lt's element order of each element of its layout)."""
+        if self._sum is None:
+            total = self._new_sum()
+            H, D, nnz = self._heads, self._head_len, self._indices.shape[0]
+            total.build([common.placeholder((self._num_cols,) + ((D,) if H == 1 else (H, D))),
+                         common.placeholder((nnz,) if H == 1 else (nnz, H))], {}, {})
+            total.out_tvm = None                    # its results go to tensors of backward()'s own
+            self._sum = total
+        if 'sum_position' not in lt:
+            csr_pos = common.to_device_i32(lt['csr_pos_host'], self._ctx).long()
+            of_csr = torch.empty(csr_pos.shape, dtype=torch.int32, device=self._ctx)
+            of_csr[csr_pos] = torch.arange(csr_pos.shape[0], dtype=torch.int32, device=self._ctx)
+            pos = self._sum.layout_positions()
+            lt['sum_position'] = of_csr if pos is None else of_csr[pos.long()]
+        return self._sum, lt['sum_position']
 
     def _dst_partitions(self, slice_row_bytes):
         if self._t_parts is not None:

@@ -354,6 +354,23 @@ class GSpMMhip(VanillaSpMMhip):
         if out is not self.out_tvm:
             self.out_tvm.copy_(out[..., :self._pad_from])
 
+    def layout_positions(self):
+        """Where each element of the built layout lies in the adjacency's CSR order (int32 on the device; None: in its place)."""
+        return self._active['edge_pos32'] if self._active['P'] > 1 else None
+
+    def run_laid_out(self, src_feat, weights, out):
+        """The weighted sum into `out` with weights that are head-major, (H, nnz), and in the layout's element order already."""
+        if self._func is None or self._bop is not None or self._reduce != 'sum' or self._pad_from is not None:
+            raise RuntimeError("run_laid_out needs a built weighted sum that pads nothing")
+        nnz = self._adj_indices.shape[0]
+        common.check_inputs([src_feat, weights, out], [self._placeholders[0], common.placeholder((self._heads, nnz)),
+                                                       common.placeholder((self._num_rows,) + self._placeholders[0].shape[1:])], self._ctx)
+        lay = self._active
+        _lib.check(self._func(lay['plan'], _lib.dev_ptr(lay['pos']), _lib.dev_ptr(lay['idx']), _lib.dev_ptr(weights),
+                              _lib.dev_ptr(src_feat), _lib.dev_ptr(out), self._feat_len, self._heads, 1, _REDUCE['sum'],
+                              self._num_feat_partitions, common.stream_ptr()))
+        return out
+
     def run_with_dots(self, src_feat, weights, own):
         """run([src_feat, weights]) and, in the same sweep, dots[e, h] = <own[row e, h, :], src_feat[col e, h, :]> per edge in
         the order of the weights given (set_weight_order) -- the two gradients of a weighted sum over the transposed graph.

@@ -374,3 +374,27 @@ def _choose_sddmm_heads(n_rows, n_cols, nnz, heads, head_len):
         if t == 1:
             return None
     return p, t
+
+
+# What attention's gradients may take for two [nnz, H] arrays while a call lasts.
+ATTENTION_EDGE_BYTES = 16 << 30
+
+
+def attention_keeps_score_gradients(nnz, num_rows, heads, head_len):
+    """Whether the gradients of dot-product attention keep the scores' gradients and take dQ from a weighted sum that
+    gathers K alone, instead of a second sweep that gathers K and V.  Saved per edge and head: a gather of head_len floats and
+    the score's second evaluation; paid: the values written, brought into the other order (in fours of heads at about 1.5 times
+    a copy's time, one to three heads a scattered 4-byte read each) and read.  Whole steps, second sweep -> kept, in us:
+      58,000 nodes, 12.5 M edges: 8x64 8335 -> 7450, 1x64 1110 -> 1020, 8x32 5565 -> 5037, 8x16 4907 -> 4244, 4x16 2296 -> 2052,
+        but 4x32 2185 -> 2219, 2x32 1003 -> 1075, 1x32 551 -> 598
+      20,000 nodes, 4 M edges: 4x64 1335 -> 1160, 4x32 696 -> 643, 2x32 332 -> 348
+      200,000 nodes, 4 M edges: 8x64 7345 -> 6221, 4x32 1857 -> 1651, 2x32 876 -> 835, 1x32 454 -> 432, 1x16 395 -> 392
+      100,000 nodes, 8 M edges: 4x32 1956 -> 1842, 2x32 930 -> 935
+      20,000 nodes, 200,000 edges (launches): 4x64 183 -> 165, 2x64 147 -> 157, 8x16 218 -> 206, 4x32 136 -> 163"""
+    if nnz * heads * head_len < 3 << 24 or 2 * 4 * nnz * heads > ATTENTION_EDGE_BYTES:
+        return False
+    if head_len == 64:
+        return True
+    if heads % 4:
+        return nnz <= 32 * num_rows
+    return head_len == 16 or heads % 8 == 0 or nnz <= 128 * num_rows

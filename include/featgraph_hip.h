@@ -262,6 +262,13 @@ int fg_gspmm_arg_f32(fg_spmm_plan *plan, const int32_t *indptr_dev, const int32_
  */
 int fg_edge_values_head_major_f32(const float *src_dev, const int32_t *edge_pos_dev, int64_t n_edges,
                                   int heads, float *dst_dev, void *stream);
+/*
+ * The same for values that are head-major already, result[h, e] = src[h, edge_pos[e]], both arrays [heads, n_edges]; src is
+ * overwritten as well, and *result tells which of the two (src_dev or dst_dev) holds the result once the stream is there.
+ * edge_pos 16-byte aligned.
+ */
+int fg_edge_values_permute_f32(float *src_dev, const int32_t *edge_pos_dev, int64_t n_edges, int heads, float *dst_dev,
+                               float **result, void *stream);
 
 /* ---- SDDMM --------------------------------------------------------------------------- */
 
@@ -445,13 +452,16 @@ int fg_graph_attention_additive_f32(fg_spmm_plan *plan, const int32_t *pos_dev, 
                                     void *stream);
 
 /*
- * Gradients of fg_graph_attention_f32, again without any [nnz, heads] array: the scores are formed anew from
- * Q and K, the softmax from row_state.
+ * Gradients of fg_graph_attention_f32: the scores are formed anew from Q and K, the softmax from row_state.
  *   fg_graph_attention_coef_f32: row_coef[h, v] = (max + log(sum), <dout[v, h, :], out[v, h, :]>), an
  *     [heads, n_dst, 2] array, from the forward pass's row_state and output (one small pass over the rows);
  *   fg_graph_attention_backward_q_f32: dq, on the plan and arrays of the forward pass (gathers K and V);
  *   fg_graph_attention_backward_kv_f32: dk and dv, on a plan and arrays of the TRANSPOSED adjacency (rows =
- *     sources; gathers Q, dout and row_coef of the destinations).
+ *     sources; gathers Q, dout and row_coef of the destinations);
+ *   fg_graph_attention_backward_kv_ds_f32: the same, and ds[h, t] = scale * the gradient of element t's score, a
+ *     [heads, nnz] array in the layout's element order.  dq[v, h, :] is the sum of ds * k over v's elements: brought into
+ *     the order of a layout of the adjacency (fg_edge_values_permute_f32) they are fg_gspmm_f32's head-major weights, and
+ *     _backward_q_f32, which gathers V as well, is not needed.
  * Same restrictions as the forward pass.
  */
 int fg_graph_attention_coef_f32(const float *out_dev, const float *dout_dev, const float *row_state_dev,
@@ -464,6 +474,10 @@ int fg_graph_attention_backward_kv_f32(fg_spmm_plan *plan_t, const int32_t *pos_
                                        const float *q_dev, const float *dout_dev, const float *k_dev,
                                        const float *v_dev, const float *row_coef_dev, float *dk_dev, float *dv_dev,
                                        int heads, int head_len, float scale, void *stream);
+int fg_graph_attention_backward_kv_ds_f32(fg_spmm_plan *plan_t, const int32_t *pos_t_dev, const int32_t *idx_t_dev,
+                                          const float *q_dev, const float *dout_dev, const float *k_dev,
+                                          const float *v_dev, const float *row_coef_dev, float *dk_dev, float *dv_dev,
+                                          float *ds_dev, int heads, int head_len, float scale, void *stream);
 
 /*
  * Gradients of fg_graph_attention_additive_f32.  row_coef is [heads, n_dst, 4] here: (max + log(sum),
