@@ -82,6 +82,7 @@ struct GenArgs {
     int ordered;                 // element positions ascend along every row (segment) of the walked layout
     int final;                   // the kernel's rows are results (one partition), not a partition's share of them
     int64_t pos_stride, col_width, out_stride, partial_stride;
+    bool src32;                  // the left operand lies on the source nodes and spans less than 4 GiB
 };
 
 // The operand features of a lane's V outputs: V consecutive ones (CONTIG: one 128-bit load) or one value V times.
@@ -142,11 +143,17 @@ enum { kFirst, kFull, kNaNs };      // how a walk finds positions, see batch() b
 // identity and no row is scaled, both being the combining kernel's business.
 // LNT / RNT: see load_operand.  RED: FG_REDUCE_SUM or FG_REDUCE_MAX; a minimum runs as the maximum of the negated
 // messages (a.sign = -1; negation is exact, so values, ties and selected positions are those of the minimum).
-template <int OP, int RED, bool ARG, int V, bool LC, bool RC, bool LNT, bool RNT, bool PART>
+// SRC32: the left operand lies on the source nodes and spans less than 4 GiB: its rows' byte offsets are formed once,
+// where the columns are staged, and the gathers add them to a scalar base.  SIGN (not 0): the sign as a compile-time constant
+// (GenArgs::sign is not read), which the comparison and the maximum take as an operand modifier.  Both for the selected
+// copies in ascending order, the walk that vector instructions bound (26 of them per gathered 128 bits without, 17 with);
+// registers still allow 4 wavefronts per SIMD, and forcing 6 spills (F=100 452 -> 530 us).  12.5M edges on 58,000 nodes, copy_u max,
+// F=64 / 100 / 128: 289 / 474 / 575 -> 270 / 452 / 544 us.
+template <int OP, int RED, bool ARG, int V, bool LC, bool RC, bool LNT, bool RNT, bool PART, bool SRC32 = false, int SIGN = 0>
 __global__ __launch_bounds__(kBlock) void gspmm_bcast_kernel(const GenArgs a) {
     static_assert(RED == FG_REDUCE_SUM || RED == FG_REDUCE_MAX, "a minimum is a maximum with a.sign = -1");
     constexpr bool kLhs = kUsesLhs<OP>, kRhs = kUsesRhs<OP>;
-    const float sign = RED == FG_REDUCE_SUM ? 1.f : a.sign;
+    const float sign = RED == FG_REDUCE_SUM ? 1.f : SIGN ? (float)SIGN : a.sign;
     const bool final = !PART || a.final != 0;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -181,7 +188,8 @@ __global__ __launch_bounds__(kBlock) void gspmm_bcast_kernel(const GenArgs a) {
     auto stage = [&](int64_t c0, int n) {
         for (int t = lane; t < n; t += 64) {
             const int col = a.indices16 ? (int)a.indices16[c0 + t] : a.indices[c0 + t];      // uniform choice
-            el[t] = make_int2(col + (int)ubase, PART ? a.edge_pos[c0 + t] : (int)(c0 + t));
+            const uint32_t src = (uint32_t)(col + (int)ubase);
+            el[t] = make_int2((int)(SRC32 ? src * ((uint32_t)a.lhs_len * 4u) : src), PART ? a.edge_pos[c0 + t] : (int)(c0 + t));
         }
         wave_lds_sync();
     };
@@ -225,7 +233,10 @@ __global__ __launch_bounds__(kBlock) void gspmm_bcast_kernel(const GenArgs a) {
                     const int2 w = el[(ALL || t < t1) ? t : tb];
                     stored[k] = w.y;
                     float l[V], r[V];
-                    if (kLhs) load_operand<V, LC, LNT>(row_at(lbase, l_on_e ? w.y : w.x, lbytes), l);
+                    if (SRC32)
+                        load_operand<V, LC, LNT>(reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.lhs) +
+                                                                                 ((uint32_t)w.x + (uint32_t)fl * 4u)), l);
+                    else if (kLhs) load_operand<V, LC, LNT>(row_at(lbase, l_on_e ? w.y : w.x, lbytes), l);
                     if (kRhs) load_operand<V, RC, RNT>(row_at(rbase, r_on_e ? w.y : w.x, rbytes), r);
 #pragma unroll
                     for (int i = 0; i < V; ++i) {
@@ -275,10 +286,10 @@ __global__ __launch_bounds__(kBlock) void gspmm_bcast_kernel(const GenArgs a) {
                     for (; tb < t1; tb += step * U) batch(std::false_type{}, find_tag, tb, t1);
                 }
             };
-            bool full_rule = ARG && !a.ordered;      // whether the groups' results need it as well
+            bool full_rule = ARG && !SRC32 && !a.ordered;      // whether the groups' results need it as well
             if constexpr (ARG) {
                 if (full_rule) {
-                    walk(std::integral_constant<int, kFull>{});
+                    if constexpr (!SRC32) walk(std::integral_constant<int, kFull>{});
                 } else {
                     walk(std::integral_constant<int, kFirst>{});
                     // Nothing above -inf though the group had elements: the first of them.  12.5M edges, F=64 / 100 / 256, 97 %
@@ -445,6 +456,13 @@ void launch_spmm_variant(int vec, bool lnt, bool rnt, dim3 grid, hipStream_t st,
     if (vec == 0) { FG_GO(1, true, true, false, false); return; }
     const bool lc = vec != 3, rc = vec != 2;
     lnt = lnt && lc; rnt = rnt && rc;
+    if constexpr (OP == FG_BIN_COPY_LHS && ARG) {
+        if (a.src32 && a.ordered && lc) {
+            if (a.sign > 0) hipLaunchKernelGGL((gspmm_bcast_kernel<OP, RED, ARG, 4, true, true, false, false, PART, true, 1>), grid, dim3(kBlock), 0, st, a);
+            else hipLaunchKernelGGL((gspmm_bcast_kernel<OP, RED, ARG, 4, true, true, false, false, PART, true, -1>), grid, dim3(kBlock), 0, st, a);
+            return;
+        }
+    }
     if constexpr (USES == 1) {             // the right operand is not read: one instantiation stands for all its modes
         if (!lc) FG_GO(4, false, true, false, false);
         else if (lnt) FG_GO(4, true, true, true, false);
@@ -849,17 +867,20 @@ int gspmm_bcast_run(fg_spmm_plan *pl, const int32_t *pos_dev, const int32_t *idx
     a.lhs = lhs_dev; a.rhs = rhs_dev; a.lhs_off = lhs_off_dev; a.rhs_off = rhs_off_dev;
     a.lhs_len = lhs_len; a.rhs_len = rhs_len; a.lhs_target = lhs_target; a.rhs_target = rhs_target;
     a.sign = reduce == FG_REDUCE_MIN ? -1.f : 1.f;
+    a.src32 = uses_l && lhs_target == FG_TARGET_U && (uint64_t)pl->n_src * (uint64_t)lhs_len * 4u < (1ull << 32);
     a.row_scale = P > 1 ? nullptr : row_scale_dev;
     a.out = P > 1 ? buf : out_dev;
     a.arg = P > 1 ? (arg_dev ? abuf : nullptr) : arg_dev;
     a.partial = values; a.partial_arg = positions;
     // Feature tiles of 64 floats over the workgroups (as for the weighted sum) when an operand is gathered from the
     // source nodes and the 128-bit paths apply: a partition's slice of a tile is what an L2 has to hold.
-    // (Not with the positions of the selected elements, whose kernels held too many registers to gain from it
-    // when each message went by the full rule, F=256 17.1 ms tiled against 14.7 ms, not measured since -- nor with an operand streamed from the edges, which sets the time.)
+    // (Not with an operand streamed from the edges, which sets the time.  With positions of the selected elements for copies
+    // only: copy_u max, F=128 / 256 / 512, 12.5M edges on 58,000 nodes 586 -> 539 / 1061 -> 1045 / 2501 -> 1963 us, 8M on 200,000
+    // 504 -> 462 / 1105 -> 896 / 2294 -> 1964; u_add_e max, which instructions bound, 669 -> 683 / 1132 -> 1270 / 2573 -> 2403 and
+    // 509 -> 549 / 1101 -> 1030 / 2320 -> 2198.)
     const bool gathers = (uses_l && lhs_target == FG_TARGET_U) || (uses_r && rhs_target == FG_TARGET_U);
     const bool streams = (uses_l && lhs_target == FG_TARGET_E && lmode == 1) || (uses_r && rhs_target == FG_TARGET_E && rmode == 1);
-    const int T = (V == 4 && gathers && !streams && !arg_dev && out_len >= 128 && out_len % 64 == 0) ? out_len / 64 : 1;
+    const int T = (V == 4 && gathers && !streams && (!arg_dev || op == FG_BIN_COPY_LHS) && out_len >= 128 && out_len % 64 == 0) ? out_len / 64 : 1;
     a.n_tiles = T; a.tile_vecs = T > 1 ? 16 : (out_len + V - 1) / V;
     a.F = out_len; a.L = lanes_for(T > 1 ? 16 : out_len / V);
     a.item_off = pl->item_off_dev; a.edge_pos = edge_pos_dev; a.n_parts = P; a.final = P == 1;

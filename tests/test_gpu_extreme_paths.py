@@ -238,3 +238,30 @@ def test_gradients_of_rows_of_a_few_elements(feat_len, degree):
             for a, b in zip(got, ref):
                 # sums of at most a few hundred fp32 products
                 assert float((a.double() - b).norm()) <= 1e-5 * float(b.norm())
+
+
+@pytest.mark.parametrize("special", ["ties", "nan", "minus_inf"])
+@pytest.mark.parametrize("reduce", ["max", "min"])
+@pytest.mark.parametrize("feat_len", [128, 192, 320])
+def test_positions_in_feature_tiles(oracle, special, reduce, feat_len):
+    """Feature lengths that the launch cuts into tiles of 64: exactly the oracle's values and positions, in every tile."""
+    import torch
+    from featgraph_amd.module import GSpMMhip, placeholder
+    rng = np.random.default_rng(feat_len)
+    adj = _graph(rng, LENS)
+    x = rng.integers(-1, 2, size=(700, feat_len)).astype(np.float32)
+    if special == "nan":
+        x[rng.random(x.shape) < 0.01] = np.nan
+    if special == "minus_inf":
+        x[rng.random(x.shape) < 0.7] = -np.inf if reduce == "max" else np.inf
+    e = rng.integers(0, 2, size=(adj.nnz, 1)).astype(np.float32)
+    for msg, arrays, o in (("copy_u", [x], ("copy_lhs", x, None, "u", "e")), ("u_add_e", [x, e], ("add", x, e, "u", "e"))):
+        ref, ref_arg = oracle.gspmm_bcast(adj.indptr, adj.indices, o[0], reduce, o[1], o[2], o[3], o[4])
+        for P in (None, 3):
+            m = GSpMMhip(adj)
+            m.build([placeholder(a.shape) for a in arrays], {'msg': msg, 'reduce': reduce, 'return_arg': True, 'broadcast': True},
+                    {'num_src_partitions': P})
+            assert m._bop.feature_tiles(True) == (feat_len // 64 if msg == "copy_u" else 1)
+            out = m.run([torch.from_numpy(a).cuda() for a in arrays]).cpu().numpy()
+            assert np.array_equal(out, ref, equal_nan=True), (msg, P)
+            assert np.array_equal(m.arg_tvm.cpu().numpy(), ref_arg), (msg, P)
