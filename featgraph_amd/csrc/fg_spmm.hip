@@ -1519,7 +1519,9 @@ extern "C" int fg_spmm_dot_f32(fg_spmm_plan *plan, const int32_t *pos_dev, const
     if (!plan) return fail(FG_ERR_ARG, "plan is null");
     if (heads < 1 || F < 1 || F % heads != 0) return fail(FG_ERR_SHAPE, "feature length %d is not divisible by %d heads", F, heads);
     if (own_len < 1 || own_len > F / heads) return fail(FG_ERR_SHAPE, "heads of %d floats in own, of %d in x", own_len, F / heads);
-    if (plan->n_dst > 0 && plan->nnz > 0 && (!own_dev || !edge_pos_dev || !dots_dev)) return fail(FG_ERR_ARG, "null device pointer");
+    // without elements there is nothing to take a dot product of: the plain sum, which reads none of the three
+    if (plan->nnz == 0) return fg_gspmm_f32(plan, pos_dev, idx_dev, vals_dev, x_dev, out_dev, F, heads, vals_head_major, FG_REDUCE_SUM, num_feat_partitions, stream);
+    if (plan->n_dst > 0 && (!own_dev || !edge_pos_dev || !dots_dev)) return fail(FG_ERR_ARG, "null device pointer");
     if (((uintptr_t)edge_pos_dev & 15) != 0) return fail(FG_ERR_ARG, "the positions of the dots must be 16-byte aligned");
     const DotRequest dot = {own_dev, (int64_t)heads * own_len, own_len, dots_dev, edge_pos_dev};
     return spmm_run(plan, pos_dev, idx_dev, vals_dev, x_dev, out_dev, F, num_feat_partitions, stream, heads, FG_REDUCE_SUM,

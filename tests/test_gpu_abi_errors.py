@@ -160,3 +160,39 @@ def test_broadcasting_entry_points(env):
     assert sddmm(op=DOT, n=2, red_len=3) == FG_ERR_SHAPE              # 8 is not a multiple of the contracted length
     assert sddmm(op=DOT, n=2, red_len=4, o=eo) == FG_OK
     assert sddmm(n_edges=0, lhs=None, rhs=None) == FG_OK              # nothing to read, nothing refused
+
+
+def test_sum_with_dots_arguments(env):
+    """fg_spmm_dot_f32: an operand that the kernel would read must be there; on a plan without elements none of the dots' is,
+    and the rows are written as those of a plain sum."""
+    import torch
+    L, lib, plan, plan2, t = env
+    p = lib.dev_ptr
+    F = 16
+    x, own = torch.ones((5, F), device="cuda"), torch.ones((4, F), device="cuda")
+    out, dots = torch.full((4, F), float("nan"), device="cuda"), torch.full((6,), float("nan"), device="cuda")
+    where = torch.arange(6, dtype=torch.int32, device="cuda")
+
+    def call(pl=plan, idx=t['indices'], w=t['vals'], x=x, own=own, own_len=F, o=out, pos=where, d=dots, heads=1):
+        return L.fg_spmm_dot_f32(pl, p(t['indptr']), p(idx), p(w), p(x), p(own), own_len, p(o), p(pos), p(d), F, heads, 0, 0, None)
+
+    assert L.fg_spmm_dot_takes(plan, F, 1, 0) == 1
+    assert call() == FG_OK
+    torch.cuda.synchronize()
+    assert out[:, 0].tolist() == [2.0, 0.0, 3.0, 1.0] and dots.tolist() == [float(F)] * 6
+    for bad in (dict(pl=None), dict(own=None), dict(pos=None), dict(d=None), dict(w=None), dict(x=None), dict(idx=None), dict(o=None),
+                dict(pos=where[1:])):
+        assert call(**bad) == FG_ERR_ARG, bad
+    for bad in (dict(own_len=0), dict(own_len=F + 1), dict(heads=3)):
+        assert call(**bad) == FG_ERR_SHAPE, bad
+    empty = ctypes.c_void_p()
+    none = np.zeros(5, dtype=np.int32)
+    assert L.fg_spmm_plan_create(lib.host_ptr(none), 4, 5, 1, None, ctypes.byref(empty)) == FG_OK
+    try:
+        pos = torch.zeros(5, dtype=torch.int32, device="cuda")
+        out.fill_(float("nan"))
+        assert L.fg_spmm_dot_f32(empty, p(pos), None, None, p(x), None, F, p(out), None, None, F, 1, 0, 0, None) == FG_OK
+        torch.cuda.synchronize()
+        assert torch.equal(out, torch.zeros_like(out))
+    finally:
+        L.fg_spmm_plan_destroy(empty)
