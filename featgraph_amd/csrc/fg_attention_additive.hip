@@ -14,7 +14,8 @@
 // float64, that dEr is closer than the edge-by-edge sum (3.4e-7 against 5.5e-7 relative, 58,000 nodes, 3 M edges); by column
 // the same form is not (cancellation that the edge-by-edge difference has not), so dEl is summed edge by edge.
 // Not in the reference (no attention operator exists there); the result is defined by the composition of
-// gather-add, leaky ReLU, edge softmax and per-head weighted SpMM.
+// gather-add, leaky ReLU, edge softmax and per-head weighted SpMM: a row with a NaN score, or one of +inf, is NaN and so is
+// every gradient it takes part in.  (A row whose scores are all -inf counts as one without edges, though: 0.)
 //
 // Layout of the work: one head (16, 32 or 64 floats) per kernel tile, the tile index fastest in the workgroup id so
 // that every XCD gathers one head's slices; items, staging and tile-by-tile copies are those of the SpMM kernels.
@@ -104,7 +105,8 @@ __device__ __forceinline__ float wave_max(float v) {
     return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(fg::rows_max(v))));
 }
 
-// Running sums of one row: over all its elements and over those with z > 0.  acc / plus: weighted rows, this lane's four
+// Running sums of one row: over all its elements and over those with z > 0.  fmaxf passes a NaN score by, so the sum of
+// exponentials alone carries it: a score makes it NaN where any is above -inf, and where none is, as the score itself (nan_term).  acc / plus: weighted rows, this lane's four
 // floats (in the totals of a row that the wavefront shared: one of them, fg::word_of_row); a / p: weights (by column a is the sum of gate * a * (da - delta)).  m: the maximum that the forward weights are
 // relative to.
 template <typename T>
@@ -113,6 +115,8 @@ struct SumsOf {
     float a, p, m;
 };
 using Sums = SumsOf<float4>;
+// s, a score that is -inf or NaN, as a term of a sum of exponentials
+__device__ __forceinline__ float nan_term(float s) { return s == -INFINITY ? 0.f : s; }
 __device__ __forceinline__ Sums sums_empty() { return {zero4(), zero4(), 0.f, 0.f, -INFINITY}; }
 
 __device__ __forceinline__ void scale4(float &a, float f) { a *= f; }
@@ -138,7 +142,7 @@ __device__ __forceinline__ void rescale(SumsOf<T> &r, float f) {
 template <bool PLUS, typename T>
 __device__ __forceinline__ void merge(SumsOf<T> &r, const SumsOf<T> &s) {
     const float m = fmaxf(r.m, s.m);
-    if (m == -INFINITY) return;               // both empty
+    if (m == -INFINITY) { r.a += s.a; return; }      // both empty, or NaN scores alone in one of them
     const float fs = __expf(s.m - m);         // exp(-inf) = 0 for the empty side
     rescale<PLUS>(r, __expf(r.m - m));
     fma4(r.acc, fs, s.acc);
@@ -251,7 +255,11 @@ __global__ __launch_bounds__(kBlock, PASS == kMerge ? 5 : 8) void additive_sweep
                 }
             }
             const float m = fmaxf(r.m, wave_max(mx));
-            if (m == -INFINITY) return false;
+            if (m == -INFINITY) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) r.a += nan_term(s[i]);
+                return false;
+            }
             if (r.m != -INFINITY) rescale<PLUS>(r, __expf(r.m - m));      // a later batch of a long row
             r.m = m;
         }
@@ -342,7 +350,11 @@ __global__ __launch_bounds__(kBlock, PASS == kMerge ? 5 : 8) void additive_sweep
             if (FWD) m = fmaxf(m, j + u < e ? s[u] : -INFINITY);
         }
         if constexpr (FWD) {
-            if (m == -INFINITY) return;         // uniform inside a lane group
+            if (m == -INFINITY) {               // uniform inside a lane group
+#pragma unroll
+                for (int u = 0; u < kU; ++u) r.a += j + u < e ? nan_term(s[u]) : 0.f;
+                return;
+            }
             rescale<PLUS>(r, __expf(r.m - m));
             r.m = m;
         }
@@ -384,9 +396,9 @@ __global__ __launch_bounds__(kBlock, PASS == kMerge ? 5 : 8) void additive_sweep
             if (PASS == kMerge) merge<PLUS>(r, old);
             float l = r.a, share = r.p;
             if (PASS == kOnly) {
-                const float inv = l > 0.f ? 1.0f / l : 0.f;
+                const float inv = l == 0.f ? 0.f : 1.0f / l;
                 rescale<PLUS>(r, inv);
-                if (!(l > 0.f)) { set_zero(r.acc); set_zero(r.plus); r.p = 0.f; }
+                if (l == 0.f) { set_zero(r.acc); set_zero(r.plus); r.p = 0.f; }
                 share = r.p;
             }
             store_nt(r.acc, out_row(row) + f);
@@ -547,19 +559,21 @@ __global__ __launch_bounds__(256) void additive_merge_kernel(float4 *out, float4
                 run.p += buf_share[p * pairs + pair] * f;
             }
         }
+    } else {
+        for (int p = 0; p < P; ++p) run.a += buf_state[(p * pairs + pair) * 2 + 1];      // 0, or NaN
     }
     const float l = run.a;
-    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    const float inv = l == 0.f ? 0.f : 1.0f / l;
     scale4(run.acc, inv);
-    out[i] = l > 0.f ? run.acc : zero4();
+    out[i] = l == 0.f ? zero4() : run.acc;
     if (plus) {
         scale4(run.plus, inv);
-        plus[i] = l > 0.f ? run.plus : zero4();
+        plus[i] = l == 0.f ? zero4() : run.plus;
     }
     // (P == 1: the state and share in place are read by the row's other words in this launch, so they are not rewritten here)
     if (P > 1 && w == h * head_words) {
         state[pair * 2] = m; state[pair * 2 + 1] = l;
-        if (plus) share[pair] = l > 0.f ? run.p * inv : 0.f;
+        if (plus) share[pair] = l == 0.f ? 0.f : run.p * inv;
     }
 }
 // share /= sum of exponentials, after the passes that merged in place
@@ -567,7 +581,7 @@ __global__ __launch_bounds__(256) void additive_share_kernel(float *share, const
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n_pairs) return;
     const float l = state[i * 2 + 1];
-    share[i] = l > 0.f ? share[i] / l : 0.f;
+    share[i] = l == 0.f ? 0.f : share[i] / l;
 }
 
 // coef[h, r] = (m + log l, <dout[r, h, :], out[r, h, :]>, er[r, h], 0), head by head so that the gathers of one head stay
@@ -589,7 +603,7 @@ __global__ __launch_bounds__(256) void additive_coef_kernel(const float *out, co
     if (on && li == 0) {
         const float m = state[pair * 2], l = state[pair * 2 + 1];
         const int64_t r = pair / H, h = pair - r * H;
-        const float c1 = l > 0.f ? m + __logf(l) : INFINITY, dl = l > 0.f ? delta : 0.f;
+        const float c1 = l == 0.f ? INFINITY : m + __logf(l), dl = l == 0.f ? 0.f : delta;
         *reinterpret_cast<float4 *>(coef + (h * n_rows + r) * 4) = make_float4(c1, dl, er[r * er_row + h * er_head], 0.f);
         if (plus) der[r * er_row + h * er_head] = (1.f - slope) * (up - dl * share[pair]);
     }
