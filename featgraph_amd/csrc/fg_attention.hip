@@ -8,7 +8,9 @@
 // scores: every lane group keeps a running maximum, a running sum of exponentials and the running
 // weighted sum of its row (rescaled whenever the maximum grows), and source-column partitions are
 // merged the same way through `out` and a small [n_dst, H, 2] state array.  Not in the reference (no
-// attention operator exists there); the result is defined by the composition of the three operators.
+// attention operator exists there); the result is defined by the composition of the three operators: a row with a NaN
+// score, or one of +inf, is NaN and so is every gradient it takes part in.  (A row whose scores are all -inf counts as one
+// without edges, though: 0.)
 //
 // Layout of the work: one head (16, 32 or 64 floats) per kernel tile, the tile index fastest in the
 // workgroup id so that every XCD gathers one head's slices of K and V; items, staging and the
@@ -55,7 +57,8 @@ struct AttnArgs {
     int64_t pos_stride = 0, kv_stride = 0, out_stride = 0, state_stride = 0;
 };
 
-// Running softmax-weighted sum of one lane group: maximum, sum of exponentials, weighted sum.
+// Running softmax-weighted sum of one lane group: maximum, sum of exponentials, weighted sum.  fmaxf passes a NaN score by: the
+// sum of exponentials alone carries it to the row's result.
 struct Running {
     float m, l;
     float4 acc;
@@ -66,7 +69,7 @@ __device__ __forceinline__ Running running_empty() { return {-INFINITY, 0.f, mak
 // r <- r and s merged (both relative to their own maxima).
 __device__ __forceinline__ void running_merge(Running &r, const Running &s) {
     const float m = fmaxf(r.m, s.m);
-    if (m == -INFINITY) return;               // both empty
+    if (m == -INFINITY) { r.l += s.l; return; }      // both empty, or NaN scores alone in one of them
     const float fr = __expf(r.m - m), fs = __expf(s.m - m);      // exp(-inf) = 0 for the empty side
     r.acc.x = r.acc.x * fr + s.acc.x * fs; r.acc.y = r.acc.y * fr + s.acc.y * fs;
     r.acc.z = r.acc.z * fr + s.acc.z * fs; r.acc.w = r.acc.w * fr + s.acc.w * fs;
@@ -95,7 +98,11 @@ __device__ __forceinline__ void update(const int32_t (&c)[NU], const bool (&vali
         s[u] = valid[u] ? t : -INFINITY;
         m = fmaxf(m, s[u]);
     }
-    if (m == -INFINITY) return;             // nothing finite so far (uniform inside a lane group)
+    if (m == -INFINITY) {                   // nothing above -inf so far (uniform inside a lane group)
+#pragma unroll
+        for (int u = 0; u < NU; ++u) r.l += s[u] == -INFINITY ? 0.f : s[u];      // what is not -inf is NaN
+        return;
+    }
     const float f = __expf(r.m - m);
     r.acc.x *= f; r.acc.y *= f; r.acc.z *= f; r.acc.w *= f;
     r.l *= f;
@@ -339,9 +346,9 @@ __global__ __launch_bounds__(256) void attention_finish_kernel(float4 *out, cons
     const uint32_t r = i / row_words, h = (i - r * row_words) / head_words;
     const float l = state[((uint64_t)r * H + h) * 2 + 1];
     float4 o = out[i];
-    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    const float inv = l == 0.f ? 0.f : 1.0f / l;
     o.x *= inv; o.y *= inv; o.z *= inv; o.w *= inv;
-    out[i] = l > 0.f ? o : make_float4(0.f, 0.f, 0.f, 0.f);
+    out[i] = l == 0.f ? make_float4(0.f, 0.f, 0.f, 0.f) : o;
 }
 
 // The partitions' buffers merged, partition after partition, and the row divided by its sum of exponentials:
@@ -368,10 +375,12 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(float4 *out, float
             run.acc.x += a.x * f; run.acc.y += a.y * f; run.acc.z += a.z * f; run.acc.w += a.w * f;
             run.l += buf_state[p * sstride + srow + 1] * f;
         }
+    } else {
+        for (int p = 0; p < P; ++p) run.l += buf_state[p * sstride + srow + 1];      // 0, or NaN
     }
-    const float inv = run.l > 0.f ? 1.0f / run.l : 0.f;
-    out[i] = run.l > 0.f ? make_float4(run.acc.x * inv, run.acc.y * inv, run.acc.z * inv, run.acc.w * inv)
-                         : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float inv = run.l == 0.f ? 0.f : 1.0f / run.l;
+    out[i] = run.l == 0.f ? make_float4(0.f, 0.f, 0.f, 0.f)
+                          : make_float4(run.acc.x * inv, run.acc.y * inv, run.acc.z * inv, run.acc.w * inv);
     if (w == h * head_words) { state[srow] = run.m; state[srow + 1] = run.l; }
 }
 

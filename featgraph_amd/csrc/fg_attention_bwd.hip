@@ -334,7 +334,7 @@ __global__ __launch_bounds__(256) void attention_coef_kernel(const float *out, c
     if (on && li == 0) {
         const float m = state[pair * 2], l = state[pair * 2 + 1];
         const int64_t r = pair / H, h = pair - r * H;
-        const float c1 = l > 0.f ? m + __logf(l) : INFINITY, dl = l > 0.f ? delta : 0.f;
+        const float c1 = l == 0.f ? INFINITY : m + __logf(l), dl = l == 0.f ? 0.f : delta;
         float *c = coef + (h * n_rows + r) * 2;             // head by head
         c[0] = c1; c[1] = dl;
     }

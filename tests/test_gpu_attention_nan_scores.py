@@ -83,6 +83,32 @@ def test_additive(monkeypatch, kind, value, parts, pass_buffers):
     assert torch.equal(torch.nan_to_num(plain, nan=7.0), torch.nan_to_num(got[0], nan=7.0))
 
 
+@pytest.mark.parametrize("kind", ["few", "edges"])
+@pytest.mark.parametrize("kept", [True, False])
+@WAYS
+def test_dot(monkeypatch, kind, kept, parts, pass_buffers):
+    import torch
+    from featgraph_amd import tuning
+    from featgraph_amd.autograd import Graph
+    _setup(monkeypatch, parts, pass_buffers)
+    monkeypatch.setattr(tuning, "attention_keeps_score_gradients", lambda *a: kept)
+    adj = _graph(kind, np.random.default_rng(3))
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    normal = lambda n: torch.randn((n, H, D), generator=gen, device="cuda")
+    q, k, v, dout = normal(adj.shape[0]), normal(adj.shape[1]), normal(adj.shape[1]), normal(adj.shape[0])
+    lens = np.diff(adj.indptr)
+    for i, n in enumerate(np.unique(lens)):
+        q[int(np.flatnonzero(lens == n)[3]), i % H, 5] = float("nan")
+    k[int(np.bincount(adj.indices).argmin()), 1, 0] = float("nan")
+    leaves = [t.clone().requires_grad_() for t in (q, k, v)]
+    out = Graph(adj).attention(*leaves, scale=0.2)
+    got = (out.detach(),) + torch.autograd.grad(out, leaves, dout)
+    a, b, w = (t.detach().double().requires_grad_() for t in (q, k, v))
+    ref = _float64(adj, lambda row, col: 0.2 * (b[col] * a[row]).sum(-1), w, dout, (a, b, w))
+    assert int(torch.isnan(ref[0]).any(2).sum()) >= 6 and not bool(torch.isnan(ref[0]).all())
+    _same(("out", "dQ", "dK", "dV"), got, ref)
+
+
 @WAYS
 def test_rows_of_minus_infinity_count_as_empty(monkeypatch, parts, pass_buffers):
     import torch
