@@ -101,6 +101,7 @@ class GSpMMhip(VanillaSpMMhip):
         self._reduce, self._msg, self._weights_at_run, self._notes = reduce, msg, weights_at_run, notes
         self._active = self._glayout(P)
         self._func = _lib.lib().fg_gspmm_f32
+        self._dots_fit = True
         common.reserve(self._active['plan'], common.OP_SPMM_SUM if _REDUCE[reduce] == 0 else common.OP_SPMM_EXTREME,
                        heads, feat_len // heads, self._num_feat_partitions, self._ctx)
         self._return_arg = return_arg
@@ -374,10 +375,11 @@ class GSpMMhip(VanillaSpMMhip):
     def run_with_dots(self, src_feat, weights, own):
         """run([src_feat, weights]) and, in the same sweep, dots[e, h] = <own[row e, h, :], src_feat[col e, h, :]> per edge in
         the order of the weights given (set_weight_order) -- the two gradients of a weighted sum over the transposed graph.
-        Returns (self.out_tvm, dots), or None where the library has no kernel for both (fg_spmm_dot_takes)."""
+        Returns (self.out_tvm, dots), or None where the library has no kernel for both (fg_spmm_dot_takes) or the scratch for
+        the dots cannot be allocated (not tried again before the next build())."""
         if self._func is None:
             raise RuntimeError("call build() before run_with_dots()")
-        if self._bop is not None or not self._weights_at_run or self._reduce != 'sum':
+        if self._bop is not None or not self._weights_at_run or self._reduce != 'sum' or not self._dots_fit:
             return None
         lay = self._active
         pos = self._given_pos(lay)
@@ -394,10 +396,14 @@ class GSpMMhip(VanillaSpMMhip):
         if self._pad_from is not None:
             self._x_pad[..., :self._pad_from].copy_(src_feat)
             src_feat, out = self._x_pad, self._out_pad
-        _lib.check(_lib.lib().fg_spmm_dot_f32(
-            lay['plan'], _lib.dev_ptr(lay['pos']), _lib.dev_ptr(lay['idx']), _lib.dev_ptr(w), _lib.dev_ptr(src_feat), _lib.dev_ptr(own),
-            own.shape[-1], _lib.dev_ptr(out), _lib.dev_ptr(pos), _lib.dev_ptr(dots), self._feat_len, self._heads, head_major,
-            self._num_feat_partitions, common.stream_ptr()))
+        try:
+            _lib.check(_lib.lib().fg_spmm_dot_f32(
+                lay['plan'], _lib.dev_ptr(lay['pos']), _lib.dev_ptr(lay['idx']), _lib.dev_ptr(w), _lib.dev_ptr(src_feat), _lib.dev_ptr(own),
+                own.shape[-1], _lib.dev_ptr(out), _lib.dev_ptr(pos), _lib.dev_ptr(dots), self._feat_len, self._heads, head_major,
+                self._num_feat_partitions, common.stream_ptr()))
+        except MemoryError:
+            self._dots_fit = False
+            return None
         if out is not self.out_tvm:
             self.out_tvm.copy_(out[..., :self._pad_from])
         return self.out_tvm, dots

@@ -1,0 +1,60 @@
+"""Gradients whose faster way needs memory that is not there take the way that needs less: the library or torch reporting that an
+allocation failed (forced from the host, no device is exhausted) must not end a training step that the other way can finish."""
+import ctypes
+
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+pytestmark = pytest.mark.gpu
+
+FG_ERR_NOMEM = -5
+
+
+def _graph(n_dst=400, n_src=300, density=0.05):
+    adj = sp.random(n_dst, n_src, density=density, format="csr", random_state=np.random.default_rng(4)).astype("float32")
+    adj.sort_indices()
+    return adj
+
+
+def _failing(calls):
+    def fail(*args):
+        calls.append(1)
+        return FG_ERR_NOMEM
+    return fail
+
+
+@pytest.mark.parametrize("tail", [(64,), (4, 32)])
+def test_weighted_sum_gradients_without_memory_for_the_dots(monkeypatch, tail):
+    import torch
+    from featgraph_amd import _lib
+    from featgraph_amd.autograd import Graph
+    adj = _graph()
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    normal = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    x, w, dy = normal(adj.shape[1], *tail).requires_grad_(), normal(adj.nnz, *tail[:-1]).requires_grad_(), normal(adj.shape[0], *tail)
+    g = Graph(adj)
+    ref = torch.autograd.grad(g.spmm(x, w), (x, w), dy)
+    calls = []
+    monkeypatch.setattr(_lib.lib(), "fg_spmm_dot_f32", _failing(calls))
+    for _ in range(2):
+        got = torch.autograd.grad(g.spmm(x, w), (x, w), dy)
+        assert torch.equal(got[0], ref[0])
+        # the dots in another order: 64 products each, 2^-24 per rounding of the sum of |terms| (standard normal: below 64)
+        assert float((got[1] - ref[1]).abs().max()) <= 64 * 2.0 ** -24 * 64
+    assert len(calls) == 1                      # a step does not try again what did not fit
+
+
+def test_dots_that_would_take_more_than_the_cap_are_refused():
+    """One array of nnz dot products per tile or head, 8 GiB of them at most.  (Plans alone: nothing is launched.)"""
+    from featgraph_amd import _lib
+    L = _lib.lib()
+    rows, per_row = 1 << 20, 1 << 10            # 2^30 elements: 4 GiB per array
+    pos = np.arange(0, rows * per_row + 1, per_row, dtype=np.int32)
+    plan = ctypes.c_void_p()
+    _lib.check(L.fg_spmm_plan_create(_lib.host_ptr(pos), rows, 4096, 1, None, ctypes.byref(plan)))
+    try:
+        for F, heads, tiles, takes in ((64, 1, 1, 1), (128, 1, 2, 1), (192, 1, 3, 0), (128, 2, 0, 1), (256, 4, 0, 0)):
+            assert L.fg_spmm_dot_takes(plan, F, heads, tiles) == takes, (F, heads, tiles)
+    finally:
+        L.fg_spmm_plan_destroy(plan)
