@@ -55,6 +55,17 @@ class Graph(object):
             m.share_layouts_with(owner)
         return m
 
+    def _built_sum(self, inputs):
+        """A weighted sum over the adjacency; one that cannot be built leaves no layouts behind."""
+        m = self._gspmm_module(False)
+        try:
+            m.build(inputs, {}, {})
+        except Exception:
+            if self._layout_owner[False] is m:
+                del self._layout_owner[False]
+            raise
+        return m
+
     def _spmm_mod(self, transposed, tail, w_heads):
         key = ('spmm', transposed, tail, w_heads)
         if key not in self._mods:
@@ -206,7 +217,7 @@ class Graph(object):
             m.build([placeholder(tuple(q.shape)), placeholder(tuple(k.shape)), placeholder(tuple(v.shape))],
                     {'scale': scale}, {})
             graph = weakref.ref(self)           # no cycle: a Graph's device memory goes when its last user does
-            m._new_sum = lambda: graph()._gspmm_module(False)
+            m._new_sum = lambda inputs: graph()._built_sum(inputs)
             self._mods[key] = m
         return self._mods[key]
 

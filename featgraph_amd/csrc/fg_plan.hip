@@ -177,7 +177,8 @@ extern "C" int fg_spmm_plan_create(const int32_t *pos, int64_t n_dst, int64_t n_
         e = hipMemcpy(pl->fixups_dev, fixups.data(), sizeof(Fixup) * fixups.size(), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         fg_spmm_plan_destroy(pl);
-        return fail(FG_ERR_HIP, "fg_spmm_plan_create: %s", hipGetErrorString(e));
+        (void)hipGetLastError();
+        return fail(e == hipErrorOutOfMemory ? FG_ERR_NOMEM : FG_ERR_HIP, "fg_spmm_plan_create: %s", hipGetErrorString(e));
     }
     *plan_out = pl;
     return FG_OK;

@@ -41,8 +41,7 @@ class GraphAttentionhip(object):
         self._csr = csr
         self._layouts = {}
         self._sum = None
-        # where the weighted sum of backward() comes from (a Graph gives one that shares its layouts)
-        self._new_sum = lambda: GSpMMhip(scipy.sparse.csr_matrix((np.ones(csr.nnz, np.float32), csr.indices, csr.indptr), shape=csr.shape))
+        self._new_sum = None        # a Graph gives a function here that builds backward()'s weighted sum on layouts it has
         self._placeholders = None
         self.out_tvm = None
 
@@ -111,6 +110,7 @@ class GraphAttentionhip(object):
         self.state_tvm = torch.zeros((self._num_rows, heads, 2), dtype=torch.float32, device=self._ctx)
         self._coef = None
         self._sum = None
+        self._scores_kept = True            # until an allocation fails
         for lay in self._layouts.values():
             lay.pop('sum_position', None)
 
@@ -210,7 +210,7 @@ class GraphAttentionhip(object):
         (out_tvm / state_tvm as they were after run() on these inputs).  The scores are formed again from Q
         and K; dK and dV come from a sweep like the forward pass over the transposed adjacency, dQ from a weighted sum
         with the scores' gradients that this sweep leaves (two arrays of nnz * H floats while the call lasts), or, where
-        that does not pay or the arrays would not fit, from a sweep of its own over the adjacency.  Returns new tensors."""
+        that does not pay or does not fit, from a sweep of its own over the adjacency.  Returns new tensors."""
         if self._placeholders is None:
             raise RuntimeError("call build() before backward()")
         common.check_inputs([q, k, v], self._placeholders, self._ctx)
@@ -227,17 +227,7 @@ class GraphAttentionhip(object):
         kv = (lt['plan'], _lib.dev_ptr(lt['pos']), _lib.dev_ptr(lt['idx']), _lib.dev_ptr(q), _lib.dev_ptr(grad_out),
               _lib.dev_ptr(k), _lib.dev_ptr(v), _lib.dev_ptr(coef), _lib.dev_ptr(dk), _lib.dev_ptr(dv))
         tail = (self._heads, self._head_len, ctypes.c_float(self._scale), s)
-        edges = self._edge_buffers()
-        if edges is not None:
-            total, position = self._query_sum(lt)
-            ds, other = edges
-            _lib.check(L.fg_graph_attention_backward_kv_ds_f32(*kv, _lib.dev_ptr(ds), *tail))
-            result = ctypes.c_void_p()
-            _lib.check(L.fg_edge_values_permute_f32(_lib.dev_ptr(ds), _lib.dev_ptr(position), ds.shape[1], self._heads,
-                                                    _lib.dev_ptr(other), ctypes.byref(result), s))
-            flat = total._placeholders[0].shape
-            total.run_laid_out(k.view(flat), ds if result.value == ds.data_ptr() else other, dq.view((self._num_rows,) + flat[1:]))
-        else:
+        if not self._backward_with_kept_scores(lt, kv, tail, k, dq):
             lay = self._active
             _lib.check(L.fg_graph_attention_backward_q_f32(lay['plan'], _lib.dev_ptr(lay['pos']), _lib.dev_ptr(lay['idx']),
                                                            _lib.dev_ptr(q), _lib.dev_ptr(k), _lib.dev_ptr(v),
@@ -246,23 +236,49 @@ class GraphAttentionhip(object):
         self._coef = coef
         return dq, dk, dv
 
-    def _edge_buffers(self):
-        """Two (H, nnz) arrays for the scores' gradients, or None where dQ is to come from a sweep of its own."""
+    def _backward_with_kept_scores(self, lt, kv, tail, k, dq):
+        """dK and dV, and dQ from the scores' gradients that their sweep leaves; False, and nothing of them to use, where that
+        does not pay or memory for it was not to be had (not tried again before the next build(): an attempt that fails
+        costs device synchronisations)."""
         nnz = self._indices.shape[0]
-        if not tuning.attention_keeps_score_gradients(nnz, self._num_rows, self._heads, self._head_len):
-            return None
+        if not self._scores_kept or not tuning.attention_keeps_score_gradients(nnz, self._num_rows, self._heads, self._head_len):
+            return False
         try:
-            return tuple(torch.empty((2, self._heads, nnz), dtype=torch.float32, device=self._ctx))
-        except torch.cuda.OutOfMemoryError:
-            return None
+            self._kept_scores_sweeps(lt, kv, tail, k, dq)
+        except (MemoryError, torch.cuda.OutOfMemoryError):
+            self._scores_kept = False
+        if not self._scores_kept:
+            # what was taken goes back to the device, where the other way's plans look for memory
+            self._sum = None
+            lt.pop('sum_position', None)
+            if not torch.cuda.is_current_stream_capturing():
+                torch.cuda.empty_cache()
+        return self._scores_kept
+
+    def _kept_scores_sweeps(self, lt, kv, tail, k, dq):
+        L, H, nnz = _lib.lib(), self._heads, self._indices.shape[0]
+        # the sum's plan and positions before the arrays: the library allocates beside torch, not from what torch holds
+        total, position = self._query_sum(lt)
+        ds, other = torch.empty((2, H, nnz), dtype=torch.float32, device=self._ctx)
+        _lib.check(L.fg_graph_attention_backward_kv_ds_f32(*kv, _lib.dev_ptr(ds), *tail))
+        result = ctypes.c_void_p()
+        _lib.check(L.fg_edge_values_permute_f32(_lib.dev_ptr(ds), _lib.dev_ptr(position), nnz, H, _lib.dev_ptr(other),
+                                                ctypes.byref(result), tail[-1]))
+        flat = total._placeholders[0].shape
+        total.run_laid_out(k.view(flat), ds if result.value == ds.data_ptr() else other, dq.view((self._num_rows,) + flat[1:]))
+
+    def _own_sum(self, inputs):
+        csr = self._csr
+        total = GSpMMhip(scipy.sparse.csr_matrix((np.ones(csr.nnz, np.float32), csr.indices, csr.indptr), shape=csr.shape))
+        total.build(inputs, {}, {})
+        return total
 
     def _query_sum(self, lt):
         """(weighted sum over the adjacency with H heads, position in lt's element order of each element of its layout)."""
         if self._sum is None:
-            total = self._new_sum()
             H, D, nnz = self._heads, self._head_len, self._indices.shape[0]
-            total.build([common.placeholder((self._num_cols,) + ((D,) if H == 1 else (H, D))),
-                         common.placeholder((nnz,) if H == 1 else (nnz, H))], {}, {})
+            total = (self._new_sum or self._own_sum)([common.placeholder((self._num_cols,) + ((D,) if H == 1 else (H, D))),
+                                                      common.placeholder((nnz,) if H == 1 else (nnz, H))])
             total.out_tvm = None                    # its results go to tensors of backward()'s own
             self._sum = total
         if 'sum_position' not in lt:

@@ -58,3 +58,62 @@ def test_dots_that_would_take_more_than_the_cap_are_refused():
             assert L.fg_spmm_dot_takes(plan, F, heads, tiles) == takes, (F, heads, tiles)
     finally:
         L.fg_spmm_plan_destroy(plan)
+
+
+@pytest.mark.parametrize("where", ["sweep", "sum", "positions", "arrays"])
+@pytest.mark.parametrize("shared", [True, False])
+def test_attention_gradients_without_memory_for_the_scores_gradients(monkeypatch, where, shared):
+    """The two arrays, the weighted sum they are for, its positions or the sweep's own scratch do not fit: the second sweep."""
+    import torch
+    from featgraph_amd import _lib, tuning
+    from featgraph_amd.autograd import Graph
+    from featgraph_amd.module import GraphAttentionhip, GSpMMhip, placeholder
+    adj = _graph()
+    H, D = 4, 32
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    normal = lambda n: torch.randn((n, H, D), generator=gen, device="cuda")
+    q, k, v, dout = normal(adj.shape[0]), normal(adj.shape[1]), normal(adj.shape[1]), normal(adj.shape[0])
+
+    def step():
+        if shared:
+            leaves = [t.clone().requires_grad_() for t in (q, k, v)]
+            return torch.autograd.grad(g.attention(*leaves, scale=0.2), leaves, dout)
+        out = m.run([q, k, v])
+        return m.backward(q, k, v, out, m.state_tvm, dout)
+
+    def build():
+        m = GraphAttentionhip(adj)
+        m.build([placeholder(q.shape), placeholder(k.shape), placeholder(v.shape)], {'scale': 0.2})
+        return m
+
+    monkeypatch.setattr(tuning, "attention_keeps_score_gradients", lambda *a: False)
+    g, m = (Graph(adj), None) if shared else (None, build())
+    ref = step()
+    g, m = (Graph(adj), None) if shared else (None, build())
+    monkeypatch.setattr(tuning, "attention_keeps_score_gradients", lambda *a: True)
+    calls = []
+    if where == "sweep":
+        monkeypatch.setattr(_lib.lib(), "fg_graph_attention_backward_kv_ds_f32", _failing(calls))
+    elif where == "sum":
+        def no_plan(self, *a):
+            calls.append(1)
+            raise MemoryError("cannot allocate the plan's scratch buffer")
+        monkeypatch.setattr(GSpMMhip, "build", no_plan)
+    elif where == "positions":
+        def no_positions(self):
+            calls.append(1)
+            raise torch.cuda.OutOfMemoryError("positions")
+        monkeypatch.setattr(GSpMMhip, "layout_positions", no_positions)
+    else:
+        real = torch.empty
+
+        def no_arrays(*a, **kw):
+            if a and a[0] == (2, H, adj.nnz):
+                calls.append(1)
+                raise torch.cuda.OutOfMemoryError("arrays")
+            return real(*a, **kw)
+        monkeypatch.setattr(torch, "empty", no_arrays)
+    for _ in range(2):
+        got = step()
+        assert all(torch.equal(a, b) for a, b in zip(got, ref))
+    assert len(calls) == 1
