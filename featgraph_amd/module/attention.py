@@ -322,16 +322,21 @@ class GraphAttentionhip(object):
         self._coef = coef
         return der_t.t().contiguous(), del_t.t().contiguous(), dv
 
+    def reserve_train(self):
+        """Sizes the plan's scratch for train_forward() of the built shape (build() sizes it for run(), which needs less): to be
+        called after build() by a program whose first train_forward() is one that it captures."""
+        if self._placeholders is None or not self._additive:
+            raise RuntimeError("build() with additive scores before reserve_train()")
+        common.reserve(self._active['plan'], common.OP_ATTENTION_ADDITIVE_TRAIN, self._heads, self._head_len, 0, self._ctx)
+
     def train_forward(self, er, el, v):
         """Additive scores: (out, saved) as new tensors, `saved` being what train_backward() starts from -- the row state and
-        the sums over the edges with a positive score (as large as `out`), with which dEr takes no sweep of its own."""
+        the sums over the edges with a positive score (as large as `out`), with which dEr takes no sweep of its own.  The first call
+        on a plan may grow its scratch: reserve_train()."""
         if self._placeholders is None or not self._additive:
             raise RuntimeError("build() with additive scores before train_forward()")
         common.check_inputs([er, el, v], self._placeholders, self._ctx)
         H, D, lay = self._heads, self._head_len, self._active
-        if not getattr(self, '_train_reserved', False):
-            common.reserve(lay['plan'], common.OP_ATTENTION_ADDITIVE_TRAIN, H, D, 0, self._ctx)
-            self._train_reserved = True
         new = lambda *shape: torch.empty(shape, dtype=torch.float32, device=self._ctx)
         n = self._num_rows
         out, plus, state, share = new(n, H, D), new(n, H, D), new(n, H, 2), new(n, H)
