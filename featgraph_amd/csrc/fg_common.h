@@ -121,6 +121,7 @@ int check_device(const fg_spmm_plan *plan);
 // What one call of each operator needs (the same functions size the buffers inside the calls).
 // Each returns FG_OK or the status the call itself would return for that shape.
 int spmm_scratch_need(const fg_spmm_plan *plan, int F, int heads, int reduce, int num_feat_partitions, ScratchNeed *need);
+int spmm_dot_scratch_need(const fg_spmm_plan *plan, int F, int heads, int num_feat_partitions, ScratchNeed *need);
 int sddmm_dds_scratch_need(const fg_spmm_plan *plan, int H, int D, int num_feat_partitions, ScratchNeed *need);
 int softmax_scratch_need(const fg_spmm_plan *plan, int heads, ScratchNeed *need);
 int gspmm_bcast_scratch_need(const fg_spmm_plan *plan, int out_len, bool with_arg, ScratchNeed *need);

@@ -414,6 +414,7 @@ extern "C" int fg_spmm_plan_reserve(fg_spmm_plan *pl, int op, int heads, int hea
         case FG_OP_ATTENTION: rc = fg::attention_scratch_need(pl, heads, head_len, 2, true, &need); break;
         case FG_OP_ATTENTION_ADDITIVE: rc = fg::additive_scratch_need(pl, heads, head_len, true, false, &need); break;
         case FG_OP_ATTENTION_ADDITIVE_TRAIN: rc = fg::additive_scratch_need(pl, heads, head_len, false, true, &need); break;
+        case FG_OP_SPMM_SUM_DOTS: rc = fg::spmm_dot_scratch_need(pl, heads * head_len, heads, num_feat_partitions, &need); break;
         case FG_OP_GSPMM_BCAST: rc = fg::gspmm_bcast_scratch_need(pl, heads * head_len, false, &need); break;
         case FG_OP_GSPMM_BCAST_ARG: rc = fg::gspmm_bcast_scratch_need(pl, heads * head_len, true, &need); break;
         default: return fail(FG_ERR_ARG, "fg_spmm_plan_reserve: unknown operator %d", op);

@@ -1198,6 +1198,14 @@ bool takes_dots(const fg_spmm_plan *pl, const SpmmConfig &c, int F, int heads) {
            (heads == 1 || c.tile_w % (F / heads) == 0) && (uint64_t)dot_arrays(c) * dot_stride(pl) * 4u <= (8ull << 30);
 }
 
+// Adds the dots to a sum's scratch, behind everything else that the call keeps there (*at).
+int add_dots(const fg_spmm_plan *pl, const SpmmConfig &c, int F, int heads, fg::ScratchNeed *need, size_t *at) {
+    if (!takes_dots(pl, c, F, heads)) return fail(FG_ERR_SHAPE, "no sum with dots for %d heads of %d floats on this plan", heads, F / heads);
+    *at = (need->partial + 3) & ~(size_t)3;
+    need->partial = *at + (size_t)dot_arrays(c) * dot_stride(pl);
+    return FG_OK;
+}
+
 // Kernel tiles per launch: 8, 4, 2 or 1 -- counts that divide the 8 XCDs, so that workgroup id % tiles-per-launch
 // always puts a tile on the same XCDs and an L2 serves one tile's slice at a time (10 tiles: 8 + 2; 5: 4 + 1).  With
 // any other count every XCD would see every tile (232,965-node graph, F=640: 27.4 ms with 10 tiles in one launch).
@@ -1225,12 +1233,8 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
     // fixed_partial: the split rows' partial sums go to this buffer of fixed size instead of the plan's,
     // X is gathered from the caller's matrix (no tile-by-tile copy), and nothing is allocated.
     fg::ScratchNeed need = scratch_need(pl, c, F, reduce);
-    // dots: behind everything else that the call keeps in the plan's scratch
-    const size_t dots_at = (need.partial + 3) & ~(size_t)3;
-    if (dot) {
-        if (!takes_dots(pl, c, F, heads)) return fail(FG_ERR_SHAPE, "no sum with dots for %d heads of %d floats on this plan", heads, F / heads);
-        need.partial = dots_at + (size_t)dot_arrays(c) * dot_stride(pl);
-    }
+    size_t dots_at = 0;
+    if (dot && (rc = add_dots(pl, c, F, heads, &need, &dots_at)) != FG_OK) return rc;
     if (fixed_partial) {
         // the limit counts pieces of 1024 elements; a plan cut finer than that fills the buffer a range of columns at a time
         need.partial = (((size_t)pl->default_pieces * (size_t)F) + 3) & ~(size_t)3;
@@ -1407,6 +1411,13 @@ int spmm_scratch_need(const fg_spmm_plan *pl, int F, int heads, int reduce, int 
     if (int rc = resolve_config(pl, F, T, heads, reduce, true, &c)) return rc;
     *need = scratch_need(pl, c, F, reduce);
     return FG_OK;
+}
+int spmm_dot_scratch_need(const fg_spmm_plan *pl, int F, int heads, int T, ScratchNeed *need) {
+    SpmmConfig c;
+    size_t at;
+    if (int rc = resolve_config(pl, F, T, heads, FG_REDUCE_SUM, true, &c)) return rc;
+    *need = scratch_need(pl, c, F, FG_REDUCE_SUM);
+    return add_dots(pl, c, F, heads, need, &at);
 }
 std::string spmm_launch_text(const fg_spmm_plan *pl, int F, int T) {
     SpmmConfig c;

@@ -372,6 +372,12 @@ class GSpMMhip(VanillaSpMMhip):
                               self._num_feat_partitions, common.stream_ptr()))
         return out
 
+    def reserve_dots(self):
+        """Sizes the plan's scratch for run_with_dots() (build() sizes it for run(), which needs less): to be called after build()
+        by a program whose first such call is one that it captures.  ValueError where the library has no kernel for both."""
+        common.reserve(self._active['plan'], common.OP_SPMM_SUM_DOTS, self._heads, self._feat_len // self._heads,
+                       self._num_feat_partitions, self._ctx)
+
     def run_with_dots(self, src_feat, weights, own):
         """run([src_feat, weights]) and, in the same sweep, dots[e, h] = <own[row e, h, :], src_feat[col e, h, :]> per edge in
         the order of the weights given (set_weight_order) -- the two gradients of a weighted sum over the transposed graph.

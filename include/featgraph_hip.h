@@ -133,7 +133,8 @@ typedef enum {
     FG_OP_ATTENTION_ADDITIVE = 5, /* fg_graph_attention_additive_f32 and its two gradient calls */
     FG_OP_GSPMM_BCAST = 6,        /* fg_gspmm_bcast_f32 / _dds_f32 without arg_dev (heads * head_len = out_len) */
     FG_OP_GSPMM_BCAST_ARG = 7,    /* fg_gspmm_bcast_f32 / _dds_f32 with arg_dev */
-    FG_OP_ATTENTION_ADDITIVE_TRAIN = 8 /* fg_graph_attention_additive_train_f32 and _train_elv_f32 */
+    FG_OP_ATTENTION_ADDITIVE_TRAIN = 8, /* fg_graph_attention_additive_train_f32 and _train_elv_f32 */
+    FG_OP_SPMM_SUM_DOTS = 9       /* fg_spmm_dot_f32 (FG_ERR_SHAPE where fg_spmm_dot_takes says no) */
 } fg_op;
 int fg_spmm_plan_reserve(fg_spmm_plan *plan, int op, int heads, int head_len, int num_feat_partitions);
 
