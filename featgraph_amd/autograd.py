@@ -199,7 +199,9 @@ class Graph(object):
         softmax_r(leaky_relu(el[col e, h] + er[r, h])) * v[col e, h, :]; er (num_rows, H), el (num_cols, H),
         v (num_cols, H, D) with D in {16, 32, 64}.  One operator forward, one sweep backward; no per-edge
         array is stored (with gradients the forward pass keeps a second array of the output's size)."""
-        return _GatAttention.apply(self, er, el, v, float(negative_slope))
+        # whether gradients will be wanted is asked here: inside the function grad mode is off, and a parameter's flag is not
+        train = torch.is_grad_enabled() and any(t.requires_grad for t in (er, el, v))
+        return _GatAttention.apply(self, er, el, v, float(negative_slope), train)
 
     def _gat_mod(self, er, el, v, slope):
         key = ('gat', tuple(v.shape[1:]), slope)
@@ -397,10 +399,10 @@ class _Attention(torch.autograd.Function):
 
 class _GatAttention(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, g, er, el, v, slope):
+    def forward(ctx, g, er, el, v, slope, train):
         er, el, v = er.contiguous(), el.contiguous(), v.contiguous()
         mod = g._gat_mod(er, el, v, slope)
-        if not any(ctx.needs_input_grad):
+        if not train:
             return _fresh_run(mod, [er, el, v])
         _let_go(mod)
         out, saved = mod.train_forward(er, el, v)
@@ -412,7 +414,7 @@ class _GatAttention(torch.autograd.Function):
     def backward(ctx, dout):
         er, el, v, out, *saved = ctx.saved_tensors
         der, del_, dv = ctx.g._gat_mod(er, el, v, ctx.slope).train_backward(er, el, v, out, saved, dout.contiguous())
-        return None, der, del_, dv, None
+        return None, der, del_, dv, None, None
 
 
 class _EdgeSoftmax(torch.autograd.Function):
