@@ -404,8 +404,17 @@ class _GatAttention(torch.autograd.Function):
         mod = g._gat_mod(er, el, v, slope)
         if not train:
             return _fresh_run(mod, [er, el, v])
-        _let_go(mod)
-        out, saved = mod.train_forward(er, el, v)
+        out = None
+        if not getattr(mod, '_sums_do_not_fit', False):
+            _let_go(mod)
+            try:
+                out, saved = mod.train_forward(er, el, v)
+            except (MemoryError, torch.cuda.OutOfMemoryError):
+                mod._sums_do_not_fit = True             # a failed attempt costs device synchronisations: not at every step
+        if out is None:
+            mod.state_tvm = torch.empty_like(mod.state_tvm)
+            out = _fresh_run(mod, [er, el, v])
+            saved = (mod.state_tvm,)
         ctx.g, ctx.slope = g, slope
         ctx.save_for_backward(er, el, v, out, *saved)
         return out
@@ -413,7 +422,11 @@ class _GatAttention(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout):
         er, el, v, out, *saved = ctx.saved_tensors
-        der, del_, dv = ctx.g._gat_mod(er, el, v, ctx.slope).train_backward(er, el, v, out, saved, dout.contiguous())
+        mod = ctx.g._gat_mod(er, el, v, ctx.slope)
+        if len(saved) == 1:                             # the row state alone: dEr by a sweep of its own
+            der, del_, dv = mod.backward(er, el, v, out, saved[0], dout.contiguous())
+        else:
+            der, del_, dv = mod.train_backward(er, el, v, out, saved, dout.contiguous())
         return None, der, del_, dv, None, None
 
 

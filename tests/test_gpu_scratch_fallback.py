@@ -117,3 +117,39 @@ def test_attention_gradients_without_memory_for_the_scores_gradients(monkeypatch
         got = step()
         assert all(torch.equal(a, b) for a, b in zip(got, ref))
     assert len(calls) == 1
+
+
+@pytest.mark.parametrize("where", ["scratch", "arrays"])
+def test_additive_attention_without_memory_for_the_kept_sums(monkeypatch, where):
+    """The training pass's buffers, or the array it keeps, do not fit: the plain forward pass and a sweep of its own for dEr."""
+    import torch
+    from featgraph_amd import _lib
+    from featgraph_amd.autograd import Graph
+    from featgraph_amd.module import GraphAttentionhip
+    adj = _graph()
+    H, D = 4, 32
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    leaves = [torch.randn(s, generator=gen, device="cuda").requires_grad_() for s in ((adj.shape[0], H), (adj.shape[1], H), (adj.shape[1], H, D))]
+    dout = torch.randn((adj.shape[0], H, D), generator=gen, device="cuda")
+
+    def step(g):
+        out = g.gat_attention(*leaves)
+        return (out.detach(),) + torch.autograd.grad(out, leaves, dout)
+
+    ref = step(Graph(adj))
+    calls = []
+    if where == "scratch":
+        monkeypatch.setattr(_lib.lib(), "fg_graph_attention_additive_train_f32", _failing(calls))
+    else:
+        def no_arrays(self, *a):
+            calls.append(1)
+            raise torch.cuda.OutOfMemoryError("plus")
+        monkeypatch.setattr(GraphAttentionhip, "train_forward", no_arrays)
+    g = Graph(adj)
+    for _ in range(2):
+        got = step(g)
+        assert torch.equal(got[0], ref[0])
+        for a, b in zip(got[1:], ref[1:]):
+            # either way within 2e-6 of float64 on such rows
+            assert float((a - b).norm()) <= 4e-6 * float(b.norm())
+    assert len(calls) == 1
