@@ -115,8 +115,7 @@ class Graph(object):
         or, where there is no kernel for that, in two."""
         dy = dy.contiguous()
         mod = self._spmm_mod(True, tuple(dy.shape[1:]), 0 if w.dim() == 1 else w.shape[1])
-        like = _let_go(mod)
-        mod.out_tvm = torch.empty(like[0], dtype=like[1], device=like[2])
+        _let_go(mod)                        # the call takes a new output, once it knows that it will write one
         both = mod.run_with_dots(dy, w.contiguous(), x.contiguous())
         mod.out_tvm = None
         return both if both is not None else (self._spmm_raw(dy, w, transposed=True), self._sddmm_raw(x, dy))

@@ -75,3 +75,20 @@ def test_non_finite_rows_stay_where_they_belong():
     hit[adj.indices[row == bad]] = True
     assert np.array_equal(~np.isfinite(dx.cpu().numpy()).all(1), hit)
     assert np.array_equal(~np.isfinite(dw.cpu().numpy()), row == bad)
+
+
+@pytest.mark.parametrize("tail,outputs", [((64,), 1), ((2, 128), 1)])
+def test_one_output_is_allocated_whichever_way_is_taken(monkeypatch, tail, outputs):
+    import torch
+    from featgraph_amd.autograd import Graph
+    adj = _graph("mixed", np.random.default_rng(1))
+    g = Graph(adj)
+    x = torch.ones((adj.shape[1],) + tail, device="cuda", requires_grad=True)
+    w = torch.ones((adj.nnz,) + tail[:-1], device="cuda", requires_grad=True)
+    dy = torch.ones((adj.shape[0],) + tail, device="cuda")
+    torch.autograd.grad(g.spmm(x, w), (x, w), dy)              # builds what it needs
+    taken, empty = [], torch.empty
+    y = g.spmm(x, w)
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: taken.append(a[0]) or empty(*a, **k))
+    torch.autograd.grad(y, (x, w), dy)
+    assert taken.count(tuple(x.shape)) == outputs
