@@ -178,18 +178,19 @@ class GraphAttentionhip(object):
         self._launch(*input_tvm_ndarrays)
         return self.out_tvm
 
+    def _transposed(self, P):
+        """Position array, column ids and, for every element, its position in the adjacency's CSR order."""
+        nnz = self._indices.shape[0]
+        tr = scipy.sparse.csr_matrix((np.arange(nnz, dtype=np.int32), self._indices, self._indptr), shape=self._csr.shape).T.tocsr()
+        tr.sort_indices()
+        return util_convert_csr_to_dds(tr, P) if P > 1 else (tr.indptr, tr.indices, tr.data)
+
     def _layout_t(self, P):
         """The transposed adjacency (rows = sources) with P partitions over the destinations."""
         key = ('t', P)
         if key in self._layouts:
             return self._layouts[key]
-        nnz = self._indices.shape[0]
-        tr = scipy.sparse.csr_matrix((np.arange(nnz, dtype=np.int32), self._indices, self._indptr), shape=self._csr.shape).T.tocsr()
-        tr.sort_indices()
-        if P > 1:
-            pos, idx, csr_pos = util_convert_csr_to_dds(tr, P)
-        else:
-            pos, idx, csr_pos = tr.indptr, tr.indices, tr.data
+        pos, idx, csr_pos = self._transposed(P)
         pos = np.ascontiguousarray(pos, dtype=np.int32)
         lay = {'P': P, 'pos': common.to_device_i32(pos, self._ctx),
                'idx': common.to_device_i32(np.ascontiguousarray(idx, dtype=np.int32), self._ctx), 'plan': ctypes.c_void_p()}
@@ -201,7 +202,8 @@ class GraphAttentionhip(object):
             _lib.check(_lib.lib().fg_spmm_plan_create(_lib.host_ptr(pos), self._num_cols, self._num_rows, P,
                                                       ctypes.byref(opts), ctypes.byref(lay['plan'])))
         common.narrow_indices(lay['plan'], lay['idx'], self._num_rows, P, self._ctx)      # the transposed graph gathers from the rows
-        lay['csr_pos_host'] = csr_pos
+        if not self._additive and self._keeps_scores():
+            lay['csr_pos_host'] = csr_pos                   # until _query_sum has made its positions of it
         self._layouts[key] = lay
         return lay
 
@@ -240,8 +242,7 @@ class GraphAttentionhip(object):
         """dK and dV, and dQ from the scores' gradients that their sweep leaves; False, and nothing of them to use, where that
         does not pay or memory for it was not to be had (not tried again before the next build(): an attempt that fails
         costs device synchronisations)."""
-        nnz = self._indices.shape[0]
-        if not self._scores_kept or not tuning.attention_keeps_score_gradients(nnz, self._num_rows, self._heads, self._head_len):
+        if not self._keeps_scores():
             return False
         try:
             self._kept_scores_sweeps(lt, kv, tail, k, dq)
@@ -254,6 +255,9 @@ class GraphAttentionhip(object):
             if not torch.cuda.is_current_stream_capturing():
                 torch.cuda.empty_cache()
         return self._scores_kept
+
+    def _keeps_scores(self):
+        return self._scores_kept and tuning.attention_keeps_score_gradients(self._indices.shape[0], self._num_rows, self._heads, self._head_len)
 
     def _kept_scores_sweeps(self, lt, kv, tail, k, dq):
         L, H, nnz = _lib.lib(), self._heads, self._indices.shape[0]
@@ -282,7 +286,10 @@ class GraphAttentionhip(object):
             total.out_tvm = None                    # its results go to tensors of backward()'s own
             self._sum = total
         if 'sum_position' not in lt:
-            csr_pos = common.to_device_i32(lt['csr_pos_host'], self._ctx).long()
+            csr_pos = lt.pop('csr_pos_host', None)
+            if csr_pos is None:                             # positions of another build were made of it
+                csr_pos = self._transposed(lt['P'])[2]
+            csr_pos = common.to_device_i32(csr_pos, self._ctx).long()
             of_csr = torch.empty(csr_pos.shape, dtype=torch.int32, device=self._ctx)
             of_csr[csr_pos] = torch.arange(csr_pos.shape[0], dtype=torch.int32, device=self._ctx)
             pos = self._sum.layout_positions()

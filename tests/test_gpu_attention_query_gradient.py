@@ -62,3 +62,30 @@ def test_both_ways_match_float64(monkeypatch, kind, heads, head_len, parts):
             # about 10: 10 * 2^-24 = 6e-7 relative)
             assert float((x.double() - y).norm()) <= 2e-6 * float(y.norm()), (name, kept)
     assert torch.equal(got[True][1], got[False][1]) and torch.equal(got[True][2], got[False][2])
+
+
+def test_host_positions_are_let_go_and_made_again(monkeypatch):
+    """The elements' CSR positions (4 bytes per edge) stay on the host only until the device has the positions made of them, not at
+    all where nothing will be, and a second build() makes its own."""
+    import torch
+    from featgraph_amd import tuning
+    from featgraph_amd.module import GraphAttentionhip, placeholder
+    adj = _graph("mixed", np.random.default_rng(1))
+    monkeypatch.setattr(tuning, "attention_keeps_score_gradients", lambda *a: True)
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    m = GraphAttentionhip(adj)
+    for heads, head_len in ((4, 16), (1, 64)):
+        q, k, v, dout = (torch.randn((n, heads, head_len), generator=gen, device="cuda") for n in adj.shape[:1] + adj.shape[1:] * 2 + adj.shape[:1])
+        m.build([placeholder(q.shape), placeholder(k.shape), placeholder(v.shape)], {'scale': 0.3}, {'num_dst_partitions': 2})
+        out = m.run([q, k, v])
+        got = m.backward(q, k, v, out, m.state_tvm, dout)
+        for x, y in zip(got, _float64(adj, q, k, v, dout, 0.3)):
+            assert float((x.double() - y).norm()) <= 2e-6 * float(y.norm())      # as above
+        assert [lay for lay in m._layouts.values() if 'csr_pos_host' in lay] == []
+        assert len([lay for lay in m._layouts.values() if 'sum_position' in lay]) == 1
+    m = GraphAttentionhip(adj)
+    er, el, v = (torch.randn(s, generator=gen, device="cuda") for s in ((adj.shape[0], 2), (adj.shape[1], 2), (adj.shape[1], 2, 32)))
+    m.build([placeholder(t.shape) for t in (er, el, v)], {'scores': 'additive'})
+    out, saved = m.train_forward(er, el, v)
+    m.train_backward(er, el, v, out, saved, torch.ones_like(out))
+    assert [lay for lay in m._layouts.values() if 'csr_pos_host' in lay] == []
