@@ -15,6 +15,7 @@ import numpy as np
 import scipy.sparse
 import torch
 
+from . import tuning
 from .module import (EdgeSoftmaxhip, GraphAttentionhip, GSDDMMhip, GSpMMhip, MultiHeadSDDMMhip, VanillaSDDMMhip,
                      placeholder)
 from .module.general import parse_message
@@ -112,12 +113,17 @@ class Graph(object):
 
     def _spmm_grads_raw(self, x, w, dy):
         """(A(w)^T dy, <dy[row e], x[col e]> per edge) in one sweep over the transposed graph, which gathers dy once for both,
-        or, where there is no kernel for that, in two."""
+        or, where that is slower or there is no kernel for it, in two."""
         dy = dy.contiguous()
         mod = self._spmm_mod(True, tuple(dy.shape[1:]), 0 if w.dim() == 1 else w.shape[1])
-        _let_go(mod)                        # the call takes a new output, once it knows that it will write one
-        both = mod.run_with_dots(dy, w.contiguous(), x.contiguous())
-        mod.out_tvm = None
+        if getattr(mod, '_one_sweep', None) is None:
+            mod._one_sweep = tuning.sum_gradients_in_one_sweep(self.shape[0], self.shape[1], self.nnz, mod._heads,
+                                                               dy.shape[-1])
+        both = None
+        if mod._one_sweep:
+            _let_go(mod)                    # the call takes a new output, once it knows that it will write one
+            both = mod.run_with_dots(dy, w.contiguous(), x.contiguous())
+            mod.out_tvm = None
         return both if both is not None else (self._spmm_raw(dy, w, transposed=True), self._sddmm_raw(x, dy))
 
     def _sddmm_raw(self, src, dst):

@@ -1187,13 +1187,11 @@ int dot_arrays(const SpmmConfig &c) { return c.n_ftiles * c.hpt; }
 size_t dot_stride(const fg_spmm_plan *pl) { return ((size_t)pl->nnz + 3) & ~(size_t)3; }
 // Whether this configuration takes the kernels with dots: whole tiles of 128-bit lanes, one load per lane, 32-bit offsets,
 // a wavefront's own place for every row of every pass, and no tile that cuts a head of several (its parts would have to be
-// added up).  Tiles of several heads keep few wavefronts in flight (104 registers): below 128 floats per row they lose on
-// large graphs what the second gather costs.  The arrays of dots are the plan's scratch from the first call on: 8 GiB of it at most,
-// as for the passes' buffers.  Step with both gradients, separate sweeps -> one: 12.5 M elements 4 x 8
-// 790 -> 874 us, 2 x 32 911 -> 957, 8 x 16 1831 -> 1808; 4 M: 357 -> 364, 602 -> 563, 950 -> 840; 400,000: 161 -> 145, 268 -> 191, 168 -> 152.
+// added up).  The arrays of dots are the plan's scratch from the first call on: 8 GiB of it at most, as for the passes' buffers.
+// Where two sweeps are faster is the caller's to know (tiles of several heads keep few wavefronts in flight: 104 registers).
 bool takes_dots(const fg_spmm_plan *pl, const SpmmConfig &c, int F, int heads) {
     return c.V == 4 && c.K == 1 && c.full && c.off32 && c.sub_per_tile == 1 &&
-           !(c.hpt > 1 && (c.L < 8 || (F < 128 && pl->nnz >= (4 << 20)))) &&
+           !(c.hpt > 1 && c.L < 8) &&
            (pl->num_col_partitions == 1 || uses_pass_buffers(pl, c, F, FG_REDUCE_SUM)) &&
            (heads == 1 || c.tile_w % (F / heads) == 0) && (uint64_t)dot_arrays(c) * dot_stride(pl) * 4u <= (8ull << 30);
 }

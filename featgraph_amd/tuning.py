@@ -398,3 +398,32 @@ def attention_keeps_score_gradients(nnz, num_rows, heads, head_len):
     if heads % 4:
         return nnz <= 32 * num_rows
     return head_len == 16 or heads % 8 == 0 or nnz <= 128 * num_rows
+
+
+def sum_gradients_in_one_sweep(num_rows, num_cols, nnz, heads, head_len):
+    """Whether the two gradients of a weighted sum come faster from one sweep over the transposed graph than from a sum and a
+    separate SDDMM (heads of head_len floats).  The kernels with dots lose where a lane group is
+    small -- tiles of one head of 16 floats, of several short heads -- and the SDDMM has whole tiles for the shape; they win
+    many times over where it has not.  Whole steps, two sweeps -> one, in us:
+      one head, 16 floats: 400,000 elements 69 -> 65 (degree 8); 4 M 179 -> 198 (30), 13 M 453 -> 492 (120); 32 floats: 2 M 161 -> 172 (8), 4 M 236 -> 240
+        (20), 216 -> 219 (30), 12.5 M 455 -> 425 (215); 24, run as 32: 4 M 302 -> 285 (20); 64: 4 M 560 -> 496 (8), 370 -> 321 (30), 238 -> 206 (120)
+      2x16: 100,000 74 -> 71, 400,000 93 -> 97, 4 M 528 -> 577 (8), 334 -> 415 (30), 212 -> 275 (120)
+      4x16: 4 M 668 -> 582 (8), 300 -> 298 (120); 13 M 2106 -> 1876 (8), 1231 -> 1130 (120), but 945 -> 973 (215)
+      4x8 / 8x8 / 2x32, 1 M: 155 -> 143 / 218 -> 194 / 178 -> 166 (8), 157 -> 150 / 161 -> 162 / 152 -> 147 (30); 4 M: 306 -> 325 / 552 -> 560 /
+        464 -> 469 (30), 225 -> 244 / 402 -> 458 / 260 -> 299 (120)
+      16x8: 4 M 1572 -> 1469 (8), 1112 -> 1039 (30), 825 -> 840 (120); 3x32, 6x32: 1020 -> 959, 1913 -> 1851 (8), 613 -> 643, 1442 -> 1449 (30);
+        13 M 1397 -> 1593, 2991 -> 3407 (120)
+      4x32, 8x32, 8x16: 4 M 852 -> 667, 1744 -> 1288, 933 -> 790 (30), 454 -> 391, 925 -> 781, 573 -> 555 (120)
+      no tile of the SDDMM's: 3x16 1128 -> 423, 6x32 1092 -> 412, 12x8 3403 -> 975 (4 M, 2 M, 4 M; 120)"""
+    feat_len = heads * head_len
+    if heads == 1:
+        return nnz < 1 << 20 or head_len > 16 and (head_len != 32 or nnz >= 24 * num_rows)
+    if head_len >= 64 or not _is_pow2(feat_len) and choose_sddmm(num_rows, num_cols, nnz, heads, head_len) is None:
+        return True
+    if head_len == 16:
+        if heads % 4:
+            return nnz < 1 << 18
+        return feat_len >= 128 or nnz < 1 << 22 or nnz <= 128 * num_rows
+    if head_len == 32 and _is_pow2(feat_len) and feat_len >= 128:
+        return True
+    return nnz < 1 << 20 or (feat_len >= 128 and nnz <= (16 if head_len == 32 else 64) * num_rows)

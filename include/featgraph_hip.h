@@ -237,7 +237,7 @@ int fg_gspmm_f32(fg_spmm_plan *plan, const int32_t *pos_dev, const int32_t *idx_
  * for every element t of the layout, own_dev [n_dst, heads, own_len] (own_len <= F / heads; columns of x beyond it count
  * as zeros of own).  Without elements this is fg_gspmm_f32: own_dev, edge_pos_dev and dots_dev are not read and may be
  * NULL.  fg_spmm_dot_takes says whether this plan and shape do (arrays 16-byte aligned): whole tiles of 16 to 256
- * floats, X below 4 GiB, with several partitions every pass in a buffer of its own, and at most 8 GiB of scratch for the
+ * floats, X below 4 GiB (whether one sweep is also the faster way depends on the graph: tuning.sum_gradients_in_one_sweep), with several partitions every pass in a buffer of its own, and at most 8 GiB of scratch for the
  * dots (nnz floats per head, or per tile with one head).  FG_ERR_NOMEM leaves a plan that a plain sum can still use.
  */
 int fg_spmm_dot_takes(const fg_spmm_plan *plan, int F, int heads, int num_feat_partitions);
