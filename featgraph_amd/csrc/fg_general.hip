@@ -875,12 +875,15 @@ int gspmm_bcast_run(fg_spmm_plan *pl, const int32_t *pos_dev, const int32_t *idx
     // Feature tiles of 64 floats over the workgroups (as for the weighted sum) when an operand is gathered from the
     // source nodes and the 128-bit paths apply: a partition's slice of a tile is what an L2 has to hold.
     // (Not with an operand streamed from the edges, which sets the time.  With positions of the selected elements for copies
-    // only: copy_u max, F=128 / 256 / 512, 12.5M edges on 58,000 nodes 586 -> 539 / 1061 -> 1045 / 2501 -> 1963 us, 8M on 200,000
-    // 504 -> 462 / 1105 -> 896 / 2294 -> 1964; u_add_e max, which instructions bound, 669 -> 683 / 1132 -> 1270 / 2573 -> 2403 and
-    // 509 -> 549 / 1101 -> 1030 / 2320 -> 2198.)
+    // only, in tiles that divide the 8 XCDs, from degree 32 on: below that a row's start and end cost each tile more than the
+    // L2s gain.  copy_u max with its gradient, untiled -> tiled, F=128 / 256 / 512, 4M edges: degree 200 219 -> 210 / 415 -> 362 / 922 -> 682 us,
+    // 80 384 -> 353 / 873 -> 724 / 1812 -> 1358, 40 (F=128 / 256) 723 -> 706 / 1491 -> 1394, 30 985 -> 974 / 1976 -> 1887 / 3919 -> 3780, 15 1857 -> 1859 / 3583 -> 3630 / 7087 -> 7231; 9M edges of
+    // degree 15 4287 -> 4385 / 8284 -> 8528 / 16374 -> 16879; F=192 / 320 at degree 200 313 -> 338 / 605 -> 614.  Below 2^15 edges
+    // launches are all there is, and either is the other's time.  u_add_e max, which instructions bound, 12.5M edges on 58,000 nodes 669 -> 683 / 1132 -> 1270 / 2573 -> 2403, 8M on 200,000 509 -> 549 / 1101 -> 1030 / 2320 -> 2198.)
     const bool gathers = (uses_l && lhs_target == FG_TARGET_U) || (uses_r && rhs_target == FG_TARGET_U);
     const bool streams = (uses_l && lhs_target == FG_TARGET_E && lmode == 1) || (uses_r && rhs_target == FG_TARGET_E && rmode == 1);
-    const int T = (V == 4 && gathers && !streams && (!arg_dev || op == FG_BIN_COPY_LHS) && out_len >= 128 && out_len % 64 == 0) ? out_len / 64 : 1;
+    int T = (V == 4 && gathers && !streams && out_len >= 128 && out_len % 64 == 0) ? out_len / 64 : 1;
+    if (arg_dev && !(op == FG_BIN_COPY_LHS && (T & (T - 1)) == 0 && pl->nnz >= 32 * pl->n_dst) && pl->nnz >= (1 << 15)) T = 1;
     a.n_tiles = T; a.tile_vecs = T > 1 ? 16 : (out_len + V - 1) / V;
     a.F = out_len; a.L = lanes_for(T > 1 ? 16 : out_len / V);
     a.item_off = pl->item_off_dev; a.edge_pos = edge_pos_dev; a.n_parts = P; a.final = P == 1;

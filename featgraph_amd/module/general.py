@@ -90,6 +90,7 @@ class BroadcastOp(object):
             if t is not None and (t not in TARGET or (t == 'v' and not allow_v)):
                 raise ValueError("operand target %r is not valid here" % (t,))
         self.op = op
+        self.num_rows, self.nnz = num_rows, nnz
         self.lhs_target, self.rhs_target = lhs_target, rhs_target
         l_shape = check_operand_shape(lhs_ph, lhs_target, num_rows, num_cols, nnz, "the left operand") if lhs_ph is not None else None
         r_shape = check_operand_shape(rhs_ph, rhs_target, num_rows, num_cols, nnz, "the right operand") if rhs_ph is not None else None
@@ -110,8 +111,8 @@ class BroadcastOp(object):
     def feature_tiles(self, return_arg=False):
         """The number of 64-float feature tiles the library's SpMM kernel will cut this message into (it does so from
         128 output features on, when an operand is gathered from the source nodes, none is streamed from the edges
-        with 4 consecutive features per lane, positions are asked for of a copy only and 4 features per lane are possible: every
-        operand's groups of 4 consecutive or equal)."""
+        with 4 consecutive features per lane and 4 features per lane are possible: every operand's groups of 4 consecutive or
+        equal; with positions for copies only: in a power of two of tiles from 32 edges per row on, or below 2^15 edges)."""
         def wide(off, length, vec_flag, splat_flag):
             if length == 0:
                 return 1                                    # operand not used
@@ -121,9 +122,13 @@ class BroadcastOp(object):
         l, r = wide(self.lhs_off, self.lhs_len, 1, 2), wide(self.rhs_off, self.rhs_len, 4, 8)
         vec = self.out_len % 4 == 0 and l and r and not (l == 2 and r == 2)
         streams = (self.lhs_target == 'e' and self.lhs_len > 0 and l == 1) or (self.rhs_target == 'e' and self.rhs_len > 0 and r == 1)
-        if vec and not streams and (not return_arg or self.op == 'copy_lhs') and self.gathered_len() > 0 and self.out_len >= 128 and self.out_len % 64 == 0:
-            return self.out_len // 64
-        return 1
+        if not vec or streams or self.gathered_len() == 0 or self.out_len < 128 or self.out_len % 64:
+            return 1
+        tiles = self.out_len // 64
+        if return_arg and (self.op != 'copy_lhs' or
+                           (self.nnz >= 1 << 15 and (tiles & (tiles - 1) or self.nnz < 32 * self.num_rows))):
+            return 1
+        return tiles
 
     def gathered_len(self):
         """Feature length of the operand that is gathered from the source nodes (0: none is)."""

@@ -265,3 +265,22 @@ def test_positions_in_feature_tiles(oracle, special, reduce, feat_len):
             out = m.run([torch.from_numpy(a).cuda() for a in arrays]).cpu().numpy()
             assert np.array_equal(out, ref, equal_nan=True), (msg, P)
             assert np.array_equal(m.arg_tvm.cpu().numpy(), ref_arg), (msg, P)
+
+
+@pytest.mark.parametrize("degree,feat_len,tiles", [(64, 128, 2), (64, 256, 4), (64, 192, 1), (20, 128, 1), (20, 256, 1)])
+@pytest.mark.parametrize("reduce", ["max", "min"])
+def test_positions_on_either_side_of_the_tiling_rule(oracle, degree, feat_len, tiles, reduce):
+    """From 2^15 edges on the feature axis is cut for positions where the degree and the number of tiles make it pay; values and
+    positions are the oracle's either way, over one and several partitions."""
+    import torch
+    from featgraph_amd.module import GSpMMhip, placeholder
+    rng = np.random.default_rng(degree + feat_len)
+    adj = _graph(rng, [degree] * ((1 << 15) // degree + 1))
+    x = rng.integers(-1, 2, size=(700, feat_len)).astype(np.float32)
+    ref, ref_arg = oracle.gspmm_bcast(adj.indptr, adj.indices, "copy_lhs", reduce, x, None, "u", "e")
+    for P in (None, 3):
+        m = GSpMMhip(adj)
+        m.build([placeholder(x.shape)], {'msg': 'copy_u', 'reduce': reduce, 'return_arg': True}, {'num_src_partitions': P})
+        assert m._bop.feature_tiles(True) == tiles
+        out = m.run([torch.from_numpy(x).cuda()]).cpu().numpy()
+        assert np.array_equal(out, ref) and np.array_equal(m.arg_tvm.cpu().numpy(), ref_arg), P
