@@ -89,3 +89,10 @@ def test_host_positions_are_let_go_and_made_again(monkeypatch):
     out, saved = m.train_forward(er, el, v)
     m.train_backward(er, el, v, out, saved, torch.ones_like(out))
     assert [lay for lay in m._layouts.values() if 'csr_pos_host' in lay] == []
+
+
+@pytest.mark.parametrize("kind", ["few", "edges"])
+@pytest.mark.parametrize("heads,head_len", [(8, 16), (8, 64), (12, 16)])
+def test_relayout_of_eight_and_of_twelve_heads(monkeypatch, kind, heads, head_len):
+    """The scores' gradients of 8 heads go through a relayout kernel of their own, those of 12 through the one for any count."""
+    test_both_ways_match_float64(monkeypatch, kind, heads, head_len, 3)

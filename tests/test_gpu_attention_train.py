@@ -68,3 +68,46 @@ def test_step_matches_float64(monkeypatch, kind, heads, head_len, parts, pass_bu
             assert float((x.double() - y).norm()) <= bound * float(y.norm()), (name, shift)
         with torch.no_grad():
             assert torch.equal(g.gat_attention(er, el, v, negative_slope=slope), got[0])
+
+
+@pytest.mark.parametrize("kind", ["few", "edges"])
+@pytest.mark.parametrize("heads,head_len", [(1, 64), (4, 16)])
+@pytest.mark.parametrize("parts,pass_buffers", [(1, 0), (3, 0), (3, 2)])
+def test_non_finite_rows_stay_where_they_belong(monkeypatch, kind, heads, head_len, parts, pass_buffers):
+    """A source with an infinite row of V, a destination with an infinite row of dout: only what the formulas give them."""
+    import torch
+    from featgraph_amd import _lib, tuning
+    from featgraph_amd.autograd import Graph
+    monkeypatch.setattr(tuning, "_partitions", lambda *a, **k: parts)
+    monkeypatch.setattr(_lib, "plan_opts", _lib.FgPlanOpts(pass_buffers=pass_buffers))
+    adj = _graph(kind, np.random.default_rng(heads + parts))
+    adj.sort_indices()
+    n_dst, n_src = adj.shape
+    row = np.repeat(np.arange(n_dst), np.diff(adj.indptr))
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    normal = lambda *shape: torch.randn(shape, generator=gen, device="cuda")
+    er, el, v, dout = normal(n_dst, heads), normal(n_src, heads), normal(n_src, heads, head_len), normal(n_dst, heads, head_len)
+    g = Graph(adj)
+
+    def step(v, dout):
+        leaves = [t.clone().requires_grad_() for t in (er, el, v)]
+        out = g.gat_attention(*leaves)
+        return (out.detach(),) + torch.autograd.grad(out, leaves, dout)
+
+    clean = step(v, dout)
+    degree = np.bincount(adj.indices, minlength=n_src)
+    c = int(np.flatnonzero(degree > 0)[degree[degree > 0].argmin()])      # referenced by few rows
+    r = int(np.flatnonzero(np.diff(adj.indptr) > 0)[0])
+    rows_of_c = np.isin(np.arange(n_dst), row[adj.indices == c])
+    cols_of = lambda rows: np.isin(np.arange(n_src), adj.indices[np.isin(row, np.flatnonzero(rows))])
+    only_r = np.arange(n_dst) == r
+    vb, db = v.clone(), dout.clone()
+    vb[c] = float("inf")
+    db[r] = float("inf")
+    none_r, none_c = np.zeros(n_dst, bool), np.zeros(n_src, bool)
+    for got, hits in ((step(vb, dout), (rows_of_c, rows_of_c, cols_of(rows_of_c), none_c)),
+                      (step(v, db), (none_r, only_r, cols_of(only_r), cols_of(only_r)))):
+        for name, x, y, hit in zip(("out", "dEr", "dEl", "dV"), got, clean, hits):
+            hit = torch.from_numpy(hit).cuda()
+            assert not bool(torch.isfinite(x[hit]).any()), name
+            assert torch.equal(x[~hit], y[~hit]), name

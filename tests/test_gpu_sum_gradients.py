@@ -92,3 +92,32 @@ def test_one_output_is_allocated_whichever_way_is_taken(monkeypatch, tail, outpu
     monkeypatch.setattr(torch, "empty", lambda *a, **k: taken.append(a[0]) or empty(*a, **k))
     torch.autograd.grad(y, (x, w), dy)
     assert taken.count(tuple(x.shape)) == outputs
+
+
+@pytest.mark.parametrize("tail", [(16,), (64,), (4, 16), (2, 32), (4, 8)])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_non_finite_rows_stay_where_they_belong_on_short_rows(tail, value):
+    """Rows of a few elements, which lane groups walk on their own: the slots past a row's end hold other groups' elements, whose
+    weights may have given way to dot products already."""
+    import torch
+    from featgraph_amd.autograd import Graph
+    adj = _graph("few", np.random.default_rng(2))
+    out_degree = np.bincount(adj.indices, minlength=adj.shape[1])
+    assert out_degree.max() <= 5 and (out_degree > 0).sum() >= 64      # whole rows of the transposed graph, many to an item
+    row = np.repeat(np.arange(adj.shape[0]), np.diff(adj.indptr))
+    bad = row[::37]                                                      # destinations of every 37th edge
+    w = torch.rand((adj.nnz,) + tail[:-1], device="cuda").add_(0.5).requires_grad_()
+    x = torch.ones((adj.shape[1],) + tail, device="cuda", requires_grad=True)
+    clean = torch.ones((adj.shape[0],) + tail, device="cuda")
+    dy = clean.clone()
+    dy[torch.from_numpy(bad).cuda()] = value
+    g = Graph(adj)
+    y = g.spmm(x, w)
+    want = torch.autograd.grad(y, (x, w), clean, retain_graph=True)
+    dx, dw = torch.autograd.grad(y, (x, w), dy)
+    hit_w = np.isin(row, bad)
+    hit_x = np.isin(np.arange(adj.shape[1]), adj.indices[hit_w])
+    for got, ref, hit in ((dx, want[0], hit_x), (dw, want[1], hit_w)):
+        hit = torch.from_numpy(hit).cuda()
+        assert not bool(torch.isfinite(got[hit]).any())
+        assert torch.equal(got[~hit], ref[~hit])
