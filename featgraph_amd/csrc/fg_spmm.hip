@@ -619,7 +619,7 @@ size_t dot_stride(const fg_spmm_plan *pl) { return ((size_t)pl->nnz + 3) & ~(siz
 // Whether this configuration takes the kernels with dots: whole tiles of 128-bit lanes, one load per lane, 32-bit offsets,
 // a wavefront's own place for every row of every pass, and no tile that cuts a head of several (its parts would have to be
 // added up).  The arrays of dots are the plan's scratch from the first call on: 8 GiB of it at most, as for the passes' buffers.
-// Where two sweeps are faster is the caller's to know (tiles of several heads keep few wavefronts in flight: 104 registers).
+// Where two sweeps are faster is the caller's to know (tiles of several heads keep few wavefronts in flight: 88 to 97 registers).
 bool takes_dots(const fg_spmm_plan *pl, const SpmmConfig &c, int F, int heads) {
     return c.V == 4 && c.K == 1 && c.full && c.off32 && c.sub_per_tile == 1 &&
            !(c.hpt > 1 && c.L < 8) &&
