@@ -390,7 +390,11 @@ def attention_keeps_score_gradients(nnz, num_rows, heads, head_len):
       20,000 nodes, 4 M edges: 4x64 1335 -> 1160, 4x32 696 -> 643, 2x32 332 -> 348
       200,000 nodes, 4 M edges: 8x64 7345 -> 6221, 4x32 1857 -> 1651, 2x32 876 -> 835, 1x32 454 -> 432, 1x16 395 -> 392
       100,000 nodes, 8 M edges: 4x32 1956 -> 1842, 2x32 930 -> 935
-      20,000 nodes, 200,000 edges (launches): 4x64 183 -> 165, 2x64 147 -> 157, 8x16 218 -> 206, 4x32 136 -> 163"""
+      20,000 nodes, 200,000 edges (launches): 4x64 183 -> 165, 2x64 147 -> 157, 8x16 218 -> 206, 4x32 136 -> 163
+      heads of 64, one / two / three / four of them: 200,000 nodes, 1.6 M edges 541 -> 468, 1054 -> 899, 1581 -> 1350, 2169 -> 1864; 400,000, 6 M
+        1594 -> 1445, 3244 -> 2921, 4960 -> 4439, 7555 -> 6419; 100,000, 8 M 1586 -> 1294, 3200 -> 2728, 5323 -> 4576, 6388 -> 5344; 10,000, 3.9 M
+        275 -> 263, 528 -> 496, 1422 -> 1148, 1119 -> 977; sources skewed, 20,000, 3.7 M 1024 -> 1017, 1205 -> 1181, 2087 -> 1842, 1677 -> 1552;
+        sources skewed, 200,000, 6 M 4624 -> 4525, 6401 -> 6215, 7746 -> 7379, 9135 -> 8549"""
     if nnz * heads * head_len < 3 << 24 or 2 * 4 * nnz * heads > ATTENTION_EDGE_BYTES:
         return False
     if head_len == 64:
