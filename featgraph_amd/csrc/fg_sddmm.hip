@@ -1,16 +1,12 @@
 // Edge-wise dot products (SDDMM) for gfx950, single- and multi-head:
 //   out[e, h] = sum_{d<D} src[col[e], h, d] * dst[row[e], h, d]
 //
-// Edge-parallel: a wavefront owns a run of consecutive stored edges.  A group of L lanes
-// covers one edge's F = H*D floats with K vector loads per operand, the 64/L groups work on
-// different edges at once, and each head's products are added across its lanes with a
-// butterfly of cross-lane shuffles.  Row/column ids are staged in LDS (up to 256 edges per
-// wavefront), results are collected in registers and written back as dense runs.  When the
-// stored order keeps equal row ids together (CSR order, 2-D partitioned order) the dst row
-// already held in registers is reused instead of fetched again.
+// Two traversals.  In stored (or row) order a wavefront owns a run of consecutive edges and works on (edge, head) pairs:
+// sddmm_coo_kernel, sddmm_csr_kernel.  Over a source-column-partitioned, feature-tiled edge list: sddmm_tiled_kernel.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "fg_common.h"
 #include "fg_device.h"
@@ -24,17 +20,10 @@ namespace {
 
 constexpr int kWavesPerBlock = 4;
 constexpr int kBlock = 64 * kWavesPerBlock;
-constexpr int kEdgesPerWave = 256;       // COO kernel: stored edges per wavefront
-constexpr int kMaxHeadsFast = 16;        // most heads the lane layouts below cover (4 loads x 4 heads)
-
-template <int V> struct Vec;
-template <> struct Vec<4> { using type = float4; };
-template <> struct Vec<1> { using type = float; };
 
 __device__ __forceinline__ float vdot(const float4 &a, const float4 &b) {
     return a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w;
 }
-__device__ __forceinline__ float vdot(const float &a, const float &b) { return a * b; }
 __device__ __forceinline__ float4 vzero4() { return make_float4(0.f, 0.f, 0.f, 0.f); }
 
 // Sum over the RW consecutive lanes of a head segment; every lane of the segment gets it.
@@ -52,182 +41,271 @@ __device__ __forceinline__ float segment_sum(float v) {
     return v;
 }
 
+// ---- stored order -----------------------------------------------------------------------------
+//
+// A group of L lanes covers one head of one edge, 4 * L floats (a chunk) at a time.  `side` heads (the largest power of two that
+// divides H and leaves every group a head) go side by side, so that a unit -- `side` heads of one edge -- is what a wavefront
+// stages and steps over: src and dst are matrices of n * H / side rows of side * D floats, unit (e, b) multiplies rows
+// col[e] * H / side + b and row[e] * H / side + b, and its results are `side` consecutive floats.  One kernel so takes every head
+// count and every length from 4 floats on.  A wavefront takes batch_steps(L) units per lane group at once (a batch), all
+// their gathers of a chunk in flight together.  The last, partly filled chunk of a head is read as 128-bit words
+// that end at its last float, and what a lane has read twice or too much is replaced by zeros in both operands: no length
+// needs padding or scalar loads.
+//
+// Bound by the rate of gathers (the texture-address path, 64 bytes per clock and CU) where the operands sit in the
+// caches, so a batch whose units multiply one and the same destination row (a uniform test; most batches of a graph in
+// row order) reads it once instead of once per unit; heads of 8 or 16 floats by vector instructions.  Measured against a kernel
+// that held a row's 256 consecutive edges per wavefront, both operands of every edge gathered, lanes masked or scalar where
+// a length did not fit, and one edge at a time for the head counts without a shape (us; nodes, edges):
+//   10,000, 170,000: F=32 7.7 -> 5.0, F=71 70 -> 9.7, F=512 84 -> 35, 4 heads of 48 139 -> 17
+//   15,500, 6.3 M (rows of 408): F=64 103 -> 75, F=71 351 -> 128, F=338 2132 -> 1007, F=512 1505 -> 1415, 3x16 1088 -> 107
+//   104,000, 530,000: F=64 22.5 -> 21.5, F=71 95 -> 35, 8x32 94 -> 90;  58,000, 12.5 M: F=16 76 -> 74, 4x48 3691 -> 1056
+
+// Units per lane group and batch.  Heads of a few lanes are bound by vector instructions and want wavefronts, not loads, in
+// flight: with 8 units on 4 lanes (96 registers, 4 units: 72) rows of 16 floats take 79.9 us for 74.3 on 12.5 M edges of 58,000 nodes.
+__host__ __device__ constexpr int batch_steps(int L) { return L <= 4 ? 4 : 8; }
+constexpr int kStageUnits = fg::kItemEdges;    // most units staged per wavefront at a time
+constexpr int kMinDot = 4;                     // shorter heads: sddmm_short_kernel
+
 struct SddmmArgs {
-    const int32_t *row;     // COO kernel: row id per stored edge
-    const int32_t *col;     // column id per stored edge
+    const int32_t *row;     // COO kernel: row id per edge
+    const int32_t *col;     // column id per edge
+    const int32_t *edge_pos;   // COO kernel: where edge e's results go (null: at e)
     const Item *items;      // CSR kernel: plan items
     int64_t n_items;
     const int32_t *pos;     // CSR kernel: row boundaries (indptr)
     int64_t n_edges;
+    int edges_per_wave;     // COO kernel
     const float *src;       // gathered by col
     const float *dst;       // gathered by row
     float *out;             // [E, H]
-    int F;                  // H * D
+    int H, D;
+    int side;               // heads of a unit
 };
 
-// Layout of one edge over its group of L lanes: lane li, load k covers floats
-// [k*L*V + li*V, +V).  A head is RW lanes wide inside one load (KH == 1, L/RW heads per
-// load) or spans KH whole loads (RW == L).  Heads per edge: (L / RW) * (K / KH).
-template <int V, int L, int K, int RW, int KH>
-struct Shape {
-    using vec = typename Vec<V>::type;
-    static constexpr int G = 64 / L;
-    static constexpr int HPL = L / RW;          // heads per load
-    static constexpr int NH = K / KH;           // head groups along k
-    static constexpr int H = HPL * NH;
-};
+using W4 = fg::Words4<float>;                  // 128 bits, aligned like a float
 
-// dot products of one edge's operands, reduced per head; result valid in every lane of the
-// head's segment, for head group kk in q[kk].
-template <int V, int L, int K, int RW, int KH, bool FULL>
-__device__ __forceinline__ void edge_heads(const typename Vec<V>::type (&s)[K], const typename Vec<V>::type (&d)[K],
-                                           const bool (&on)[K], float (&q)[K / KH]) {
+// U values per lane, each to be summed over the L lanes of a lane group: at every step a lane keeps half of its values
+// and hands the other half to its partner, so that the sums end up spread over the group: lane i holds the value(s)
+// kept(i) .. kept(i) + n - 1 (n = U / L, or 1) and, where L > U, several lanes hold the same one.  22 operations for
+// eight values over 16 lanes instead of 8 butterflies of 4.
+template <int CTRL, int N>
+__device__ __forceinline__ void trade_half(float *p, bool hi) {
+    if constexpr (N > 1) {
 #pragma unroll
-    for (int kk = 0; kk < K / KH; ++kk) {
-        float p = 0.f;
-#pragma unroll
-        for (int k = kk * KH; k < (kk + 1) * KH; ++k)
-            if (FULL || on[k]) p += vdot(s[k], d[k]);
-        q[kk] = segment_sum<RW>(p);
+        for (int i = 0; i < N / 2; ++i) p[i] = (hi ? p[N / 2 + i] : p[i]) + dpp_move<CTRL>(hi ? p[i] : p[N / 2 + i]);
+    } else {
+        p[0] += dpp_move<CTRL>(p[0]);
     }
 }
+template <int L, int U>
+__device__ __forceinline__ void spread_sums(float (&p)[U], int lane) {
+    static_assert(L <= 32 && (L < 32 || U > 1), "lane groups of up to 32");
+    constexpr int n32 = L >= 32 ? U / 2 : U, n16 = L >= 16 ? (n32 + 1) / 2 : n32, n8 = L >= 8 ? (n16 + 1) / 2 : n16,
+                  n4 = L >= 4 ? (n8 + 1) / 2 : n8;
+    if constexpr (L >= 32) {                   // lanes i and i ^ 16: even 16-lane rows keep the first half of the values
+#pragma unroll
+        for (int i = 0; i < n32; ++i) {
+            fg::swap_rows(p[i], p[n32 + i]);
+            p[i] += p[n32 + i];
+        }
+    }
+    if constexpr (L >= 16) trade_half<0x140, n32>(p, (lane & 8) != 0);     // lane 15 - i
+    if constexpr (L >= 8) trade_half<0x141, n16>(p, (lane & 4) != 0);      // lane 7 - i
+    if constexpr (L >= 4) trade_half<0x4E, n8>(p, (lane & 2) != 0);        // lane i ^ 2
+    trade_half<0xB1, n4>(p, (lane & 1) != 0);                              // lane i ^ 1
+}
+template <int L, int U>
+struct Spread {
+    static constexpr int per_lane = L >= U ? 1 : U / L, lanes = L >= U ? L / U : 1;      // lanes that hold one value
+    // the first value that lane `i` of a group ends up with, and whether it is the one to store it
+    static __device__ __forceinline__ int kept(int i) { return L >= U ? i / lanes : i * per_lane; }
+    static __device__ __forceinline__ bool stores(int i) { return i % lanes == 0; }
+};
 
-// Dot products of the staged edges [0, n) of `edge` (x = column id, y = row id); results go to
-// out[j * H + head] for staged edge j.  The G lane groups take edges g, g+G, ...; U steps' src
-// loads are issued back to back.  Per-head results are collected in registers -- the lane
-// whose position in its head segment equals the step number (mod RW) keeps that step's value
-// -- and written out every RW steps as one dense run of RW*G*H floats.
-template <int V, int L, int K, int RW, int KH, bool FULL>
-__device__ __forceinline__ void sddmm_staged(const int2 *edge, int n, int g, int li, const float *sb,
-                                             const float *db, int64_t F, const bool (&on)[K], float *out,
-                                             int32_t &held_row, typename Vec<V>::type (&dv)[K]) {
-    using S = Shape<V, L, K, RW, KH>;
-    using vec = typename S::vec;
-    constexpr int G = S::G, H = S::H, NH = S::NH;
-    constexpr int U = (K >= 2) ? 2 : 4;
-    const int seg_pos = li % RW, head0 = li / RW;
-    (void)held_row;
-    float res[NH];
-#pragma unroll
-    for (int kk = 0; kk < NH; ++kk) res[kk] = 0.f;
-    const int nsteps = (n + G - 1) / G;
-    for (int s0 = 0; s0 < nsteps; s0 += U) {
-        int2 rc[U];
-        vec sv[U][K], dw[U][K];
-        // no load sits under a branch: a group without an edge in this step re-reads the last edge
-        // (its result is not stored), and both operands are fetched for every edge -- when the row
-        // repeats, the destination row comes from the cache
-#pragma unroll
-        for (int u = 0; u < U; ++u) rc[u] = edge[min((s0 + u) * G + g, n - 1)];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int k = 0; k < K; ++k)
-                if (FULL || on[k]) {
-                    sv[u][k] = *reinterpret_cast<const vec *>(sb + (int64_t)rc[u].x * F + k * L * V);
-                    dw[u][k] = *reinterpret_cast<const vec *>(db + (int64_t)rc[u].y * F + k * L * V);
-                }
+// The staged units [0, n) of `unit` (x / y: the operands' rows, as byte offsets with OFF32, else as column and row ids whose
+// block of heads is in `block`; valid entries up to the next multiple of a batch); unit j's results go to out[j * side ..], or with
+// `edge_pos` (of the edge of unit 0, whose block is first_block) to the place of its edge.  ONE: a head is one chunk at most.
+template <int L, bool OFF32, bool ONE>
+__device__ __forceinline__ void dot_units(const uint2 *unit, const uint32_t *block, int n, int lane, const SddmmArgs &a, float *out,
+                                          const int32_t *edge_pos, int first_block) {
+    constexpr int U = batch_steps(L), CH = 4 * L;
+    using S = Spread<L, U>;
+    const int li = lane % L;
+    const int head = (lane / L) & (a.side - 1), g = (lane / L) / a.side, G = 64 / L / a.side;     // side: a power of two
+    const int blocks = a.H / a.side;
+    const char *const sb = reinterpret_cast<const char *>(a.src), *const db = reinterpret_cast<const char *>(a.dst);
+    const int full_chunks = a.D / CH;
+    const bool ragged = a.D % CH != 0;         // uniform
+    // the lane's words of the last chunk: read from `from`, words below `skip` belong to an earlier lane (or to nobody)
+    const int c0 = full_chunks * CH + 4 * li;
+    const int from = min(c0, a.D - 4), skip = c0 - from;
+    const uint32_t head_bytes = (uint32_t)(head * a.D) * 4u;
+    auto at = [&](const char *base, uint32_t row, uint32_t b, uint32_t bytes) -> const W4 * {
+        if (OFF32) return reinterpret_cast<const W4 *>(base + (row + bytes));
+        return reinterpret_cast<const W4 *>(base + ((int64_t)row * a.H + (int64_t)b * a.side) * a.D * 4 + bytes);
+    };
+    for (int s0 = 0; s0 < n; s0 += G * U) {
+        uint2 rc[U];
+        uint32_t rb[U];
+        uint32_t differ = 0;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int step = s0 + u;
-            if (step < nsteps) {                       // uniform
+            const int j = s0 + u * G + g;      // past the end: the last unit again; no result is stored
+            rc[u] = unit[j];
+            rb[u] = OFF32 ? 0u : block[j];
+            differ |= (rc[u].y ^ rc[0].y) | (rb[u] ^ rb[0]);
+        }
+        int place[S::per_lane];
+        if (edge_pos) {                        // the results' places, on their way while the dot products are formed
 #pragma unroll
-                for (int k = 0; k < K; ++k) dv[k] = dw[u][k];
-                float q[NH];
-                edge_heads<V, L, K, RW, KH, FULL>(sv[u], dv, on, q);
-                if ((step % RW) == seg_pos) {
+            for (int i = 0; i < S::per_lane; ++i) {
+                const int j = min(s0 + (S::kept(li) + i) * G + g, n - 1);
+                place[i] = edge_pos[blocks == 1 ? j : (first_block + j) / blocks];
+            }
+        }
+        float p[U];
+        auto batch = [&](auto one_row) {
+            constexpr bool SAME = decltype(one_row)::value;
+            float4 acc[ONE ? 1 : U];
+            if constexpr (!ONE) {
 #pragma unroll
-                    for (int kk = 0; kk < NH; ++kk) res[kk] = q[kk];
-                }
-                if ((step % RW) == RW - 1 || step == nsteps - 1) {   // uniform: write the collected block
-                    const int my_step = (step / RW) * RW + seg_pos;
-                    const int j = my_step * G + g;
-                    if (my_step <= step && j < n) {
+                for (int u = 0; u < U; ++u) acc[u] = vzero4();
+            }
+            auto chunk = [&](uint32_t bytes, auto last_one) {
+                auto words = [&](const W4 &w) {
+                    return decltype(last_one)::value ? make_float4(0 >= skip ? w.v[0] : 0.f, 1 >= skip ? w.v[1] : 0.f,
+                                                                   2 >= skip ? w.v[2] : 0.f, 3 >= skip ? w.v[3] : 0.f)
+                                                     : make_float4(w.v[0], w.v[1], w.v[2], w.v[3]);
+                };
+                auto use = [&](int u, const W4 &s, const float4 &d) {
+                    const float4 x = words(s);
+                    if constexpr (ONE) p[u] = vdot(x, d);
+                    else { acc[u].x += x.x * d.x; acc[u].y += x.y * d.y; acc[u].z += x.z * d.z; acc[u].w += x.w * d.w; }
+                };
+                if constexpr (SAME) {
+                    W4 s[U];
+                    const W4 d = *at(db, rc[0].y, rb[0], bytes);
 #pragma unroll
-                        for (int kk = 0; kk < NH; ++kk) out[(int64_t)j * H + kk * S::HPL + head0] = res[kk];
+                    for (int u = 0; u < U; ++u) s[u] = *at(sb, rc[u].x, rb[u], bytes);
+                    const float4 dv = words(d);
+#pragma unroll
+                    for (int u = 0; u < U; ++u) use(u, s[u], dv);
+                } else {
+                    // half a batch at a time: as many loads in flight, in half the registers
+#pragma unroll
+                    for (int h = 0; h < U; h += U / 2) {
+                        W4 s[U / 2], d[U / 2];
+#pragma unroll
+                        for (int u = 0; u < U / 2; ++u) {
+                            s[u] = *at(sb, rc[h + u].x, rb[h + u], bytes);
+                            d[u] = *at(db, rc[h + u].y, rb[h + u], bytes);
+                        }
+#pragma unroll
+                        for (int u = 0; u < U / 2; ++u) use(h + u, s[u], words(d[u]));
+                        __builtin_amdgcn_sched_barrier(0);      // the compiler would issue both halves' loads first
                     }
                 }
+            };
+            if constexpr (ONE) {
+                if (ragged) chunk(head_bytes + (uint32_t)from * 4u, std::true_type());
+                else chunk(head_bytes + (uint32_t)li * 16u, std::false_type());
+            } else {
+#pragma unroll 1
+                for (int k = 0; k < full_chunks; ++k) chunk(head_bytes + (uint32_t)(k * CH + 4 * li) * 4u, std::false_type());
+                if (ragged) chunk(head_bytes + (uint32_t)from * 4u, std::true_type());
+#pragma unroll
+                for (int u = 0; u < U; ++u) p[u] = (acc[u].x + acc[u].y) + (acc[u].z + acc[u].w);
+            }
+        };
+        if (!__any(differ != 0)) batch(std::true_type());
+        else batch(std::false_type());
+        spread_sums<L, U>(p, lane);
+#pragma unroll
+        for (int i = 0; i < S::per_lane; ++i) {
+            const int j = s0 + (S::kept(li) + i) * G + g;
+            if (S::stores(li) && j < n) {
+                if (edge_pos) out[(int64_t)place[i] * a.H + (blocks == 1 ? 0 : (first_block + j) % blocks * a.side) + head] = p[i];
+                else out[j * a.side + head] = p[i];
             }
         }
     }
 }
 
-// Stored-order (COO) kernel: a wavefront takes kEdgesPerWave consecutive stored edges.
-template <int V, int L, int K, int RW, int KH, bool FULL>
-__global__ __launch_bounds__(kBlock) void sddmm_coo_kernel(const SddmmArgs a) {
-    using S = Shape<V, L, K, RW, KH>;
-    using vec = typename S::vec;
-    constexpr int H = S::H;
-    static_assert(kEdgesPerWave <= fg::kItemEdges, "staging row too small");
-    __shared__ int2 s_edge[kWavesPerBlock][fg::kItemEdges];
+// Stages the units of n_edges consecutive edges and multiplies them.  Edge e's column is col[e]; its row is row[e] (COO), or, without
+// `row`, row_of(e).  OFF32: row numbers and the bytes of a unit's row fit 24 bits, their product 32.
+template <int L, bool OFF32, bool ONE, typename RowOf>
+__device__ __forceinline__ void dot_run(uint2 *unit, uint32_t *block, int n_edges, int lane, const SddmmArgs &a, const int32_t *col,
+                                        const int32_t *row, float *out, const int32_t *edge_pos, RowOf row_of) {
+    const uint32_t blocks = (uint32_t)(a.H / a.side);
+    const int batch = 64 / L / a.side * batch_steps(L);
+    const uint32_t row_bytes = (uint32_t)(a.side * a.D) * 4u;
+    const int64_t n_units = (int64_t)n_edges * blocks;
+    for (int64_t v0 = 0; v0 < n_units; v0 += kStageUnits) {
+        // more units than are staged at a time: one edge's (COO), or those of many (CSR)
+        const int n = (int)min((int64_t)kStageUnits, n_units - v0);
+        uint32_t e0 = (uint32_t)v0, b0 = 0;
+        wave_lds_sync();                       // earlier reads of the staging row are done
+        if (row && blocks == 1 && n > 64) {    // lane l stages units 4l .. 4l + 3 (past the end: the last one)
+            int32_t c[4], r[4];
+            fg::load_four(col + v0, n, lane, 1, c);
+            fg::load_four(row + v0, n, lane, 1, r);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (OFF32) { c[i] = (int)__umul24((uint32_t)c[i], row_bytes); r[i] = (int)__umul24((uint32_t)r[i], row_bytes); }
+                else block[4 * lane + i] = 0;
+            }
+            uint4 *u4 = reinterpret_cast<uint4 *>(unit);
+            u4[2 * lane] = make_uint4((uint32_t)c[0], (uint32_t)r[0], (uint32_t)c[1], (uint32_t)r[1]);
+            u4[2 * lane + 1] = make_uint4((uint32_t)c[2], (uint32_t)r[2], (uint32_t)c[3], (uint32_t)r[3]);
+        } else {
+            e0 = blocks == 1 ? (uint32_t)v0 : (uint32_t)(v0 / blocks); b0 = (uint32_t)(v0 - (int64_t)e0 * blocks);
+            for (int t = lane; t < (n + batch - 1) / batch * batch; t += 64) {
+                const uint32_t v = b0 + (uint32_t)min(t, n - 1), q = blocks == 1 ? v : v / blocks, e = e0 + q, b = v - q * blocks;
+                const uint32_t c = (uint32_t)col[e], r = (uint32_t)(row ? row[e] : row_of((int)e));
+                if (OFF32) unit[t] = make_uint2(__umul24(__umul24(c, blocks) + b, row_bytes), __umul24(__umul24(r, blocks) + b, row_bytes));
+                else { unit[t] = make_uint2(c, r); block[t] = b; }
+            }
+        }
+        wave_lds_sync();
+        dot_units<L, OFF32, ONE>(unit, block, n, lane, a, edge_pos ? out : out + v0 * a.side, edge_pos ? edge_pos + e0 : nullptr, (int)b0);
+    }
+}
 
+// A wavefront takes edges_per_wave consecutive edges.
+template <int L, bool OFF32, bool ONE>
+__global__ __launch_bounds__(kBlock) void sddmm_coo_kernel(const SddmmArgs a) {
+    __shared__ __align__(16) uint2 s_unit[kWavesPerBlock][kStageUnits];
+    __shared__ uint32_t s_block[kWavesPerBlock][OFF32 ? 1 : kStageUnits];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int g = lane / L, li = lane % L;
-    const int64_t e_begin = ((int64_t)blockIdx.x * kWavesPerBlock + wave) * kEdgesPerWave;
+    const int64_t e_begin = ((int64_t)blockIdx.x * kWavesPerBlock + wave) * a.edges_per_wave;
     if (e_begin >= a.n_edges) return;
-    const int n = (int)min((int64_t)kEdgesPerWave, a.n_edges - e_begin);
-    bool on[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) on[k] = FULL || (k * L * V + li * V < a.F);
-    int2 *edge = s_edge[wave];
-    for (int t = lane; t < n; t += 64) edge[t] = make_int2(a.col[e_begin + t], a.row[e_begin + t]);
-    wave_lds_sync();
-    int32_t held_row = -1;
-    vec dv[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) dv[k] = vec();
-    sddmm_staged<V, L, K, RW, KH, FULL>(edge, n, g, li, a.src + li * V, a.dst + li * V, a.F, on,
-                                        a.out + e_begin * H, held_row, dv);
+    const int n = (int)min((int64_t)a.edges_per_wave, a.n_edges - e_begin);
+    dot_run<L, OFF32, ONE>(s_unit[wave], s_block[wave], n, lane, a, a.col + e_begin, a.row + e_begin,
+                           a.edge_pos ? a.out : a.out + e_begin * a.H, a.edge_pos ? a.edge_pos + e_begin : nullptr, [](int) { return 0; });
 }
 
 // CSR-order kernel over plan items: a run of whole rows, one row, or a piece of a long row.
-template <int V, int L, int K, int RW, int KH, bool FULL>
+template <int L, bool OFF32, bool ONE>
 __global__ __launch_bounds__(kBlock) void sddmm_csr_kernel(const SddmmArgs a) {
-    using S = Shape<V, L, K, RW, KH>;
-    using vec = typename S::vec;
-    constexpr int H = S::H;
-    __shared__ int2 s_edge[kWavesPerBlock][fg::kItemEdges];
+    __shared__ __align__(16) uint2 s_unit[kWavesPerBlock][kStageUnits];
+    __shared__ uint32_t s_block[kWavesPerBlock][OFF32 ? 1 : kStageUnits];
     __shared__ int32_t s_end[kWavesPerBlock][fg::kItemRows];
-
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int g = lane / L, li = lane % L;
     const int64_t item_id = (int64_t)blockIdx.x * kWavesPerBlock + wave;
     if (item_id >= a.n_items) return;
     const Item it = a.items[item_id];
     if (it.len == 0) return;
-    bool on[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) on[k] = FULL || (k * L * V + li * V < a.F);
-    int2 *edge = s_edge[wave];
-    int32_t held_row = -1;
-    vec dv[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) dv[k] = vec();
-    const float *sb = a.src + li * V, *db = a.dst + li * V;
-
-    if (it.info < -1) {
-        // several whole rows: the row of staged edge t is the first row whose end exceeds t
-        const int nrows = -it.info;
-        if (lane < nrows) s_end[wave][lane] = a.pos[it.row + lane + 1] - it.start;
-        wave_lds_sync();
-        for (int t = lane; t < it.len; t += 64) {
-            int lo = 0, hi = nrows - 1;
-            while (lo < hi) { const int mid = (lo + hi) >> 1; if (s_end[wave][mid] > t) hi = mid; else lo = mid + 1; }
-            edge[t] = make_int2(a.col[it.start + t], it.row + lo);
-        }
-        wave_lds_sync();
-        sddmm_staged<V, L, K, RW, KH, FULL>(edge, it.len, g, li, sb, db, a.F, on, a.out + (int64_t)it.start * H,
-                                            held_row, dv);
-        return;
-    }
-    for (int32_t base = 0; base < it.len; base += fg::kItemEdges) {
-        const int n = min(fg::kItemEdges, it.len - base);
-        wave_lds_sync();
-        for (int t = lane; t < n; t += 64) edge[t] = make_int2(a.col[it.start + base + t], it.row);
-        wave_lds_sync();
-        sddmm_staged<V, L, K, RW, KH, FULL>(edge, n, g, li, sb, db, a.F, on,
-                                            a.out + ((int64_t)it.start + base) * H, held_row, dv);
-    }
+    const int nrows = it.info < -1 ? -it.info : 1;
+    if (lane < nrows) s_end[wave][lane] = nrows > 1 ? a.pos[it.row + lane + 1] - it.start : it.len;
+    wave_lds_sync();
+    dot_run<L, OFF32, ONE>(s_unit[wave], s_block[wave], it.len, lane, a, a.col + it.start, nullptr, a.out + (int64_t)it.start * a.H, nullptr,
+                           [&](int e) {
+        // the row of the item's edge e: the first whose end exceeds it
+        int lo = 0, hi = nrows - 1;
+        while (lo < hi) { const int mid = (lo + hi) >> 1; if (s_end[wave][mid] > e) hi = mid; else lo = mid + 1; }
+        return it.row + lo;
+    });
 }
 
 // ---- feature-tiled, source-column-partitioned traversal ---------------------------------------
@@ -687,159 +765,106 @@ bool launch_tiled_l(int L, int K, int RW, int KH, bool off32, dim3 grid, hipStre
     return false;
 }
 
-// Any H, D (odd lengths, unaligned pointers): one edge at a time per wavefront, lanes stride
-// over the head's D floats, full-wavefront reduction per head.
-__global__ __launch_bounds__(kBlock) void sddmm_generic_kernel(const int32_t *row, const int32_t *col,
-                                                               const int32_t *indptr, int64_t n_rows,
-                                                               int64_t n_edges, const float *src,
-                                                               const float *dst, float *out, int H, int D) {
-    const int lane = threadIdx.x & 63;
-    const int64_t wave_id = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int64_t e0 = wave_id * 64;
-    const int64_t F = (int64_t)H * D;
-    for (int64_t e = e0; e < min(e0 + 64, n_edges); ++e) {
-        int64_t r;
-        if (row) r = row[e];
-        else {                                   // CSR order: last row with indptr[r] <= e
-            int64_t lo = 0, hi = n_rows;
-            while (hi - lo > 1) { const int64_t mid = (lo + hi) >> 1; if (indptr[mid] <= e) lo = mid; else hi = mid; }
-            r = lo;
-        }
-        const float *s = src + (int64_t)col[e] * F;
-        const float *d = dst + r * F;
-        for (int h = 0; h < H; ++h) {
-            float p = 0.f;
-            for (int k = lane; k < D; k += 64) p += s[h * D + k] * d[h * D + k];
-            p = segment_sum<64>(p);
-            if (lane == 0) out[e * H + h] = p;
-        }
+// Rows of fewer than kMinDot floats: a thread per (edge, head) pair.  row == null: row ids from the boundaries `indptr`.
+__global__ __launch_bounds__(kBlock) void sddmm_short_kernel(const SddmmArgs a, const int32_t *indptr, int64_t n_rows) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t e = t / a.H;
+    if (e >= a.n_edges) return;
+    const int64_t h = t - e * a.H;
+    int64_t r;
+    if (a.row) {
+        r = a.row[e];
+    } else {                                    // CSR order: the last row with indptr[r] <= e
+        int64_t lo = 0, hi = n_rows;
+        while (hi - lo > 1) { const int64_t mid = (lo + hi) >> 1; if (indptr[mid] <= e) lo = mid; else hi = mid; }
+        r = lo;
     }
+    const float *s = a.src + ((int64_t)a.col[e] * a.H + h) * a.D, *d = a.dst + (r * a.H + h) * a.D;
+    float p = 0.f;
+    for (int k = 0; k < a.D; ++k) p += s[k] * d[k];
+    a.out[a.edge_pos ? (int64_t)a.edge_pos[e] * a.H + h : t] = p;
 }
 
-struct SddmmConfig { int V, L, K, RW, KH; bool full; bool generic; };
-
-int pow2_ceil(int v) { int p = 1; while (p < v) p <<= 1; return p; }
 bool is_pow2(int v) { return v > 0 && (v & (v - 1)) == 0; }
 
-void choose_config(int H, int D, bool aligned16, SddmmConfig *c) {
-    const int F = H * D;
-    c->generic = true;
-    c->full = false;
-    if (H == 1) {
-        c->V = (aligned16 && F % 4 == 0) ? 4 : 1;
-        const int lanes = (F + c->V - 1) / c->V;
-        if (lanes <= 64) { c->L = pow2_ceil(lanes) < 4 ? 4 : pow2_ceil(lanes); c->K = 1; }
-        else if (lanes <= 128) { c->L = 64; c->K = 2; }
-        else if (lanes <= 256) { c->L = 64; c->K = 4; }
-        else return;
-        c->RW = c->L; c->KH = c->K;
-        c->full = (F == c->V * c->L * c->K);
-        c->generic = false;
-        return;
+// Lanes per head: up to 32 floats, the 2 / 4 / 8 lanes that cover it with one chunk; beyond, the 8, 16 or 32 lanes whose loads touch the
+// fewest 128-byte lines (a chunk of a row that does not start on one touches one more), then those with one chunk, then the fewest.
+// 15,500 nodes, 6.3 M edges, us with 8 / 16 / 32 lanes: F=71 158 / 147 / 129, F=130 309 / 261 / 266, F=160 278 / 287 / 296, F=338 1236 / 1027 /
+// 1008, F=512 1419 / 1469 / 1525; with 4 lanes 202, 428, 370, 2057, 2161.
+int lanes_per_head(int D) {
+    if (D <= 8) return 2;
+    if (D <= 16) return 4;
+    if (D <= 32) return 8;
+    int best = 8, best_lines = 1 << 30;
+    for (int L = 8; L <= 32; L *= 2) {
+        const int chunks = (D + 4 * L - 1) / (4 * L);
+        const int lines = chunks * (L / 8 + (D % 32 != 0));
+        if (lines < best_lines || (lines == best_lines && chunks == 1)) { best = L; best_lines = lines; }
     }
-    if (!aligned16 || D % 4 != 0 || H > kMaxHeadsFast) return;
-    const int rw = D / 4;                       // lanes per head
-    if (!is_pow2(rw) || rw > 64 || rw < 2) return;
-    const int lanes = H * rw;
-    c->V = 4; c->RW = rw; c->KH = 1;
-    if (lanes <= 64) {
-        if (!is_pow2(lanes)) return;
-        c->L = lanes < 4 ? 4 : lanes; c->K = 1;
-        if (c->L != lanes) return;
-    } else {
-        if (lanes != 128 && lanes != 256) return;
-        c->L = 64; c->K = lanes / 64;
-    }
-    c->full = true;
-    c->generic = false;
+    return best;
 }
 
-template <int V, int L, int K, int RW, int KH>
-void launch_one(bool csr, bool full, dim3 grid, hipStream_t st, const SddmmArgs &a) {
+template <int L, bool OFF32>
+void launch_units(bool csr, dim3 grid, hipStream_t st, const SddmmArgs &a) {
+    const bool one = a.D <= 4 * L;
     if (csr) {
-        if (full) hipLaunchKernelGGL((sddmm_csr_kernel<V, L, K, RW, KH, true>), grid, dim3(kBlock), 0, st, a);
-        else hipLaunchKernelGGL((sddmm_csr_kernel<V, L, K, RW, KH, false>), grid, dim3(kBlock), 0, st, a);
+        if (one) hipLaunchKernelGGL((sddmm_csr_kernel<L, OFF32, true>), grid, dim3(kBlock), 0, st, a);
+        else hipLaunchKernelGGL((sddmm_csr_kernel<L, OFF32, false>), grid, dim3(kBlock), 0, st, a);
     } else {
-        if (full) hipLaunchKernelGGL((sddmm_coo_kernel<V, L, K, RW, KH, true>), grid, dim3(kBlock), 0, st, a);
-        else hipLaunchKernelGGL((sddmm_coo_kernel<V, L, K, RW, KH, false>), grid, dim3(kBlock), 0, st, a);
+        if (one) hipLaunchKernelGGL((sddmm_coo_kernel<L, OFF32, true>), grid, dim3(kBlock), 0, st, a);
+        else hipLaunchKernelGGL((sddmm_coo_kernel<L, OFF32, false>), grid, dim3(kBlock), 0, st, a);
     }
 }
 
-// single head: the head spans the whole lane group and all K loads
-template <int V>
-bool launch_vanilla(const SddmmConfig &c, bool csr, dim3 grid, hipStream_t st, const SddmmArgs &a) {
-    if (c.K == 1) {
-        switch (c.L) {
-            case 4: launch_one<V, 4, 1, 4, 1>(csr, c.full, grid, st, a); return true;
-            case 8: launch_one<V, 8, 1, 8, 1>(csr, c.full, grid, st, a); return true;
-            case 16: launch_one<V, 16, 1, 16, 1>(csr, c.full, grid, st, a); return true;
-            case 32: launch_one<V, 32, 1, 32, 1>(csr, c.full, grid, st, a); return true;
-            case 64: launch_one<V, 64, 1, 64, 1>(csr, c.full, grid, st, a); return true;
-        }
-    } else if (c.K == 2) { launch_one<V, 64, 2, 64, 2>(csr, c.full, grid, st, a); return true; }
-    else if (c.K == 4) { launch_one<V, 64, 4, 64, 4>(csr, c.full, grid, st, a); return true; }
-    return false;
-}
-
-template <int L, int K>
-bool launch_heads_lk(const SddmmConfig &c, bool csr, dim3 grid, hipStream_t st, const SddmmArgs &a) {
-    switch (c.RW) {
-        case 2: if constexpr (L >= 2) { launch_one<4, L, K, 2, 1>(csr, true, grid, st, a); return true; } break;
-        case 4: if constexpr (L >= 4) { launch_one<4, L, K, 4, 1>(csr, true, grid, st, a); return true; } break;
-        case 8: if constexpr (L >= 8) { launch_one<4, L, K, 8, 1>(csr, true, grid, st, a); return true; } break;
-        case 16: if constexpr (L >= 16) { launch_one<4, L, K, 16, 1>(csr, true, grid, st, a); return true; } break;
-        case 32: if constexpr (L >= 32) { launch_one<4, L, K, 32, 1>(csr, true, grid, st, a); return true; } break;
-        case 64: if constexpr (L >= 64) { launch_one<4, L, K, 64, 1>(csr, true, grid, st, a); return true; } break;
+template <bool OFF32>
+void launch_units_l(int L, bool csr, dim3 grid, hipStream_t st, const SddmmArgs &a) {
+    switch (L) {
+        case 2: launch_units<2, OFF32>(csr, grid, st, a); break;
+        case 4: launch_units<4, OFF32>(csr, grid, st, a); break;
+        case 8: launch_units<8, OFF32>(csr, grid, st, a); break;
+        case 16: launch_units<16, OFF32>(csr, grid, st, a); break;
+        default: launch_units<32, OFF32>(csr, grid, st, a); break;
     }
-    return false;
 }
 
-bool launch_heads(const SddmmConfig &c, bool csr, dim3 grid, hipStream_t st, const SddmmArgs &a) {
-    if (c.K == 1) {
-        switch (c.L) {
-            case 4: return launch_heads_lk<4, 1>(c, csr, grid, st, a);
-            case 8: return launch_heads_lk<8, 1>(c, csr, grid, st, a);
-            case 16: return launch_heads_lk<16, 1>(c, csr, grid, st, a);
-            case 32: return launch_heads_lk<32, 1>(c, csr, grid, st, a);
-            case 64: return launch_heads_lk<64, 1>(c, csr, grid, st, a);
-        }
-    } else if (c.K == 2) return launch_heads_lk<64, 2>(c, csr, grid, st, a);
-    else if (c.K == 4) return launch_heads_lk<64, 4>(c, csr, grid, st, a);
-    return false;
-}
-
-int sddmm_run(const fg_spmm_plan *pl, const int32_t *row, const int32_t *col, const int32_t *indptr,
-              int64_t n_rows, int64_t n_edges, const float *src, const float *dst, float *out, int H,
-              int D, void *stream) {
+// n_src, n_dst: rows of the operands (0: not known; rows are then addressed with 64 bits).
+int sddmm_run(const fg_spmm_plan *pl, const int32_t *row, const int32_t *col, const int32_t *indptr, const int32_t *edge_pos,
+              int64_t n_edges, int64_t n_src, int64_t n_dst, const float *src, const float *dst, float *out, int H, int D, void *stream) {
     if (H < 1 || D < 1) return fail(FG_ERR_SHAPE, "heads and head length must be positive, got H=%d D=%d", H, D);
     if (n_edges < 0) return fail(FG_ERR_ARG, "negative edge count");
     if (n_edges == 0) return FG_OK;
     if (!col || !src || !dst || !out || (!row && !pl) || (pl && !indptr)) return fail(FG_ERR_ARG, "null device pointer");
     if ((int64_t)H * D > INT32_MAX) return fail(FG_ERR_SHAPE, "H*D too large");
     hipStream_t st = (hipStream_t)stream;
-    const bool aligned16 = (((uintptr_t)src | (uintptr_t)dst) & 15) == 0;
-    SddmmConfig c;
-    choose_config(H, D, aligned16, &c);
-    SddmmArgs a;
-    a.row = row; a.col = col; a.items = pl ? pl->items_dev : nullptr; a.n_items = pl ? pl->n_items : 0;
-    a.pos = indptr;
-    a.n_edges = n_edges; a.src = src; a.dst = dst; a.out = out; a.F = H * D;
     const bool csr = pl != nullptr;
-    bool launched = false;
-    if (!c.generic) {
-        const int64_t waves = csr ? pl->n_items : (n_edges + kEdgesPerWave - 1) / kEdgesPerWave;
-        const int64_t blocks = (waves + kWavesPerBlock - 1) / kWavesPerBlock;
+    SddmmArgs a;
+    a.row = row; a.col = col; a.edge_pos = edge_pos; a.items = csr ? pl->items_dev : nullptr; a.n_items = csr ? pl->n_items : 0;
+    a.pos = indptr; a.n_edges = n_edges; a.src = src; a.dst = dst; a.out = out; a.H = H; a.D = D;
+    int64_t blocks;
+    if (D < kMinDot) {
+        blocks = (n_edges * H + kBlock - 1) / kBlock;
         if (blocks > 0x7fffffffLL) return fail(FG_ERR_SHAPE, "grid too large");
-        const dim3 grid((unsigned)blocks);
-        if (H == 1) launched = (c.V == 4) ? launch_vanilla<4>(c, csr, grid, st, a) : launch_vanilla<1>(c, csr, grid, st, a);
-        else launched = launch_heads(c, csr, grid, st, a);
-    }
-    if (!launched) {
-        const int64_t waves = (n_edges + 63) / 64;
-        const int64_t blocks = (waves + kWavesPerBlock - 1) / kWavesPerBlock;
+        hipLaunchKernelGGL(sddmm_short_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, st, a, indptr, csr ? pl->n_dst : 0);
+    } else {
+        const int L = lanes_per_head(D);
+        a.side = 1;
+        while (a.side * 2 <= 64 / L && H % (a.side * 2) == 0) a.side *= 2;
+        const int batch = 64 / L / a.side * batch_steps(L), blocks_per_edge = H / a.side;
+        // fewer units per wavefront where there are not enough to keep every SIMD's 8 slots full, down to 64 (ids staged by
+        // one load per lane), and to one batch where even that leaves SIMDs empty (F=128, us with 256 / 128 / 64 / 32 units: 16,400 nodes,
+        // 93,000 edges 18.2 / - / - / 7.7; 10,000, 170,000 18.7 / - / 9.8 / 11.4; 4,700, 1.1 M 30.1 / 26.5 / 30.1 / -)
+        int units = kStageUnits;
+        while (units > batch && n_edges * blocks_per_edge / units < (units > 64 ? 8192 : 2048)) units /= 2;
+        a.edges_per_wave = std::max(1, units / blocks_per_edge);
+        const int64_t waves = csr ? pl->n_items : (n_edges + a.edges_per_wave - 1) / a.edges_per_wave;
+        blocks = (waves + kWavesPerBlock - 1) / kWavesPerBlock;
         if (blocks > 0x7fffffffLL) return fail(FG_ERR_SHAPE, "grid too large");
-        hipLaunchKernelGGL(sddmm_generic_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, st, row, col, indptr,
-                           n_rows, n_edges, src, dst, out, H, D);
+        const uint64_t row_bytes = (uint64_t)H * D * 4u;
+        const uint64_t rows = (uint64_t)std::max(n_src, n_dst);
+        const bool off32 = n_src > 0 && n_dst > 0 && rows * row_bytes < (1ull << 32) && rows * blocks_per_edge < (1u << 24) &&
+                           row_bytes < (1u << 24);
+        if (off32) launch_units_l<true>(L, csr, dim3((unsigned)blocks), st, a);
+        else launch_units_l<false>(L, csr, dim3((unsigned)blocks), st, a);
     }
     FG_HIP_TRY(hipGetLastError());
     return FG_OK;
@@ -851,7 +876,15 @@ extern "C" int fg_sddmm_coo_f32(const int32_t *row_dev, const int32_t *col_dev, 
                                 const float *src_dev, const float *dst_dev, float *out_dev, int H,
                                 int D, void *stream) {
     if (n_edges > 0 && !row_dev) return fail(FG_ERR_ARG, "row_dev is null");
-    return sddmm_run(nullptr, row_dev, col_dev, nullptr, 0, n_edges, src_dev, dst_dev, out_dev, H, D, stream);
+    return sddmm_run(nullptr, row_dev, col_dev, nullptr, nullptr, n_edges, 0, 0, src_dev, dst_dev, out_dev, H, D, stream);
+}
+
+extern "C" int fg_sddmm_edges_f32(const int32_t *row_dev, const int32_t *col_dev, const int32_t *edge_pos_dev, int64_t n_edges,
+                                  int64_t n_src, int64_t n_dst, const float *src_dev, const float *dst_dev, float *out_dev,
+                                  int H, int D, void *stream) {
+    if (n_src < 0 || n_dst < 0) return fail(FG_ERR_ARG, "negative row count");
+    if (n_edges > 0 && !row_dev) return fail(FG_ERR_ARG, "row_dev is null");
+    return sddmm_run(nullptr, row_dev, col_dev, nullptr, edge_pos_dev, n_edges, n_src, n_dst, src_dev, dst_dev, out_dev, H, D, stream);
 }
 
 extern "C" int fg_sddmm_csr_f32(const fg_spmm_plan *plan, const int32_t *indptr_dev,
@@ -860,8 +893,9 @@ extern "C" int fg_sddmm_csr_f32(const fg_spmm_plan *plan, const int32_t *indptr_
     if (!plan) return fail(FG_ERR_ARG, "plan is null");
     if (int drc = fg::check_device(plan)) return drc;
     if (plan->num_col_partitions != 1) return fail(FG_ERR_ARG, "fg_sddmm_csr_f32 needs a plan with one column partition");
-    return sddmm_run(plan, nullptr, indices_dev, indptr_dev, plan->n_dst, plan->nnz, src_dev, dst_dev,
-                     out_dev, H, D, stream);
+    const bool wide = plan->wide_offsets;
+    return sddmm_run(plan, nullptr, indices_dev, indptr_dev, nullptr, plan->nnz, wide ? 0 : plan->n_src, wide ? 0 : plan->n_dst, src_dev,
+                     dst_dev, out_dev, H, D, stream);
 }
 
 namespace {

@@ -252,14 +252,17 @@ class SDDMMbase(object):
             raise ValueError("order must be 'auto', 'csr', 'coo' or 'tiled'")
         if order == 'csr' and not self._row_sorted:
             raise ValueError("order='csr' needs stored edges with non-decreasing row ids")
-        # 'auto' takes the stored edges as they are (the COO kernel): on five graphs it is level with the CSR-order kernel
-        # at F <= 128 and 4-15 % ahead at F = 512 or on low-degree graphs; order='csr' asks for the CSR-order kernel
+        # 'auto' takes the stored edges as they are (the edge-list kernel); order='csr' asks for the CSR-order kernel
         use_csr = self._row_sorted and order == 'csr'
         # Tiled traversal for feature matrices beyond the L2: (source partitions, feature tiles)
         tiled = None
         nnz = self._adj_row_indices.shape[0]
         if order in ('auto', 'tiled') and nnz > 0:
             tiled = tuning.choose_sddmm(self._num_rows, self._num_cols, nnz, H, D, self._graph_stats() if H == 1 else None)
+            if H > 1 and getattr(self, '_pad_from', None) is not None and tiled is not None and tiled[0] == 1:
+                # padded heads without source partitions: the edge-list kernel reads them unpadded (40,000 nodes of degree 4, 8 x 48:
+                # 131 -> 44 us; 193,000 of degree 17 1289 -> 706; 172,000 of degree 16, 2 x 20 141 -> 81)
+                tiled = None
             p_arg, t_arg = schedule_args.get('num_src_partitions'), schedule_args.get('num_feat_tiles')
             if t_arg is None and knob_tiles is not None and order != 'coo' and order != 'csr':
                 t_arg = knob_tiles
@@ -339,8 +342,9 @@ class SDDMMbase(object):
                 and (compute_args.get('num_feat_partitions', 1) or 1) == 1 and self._adj_row_indices.shape[0] > 0:
             schedule_args = self._tune(list(input_placeholders), dict(compute_args), dict(schedule_args), 6 if tune is True else int(tune))
         schedule_args = {k: v for k, v in schedule_args.items() if k != 'tune'}
-        # Single-head rows of an awkward length run at the next friendly one, on zero-padded copies of both operands
-        # (tuning.padded_feature_len): the extra columns add zeros to every dot product.
+        # Single-head rows of an awkward length run at the next friendly one (tuning.padded_feature_len): the extra columns
+        # add zeros to every dot product.  The tiled traversal reads them from zero-padded copies of both operands; the
+        # edge-list kernel reads the operands as they are and fills up in registers.
         self._pad_from = None
         given = list(input_placeholders)
         if len(given) == 2 and len(given[0].shape) == 2 and len(given[1].shape) == 2 and given[0].shape[1] == given[1].shape[1] \
@@ -364,8 +368,9 @@ class SDDMMbase(object):
         phs, H, D, use_csr, tiled, notes = self._resolve(input_placeholders, compute_args, schedule_args)
         self._src_pad = self._dst_pad = None
         if self._pad_from is not None:
-            notes.append("rows of %d floats run as rows of %d on zero-padded copies" % (self._pad_from, D))
             phs = given
+        if self._pad_from is not None and tiled is not None:
+            notes.append("rows of %d floats run as rows of %d on zero-padded copies" % (self._pad_from, D))
             tail = (D,) if len(given[0].shape) == 2 else (H, D)
             self._src_pad = torch.zeros((self._num_cols,) + tail, dtype=torch.float32, device=self._ctx)
             self._dst_pad = torch.zeros((self._num_rows,) + tail, dtype=torch.float32, device=self._ctx)
@@ -378,7 +383,7 @@ class SDDMMbase(object):
                 for P in [P for P in self._dds if P != tiled[0]]:
                     self._drop_dds(P)          # partitioned copies the built configuration does not use
             common.reserve(self._tiled[0]['plan'], common.OP_SDDMM_DDS, H, D, tiled[1], self._ctx)
-        self._func = _lib.lib().fg_sddmm_csr_f32 if use_csr else _lib.lib().fg_sddmm_coo_f32
+        self._func = _lib.lib().fg_sddmm_csr_f32 if use_csr else _lib.lib().fg_sddmm_edges_f32
         if self._tiled is None:
             self._upload_edge_list()           # the stored-order kernels read it; run() itself must not upload anything
         nnz = self._adj_row_indices.shape[0]
@@ -395,7 +400,7 @@ class SDDMMbase(object):
         text += "  features         : %d head(s) x %d floats\n" % (H, D)
         text += "  kernel           : %s\n" % ("sddmm_tiled_kernel over a source-column-partitioned edge list" if tiled
                                                else "sddmm_csr_kernel over row pieces (dst row held in registers)"
-                                               if use_csr else "sddmm_coo_kernel, 256 stored edges per wavefront")
+                                               if use_csr else "sddmm_coo_kernel over runs of consecutive stored edges")
         if tiled:
             P, T = tiled
             conc = min(8 // T, P) if (T < 8 and 8 % T == 0) else 1
@@ -407,7 +412,7 @@ class SDDMMbase(object):
 
     def _launch(self, src_feat, dst_feat):
         s = common.stream_ptr()
-        if getattr(self, '_pad_from', None) is not None:
+        if getattr(self, '_src_pad', None) is not None:
             self._src_pad[..., :self._pad_from].copy_(src_feat)     # the padding columns stay zero
             self._dst_pad[..., :self._pad_from].copy_(dst_feat)
             src_feat, dst_feat = self._src_pad, self._dst_pad
@@ -417,14 +422,18 @@ class SDDMMbase(object):
                                                    _lib.dev_ptr(d['edge_pos']), _lib.dev_ptr(src_feat),
                                                    _lib.dev_ptr(dst_feat), _lib.dev_ptr(self.out_tvm),
                                                    self._heads, self._head_len, T, s))
-        elif self._use_csr:
+            return
+        D = self._head_len if self._pad_from is None else self._pad_from
+        if self._use_csr:
             _lib.check(self._func(self._plan, _lib.dev_ptr(self._adj_indptr_dev), _lib.dev_ptr(self._adj_col_indices_dev),
                                   _lib.dev_ptr(src_feat), _lib.dev_ptr(dst_feat), _lib.dev_ptr(self.out_tvm),
-                                  self._heads, self._head_len, s))
+                                  self._heads, D, s))
         else:
-            _lib.check(self._func(_lib.dev_ptr(self._adj_row_indices_dev), _lib.dev_ptr(self._adj_col_indices_dev),
-                                  self._adj_row_indices.shape[0], _lib.dev_ptr(src_feat), _lib.dev_ptr(dst_feat),
-                                  _lib.dev_ptr(self.out_tvm), self._heads, self._head_len, s))
+            row, col = self._upload_edge_list()
+            wide = _lib.plan_opts is not None and _lib.plan_opts.wide_offsets
+            _lib.check(self._func(_lib.dev_ptr(row), _lib.dev_ptr(col), None, self._adj_row_indices.shape[0],
+                                  0 if wide else self._num_cols, 0 if wide else self._num_rows, _lib.dev_ptr(src_feat),
+                                  _lib.dev_ptr(dst_feat), _lib.dev_ptr(self.out_tvm), self._heads, D, s))
 
     def run(self, input_tvm_ndarrays):
         """Run the built func with the given inputs [SrcFeat, DstFeat] (float32 torch tensors on

@@ -288,6 +288,15 @@ int fg_sddmm_coo_f32(const int32_t *row_dev, const int32_t *col_dev, int64_t n_e
                      int D, void *stream);
 
 /*
+ * The same for edges listed in an order of the caller's choice, best by row (a destination row is then read once for many
+ * edges): the results of edge e go to out[edge_pos[e] * H ..] (edge_pos null: to out[e * H ..]).  n_src / n_dst: rows of src and
+ * dst, which let the kernel address them with 32 bits; 0: not known.
+ */
+int fg_sddmm_edges_f32(const int32_t *row_dev, const int32_t *col_dev, const int32_t *edge_pos_dev, int64_t n_edges,
+                       int64_t n_src, int64_t n_dst, const float *src_dev, const float *dst_dev, float *out_dev, int H, int D,
+                       void *stream);
+
+/*
  * Same result for edges in CSR order (edge e of row v at position indptr[v] + k), using the
  * SpMM plan's row items so that dst[v] is fetched once per row piece and no row-id array
  * is read.  The plan must have num_col_partitions == 1.
