@@ -46,6 +46,26 @@ TIE = 0.03                       # predicted times closer than this are equal: f
 SPMM_COEF = dict(cache=2.12, hit=24.0e12, miss=7.07e12, span=0.011, seg=1.64e-11, edge=1.04e-12, stream=4.15e12)
 SDDMM_COEF = dict(cache=2.26, hit=23.5e12, miss=6.58e12, span=0.0, seg=3.82e-11, edge=0.0, stream=3.86e12)
 
+# Below this many stored elements the launches, the sums that follow them and the caches' real size weigh more.  A second set of
+# coefficients is fitted to sweeps of P (1 .. 16) x T on 23 graphs of 3,000 to 390,000 nodes and 100,000 to 22 M elements (degrees 7 to 430,
+# power-law and uniform; feature lengths 16 .. 512) and overrules the first where it sees 15 % (SpMM) or 5 % (SDDMM) less time for
+# its own choice: over the sweeps the time falls by 4.3 % (SpMM) and 8.7 % (SDDMM) on average, the worst point loses 6 % and 8 %, and
+# what is left to the best is 1.5 % and 3.8 %.  With the second set alone: 3.7 % and 9.2 %, the worst 54 % and 14 %.  The largest, us: 17,600 nodes of
+# degree 266, uniform, F=512: SpMM 723 -> 360, SDDMM 1128 -> 400; 12,000 of degree 200, F=512: SpMM 232 -> 190, SDDMM 473 -> 195.
+SMALL_NNZ = 1 << 25
+# pass / sum: seconds that a second pass over the graph (SpMM) and the sum of the tiles' scores (SDDMM) cost whatever their size;
+# seg_tiled: per row segment and tile where there are several; edges_dst: the edge-list kernel's reads of destination rows, as
+# a share of the gathered bytes at the hit rate.
+SPMM_SMALL_COEF = dict(cache=0.99, hit=29.95e12, miss=6.55e12, span=0.041, seg=2.86e-11, seg_tiled=6.2e-11, edge=1.37e-12, stream=3.93e12,
+                       **{'pass': 7.0e-6})
+SDDMM_SMALL_COEF = dict(cache=1.32, hit=24.7e12, miss=8.49e12, span=0.006, seg=2.85e-11, edge=0.21e-12, stream=3.85e12, sum=9.7e-6,
+                        edges_dst=0.26)
+
+
+def _is_small(stats):
+    return stats.nnz < SMALL_NNZ
+
+
 # legacy names (attention module): per-XCD slice that two L2s' worth of slices add up to
 SPMM_SLICE_BYTES = 7.5e6
 SDDMM_SLICE_BYTES = 7.5e6
@@ -183,7 +203,7 @@ def _gather_seconds(stats, feat_len, P, T, c):
     slow = 1.0 + c['span'] * max(0.0, math.log2(span / (128.0 * (1 << 20))))
     gathered = 4.0 * stats.nnz * feat_len
     t = gathered * (h / c['hit'] + (1.0 - h) * slow / c['miss'])
-    t += stats.segments(P) * T * c['seg'] + stats.nnz * T * c['edge']
+    t += stats.segments(P) * T * (c.get('seg_tiled', c['seg']) if T > 1 else c['seg']) + stats.nnz * T * c['edge']
     if tiled:
         t += 2.0 * 4.0 * stats.n_src * feat_len / COPY_BYTES_PER_S
     return t
@@ -191,16 +211,19 @@ def _gather_seconds(stats, feat_len, P, T, c):
 
 def predict_spmm(stats, feat_len, P, T, coef=SPMM_COEF):
     """Modelled seconds of one SpMM with P source-column partitions and T feature tiles."""
-    t = _gather_seconds(stats, feat_len, P, T, coef)
+    t = _gather_seconds(stats, feat_len, P, T, coef) + (coef.get('pass', 0.0) if P > 1 else 0.0)
     # out: one buffer written per pass and read back once by the sum (fitted as (2P - 1) when later passes re-read `out`)
     return t + 4.0 * stats.n_dst * feat_len * (2 * P - 1) / coef['stream']
 
 
 def predict_sddmm(stats, feat_len, P, T, coef=SDDMM_COEF):
     """Modelled seconds of one single-head SDDMM over the tiled traversal ((1, 1): the row-order kernel)."""
-    t = _gather_seconds(stats, feat_len, P, T, coef)
+    t = _gather_seconds(stats, feat_len, P, T, coef) + (coef.get('sum', 0.0) if T > 1 else 0.0)
     t += stats.segments(P) * 4.0 * feat_len / coef['stream']                    # destination rows: once per segment
-    out_bytes = 4.0 * stats.nnz * ((2 * T + 2) if T > 1 else 1)                 # per-tile partial sums: written, read, scattered
+    if (P, T) == (1, 1) and 'edges_dst' in coef:
+        t += 4.0 * stats.nnz * feat_len * coef['edges_dst'] / coef['hit']
+    # per-tile partial sums: written, read, scattered; results of several partitions go through a position
+    out_bytes = 4.0 * stats.nnz * ((2 * T + 2) if T > 1 else (2 if P > 1 and 'edges_dst' in coef else 1))
     return t + out_bytes / coef['stream']
 
 
@@ -211,14 +234,24 @@ def _candidates(feat_len, max_tile=256):
     return [(p, t) for p in parts for t in tiles]
 
 
-def _rank(stats, feat_len, predict, cands, tie_key):
-    timed = sorted(((predict(stats, feat_len, p, t), p, t) for p, t in cands))
+def _rank(stats, feat_len, predict, cands, tie_key, coef):
+    timed = sorted(((predict(stats, feat_len, p, t, coef), p, t) for p, t in cands))
     if not timed:
         return []
     best = timed[0][0]
     near = sorted(((s, p, t) for s, p, t in timed if s <= best * (1.0 + TIE)), key=lambda e: tie_key(e[1], e[2]) + (e[0],))
     rest = [(s, p, t) for s, p, t in timed if s > best * (1.0 + TIE)]
     return [(p, t) for s, p, t in near] + [(p, t) for s, p, t in rest]
+
+
+def _overrule(stats, feat_len, predict, ranked, cands, coef, margin):
+    """On a small graph: the candidates in the order of the coefficients fitted to such graphs, behind the first choice `ranked[0]` of
+    the others unless these see `margin` less time for their own."""
+    order = [c for _, c in sorted((predict(stats, feat_len, p, t, coef), (p, t)) for p, t in cands)]
+    first = ranked[0]
+    if predict(stats, feat_len, *first, coef) > (1.0 + margin) * predict(stats, feat_len, *order[0], coef):
+        return order
+    return [first] + [c for c in order if c != first]
 
 
 # predicted times within TIE of the best: SpMM takes fewer tiles (fewer passes over the edge list), SDDMM fewer
@@ -232,14 +265,28 @@ def rank_spmm(stats, feat_len):
     cands = [(p, t) for p, t in _candidates(feat_len) if p <= max(1, stats.n_src)]
     if feat_len > 256:
         cands = [(p, t) for p, t in cands if t > 1]          # rows wider than 256 floats are always tiled
-    return _rank(stats, feat_len, predict_spmm, cands, _spmm_tie)
+    ranked = _rank(stats, feat_len, predict_spmm, cands, _spmm_tie, SPMM_COEF)
+    if not ranked or not _is_small(stats):
+        return ranked
+    if feat_len % 64 == 0 and stats.nnz < 36 * stats.n_dst:
+        # short rows: 32-float tiles, which the model likes for their hit rate, are behind (30,000 nodes of degree 30, us with tiles of 64 / 32
+        # floats: F=64 25 / 28, F=256 65 / 78, F=512 116 / 150; 60,000 of degree 40, F=512 385 / 333)
+        cands = [(p, t) for p, t in cands if feat_len // t >= 64]
+    return _overrule(stats, feat_len, predict_spmm, ranked, cands, SPMM_SMALL_COEF, 0.15)
 
 
 def rank_sddmm(stats, feat_len):
     """(num_src_partitions, num_feat_tiles) candidates of the tiled traversal, most promising first;
-    (1, 1) stands for the plain row-order kernel."""
+    (1, 1) stands for the edge-list kernel."""
     cands = [(p, t) for p, t in _candidates(feat_len) if not (t == 1 and p > 1 and feat_len > 256)]
-    return _rank(stats, feat_len, predict_sddmm, cands, _sddmm_tie)
+    ranked = _rank(stats, feat_len, predict_sddmm, cands, _sddmm_tie, SDDMM_COEF)
+    if not ranked or not _is_small(stats):
+        return ranked
+    takes = [(p, t) for p, t in cands if (p, t) == (1, 1) or feat_len // t <= 256 and _is_pow2(feat_len // t) and feat_len // t >= 16]
+    ranked = [c for c in ranked if c in takes]
+    if 4.0 * stats.n_src * feat_len <= N_XCD * L2_BYTES / 4 or ranked[0][0] == 1:
+        ranked = [(1, 1)]
+    return _overrule(stats, feat_len, predict_sddmm, ranked, takes, SDDMM_SMALL_COEF, 0.05)
 
 
 def choose_spmm(n_dst, n_src, nnz, feat_len, stats=None):
@@ -253,7 +300,7 @@ def choose_spmm(n_dst, n_src, nnz, feat_len, stats=None):
     if feat_len >= 2048 and feat_len % 128 == 0:
         # rows of 8 KB and more: 128-float tiles (measured at F=2048: 57.0 ms against 68.7 ms with 64-float tiles)
         cands = [(p, feat_len // 128) for p in (1, 2, 4, 8, 16, 32)]
-        p, t = _rank(stats, feat_len, predict_spmm, cands, _spmm_tie)[0]
+        p, t = _rank(stats, feat_len, predict_spmm, cands, _spmm_tie, SPMM_COEF)[0]
         return p, t
     ranked = rank_spmm(stats, feat_len)
     if not ranked:
@@ -289,19 +336,35 @@ def choose_gather_partitions(n_dst, n_src, nnz, gathered_len, out_len, stats=Non
     cands = [(p, tiles) for p in (1, 2, 4, 8, 16, 32)
              if p <= min(MAX_PARTITIONS, max(1, n_src)) and (p == 1 or 4.0 * p * n_dst * out_len <= float(8 << 30))]
     coef = BCAST_TILED_COEF if tiles > 1 else BCAST_COEF
-    predict = lambda st, f, p, t: predict_spmm(st, f, p, t, coef)
-    return _rank(stats, gathered_len, predict, cands, _spmm_tie)[0][0]
+    return _rank(stats, gathered_len, predict_spmm, cands, _spmm_tie, coef)[0][0]
 
 
-def choose_sddmm(n_rows, n_cols, nnz, heads, head_len, stats=None):
+# What a row that starts inside a 128-byte line costs the edge-list kernel, in floats (us at F=64 / 71 / 100 / 128: 120,000 nodes of degree
+# 100 394 / 598 / 785 / 820, 12,000 of degree 200 37 / 61 / 66 / 69).
+EDGES_MISALIGNED = 16
+
+
+def choose_sddmm(n_rows, n_cols, nnz, heads, head_len, stats=None, given_len=None):
     """(num_src_partitions, num_feat_tiles) for the tiled traversal, or None when the plain
-    kernels should be used (small feature matrices, or a shape the tiled kernel does not take)."""
+    kernels should be used (small feature matrices, or a shape the tiled kernel does not take).  given_len: the rows' length where
+    head_len is what the tiled traversal would pad them to."""
     feat_len = heads * head_len
     if heads == 1:
         if nnz == 0 or feat_len % 4 != 0:
             return None
         if stats is None:
             stats = GraphStats(n_rows, n_cols, nnz)
+        if _is_small(stats):
+            ranked = rank_sddmm(stats, feat_len)
+            if given_len is not None and given_len != feat_len:
+                # unpadded on the edge-list kernel, or padded copies of both operands and the tiled traversal
+                tiled = [c for c in ranked if c != (1, 1)]
+                if not tiled:
+                    return None
+                copies = 2 * 4e-6 + 8.0 * max(n_rows, n_cols) * (given_len + feat_len) / SDDMM_SMALL_COEF['stream']
+                edges = predict_sddmm(stats, given_len + EDGES_MISALIGNED, 1, 1, SDDMM_SMALL_COEF)
+                return tiled[0] if copies + predict_sddmm(stats, feat_len, *tiled[0], SDDMM_SMALL_COEF) < edges else None
+            return None if not ranked or ranked[0] == (1, 1) else ranked[0]
         if 4.0 * n_cols * feat_len <= N_XCD * L2_BYTES / 4:
             return None                                # the whole operand sits in every L2: nothing to tile
         ranked = [(p, t) for p, t in rank_sddmm(stats, feat_len)
