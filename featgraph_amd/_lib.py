@@ -66,6 +66,8 @@ SIGNATURES = {
     "fg_gspmm_bcast_dds_f32": (_int, [_vp, _vp, _vp, _vp, _int, _int, _vp, _int, _int, _vp, _vp, _int, _int, _vp, _int, _vp, _vp, _vp, _int, _vp]),
     "fg_gsddmm_bcast_f32": (_int, [_vp, _vp, _i64, _int, _vp, _int, _int, _vp, _vp, _int, _int, _vp, _int, _vp, _int, _int, _vp]),
     "fg_gspmm_select_backward_f32": (_int, [_vp, _vp, _i64, _i64, _int, _vp, _int, _int, _vp, _vp, _int, _int, _vp, _vp, _int, _vp, _vp, _vp]),
+    "fg_select_sources_f32": (_int, [_vp, _vp, _vp, _vp, _int, _vp, _vp, _vp, _int, _vp, _int, _vp]),
+    "fg_select_edges_f32": (_int, [_vp, _vp, _vp, _int, _vp, _vp, _vp, _int, _vp, _int, _int, _vp]),
     "fg_edge_softmax_f32": (_int, [_vp, _vp, _vp, _vp, _int, _vp]),
     "fg_edge_softmax_backward_f32": (_int, [_vp, _vp, _vp, _vp, _vp, _int, _vp]),
     "fg_edge_softmax_stats_f32": (_int, [_vp, _vp, _vp, _vp, _int, _vp]),

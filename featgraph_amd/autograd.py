@@ -16,6 +16,7 @@ import scipy.sparse
 import torch
 
 from . import tuning
+from .module import common
 from .module import (EdgeSoftmaxhip, GraphAttentionhip, GSDDMMhip, GSpMMhip, MultiHeadSDDMMhip, VanillaSDDMMhip,
                      placeholder)
 from .module.general import parse_message
@@ -162,6 +163,43 @@ class Graph(object):
         if getattr(self, "_cols_dev", None) is None or self._cols_dev.device != device:
             self._cols_dev = torch.from_numpy(np.ascontiguousarray(self._csr.indices, dtype=np.int32)).to(device)
         return self._cols_dev
+
+    def _sweep_layout(self, transposed, feat_len):
+        """The unpartitioned layout of one orientation with scratch for sweeps over rows of `feat_len`, and (transposed) its
+        elements' CSR positions."""
+        key = ('sweep', transposed)
+        if key not in self._mods:
+            m = self._gspmm_module(transposed)
+            m.set_weight_order(self._tr_pos_host if transposed else None)
+            m.swept = set()
+            self._mods[key] = m
+        m = self._mods[key]
+        lay = m._layout(1)
+        if transposed and feat_len not in m.swept:
+            common.reserve(lay['plan'], common.OP_GSPMM_BCAST, 1, feat_len, 0, m.ctx)
+            m.swept.add(feat_len)
+        return lay, m._weight_perm
+
+    def _sweep_selected(self, message, side, arg, other, dout, grads, shape):
+        """Puts the gradient of a max / min aggregation's operand `side` into grads[side] by a sweep over the edges; False where
+        the other way is to be taken."""
+        sweep = message.sweep_of(side)
+        if sweep is None or self.nnz == 0 or self.shape[0] == 0:
+            return False
+        sources, own_len = sweep[0] == 'u', (message.lhs_len, message.rhs_len)[side]
+        if not tuning.select_by_sweep(self.nnz, self.shape[0], message.out_len, sweep[0], own_len, sweep[2]):
+            return False
+        try:
+            layout, edge_pos = self._sweep_layout(sources, message.out_len)
+            grad = torch.empty(shape, dtype=dout.dtype, device=dout.device)
+            if sources:
+                message.select_sources(sweep, layout, edge_pos, arg, other, dout, grad)
+            else:
+                message.select_edges(sweep, layout, arg, other, dout, grad, own_len)
+        except MemoryError:
+            return False
+        grads[side] = grad
+        return True
 
     def _degrees(self, device):
         """Edges into every destination, at least 1, float32."""
@@ -541,11 +579,19 @@ def _wants_torch_grads():
 
 def _selected_grads(g, message, arg, arrays, shapes, dout, needed):
     """Gradients of a max / min aggregation for operands of `shapes`, None where not needed; `arrays` are the operands' values
-    (None: the message copies its one operand)."""
-    grads = [torch.zeros(s, dtype=dout.dtype, device=dout.device) if need else None for s, need in zip(shapes, needed)]
+    (None: the message copies its one operand).  By sweeps over the edges where the rows are short, else (and where there is
+    no sweep) result by result."""
+    dout = dout.contiguous()
     values = [None, None] if arrays is None else [a.contiguous() for a in arrays] + [None]
-    message.select_backward(arg, g._cols(dout.device), g.nnz, values[0], values[1], dout.contiguous(),
-                            grads[0], grads[1] if len(grads) > 1 else None)
+    grads = [None] * len(shapes)
+    left = list(needed)
+    for i, need in enumerate(needed):
+        if need and g._sweep_selected(message, i, arg, values[1 - i], dout, grads, shapes[i]):
+            left[i] = False
+    if any(left):
+        rest = [torch.zeros(s, dtype=dout.dtype, device=dout.device) if need else None for s, need in zip(shapes, left)]
+        message.select_backward(arg, g._cols(dout.device), g.nnz, values[0], values[1], dout, rest[0], rest[1] if len(rest) > 1 else None)
+        grads = [r if need else d for r, d, need in zip(rest, grads, left)]
     return grads
 
 

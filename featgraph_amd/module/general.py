@@ -157,6 +157,31 @@ class BroadcastOp(object):
             _lib.dev_ptr(rhs), TARGET[self.rhs_target or 'e'], self.rhs_len, _lib.dev_ptr(self.rhs_off),
             _lib.dev_ptr(dout), self.out_len, _lib.dev_ptr(dlhs), _lib.dev_ptr(drhs), common.stream_ptr()))
 
+    def sweep_of(self, side):
+        """How a sweep over the edges forms a max / min aggregation's gradient of operand `side` (0 / 1): (the operand's target, the
+        library's operator, features of the other operand or 0), or None where there is no sweep for it."""
+        operands = [(self.lhs_target, self.lhs_len, self.lhs_off), (self.rhs_target, self.rhs_len, self.rhs_off)]
+        (target, own_len, own_off), (other_target, other_len, other_off) = operands[side], operands[1 - side]
+        if self.out_len < 4 or self.op == 'div' and side == 1 or self.op not in ('add', 'sub', 'mul', 'div', 'copy_lhs'):
+            return None
+        if own_len != self.out_len and not (target == 'e' and own_len == 1 and self.out_len <= 256) or own_len == self.out_len and own_off is not None:
+            return None
+        if self.op not in ('mul', 'div'):
+            return target, BINARY['sub' if self.op == 'sub' and side == 1 else 'add'], 0
+        if other_target == target or other_len != 1 and (other_off is not None or other_len != self.out_len):
+            return None                             # the sweeps read sources for edges and edges for sources
+        return target, BINARY[self.op], other_len
+
+    def select_sources(self, sweep, layout, edge_pos, arg, other, dout, grad):
+        _lib.check(_lib.lib().fg_select_sources_f32(
+            layout['plan'], _lib.dev_ptr(layout['pos']), _lib.dev_ptr(layout['idx']), _lib.dev_ptr(edge_pos), sweep[1], _lib.dev_ptr(arg),
+            _lib.dev_ptr(dout), _lib.dev_ptr(other if sweep[2] else None), sweep[2], _lib.dev_ptr(grad), self.out_len, common.stream_ptr()))
+
+    def select_edges(self, sweep, layout, arg, other, dout, grad, grad_len):
+        _lib.check(_lib.lib().fg_select_edges_f32(
+            layout['plan'], _lib.dev_ptr(layout['pos']), _lib.dev_ptr(layout['idx']), sweep[1], _lib.dev_ptr(arg), _lib.dev_ptr(dout),
+            _lib.dev_ptr(other if sweep[2] else None), sweep[2], _lib.dev_ptr(grad), grad_len, self.out_len, common.stream_ptr()))
+
     def run_sddmm(self, row_dev, col_dev, n_edges, lhs, rhs, out):
         _lib.check(_lib.lib().fg_gsddmm_bcast_f32(
             _lib.dev_ptr(row_dev), _lib.dev_ptr(col_dev), n_edges, BINARY[self.op],

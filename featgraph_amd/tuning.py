@@ -492,3 +492,27 @@ def sum_gradients_in_one_sweep(num_rows, num_cols, nnz, heads, head_len):
     if head_len == 32 and _is_pow2(feat_len) and feat_len >= 128:
         return True
     return nnz < 1 << 20 or (feat_len >= 128 and nnz <= (16 if head_len == 32 else 64) * num_rows)
+
+
+def select_by_sweep(nnz, num_rows, feat_len, target, own_len, other_len):
+    """Whether the gradient of a max / min aggregation for an operand on `target` comes from a sweep over the edges (own_len features, 1 where
+    it was broadcast over feat_len; other_len features of the other operand of a product or quotient, 0 without one) instead of an
+    atomic per result.  Whole gradient calls, atomics -> sweep, in us, uniform graphs / power-law ones:
+      120,000 rows, sources, F=64, 4 / 8 / 16 / 32 elements per row: copies 106 -> 43, 344 -> 76, 348 -> 138, 331 -> 259 / 98 -> 45, 324 -> 75, 338 -> 135,
+        318 -> 251; times F edge features 108 -> 63, 377 -> 119, 396 -> 215, 410 -> 405 / 101 -> 70, 362 -> 132, 396 -> 231, 406 -> 411; times one 362 -> 332 / 360 -> 327 (32)
+      F=16: copies 104 -> 33, 105 -> 57, 104 -> 102 (8, 16, 32) / 104 -> 51, 104 -> 76, 103 -> 118; times F 112 -> 56, 118 -> 98 / 113 -> 87, 122 -> 133 (8, 16)
+      20,000 rows of 32, F=128: copies 107 -> 78 / 112 -> 69; of 64 90 -> 137 / 93 -> 125
+      edges, F features, no other operand: F=64 136 -> 96, 298 -> 161, 443 -> 253 / 122 -> 101, 257 -> 176, 398 -> 293 (8, 16, 32); 20,000 rows of 128 195 -> 153 / 189 ->
+        158; F=16 41 -> 27 / 36 -> 43 (8), 96 -> 67 / 82 -> 101 (32); with a product F=64 161 -> 119 / 139 -> 156 (8), F=16 46 -> 38 / 40 -> 97
+      edges, one value: F=64 264 -> 34, 333 -> 72 / 294 -> 51, 308 -> 117 (8, 32), F=16 79 -> 25 / 78 -> 35 (8), 102 -> 76 / 102 -> 100 (64); with a product F=64 79 -> 67,
+        293 -> 65, 350 -> 160 / 83 -> 91, 307 -> 104, 327 -> 227 (4, 8, 32), 20,000 rows of 64 84 -> 50 / 90 -> 99; F=16 93 -> 30 / 90 -> 82 (8), 107 -> 73 / 105 -> 161 (32)"""
+    wide, degree = feat_len >= 48, nnz / max(1, num_rows)
+    if target == 'u':
+        if other_len == 0:
+            return degree <= (32 if wide else 24)
+        return degree <= ((24 if other_len > 1 else 32) if wide else 12)
+    if own_len == feat_len:
+        return wide and other_len == 0 and degree <= 128
+    if other_len == 0:
+        return degree <= 64
+    return wide and 6 <= degree <= 48

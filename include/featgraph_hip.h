@@ -398,6 +398,23 @@ int fg_gspmm_select_backward_f32(const int32_t *arg_dev, const int32_t *col_dev,
                                  const float *lhs_dev, int lhs_target, int lhs_len, const int32_t *lhs_off_dev,
                                  const float *rhs_dev, int rhs_target, int rhs_len, const int32_t *rhs_off_dev,
                                  const float *dout_dev, int out_len, float *dlhs_dev, float *drhs_dev, void *stream);
+/*
+ * The same gradient of one operand by a sweep over the edges, in a fixed order and without atomics, for graphs of few edges per
+ * row.  op: FG_BIN_ADD (also for copies), FG_BIN_SUB (the operand that is subtracted), FG_BIN_MUL, FG_BIN_DIV (the numerator); other_dev: the other
+ * operand of FG_BIN_MUL / _DIV, other_len = out_len or 1 features (other_len 0: none).  Every element of grad is written.
+ *   _sources : the operand on FG_TARGET_U, out_len features.  `plan`, pos, idx and edge_pos are the TRANSPOSED adjacency's (one column
+ *              partition): its elements' rows of arg / dout and their positions in the order that arg refers to.
+ *   _edges   : the operand on FG_TARGET_E, grad_len = out_len features, or 1 (the sum over up to 256).  `plan`, pos, idx: the adjacency's, whose
+ *              element order is the one that arg refers to.
+ * Rows of 4 features or more.  _sources keeps rows' pieces in the plan's scratch, as FG_OP_GSPMM_BCAST with out_len sizes it.
+ */
+int fg_select_sources_f32(fg_spmm_plan *plan, const int32_t *pos_dev, const int32_t *idx_dev, const int32_t *edge_pos_dev, int op,
+                          const int32_t *arg_dev, const float *dout_dev, const float *other_dev, int other_len, float *grad_dev,
+                          int out_len, void *stream);
+int fg_select_edges_f32(const fg_spmm_plan *plan, const int32_t *pos_dev, const int32_t *idx_dev, int op, const int32_t *arg_dev,
+                        const float *dout_dev, const float *other_dev, int other_len, float *grad_dev, int grad_len, int out_len,
+                        void *stream);
+
 int fg_gsddmm_bcast_f32(const int32_t *row_dev, const int32_t *col_dev, int64_t n_edges, int op,
                         const float *lhs_dev, int lhs_target, int lhs_len, const int32_t *lhs_off_dev,
                         const float *rhs_dev, int rhs_target, int rhs_len, const int32_t *rhs_off_dev,
