@@ -53,6 +53,8 @@ SIGNATURES = {
     "fg_spmm_dds_f32": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _int, _int, _vp]),
     "fg_gspmm_f32": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _int, _int, _int, _int, _int, _vp]),
     "fg_spmm_dot_takes": (_int, [_vp, _int, _int, _int]),
+    "fg_gspmm_padded_f32": (_int, [_vp, _vp, _vp, _vp, _vp, _int, _vp, _int, _int, _int, _int, _vp]),
+    "fg_spmm_dot_padded_f32": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _int, _vp, _vp, _vp, _int, _int, _int, _int, _vp]),
     "fg_spmm_dot_f32": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _int, _vp, _vp, _vp, _int, _int, _int, _int, _vp]),
     "fg_gspmm_arg_f32": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _int, _int, _int, _int, _int, _vp]),
     "fg_edge_values_head_major_f32": (_int, [_vp, _vp, _i64, _int, _vp, _vp]),

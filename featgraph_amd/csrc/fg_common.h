@@ -104,6 +104,9 @@ bool wants_tile_major(const fg_spmm_plan *plan, int n_tiles, uint64_t x_bytes);
 // the call fills copy `slot`.  The buffer must already be large enough (ensure_scratch).
 int make_tile_major(const fg_spmm_plan *plan, const float *x, int64_t n_rows, int F, int tile, void *stream,
                     int slot = 0, int n_slots = 1);
+// plan->tiled_dev = an [n_rows, heads, given] matrix (any alignment) with every head zero-padded to F / heads floats, tile by tile
+// as make_tile_major (tile = F: row by row; F, F / heads and tile multiples of 4).
+int make_padded_copy(const fg_spmm_plan *plan, const float *x, int64_t n_rows, int heads, int given, int F, int tile, void *stream);
 // The plan's 16-bit copy of `idx` when it has one of exactly this array (same address), else null.  With
 // fg_debug_checks(1) the array's fingerprint is compared as well (a device round trip per call): an array that was
 // rewritten or replaced at the same address is then read as int32 and the mismatch is left in fg_last_error().
@@ -121,7 +124,8 @@ int check_device(const fg_spmm_plan *plan);
 // What one call of each operator needs (the same functions size the buffers inside the calls).
 // Each returns FG_OK or the status the call itself would return for that shape.
 int spmm_scratch_need(const fg_spmm_plan *plan, int F, int heads, int reduce, int num_feat_partitions, ScratchNeed *need);
-int spmm_dot_scratch_need(const fg_spmm_plan *plan, int F, int heads, int num_feat_partitions, ScratchNeed *need);
+int spmm_padded_scratch_need(const fg_spmm_plan *plan, int F, int heads, int num_feat_partitions, ScratchNeed *need);
+int spmm_dot_scratch_need(const fg_spmm_plan *plan, int F, int heads, int num_feat_partitions, bool padded, ScratchNeed *need);
 int sddmm_dds_scratch_need(const fg_spmm_plan *plan, int H, int D, int num_feat_partitions, ScratchNeed *need);
 int softmax_scratch_need(const fg_spmm_plan *plan, int heads, ScratchNeed *need);
 int gspmm_bcast_scratch_need(const fg_spmm_plan *plan, int out_len, bool with_arg, ScratchNeed *need);

@@ -9,6 +9,7 @@
 #include <string>
 
 #include "fg_common.h"
+#include "fg_device.h"
 
 using fg::fail;
 using fg::Fixup;
@@ -206,9 +207,46 @@ __global__ __launch_bounds__(256) void tile_major_kernel(const float4 *x, float4
     const uint32_t t = c / tile_words, w = c - t * tile_words;
     dst[((uint64_t)t * n_rows + r) * tile_words + w] = x[i];
 }
+// The same from rows of heads of `given` floats, every head zero-padded to head_words: 64-bit word numbers, of which a block
+// divides its first by one scalar division and a lane the rest in 32 bits.
+__global__ __launch_bounds__(256) void padded_copy_kernel(const float *x, float4 *dst, int64_t n_rows, uint32_t row_words, uint32_t tile_words,
+                                                          uint32_t head_words, int given, int64_t n_words) {
+    const int64_t i0 = (int64_t)blockIdx.x * 256;
+    if (i0 + threadIdx.x >= n_words) return;
+    const int64_t r0 = i0 / row_words;
+    const uint32_t at = (uint32_t)(i0 - r0 * row_words) + threadIdx.x, dr = at / row_words, c = at - dr * row_words;
+    const uint32_t t = c / tile_words, w = c - t * tile_words, h = c / head_words;
+    const int64_t r = r0 + dr;
+    const int d = (int)(c - h * head_words) * 4, left = given - d;
+    const float *p = x + r * (int64_t)(row_words / head_words) * given + (int64_t)h * given + d;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (left >= 4) {
+        const fg::Words4<float> q = *reinterpret_cast<const fg::Words4<float> *>(p);
+        v = make_float4(q.v[0], q.v[1], q.v[2], q.v[3]);
+    } else {
+        if (left > 0) v.x = p[0];
+        if (left > 1) v.y = p[1];
+        if (left > 2) v.z = p[2];
+    }
+    dst[((int64_t)t * n_rows + r) * tile_words + w] = v;
+}
 }  // namespace
 
 namespace fg {
+int make_padded_copy(const fg_spmm_plan *pl, const float *x, int64_t n_rows, int heads, int given, int F, int tile, void *stream) {
+    const uint64_t floats = (uint64_t)n_rows * (uint64_t)F;
+    if (heads < 1 || F % heads != 0 || F / heads % 4 != 0 || tile % 4 != 0 || F % tile != 0 || given < 1 || given > F / heads)
+        return fail(FG_ERR_SHAPE, "padded copy of %d heads of %d floats in rows of %d and tiles of %d", heads, given, F, tile);
+    if (floats > pl->tiled_floats)
+        return fail(FG_ERR_ARG, "padded copy: the plan's buffer holds %zu floats, %llu needed", pl->tiled_floats, (unsigned long long)floats);
+    const uint64_t blocks = (floats / 4 + 255) / 256;
+    if (blocks > 0x7fffffffull) return fail(FG_ERR_SHAPE, "padded copy: grid too large");
+    if (blocks == 0) return FG_OK;
+    hipLaunchKernelGGL(padded_copy_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, x, reinterpret_cast<float4 *>(pl->tiled_dev),
+                       n_rows, (uint32_t)(F / 4), (uint32_t)(tile / 4), (uint32_t)(F / heads / 4), given, (int64_t)(floats / 4));
+    FG_HIP_TRY(hipGetLastError());
+    return FG_OK;
+}
 bool wants_tile_major(const fg_spmm_plan *pl, int n_tiles, uint64_t x_bytes) {
     if (pl->tile_major == 2 || n_tiles < 2) return false;
     if (pl->tile_major == 1) return true;
@@ -414,7 +452,9 @@ extern "C" int fg_spmm_plan_reserve(fg_spmm_plan *pl, int op, int heads, int hea
         case FG_OP_ATTENTION: rc = fg::attention_scratch_need(pl, heads, head_len, 2, true, &need); break;
         case FG_OP_ATTENTION_ADDITIVE: rc = fg::additive_scratch_need(pl, heads, head_len, true, false, &need); break;
         case FG_OP_ATTENTION_ADDITIVE_TRAIN: rc = fg::additive_scratch_need(pl, heads, head_len, false, true, &need); break;
-        case FG_OP_SPMM_SUM_DOTS: rc = fg::spmm_dot_scratch_need(pl, heads * head_len, heads, num_feat_partitions, &need); break;
+        case FG_OP_SPMM_SUM_DOTS: rc = fg::spmm_dot_scratch_need(pl, heads * head_len, heads, num_feat_partitions, false, &need); break;
+        case FG_OP_SPMM_SUM_PADDED: rc = fg::spmm_padded_scratch_need(pl, heads * head_len, heads, num_feat_partitions, &need); break;
+        case FG_OP_SPMM_SUM_DOTS_PADDED: rc = fg::spmm_dot_scratch_need(pl, heads * head_len, heads, num_feat_partitions, true, &need); break;
         case FG_OP_GSPMM_BCAST: rc = fg::gspmm_bcast_scratch_need(pl, heads * head_len, false, &need); break;
         case FG_OP_GSPMM_BCAST_ARG: rc = fg::gspmm_bcast_scratch_need(pl, heads * head_len, true, &need); break;
         default: return fail(FG_ERR_ARG, "fg_spmm_plan_reserve: unknown operator %d", op);

@@ -375,10 +375,11 @@ int launch_arg_v(int L, int K, bool full, dim3 grid, hipStream_t st, const SpmmA
 // to an array of fixed size, a range of columns at a time).
 // part_stride / out_stride (floats; 0 for a launch over one partition's fix-ups): with every pass in a buffer of
 // its own, partition p's pieces start at partial + p * part_stride and its rows at out + p * out_stride.
-template <int V>
+// SHORT: rows of `out` lie F floats apart and hold heads of out_len floats, the pieces' heads head_len.
+template <int V, bool SHORT = false>
 __global__ __launch_bounds__(256) void spmm_fixup_kernel(const Fixup *fixups, int64_t n_fixups,
                                                          const float *partial, int partial_ld, float *out, int F, int f0, int width,
-                                                         int accumulate, int64_t part_stride, int64_t out_stride) {
+                                                         int accumulate, int64_t part_stride, int64_t out_stride, int head_len = 0, int out_len = 0) {
     using vec = typename Vec<V>::type;
     const int per_row = width / V;
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -390,6 +391,14 @@ __global__ __launch_bounds__(256) void spmm_fixup_kernel(const Fixup *fixups, in
     vec sum = *reinterpret_cast<const vec *>(partial + (int64_t)fx.slot0 * partial_ld + f);
     fg::each_piece(1, fx.n_pieces, [&](int p) { return *reinterpret_cast<const vec *>(partial + (int64_t)(fx.slot0 + p) * partial_ld + f); },
                    [&](int, const vec &v) { vadd(sum, v); });
+    if constexpr (SHORT) {
+        const int h = f / head_len, d = f - h * head_len;
+        const float v[4] = {sum.x, sum.y, sum.z, sum.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (d + i < out_len) out[(int64_t)fx.row * F + h * out_len + d + i] = v[i];
+        return;
+    }
     vec *o = reinterpret_cast<vec *>(out + (int64_t)fx.row * F + f0 + f);
     if (accumulate) vadd(sum, *o);
     *o = sum;
@@ -406,6 +415,30 @@ __global__ __launch_bounds__(256) void spmm_pass_sum_kernel(const float4 *buf, f
     f4 s = __builtin_nontemporal_load(b + i);
     for (int p = 1; p < P; ++p) s += __builtin_nontemporal_load(b + (size_t)p * words + i);
     __builtin_nontemporal_store(s, reinterpret_cast<f4 *>(out) + i);
+}
+
+// The same into rows that hold heads of out_len floats, out_len <= head_len (row_words: 16-byte words of a buffer's row).
+__global__ __launch_bounds__(256) void spmm_pass_sum_short_kernel(const float4 *buf, float *out, size_t words, int P, uint32_t row_words, uint32_t head_words,
+                                                                  int out_len) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= words) return;
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    const f4 *b = reinterpret_cast<const f4 *>(buf);
+    f4 s = __builtin_nontemporal_load(b + i);
+    for (int p = 1; p < P; ++p) s += __builtin_nontemporal_load(b + (size_t)p * words + i);
+    // the block's first word's row by one scalar division, the lane's from there in 32 bits
+    const size_t i0 = (size_t)blockIdx.x * 256, r0 = i0 / row_words;
+    const uint32_t at = (uint32_t)(i0 - r0 * row_words) + threadIdx.x, dr = at / row_words, c = at - dr * row_words;
+    const uint32_t h = c / head_words;
+    const int d = (int)(c - h * head_words) * 4, left = out_len - d;
+    float *o = out + (r0 + dr) * (size_t)(row_words / head_words) * out_len + (size_t)h * out_len + d;
+    if (left >= 4) {
+        *reinterpret_cast<fg::Words4<float> *>(o) = {{s.x, s.y, s.z, s.w}};
+    } else {
+        if (left > 0) o[0] = s.x;
+        if (left > 1) o[1] = s.y;
+        if (left > 2) o[2] = s.z;
+    }
 }
 
 struct SpmmConfig {
@@ -602,6 +635,14 @@ fg::ScratchNeed scratch_need(const fg_spmm_plan *pl, const SpmmConfig &c, int F,
     return need;
 }
 
+// A sum over padded rows: a zero-padded copy of x, and with several passes that add to one another a buffer of padded results.
+fg::ScratchNeed padded_scratch_need(const fg_spmm_plan *pl, const SpmmConfig &c, int F) {
+    fg::ScratchNeed need = scratch_need(pl, c, F, FG_REDUCE_SUM);
+    if (pl->num_col_partitions > 1 && !uses_pass_buffers(pl, c, F, FG_REDUCE_SUM)) need.partial += (size_t)pl->n_dst * (size_t)F;
+    need.tiled = (size_t)pl->n_src * (size_t)F;
+    return need;
+}
+
 // What a sum with dots is asked for besides the sum (SpmmArgs: own, own_ld, own_len); out[pos[element], head].
 struct DotRequest {
     const float *own;
@@ -643,25 +684,28 @@ int tiles_this_launch(int remaining) {
 }
 
 // reduce: FG_REDUCE_SUM / MAX / MIN.  heads > 1: vals is [nnz, heads] (or [heads, nnz] when
-// head_major).  vals == nullptr with allow_no_vals: every weight is 1.
+// head_major).  vals == nullptr with allow_no_vals: every weight is 1.  given > 0 (sums only): x and out hold heads of `given`
+// floats, fewer than the F / heads that the kernels run at; the columns beyond are zeros.
 int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const float *vals,
              const float *x, float *out, int F, int T, void *stream, int heads = 1,
              int reduce = FG_REDUCE_SUM, bool allow_no_vals = false, bool head_major = false,
              int32_t *arg_out = nullptr, float *fixed_partial = nullptr, size_t fixed_partial_floats = 0,
-             const DotRequest *dot = nullptr) {
+             const DotRequest *dot = nullptr, int given = 0) {
     if (!pl) return fail(FG_ERR_ARG, "plan is null");
     if (arg_out && reduce == FG_REDUCE_SUM) return fail(FG_ERR_ARG, "positions of the selected elements exist for max / min only");
     if (int drc = fg::check_device(pl)) return drc;
     if (pl->n_dst == 0) return FG_OK;
     if (!out || !pos || (pl->nnz > 0 && (!idx || (!vals && !allow_no_vals) || !x)))
         return fail(FG_ERR_ARG, "null device pointer");
-    const bool aligned16 = (((uintptr_t)x | (uintptr_t)out | (uintptr_t)arg_out) & 15) == 0;
+    const bool padded = given > 0;           // the kernels then read the copy, which is aligned, and store at any alignment
+    const bool aligned16 = padded || (((uintptr_t)x | (uintptr_t)out | (uintptr_t)arg_out) & 15) == 0;
     SpmmConfig c;
     int rc = resolve_config(pl, F, T, heads, reduce, aligned16, &c);
     if (rc != FG_OK) return rc;
+    if (padded && c.V != 4) return fail(FG_ERR_SHAPE, "padded rows need tiles of a multiple of 4 floats, got %d", c.tile_w);
     // fixed_partial: the split rows' partial sums go to this buffer of fixed size instead of the plan's,
     // X is gathered from the caller's matrix (no tile-by-tile copy), and nothing is allocated.
-    fg::ScratchNeed need = scratch_need(pl, c, F, reduce);
+    fg::ScratchNeed need = padded ? padded_scratch_need(pl, c, F) : scratch_need(pl, c, F, reduce);
     size_t dots_at = 0;
     if (dot && (rc = add_dots(pl, c, F, heads, &need, &dots_at)) != FG_OK) return rc;
     if (fixed_partial) {
@@ -681,6 +725,9 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
     const size_t piece = piece_floats(pl, F);
     float *const pass_buf = (!fixed_partial && uses_pass_buffers(pl, c, F, reduce)) ? pl->partial_dev + (size_t)P * piece : nullptr;
     const size_t pass_stride = (size_t)pl->n_dst * (size_t)F;
+    // padded rows in several passes: the last kernel shortens them, from the passes' buffers or from one that the passes add to
+    float *const padded_out = padded && P > 1 && !pass_buf ? pl->partial_dev + piece : nullptr;
+    float *const row_out = padded_out ? padded_out : out;
     hipStream_t st = (hipStream_t)stream;
     const int64_t width = (pl->n_src + P - 1) / P;
     // With several feature tiles an XCD gathers one tile's 256 bytes (or less) out of every source
@@ -696,10 +743,16 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
         a.dots_stride = (int64_t)dot_stride(pl);
     };
     auto launch_sum = [&](dim3 grid, const SpmmArgs &a) {
+        if (a.out_len > 0 && !dot) return fg_items::launch_padded(c.L, c.K, c.full, c.off32, c.hpt, grid, st, a);
         return dot ? fg_items::launch_dot(c.L, c.hpt, grid, st, a) : c.V == 4 ? launch_v<4>(c, grid, st, a) : launch_v<1>(c, grid, st, a);
     };
-    const bool tiled = need.tiled > 0;
-    if (tiled && (rc = fg::make_tile_major(pl, x, pl->n_src, F, ft, stream)) != FG_OK) return rc;
+    const bool tiled = padded ? gathers_tile_major(pl, c, F) : need.tiled > 0;
+    if (padded) {
+        if (pl->nnz > 0 && (rc = fg::make_padded_copy(pl, x, pl->n_src, heads, given, F, tiled ? ft : F, stream)) != FG_OK) return rc;
+        x = pl->tiled_dev;
+    } else if (tiled && (rc = fg::make_tile_major(pl, x, pl->n_src, F, ft, stream)) != FG_OK) {
+        return rc;
+    }
     if (pass_buf && pl->n_items > 0) {
         // The passes are independent (each writes a buffer and pieces of its own), so one launch walks the items of all
         // partitions, partition by partition in workgroup order: the next partition's first workgroups fill the
@@ -758,7 +811,8 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
             a.x = tiled ? pl->tiled_dev + (int64_t)p * width * ft : x + (int64_t)p * width * F;
             a.x_row_bytes = (uint32_t)(tiled ? ft : F) * 4u;
             a.x_tile_bytes = tiled ? (uint32_t)((uint64_t)pl->n_src * ft * 4u) : 0u;
-            a.out = out; a.partial = partial; a.partial_ld = piece_ld; a.partial_f0 = f0;
+            a.out = row_out; a.partial = partial; a.partial_ld = piece_ld; a.partial_f0 = f0;
+            if (padded && P == 1) { a.out_ld = heads * given; a.out_len = given; }
             a.F = F; a.tile_w = c.tile_w; a.sub_per_tile = c.sub_per_tile;
             a.heads = heads; a.head_len = F / heads;
             a.vstride = head_major ? 1 : heads; a.head_stride = head_major ? pl->nnz : 1;
@@ -787,8 +841,10 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
             const Fixup *fx = pl->fixups_dev + x0;
             if (reduce == FG_REDUCE_SUM) {
                 const int add = p > 0 ? 1 : 0;
-                if (fv == 4) hipLaunchKernelGGL(spmm_fixup_kernel<4>, dim3(blocks), dim3(256), 0, st, fx, x1 - x0, partial, piece_ld, out, F, f0, piece_ld, add, (int64_t)0, (int64_t)0);
-                else hipLaunchKernelGGL(spmm_fixup_kernel<1>, dim3(blocks), dim3(256), 0, st, fx, x1 - x0, partial, piece_ld, out, F, f0, piece_ld, add, (int64_t)0, (int64_t)0);
+                if (padded && P == 1)
+                    hipLaunchKernelGGL((spmm_fixup_kernel<4, true>), dim3(blocks), dim3(256), 0, st, fx, x1 - x0, partial, piece_ld, out, heads * given, 0, piece_ld, 0, (int64_t)0, (int64_t)0, F / heads, given);
+                else if (fv == 4) hipLaunchKernelGGL(spmm_fixup_kernel<4>, dim3(blocks), dim3(256), 0, st, fx, x1 - x0, partial, piece_ld, row_out, F, f0, piece_ld, add, (int64_t)0, (int64_t)0);
+                else hipLaunchKernelGGL(spmm_fixup_kernel<1>, dim3(blocks), dim3(256), 0, st, fx, x1 - x0, partial, piece_ld, row_out, F, f0, piece_ld, add, (int64_t)0, (int64_t)0);
             } else if (reduce == FG_REDUCE_MAX) {
                 if (fv == 4) hipLaunchKernelGGL((gspmm_extreme_fixup_kernel<4, true>), dim3(blocks), dim3(256), 0, st, fx, x1 - x0, partial, out, F);
                 else hipLaunchKernelGGL((gspmm_extreme_fixup_kernel<1, true>), dim3(blocks), dim3(256), 0, st, fx, x1 - x0, partial, out, F);
@@ -798,9 +854,13 @@ int spmm_run(fg_spmm_plan *pl, const int32_t *pos, const int32_t *idx, const flo
             }
         }
     }
-    if (pass_buf) {
+    if (pass_buf || padded_out) {
         const size_t words = pass_stride / 4;
-        hipLaunchKernelGGL(spmm_pass_sum_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st,
+        if (padded)
+            hipLaunchKernelGGL(spmm_pass_sum_short_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st,
+                               reinterpret_cast<const float4 *>(pass_buf ? pass_buf : padded_out), out, words, pass_buf ? P : 1,
+                               (uint32_t)(F / 4), (uint32_t)(F / heads / 4), given);
+        else hipLaunchKernelGGL(spmm_pass_sum_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st,
                            reinterpret_cast<const float4 *>(pass_buf), reinterpret_cast<float4 *>(out), words, P);
     }
     if (dot && pl->nnz > 0) {
@@ -841,11 +901,17 @@ int spmm_scratch_need(const fg_spmm_plan *pl, int F, int heads, int reduce, int 
     *need = scratch_need(pl, c, F, reduce);
     return FG_OK;
 }
-int spmm_dot_scratch_need(const fg_spmm_plan *pl, int F, int heads, int T, ScratchNeed *need) {
+int spmm_padded_scratch_need(const fg_spmm_plan *pl, int F, int heads, int T, ScratchNeed *need) {
+    SpmmConfig c;
+    if (int rc = resolve_config(pl, F, T, heads, FG_REDUCE_SUM, true, &c)) return rc;
+    *need = padded_scratch_need(pl, c, F);
+    return FG_OK;
+}
+int spmm_dot_scratch_need(const fg_spmm_plan *pl, int F, int heads, int T, bool padded, ScratchNeed *need) {
     SpmmConfig c;
     size_t at;
     if (int rc = resolve_config(pl, F, T, heads, FG_REDUCE_SUM, true, &c)) return rc;
-    *need = scratch_need(pl, c, F, FG_REDUCE_SUM);
+    *need = padded ? padded_scratch_need(pl, c, F) : scratch_need(pl, c, F, FG_REDUCE_SUM);
     return add_dots(pl, c, F, heads, need, &at);
 }
 std::string spmm_launch_text(const fg_spmm_plan *pl, int F, int T) {
@@ -953,20 +1019,51 @@ extern "C" int fg_spmm_dot_takes(const fg_spmm_plan *plan, int F, int heads, int
     return takes_dots(plan, c, F, heads) ? 1 : 0;
 }
 
-extern "C" int fg_spmm_dot_f32(fg_spmm_plan *plan, const int32_t *pos_dev, const int32_t *idx_dev, const float *vals_dev,
-                               const float *x_dev, const float *own_dev, int own_len, float *out_dev,
-                               const int32_t *edge_pos_dev, float *dots_dev, int F, int heads, int vals_head_major,
-                               int num_feat_partitions, void *stream) {
+// fg_gspmm_f32 (sum) over rows of `heads` heads of given_len floats, computed at F / heads.
+extern "C" int fg_gspmm_padded_f32(fg_spmm_plan *plan, const int32_t *pos_dev, const int32_t *idx_dev, const float *vals_dev,
+                                   const float *x_dev, int given_len, float *out_dev, int F, int heads, int vals_head_major,
+                                   int num_feat_partitions, void *stream) {
+    if (heads < 1 || F < 1 || F % heads != 0) return fail(FG_ERR_SHAPE, "feature length %d is not divisible by %d heads", F, heads);
+    if (given_len < 1 || given_len > F / heads) return fail(FG_ERR_SHAPE, "heads of %d floats, computed at %d", given_len, F / heads);
+    return spmm_run(plan, pos_dev, idx_dev, vals_dev, x_dev, out_dev, F, num_feat_partitions, stream, heads, FG_REDUCE_SUM,
+                    /*allow_no_vals=*/true, vals_head_major != 0, nullptr, nullptr, 0, nullptr, given_len < F / heads ? given_len : 0);
+}
+
+namespace {
+// given: floats per head of x and out (0: F / heads)
+int spmm_dot_run(fg_spmm_plan *plan, const int32_t *pos_dev, const int32_t *idx_dev, const float *vals_dev, const float *x_dev, int given,
+                 const float *own_dev, int own_len, float *out_dev, const int32_t *edge_pos_dev, float *dots_dev, int F, int heads,
+                 int vals_head_major, int num_feat_partitions, void *stream) {
     if (!plan) return fail(FG_ERR_ARG, "plan is null");
     if (heads < 1 || F < 1 || F % heads != 0) return fail(FG_ERR_SHAPE, "feature length %d is not divisible by %d heads", F, heads);
     if (own_len < 1 || own_len > F / heads) return fail(FG_ERR_SHAPE, "heads of %d floats in own, of %d in x", own_len, F / heads);
     // without elements there is nothing to take a dot product of: the plain sum, which reads none of the three
-    if (plan->nnz == 0) return fg_gspmm_f32(plan, pos_dev, idx_dev, vals_dev, x_dev, out_dev, F, heads, vals_head_major, FG_REDUCE_SUM, num_feat_partitions, stream);
+    if (plan->nnz == 0)
+        return fg_gspmm_padded_f32(plan, pos_dev, idx_dev, vals_dev, x_dev, given ? given : F / heads, out_dev, F, heads, vals_head_major, num_feat_partitions, stream);
     if (plan->n_dst > 0 && (!own_dev || !edge_pos_dev || !dots_dev)) return fail(FG_ERR_ARG, "null device pointer");
     if (((uintptr_t)edge_pos_dev & 15) != 0) return fail(FG_ERR_ARG, "the positions of the dots must be 16-byte aligned");
     const DotRequest dot = {own_dev, (int64_t)heads * own_len, own_len, dots_dev, edge_pos_dev};
     return spmm_run(plan, pos_dev, idx_dev, vals_dev, x_dev, out_dev, F, num_feat_partitions, stream, heads, FG_REDUCE_SUM,
-                    /*allow_no_vals=*/false, vals_head_major != 0, nullptr, nullptr, 0, &dot);
+                    /*allow_no_vals=*/false, vals_head_major != 0, nullptr, nullptr, 0, &dot, given);
+}
+}  // namespace
+
+extern "C" int fg_spmm_dot_f32(fg_spmm_plan *plan, const int32_t *pos_dev, const int32_t *idx_dev, const float *vals_dev,
+                               const float *x_dev, const float *own_dev, int own_len, float *out_dev,
+                               const int32_t *edge_pos_dev, float *dots_dev, int F, int heads, int vals_head_major,
+                               int num_feat_partitions, void *stream) {
+    return spmm_dot_run(plan, pos_dev, idx_dev, vals_dev, x_dev, 0, own_dev, own_len, out_dev, edge_pos_dev, dots_dev, F, heads,
+                        vals_head_major, num_feat_partitions, stream);
+}
+
+// fg_spmm_dot_f32 with x, own and out of heads of given_len floats.
+extern "C" int fg_spmm_dot_padded_f32(fg_spmm_plan *plan, const int32_t *pos_dev, const int32_t *idx_dev, const float *vals_dev,
+                                      const float *x_dev, const float *own_dev, int given_len, float *out_dev,
+                                      const int32_t *edge_pos_dev, float *dots_dev, int F, int heads, int vals_head_major,
+                                      int num_feat_partitions, void *stream) {
+    const int given = heads >= 1 && given_len < F / heads ? given_len : 0;
+    return spmm_dot_run(plan, pos_dev, idx_dev, vals_dev, x_dev, given, own_dev, given_len, out_dev, edge_pos_dev, dots_dev, F, heads,
+                        vals_head_major, num_feat_partitions, stream);
 }
 
 extern "C" int fg_gspmm_arg_f32(fg_spmm_plan *plan, const int32_t *indptr_dev, const int32_t *indices_dev,

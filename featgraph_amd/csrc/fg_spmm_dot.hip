@@ -14,9 +14,16 @@ namespace {
 // of 602 floats: 1.80 ms and 0.17 ms to add the tiles' parts up, in the place of a sum of 1.47 ms and an SDDMM of 1.72 (whole
 // step 5194 -> 3850 us); 7 wavefronts per SIMD without spills beat 8 with them (step 4172 against 3990 before the last kernel's
 // own gain).
-template <int L, int HPT>
+template <int L, int HPT, bool SHORT>
 __global__ __launch_bounds__(kBlock, HPT == 1 ? 7 : 4) void spmm_dot_kernel(const SpmmArgs a) {
-    spmm_items_body<4, L, 1, true, false, true, HPT, true>(a);
+    spmm_items_body<4, L, 1, true, false, true, HPT, true, SHORT>(a);
+}
+
+template <int L, int HPT>
+int launch(dim3 grid, hipStream_t st, const SpmmArgs &a) {
+    if (a.out_len > 0) hipLaunchKernelGGL((spmm_dot_kernel<L, HPT, true>), grid, dim3(kBlock), 0, st, a);
+    else hipLaunchKernelGGL((spmm_dot_kernel<L, HPT, false>), grid, dim3(kBlock), 0, st, a);
+    return FG_OK;
 }
 
 }  // namespace
@@ -25,15 +32,15 @@ namespace fg_items {
 int launch_dot(int L, int hpt, dim3 grid, hipStream_t st, const SpmmArgs &a) {
     if (hpt == 1) {
         switch (L) {
-            case 4: hipLaunchKernelGGL((spmm_dot_kernel<4, 1>), grid, dim3(kBlock), 0, st, a); return FG_OK;
-            case 8: hipLaunchKernelGGL((spmm_dot_kernel<8, 1>), grid, dim3(kBlock), 0, st, a); return FG_OK;
-            case 16: hipLaunchKernelGGL((spmm_dot_kernel<16, 1>), grid, dim3(kBlock), 0, st, a); return FG_OK;
-            case 32: hipLaunchKernelGGL((spmm_dot_kernel<32, 1>), grid, dim3(kBlock), 0, st, a); return FG_OK;
-            case 64: hipLaunchKernelGGL((spmm_dot_kernel<64, 1>), grid, dim3(kBlock), 0, st, a); return FG_OK;
+            case 4: return launch<4, 1>(grid, st, a);
+            case 8: return launch<8, 1>(grid, st, a);
+            case 16: return launch<16, 1>(grid, st, a);
+            case 32: return launch<32, 1>(grid, st, a);
+            case 64: return launch<64, 1>(grid, st, a);
         }
-    } else if (L == 16 && hpt == 2) { hipLaunchKernelGGL((spmm_dot_kernel<16, 2>), grid, dim3(kBlock), 0, st, a); return FG_OK; }
-    else if (L == 16 && hpt == 4) { hipLaunchKernelGGL((spmm_dot_kernel<16, 4>), grid, dim3(kBlock), 0, st, a); return FG_OK; }
-    else if (L == 8 && hpt == 4) { hipLaunchKernelGGL((spmm_dot_kernel<8, 4>), grid, dim3(kBlock), 0, st, a); return FG_OK; }
+    } else if (L == 16 && hpt == 2) { return launch<16, 2>(grid, st, a); }
+    else if (L == 16 && hpt == 4) { return launch<16, 4>(grid, st, a); }
+    else if (L == 8 && hpt == 4) { return launch<8, 4>(grid, st, a); }
     return fail(FG_ERR_SHAPE, "no SpMM kernel with dots for %d heads per tile with L=%d", hpt, L);
 }
 }  // namespace fg_items

@@ -81,6 +81,9 @@ struct SpmmArgs {
     int own_len = 0;
     float *dots = nullptr;
     int64_t dots_stride = 0;
+    // Kernels that store rows shorter than the ones they compute (x is a zero-padded copy): rows of `out` lie out_ld floats
+    // apart and hold heads of out_len <= head_len floats.
+    int out_ld = 0, out_len = 0;
 };
 
 
@@ -214,16 +217,42 @@ __device__ __forceinline__ void gather_rows(int2 *s_edge, float *wrow, int b, in
         gather_tail<V, L, K, FULL, U, OFF32, HPT>((e - s0 + G - 1) / G, s_edge, wrow, s0, e, g, x, lane_bytes, F, on, acc, dots);
 }
 
-// Adds the lane groups' sums (group 0 gets the total) and stores one output row; `old` is what
-// the row held before (only read when ADD).
-template <int V, int L, int K, bool FULL, bool ADD>
-__device__ __forceinline__ void finish_row(typename Vec<V>::type (&acc)[K], const typename Vec<V>::type (&old)[K],
-                                           int g, const bool (&on)[K], float *dst) {
-    using vec = typename Vec<V>::type;
+// Stores a lane's columns f_lo, f_lo + L * V, .. of a row that holds heads of out_len floats, out_len <= head_len: 16-byte stores
+// at 4-byte alignment, the head's last words one by one.
+template <int V, int L, int K, bool FULL>
+__device__ __forceinline__ void store_short(const SpmmArgs &a, const typename Vec<V>::type (&v)[K], const bool (&on)[K], float *row, int f_lo) {
+    if constexpr (V == 4) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            if (!(FULL || on[k])) continue;
+            const int f = f_lo + k * L * V, h = a.heads == 1 ? 0 : f / a.head_len, d = f - h * a.head_len, left = a.out_len - d;
+            float *p = row + h * a.out_len + d;
+            if (left >= 4) {
+                *reinterpret_cast<fg::Words4<float> *>(p) = {{v[k].x, v[k].y, v[k].z, v[k].w}};
+            } else {
+                if (left > 0) p[0] = v[k].x;
+                if (left > 1) p[1] = v[k].y;
+                if (left > 2) p[2] = v[k].z;
+            }
+        }
+    }
+}
+
+// Adds the lane groups' sums (group 0 gets the total).
+template <int V, int L, int K>
+__device__ __forceinline__ void add_groups(typename Vec<V>::type (&acc)[K]) {
 #pragma unroll
     for (int off = L; off < 64; off <<= 1)
 #pragma unroll
         for (int k = 0; k < K; ++k) vadd(acc[k], vshfl_xor(acc[k], off));
+}
+
+// Adds the lane groups' sums and stores one output row; `old` is what the row held before (only read when ADD).
+template <int V, int L, int K, bool FULL, bool ADD>
+__device__ __forceinline__ void finish_row(typename Vec<V>::type (&acc)[K], const typename Vec<V>::type (&old)[K],
+                                           int g, const bool (&on)[K], float *dst) {
+    using vec = typename Vec<V>::type;
+    add_groups<V, L, K>(acc);
     if (g == 0) {
 #pragma unroll
         for (int k = 0; k < K; ++k)
@@ -292,8 +321,8 @@ __device__ __forceinline__ void stage_store_w(float (*rows)[ROW], int lane, cons
 // FULL: every lane's columns are inside the tile (no masking needed); ACC: add to out;
 // OFF32: X spans less than 4 GiB, rows are addressed by 32-bit byte offsets; HPT: heads (with
 // their own weights) per kernel tile, each covered by L / HPT lanes; DOT: each element's dot product with the output
-// row's row of `own` as well.
-template <int V, int L, int K, bool FULL, bool ACC, bool OFF32, int HPT = 1, bool DOT = false>
+// row's row of `own` as well; SHORT: the rows of out are shorter than the computed ones (SpmmArgs: out_ld, out_len).
+template <int V, int L, int K, bool FULL, bool ACC, bool OFF32, int HPT = 1, bool DOT = false, bool SHORT = false>
 __device__ __forceinline__ void spmm_items_body(const SpmmArgs &a) {
     using vec = typename Vec<V>::type;
     static_assert(fg::kItemEdges == 256, "stage_load/stage_store move 4 x 64 elements");
@@ -308,6 +337,7 @@ __device__ __forceinline__ void spmm_items_body(const SpmmArgs &a) {
     constexpr int kWRow = HPT > 1 ? fg::kItemEdges + kPad : 1;
     __shared__ __align__(16) float s_w[kWavesPerBlock][HPT][kWRow];
     static_assert(HPT == 1 || (L % HPT == 0 && K == 1 && FULL), "heads of a tile split its lanes evenly");
+    static_assert(!SHORT || (V == 4 && !ACC), "short rows: 128-bit lanes, one pass");
     static_assert(!DOT || (V == 4 && K == 1 && FULL && !ACC), "dots: whole tiles of 128-bit lanes, every pass in its own buffer");
 
     const int lane = threadIdx.x & 63;
@@ -445,7 +475,12 @@ __device__ __forceinline__ void spmm_items_body(const SpmmArgs &a) {
                     for (int k = 0; k < K; ++k) acc[k] = vzero(vec());
                     load_own(it.row + q);
                     gather_rows<V, L, K, FULL, U, OFF32, HPT>(edge, wrow, b, e, g, x_p, lane_bytes, F, on, acc, dots);
-                    finish_row<V, L, K, FULL, ACC>(acc, old, g, on, dst);
+                    if constexpr (SHORT) {
+                        add_groups<V, L, K>(acc);
+                        if (g == 0) store_short<V, L, K, FULL>(a, acc, on, out_p + (int64_t)(it.row + q) * a.out_ld, f_lo);
+                    } else {
+                        finish_row<V, L, K, FULL, ACC>(acc, old, g, on, dst);
+                    }
                 }
                 b = e;
             }
@@ -459,7 +494,9 @@ __device__ __forceinline__ void spmm_items_body(const SpmmArgs &a) {
         bool done = false, nonempty = false;
         for (;;) {
             if (!done && j >= e) {
-                if (q >= 0 && (!ACC || nonempty)) {       // the row this group just finished
+                if (SHORT && q >= 0) {
+                    store_short<V, L, K, FULL>(a, acc, on, out_p + (int64_t)(it.row + q) * a.out_ld, f_lo);
+                } else if (q >= 0 && (!ACC || nonempty)) {       // the row this group just finished
                     float *dst = out_p + (int64_t)(it.row + q) * F + f_lo;
 #pragma unroll
                     for (int k = 0; k < K; ++k)
@@ -556,10 +593,19 @@ __device__ __forceinline__ void spmm_items_body(const SpmmArgs &a) {
         gather_rows<V, L, K, FULL, U, OFF32, HPT>(edge, wrow, 0, n, g, x_p, lane_bytes, F, on, acc, dots);
         flush_dots((int64_t)it.start + base, n);
     }
+    if constexpr (SHORT) {
+        if (it.info < 0) {
+            add_groups<V, L, K>(acc);
+            if (g == 0) store_short<V, L, K, FULL>(a, acc, on, out_p + (int64_t)it.row * a.out_ld, f_lo);
+            return;
+        }
+    }
     finish_row<V, L, K, FULL, ACC>(acc, old, g, on, dst);
 }
 
-// The sum with dots: hpt heads per kernel tile, L lanes per source row (fg_spmm_dot.hip).
+// The sum with dots: hpt heads per kernel tile, L lanes per source row (fg_spmm_dot.hip).  a.out_len > 0: short rows of out.
 int launch_dot(int L, int hpt, dim3 grid, hipStream_t st, const SpmmArgs &a);
+// The sum with short rows of out, one pass: L lanes of K loads of 4 floats per source row (fg_spmm_padded.hip).
+int launch_padded(int L, int K, bool full, bool off32, int hpt, dim3 grid, hipStream_t st, const SpmmArgs &a);
 
 }  // namespace fg_items

@@ -101,7 +101,7 @@ def timed_mean_seconds(fn, num_runs):
 
 # fg_op of include/featgraph_hip.h
 (OP_SPMM_SUM, OP_SPMM_EXTREME, OP_SDDMM_DDS, OP_EDGE_SOFTMAX, OP_ATTENTION, OP_ATTENTION_ADDITIVE,
- OP_GSPMM_BCAST, OP_GSPMM_BCAST_ARG, OP_ATTENTION_ADDITIVE_TRAIN, OP_SPMM_SUM_DOTS) = range(10)
+ OP_GSPMM_BCAST, OP_GSPMM_BCAST_ARG, OP_ATTENTION_ADDITIVE_TRAIN, OP_SPMM_SUM_DOTS, OP_SPMM_SUM_PADDED, OP_SPMM_SUM_DOTS_PADDED) = range(12)
 
 
 def reserve(plan, op, heads, head_len, num_feat_partitions, dev):

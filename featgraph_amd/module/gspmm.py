@@ -102,7 +102,10 @@ class GSpMMhip(VanillaSpMMhip):
         self._active = self._glayout(P)
         self._func = _lib.lib().fg_gspmm_f32
         self._dots_fit = True
-        common.reserve(self._active['plan'], common.OP_SPMM_SUM if _REDUCE[reduce] == 0 else common.OP_SPMM_EXTREME,
+        # the sum's kernels pad and shorten the rows themselves, max / min run between padded copies made here
+        self._pads_inside = self._pad_from is not None and _REDUCE[reduce] == 0
+        common.reserve(self._active['plan'], common.OP_SPMM_SUM_PADDED if self._pads_inside else
+                       common.OP_SPMM_SUM if _REDUCE[reduce] == 0 else common.OP_SPMM_EXTREME,
                        heads, feat_len // heads, self._num_feat_partitions, self._ctx)
         self._return_arg = return_arg
         self._inv_deg_edge = None
@@ -113,7 +116,7 @@ class GSpMMhip(VanillaSpMMhip):
             inv = np.where(deg > 0, 1.0 / np.maximum(deg, 1), 0).astype(np.float32)
             self._inv_deg_edge = common.to_device_f32(np.repeat(inv, np.diff(self._adj_indptr)), self._ctx)
         self._x_pad = self._out_pad = None
-        if self._pad_from is not None:
+        if self._pad_from is not None and not self._pads_inside:
             tail = (feat_len,) if heads == 1 else (heads, feat_len // heads)
             self._x_pad = torch.zeros((self._num_cols,) + tail, dtype=torch.float32, device=self._ctx)
             self._out_pad = torch.zeros((self._num_rows,) + tail, dtype=torch.float32, device=self._ctx)
@@ -347,6 +350,11 @@ class GSpMMhip(VanillaSpMMhip):
             return
         out = self.out_tvm
         if getattr(self, '_pad_from', None) is not None:
+            if self._pads_inside:
+                _lib.check(_lib.lib().fg_gspmm_padded_f32(
+                    lay['plan'], _lib.dev_ptr(lay['pos']), _lib.dev_ptr(lay['idx']), _lib.dev_ptr(w), _lib.dev_ptr(src_feat), self._pad_from,
+                    _lib.dev_ptr(out), self._feat_len, heads, head_major, self._num_feat_partitions, common.stream_ptr()))
+                return
             self._x_pad[..., :self._pad_from].copy_(src_feat)       # the padding columns stay zero
             src_feat, out = self._x_pad, self._out_pad
         _lib.check(self._func(lay['plan'], _lib.dev_ptr(lay['pos']), _lib.dev_ptr(lay['idx']), _lib.dev_ptr(w),
@@ -375,7 +383,7 @@ class GSpMMhip(VanillaSpMMhip):
     def reserve_dots(self):
         """Sizes the plan's scratch for run_with_dots() (build() sizes it for run(), which needs less): to be called after build()
         by a program whose first such call is one that it captures.  ValueError where the library has no kernel for both."""
-        common.reserve(self._active['plan'], common.OP_SPMM_SUM_DOTS, self._heads, self._feat_len // self._heads,
+        common.reserve(self._active['plan'], common.OP_SPMM_SUM_DOTS if self._pad_from is None else common.OP_SPMM_SUM_DOTS_PADDED, self._heads, self._feat_len // self._heads,
                        self._num_feat_partitions, self._ctx)
 
     def run_with_dots(self, src_feat, weights, own):
@@ -398,20 +406,15 @@ class GSpMMhip(VanillaSpMMhip):
         w, head_major = self._weights(weights)
         self._w_keepalive = w
         dots = torch.empty_like(weights)
-        out = self.out_tvm
-        if self._pad_from is not None:
-            self._x_pad[..., :self._pad_from].copy_(src_feat)
-            src_feat, out = self._x_pad, self._out_pad
+        call = _lib.lib().fg_spmm_dot_f32 if self._pad_from is None else _lib.lib().fg_spmm_dot_padded_f32
         try:
-            _lib.check(_lib.lib().fg_spmm_dot_f32(
+            _lib.check(call(
                 lay['plan'], _lib.dev_ptr(lay['pos']), _lib.dev_ptr(lay['idx']), _lib.dev_ptr(w), _lib.dev_ptr(src_feat), _lib.dev_ptr(own),
-                own.shape[-1], _lib.dev_ptr(out), _lib.dev_ptr(pos), _lib.dev_ptr(dots), self._feat_len, self._heads, head_major,
+                own.shape[-1], _lib.dev_ptr(self.out_tvm), _lib.dev_ptr(pos), _lib.dev_ptr(dots), self._feat_len, self._heads, head_major,
                 self._num_feat_partitions, common.stream_ptr()))
         except MemoryError:
             self._dots_fit = False
             return None
-        if out is not self.out_tvm:
-            self.out_tvm.copy_(out[..., :self._pad_from])
         return self.out_tvm, dots
 
     def run(self, input_tvm_ndarrays):

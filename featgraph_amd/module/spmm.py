@@ -282,11 +282,8 @@ class SpMMbase(object):
         if not getattr(self, '_tuning', False):
             self._release_unused_layouts()
         self._func = _lib.lib().fg_spmm_dds_f32 if P > 1 else _lib.lib().fg_spmm_csr_f32
-        common.reserve(self._active['plan'], common.OP_SPMM_SUM, 1, feat_len, T, self._ctx)
-        self._x_pad = self._out_pad = None
-        if self._pad_from is not None:
-            self._x_pad = torch.zeros((self._num_cols, feat_len), dtype=torch.float32, device=self._ctx)
-            self._out_pad = torch.zeros((self._num_rows, feat_len), dtype=torch.float32, device=self._ctx)
+        common.reserve(self._active['plan'], common.OP_SPMM_SUM if self._pad_from is None else common.OP_SPMM_SUM_PADDED,
+                       1, feat_len, T, self._ctx)
         self.out_tvm = torch.zeros((self._num_rows, self._pad_from or feat_len), dtype=torch.float32, device=self._ctx)
 
     def lower_to_ir(self, input_placeholders, compute_args, schedule_args):
@@ -301,15 +298,12 @@ class SpMMbase(object):
 
     def _launch(self, src_feat):
         lay = self._active
-        out = self.out_tvm
+        arrays = (lay['plan'], _lib.dev_ptr(lay['pos']), _lib.dev_ptr(lay['idx']), _lib.dev_ptr(lay['vals']), _lib.dev_ptr(src_feat))
         if getattr(self, '_pad_from', None) is not None:
-            self._x_pad[:, :self._pad_from].copy_(src_feat)         # the padding columns stay zero
-            src_feat, out = self._x_pad, self._out_pad
-        _lib.check(self._func(lay['plan'], _lib.dev_ptr(lay['pos']), _lib.dev_ptr(lay['idx']), _lib.dev_ptr(lay['vals']),
-                              _lib.dev_ptr(src_feat), _lib.dev_ptr(out), self._feat_len,
-                              self._num_feat_partitions, common.stream_ptr()))
-        if out is not self.out_tvm:
-            self.out_tvm.copy_(out[:, :self._pad_from])
+            _lib.check(_lib.lib().fg_gspmm_padded_f32(*arrays, self._pad_from, _lib.dev_ptr(self.out_tvm), self._feat_len, 1, 0,
+                                                      self._num_feat_partitions, common.stream_ptr()))
+            return
+        _lib.check(self._func(*arrays, _lib.dev_ptr(self.out_tvm), self._feat_len, self._num_feat_partitions, common.stream_ptr()))
 
     def run(self, input_tvm_ndarrays):
         """Run the built func with the given inputs.

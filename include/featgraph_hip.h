@@ -134,7 +134,9 @@ typedef enum {
     FG_OP_GSPMM_BCAST = 6,        /* fg_gspmm_bcast_f32 / _dds_f32 without arg_dev (heads * head_len = out_len) */
     FG_OP_GSPMM_BCAST_ARG = 7,    /* fg_gspmm_bcast_f32 / _dds_f32 with arg_dev */
     FG_OP_ATTENTION_ADDITIVE_TRAIN = 8, /* fg_graph_attention_additive_train_f32 and _train_elv_f32 */
-    FG_OP_SPMM_SUM_DOTS = 9       /* fg_spmm_dot_f32 (FG_ERR_SHAPE where fg_spmm_dot_takes says no) */
+    FG_OP_SPMM_SUM_DOTS = 9,      /* fg_spmm_dot_f32 (FG_ERR_SHAPE where fg_spmm_dot_takes says no) */
+    FG_OP_SPMM_SUM_PADDED = 10,   /* fg_gspmm_padded_f32 (head_len: F / heads) */
+    FG_OP_SPMM_SUM_DOTS_PADDED = 11 /* fg_spmm_dot_padded_f32 (likewise) */
 } fg_op;
 int fg_spmm_plan_reserve(fg_spmm_plan *plan, int op, int heads, int head_len, int num_feat_partitions);
 
@@ -244,6 +246,18 @@ int fg_spmm_dot_takes(const fg_spmm_plan *plan, int F, int heads, int num_feat_p
 int fg_spmm_dot_f32(fg_spmm_plan *plan, const int32_t *pos_dev, const int32_t *idx_dev, const float *vals_dev,
                     const float *x_dev, const float *own_dev, int own_len, float *out_dev, const int32_t *edge_pos_dev,
                     float *dots_dev, int F, int heads, int vals_head_major, int num_feat_partitions, void *stream);
+
+/*
+ * fg_gspmm_f32 (sum) and fg_spmm_dot_f32 over rows whose length suits no tile: x, out and own hold heads of given_len floats, at any
+ * 4-byte alignment, and the kernels run at heads of F / heads >= given_len floats (a length that fg_gspmm_f32 takes, tiles of a
+ * multiple of 4), on a zero-padded copy of x in the plan's scratch (n_src * F floats).  Zero columns change no sum.
+ */
+int fg_gspmm_padded_f32(fg_spmm_plan *plan, const int32_t *pos_dev, const int32_t *idx_dev, const float *vals_dev,
+                        const float *x_dev, int given_len, float *out_dev, int F, int heads, int vals_head_major,
+                        int num_feat_partitions, void *stream);
+int fg_spmm_dot_padded_f32(fg_spmm_plan *plan, const int32_t *pos_dev, const int32_t *idx_dev, const float *vals_dev,
+                           const float *x_dev, const float *own_dev, int given_len, float *out_dev, const int32_t *edge_pos_dev,
+                           float *dots_dev, int F, int heads, int vals_head_major, int num_feat_partitions, void *stream);
 
 /*
  * fg_gspmm_f32 with FG_REDUCE_MAX / FG_REDUCE_MIN that also reports which element was selected (no
