@@ -259,7 +259,7 @@ class SDDMMbase(object):
         nnz = self._adj_row_indices.shape[0]
         if order in ('auto', 'tiled') and nnz > 0:
             tiled = tuning.choose_sddmm(self._num_rows, self._num_cols, nnz, H, D, self._graph_stats() if H == 1 else None,
-                                        given_len=getattr(self, '_pad_from', None))
+                                        given_len=getattr(self, '_pad_from', None), scattered=not self._row_sorted)
             if H > 1 and getattr(self, '_pad_from', None) is not None and tiled is not None and tiled[0] == 1:
                 # padded heads without source partitions: the edge-list kernel reads them unpadded (40,000 nodes of degree 4, 8 x 48:
                 # 131 -> 44 us; 193,000 of degree 17 1289 -> 706; 172,000 of degree 16, 2 x 20 141 -> 81)

@@ -344,16 +344,42 @@ def choose_gather_partitions(n_dst, n_src, nnz, gathered_len, out_len, stats=Non
 EDGES_MISALIGNED = 16
 
 
-def choose_sddmm(n_rows, n_cols, nnz, heads, head_len, stats=None, given_len=None):
+def _choose_sddmm_scattered(stats, feat_len, given_len):
+    """A small graph whose edges are stored in no order: the edge-list kernel gathers both operands and meets no row twice in a row, the
+    tiled traversal scatters its results.  us, edge list / tiled, uniform graphs unless said: 30,000 nodes of degree 8, F=128 33 / 30
+    (power-law 28 / 37), F=512 125 / 74; of degree 40, F=64 66 / 41, F=222 333 / 127; of degree 160, F=16 52 / 71, F=37 194 / 137;
+    140,000 of degree 8, F=37 79 / 93, F=64 79 / 74, F=128 157 / 119, F=256 330 / 213; of degree 40, F=222 1642 / 763."""
+    # (partitions with one tile scatter from short segments: 30,000 nodes of degree 8, power-law, F=256 edge list 52, 2 x 1 63)
+    takes = [(p, t) for p, t in rank_sddmm(stats, feat_len) if (p, t) != (1, 1) and (t > 1 or stats.nnz >= 12 * stats.n_dst)]
+    if not takes:
+        return None
+    coef, tiled = SDDMM_SMALL_COEF, takes[0]
+    best = predict_sddmm(stats, feat_len, *tiled, coef) + 12e-6 + 7e-12 * stats.nnz
+    edges_len = feat_len
+    if given_len is not None and given_len != feat_len:
+        edges_len = given_len + EDGES_MISALIGNED
+        best += _padding_seconds(stats, given_len, feat_len)
+    edges = 1.15 * (predict_sddmm(stats, edges_len, 1, 1, coef) + _gather_seconds(stats, edges_len, 1, 1, coef))
+    return tiled if best < edges else None
+
+
+def _padding_seconds(stats, given_len, feat_len):
+    """Padded copies of both operands."""
+    return 2 * 4e-6 + 8.0 * max(stats.n_dst, stats.n_src) * (given_len + feat_len) / SDDMM_SMALL_COEF['stream']
+
+
+def choose_sddmm(n_rows, n_cols, nnz, heads, head_len, stats=None, given_len=None, scattered=False):
     """(num_src_partitions, num_feat_tiles) for the tiled traversal, or None when the plain
     kernels should be used (small feature matrices, or a shape the tiled kernel does not take).  given_len: the rows' length where
-    head_len is what the tiled traversal would pad them to."""
+    head_len is what the tiled traversal would pad them to.  scattered: the edges are stored in no order of their rows."""
     feat_len = heads * head_len
     if heads == 1:
         if nnz == 0 or feat_len % 4 != 0:
             return None
         if stats is None:
             stats = GraphStats(n_rows, n_cols, nnz)
+        if _is_small(stats) and scattered:
+            return _choose_sddmm_scattered(stats, feat_len, given_len)
         if _is_small(stats):
             ranked = rank_sddmm(stats, feat_len)
             if given_len is not None and given_len != feat_len:
@@ -361,7 +387,7 @@ def choose_sddmm(n_rows, n_cols, nnz, heads, head_len, stats=None, given_len=Non
                 tiled = [c for c in ranked if c != (1, 1)]
                 if not tiled:
                     return None
-                copies = 2 * 4e-6 + 8.0 * max(n_rows, n_cols) * (given_len + feat_len) / SDDMM_SMALL_COEF['stream']
+                copies = _padding_seconds(stats, given_len, feat_len)
                 edges = predict_sddmm(stats, given_len + EDGES_MISALIGNED, 1, 1, SDDMM_SMALL_COEF)
                 return tiled[0] if copies + predict_sddmm(stats, feat_len, *tiled[0], SDDMM_SMALL_COEF) < edges else None
             return None if not ranked or ranked[0] == (1, 1) else ranked[0]

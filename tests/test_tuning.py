@@ -1,0 +1,20 @@
+"""Rules of the default tilings that hold for every graph."""
+from featgraph_amd import tuning
+
+
+def test_scattered_edges_take_the_tiled_walk_sooner():
+    """Edges in no order of their rows: the edge-list kernel gathers both operands, so whatever row-ordered edges are tiled for, scattered ones
+    of more than a few per row are tiled for as well; every choice is one that the kernel takes."""
+    for n in (5000, 30000, 140000):
+        for deg in (16, 40, 160):
+            for F, given in ((64, None), (128, None), (256, 222), (512, None)):
+                if n * deg > 2e7:
+                    continue
+                args = (n, n, n * deg, 1, F, None, given)
+                ordered, scattered = tuning.choose_sddmm(*args), tuning.choose_sddmm(*args, scattered=True)
+                assert scattered is not None or ordered is None or n == 5000
+                if scattered is not None:
+                    tile = F // scattered[1]
+                    assert F % scattered[1] == 0 and 16 <= tile <= 256 and tile & (tile - 1) == 0
+    assert tuning.choose_sddmm(140000, 140000, 5_600_000, 1, 256, None, 222, scattered=True) is not None
+    assert tuning.choose_sddmm(30000, 30000, 240_000, 1, 32, None, None, scattered=True) is None
