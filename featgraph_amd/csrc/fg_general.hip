@@ -70,6 +70,7 @@ struct GenArgs {
     float *partial;              // pieces of split rows: [slot][F] values
     int32_t *partial_arg;        //                       [slot][F] positions
     int F, L;
+    int spread;                  // a row of an item of n rows is shared by the fewest lane groups (a power of two) that are spread / n of all
     // PART: the elements are not addressed by their own positions -- several source-column partitions (indptr /
     // indices are the partitioned layout's position and local column arrays, item_off the plan's item ranges per
     // partition, out / arg the partitions' buffers; strides in elements, per partition), or edge operands that the
@@ -88,14 +89,15 @@ struct GenArgs {
 // The operand features of a lane's V outputs: V consecutive ones (CONTIG: one 128-bit load) or one value V times.
 // NT: a non-temporal load, for an operand on the stored elements, which is read once from end to end and should not
 // displace the gathered operand's rows from the L2.
-typedef float nt_f4 __attribute__((ext_vector_type(4)));
+// (At 4-byte alignment: one 128-bit load all the same.)
+typedef float nt_f4 __attribute__((ext_vector_type(4), aligned(4)));
 template <int V, bool CONTIG, bool NT = false>
 __device__ __forceinline__ void load_operand(const float *p, float (&o)[V]) {
     if (V == 4 && CONTIG && NT) {
         const nt_f4 t = __builtin_nontemporal_load(reinterpret_cast<const nt_f4 *>(p));
         o[0] = t.x; o[1 % V] = t.y; o[2 % V] = t.z; o[3 % V] = t.w;
     } else if (V == 4 && CONTIG) {
-        const float4 t = *reinterpret_cast<const float4 *>(p);
+        const nt_f4 t = *reinterpret_cast<const nt_f4 *>(p);
         o[0] = t.x; o[1 % V] = t.y; o[2 % V] = t.z; o[3 % V] = t.w;
     } else {
         const float s = *p;
@@ -108,6 +110,12 @@ __device__ __forceinline__ void load_operand(const float *p, float (&o)[V]) {
 __device__ __forceinline__ const float *row_at(const char *lane_base, int row, uint32_t row_bytes) {
     return reinterpret_cast<const float *>(lane_base + (uint64_t)(uint32_t)row * row_bytes);
 }
+
+// The first of the V features that vector `i` of a row of F covers.  F need not be a multiple of V: the last vector then starts earlier and
+// shares features with the one before it, and the two lanes form and store the same values.  One feature per
+// lane -> so, us on 20,000 rows of 60 elements, F=65 / 145: copy_u max 90 -> 60 / 142 -> 91, u_mul_e sum 141 -> 118 / 304 -> 212, per edge u_mul_e 149 -> 139
+// / 327 -> 307, with one value per edge 182 -> 88 / 385 -> 210; F=11 28 -> 21, 25 -> 16.
+template <int V> __device__ __forceinline__ int first_feature(int i, int F) { return V == 1 ? i : min(i * V, F - V); }
 
 template <int OP> __device__ __forceinline__ float binary(float l, float r) {
     return OP == FG_BIN_ADD ? l + r : OP == FG_BIN_SUB ? l - r : OP == FG_BIN_MUL ? l * r
@@ -164,7 +172,7 @@ __global__ __launch_bounds__(kBlock) void gspmm_bcast_kernel(const GenArgs a) {
     if (item_id >= a.n_items) return;
     const Item it = a.items[item_id];
     const int L = a.L, G = 64 / L, g = lane / L, li = lane % L;
-    const int F = a.F, FV = F / V;
+    const int F = a.F, FV = (F + V - 1) / V;
     const int fv_lo = tile * a.tile_vecs, fv_hi = min(FV, fv_lo + a.tile_vecs);
     int part = 0;
     if (PART) {
@@ -198,16 +206,16 @@ __global__ __launch_bounds__(kBlock) void gspmm_bcast_kernel(const GenArgs a) {
     // staged_at >= 0: the range lies inside the elements staged from that position on; else it is staged here, kStage
     // elements at a time (a lane group keeps its elements and their order: kStage is a multiple of the groups).
     // own (a std::bool_constant): false = the wavefront's lane groups share the row, taking every G-th element each, and
-    // their results are combined; true = every lane group has a row of its own (e0, e1, v and the destinations differ
-    // from group to group, `mine` says whether the group has a row at all), walks it element by element in stored
-    // order and stores it itself -- for items of many short rows, whose elements are all staged.
-    auto reduce_range = [&](auto own, bool mine, int64_t e0, int64_t e1, int64_t staged_at, int v, float *dst_v, int32_t *dst_a,
+    // their results are combined; true = every `share` (a power of two) neighbouring lane groups have a row of their own (e0,
+    // e1, v and the destinations differ, `mine` says whether they have a row at all), of whose elements each takes every
+    // share-th, and the first of them stores it -- for items of several rows, whose elements are all staged.
+    auto reduce_range = [&](auto own, int share, bool mine, int64_t e0, int64_t e1, int64_t staged_at, int v, float *dst_v, int32_t *dst_a,
                             bool done) {
         constexpr bool OWN = decltype(own)::value;
-        const int first = OWN ? 0 : g, step = OWN ? 1 : G;
+        const int first = OWN ? g & (share - 1) : g, step = OWN ? share : G, lanes = OWN ? L * share : 64;
         for (int f0 = fv_lo; f0 < fv_hi; f0 += L) {
             const bool active = f0 + li < fv_hi;
-            const int fc = (active ? f0 + li : fv_hi - 1) * V;       // the lane's first output feature
+            const int fc = first_feature<V>(active ? f0 + li : fv_hi - 1, F);       // the lane's first output feature
             const int fl = kLhs ? (a.lhs_off ? a.lhs_off[fc] : fc) : 0;
             const int fr = kRhs ? (a.rhs_off ? a.rhs_off[fc] : fc) : 0;
             const char *const lbase = reinterpret_cast<const char *>(kLhs ? a.lhs + fl : nullptr);
@@ -316,21 +324,21 @@ __global__ __launch_bounds__(kBlock) void gspmm_bcast_kernel(const GenArgs a) {
             } else {
                 walk(std::integral_constant<int, kFirst>{});
             }
-            if (ARG && !OWN && !full_rule) {
+            if (ARG && !full_rule) {
                 // no NaN anywhere: the groups' largest value first, then the earliest position that has it
                 float best[V];
 #pragma unroll
                 for (int i = 0; i < V; ++i) best[i] = acc[i];
-                for (int off = L; off < 64; off <<= 1)
+                for (int off = L; off < lanes; off <<= 1)
 #pragma unroll
                     for (int i = 0; i < V; ++i) best[i] = extreme<RED>(best[i], __shfl_xor(best[i], off));
 #pragma unroll
                 for (int i = 0; i < V; ++i) { at[i] = acc[i] == best[i] ? at[i] : INT_MAX; acc[i] = best[i]; }
-                for (int off = L; off < 64; off <<= 1)
+                for (int off = L; off < lanes; off <<= 1)
 #pragma unroll
                     for (int i = 0; i < V; ++i) at[i] = min(at[i], __shfl_xor(at[i], off));
             } else
-            for (int off = L; !OWN && off < 64; off <<= 1) {
+            for (int off = L; off < lanes; off <<= 1) {
 #pragma unroll
                 for (int i = 0; i < V; ++i) {
                     const float o = __shfl_xor(acc[i], off);
@@ -341,7 +349,7 @@ __global__ __launch_bounds__(kBlock) void gspmm_bcast_kernel(const GenArgs a) {
                     } else acc[i] = extreme<RED>(acc[i], o);
                 }
             }
-            if ((OWN ? mine : g == 0) && active) {
+            if (mine && first == 0 && active) {
                 const bool empty = e1 <= e0;
                 const float scale = (done && a.row_scale) ? a.row_scale[v] : 1.f;
 #pragma unroll
@@ -352,8 +360,8 @@ __global__ __launch_bounds__(kBlock) void gspmm_bcast_kernel(const GenArgs a) {
                     if (ARG) at[i] = (at[i] == INT_MAX) ? -1 : at[i];
                 }
                 if (V == 4) {
-                    *reinterpret_cast<float4 *>(dst_v + fc) = make_float4(acc[0], acc[1 % V], acc[2 % V], acc[3 % V]);
-                    if (ARG) *reinterpret_cast<int4 *>(dst_a + fc) = make_int4(at[0], at[1 % V], at[2 % V], at[3 % V]);
+                    *reinterpret_cast<fg::Words4<float> *>(dst_v + fc) = {{acc[0], acc[1 % V], acc[2 % V], acc[3 % V]}};
+                    if (ARG) *reinterpret_cast<fg::Words4<int32_t> *>(dst_a + fc) = {{at[0], at[1 % V], at[2 % V], at[3 % V]}};
                 } else {
                     dst_v[fc] = acc[0];
                     if (ARG) dst_a[fc] = at[0];
@@ -366,13 +374,16 @@ __global__ __launch_bounds__(kBlock) void gspmm_bcast_kernel(const GenArgs a) {
         const int nrows = -it.info;
         const bool fits = it.len <= kStage;       // always, for an item of several rows
         if (fits) stage(it.start, it.len);
-        if (fits && nrows >= 2 * G) {
-            // many short rows: a lane group per row, G rows at a time
-            for (int q0 = 0; q0 < nrows; q0 += G) {
-                const bool mine = q0 + g < nrows;
-                const int v = it.row + min(q0 + g, nrows - 1);
+        // as many rows at a time as there are, if the groups suffice
+        int share = 1;
+        while (share < G && share * nrows < a.spread * G) share *= 2;
+        if (fits && share < G) {
+            for (int q0 = 0; q0 < nrows; q0 += G / share) {
+                const int q = q0 + g / share;
+                const bool mine = q < nrows;
+                const int v = it.row + min(q, nrows - 1);
                 const int64_t e0 = pos_p[v], e1 = mine ? pos_p[v + 1] : e0;
-                reduce_range(std::true_type{}, mine, e0, e1, it.start, v, out_p + (int64_t)v * F,
+                reduce_range(std::true_type{}, share, mine, e0, e1, it.start, v, out_p + (int64_t)v * F,
                              ARG ? arg_p + (int64_t)v * F : nullptr, final);
             }
             return;
@@ -380,12 +391,12 @@ __global__ __launch_bounds__(kBlock) void gspmm_bcast_kernel(const GenArgs a) {
         for (int q = 0; q < nrows; ++q) {
             const int v = it.row + q;
             const int64_t e0 = pos_p[v], e1 = pos_p[v + 1];
-            reduce_range(std::false_type{}, true, e0, e1, fits ? (int64_t)it.start : -1, v, out_p + (int64_t)v * F,
+            reduce_range(std::false_type{}, G, true, e0, e1, fits ? (int64_t)it.start : -1, v, out_p + (int64_t)v * F,
                          ARG ? arg_p + (int64_t)v * F : nullptr, final);
         }
         return;
     }
-    reduce_range(std::false_type{}, true, it.start, (int64_t)it.start + it.len, -1, it.row, partial_p + (int64_t)it.info * F,
+    reduce_range(std::false_type{}, G, true, it.start, (int64_t)it.start + it.len, -1, it.row, partial_p + (int64_t)it.info * F,
                  ARG ? partial_arg_p + (int64_t)it.info * F : nullptr, false);
 }
 
@@ -511,11 +522,13 @@ void launch_spmm(int op, int reduce, bool with_arg, int vec, bool lnt, bool rnt,
 
 // How one operand can be read when a lane holds 4 consecutive output features: 1 = 4 consecutive features by one
 // 128-bit load, 2 = one feature 4 times, 0 = neither (scalar kernel).  Without an offset array the operand has the
-// output's layout; with one, the caller's flags say which pattern every aligned group of 4 follows.
-int vector_mode(bool used, const float *p, int len, const int32_t *off, int flags, int vec_flag, int splat_flag) {
-    if (!used) return 1;
-    if (!off || (flags & vec_flag)) return (len % 4 == 0 && ((uintptr_t)p & 15) == 0) ? 1 : 0;
-    return (flags & splat_flag) ? 2 : 0;
+// output's layout, and an operand of one feature repeats it; with one, the caller's flags say which pattern every aligned group of 4
+// follows, which holds for every lane's group where F is a multiple of 4.
+int vector_mode(bool used, int len, const int32_t *off, int F, int flags, int vec_flag, int splat_flag) {
+    if (!used || !off) return 1;
+    if (len == 1) return 2;
+    if (F % 4 != 0) return 0;
+    return (flags & vec_flag) ? 1 : (flags & splat_flag) ? 2 : 0;
 }
 // The launchers' `vec` from the two operands' modes (0: scalar kernel).
 int vector_variant(bool can_vec, int lmode, int rmode) {
@@ -676,7 +689,7 @@ __global__ __launch_bounds__(kBlock) void gsddmm_bcast_kernel(const EdgeArgs a) 
     const int lane = threadIdx.x & 63;
     const int64_t wave_id = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int L = a.L, G = 64 / L;
-    const int FV = a.F / V;
+    const int FV = (a.F + V - 1) / V;
     const int64_t e0 = wave_id * 64;
     if (e0 >= a.n_edges) return;
     const int n = (int)min((int64_t)64, a.n_edges - e0);
@@ -722,7 +735,7 @@ __global__ __launch_bounds__(kBlock) void gsddmm_bcast_kernel(const EdgeArgs a) 
                 ok[k] = p0 + 64 * k < total;
                 const uint32_t p = ok[k] ? p0 + 64 * k : total - 1;
                 t[k] = FV == 1 ? (int)p : (int)__umulhi(p, a.vec_magic);
-                fc[k] = fl[k] = fr[k] = ((int)p - t[k] * FV) * V;
+                fc[k] = fl[k] = fr[k] = first_feature<V>((int)p - t[k] * FV, a.F);
             }
             step(t, ok, fc, fl, fr);
         }
@@ -730,7 +743,7 @@ __global__ __launch_bounds__(kBlock) void gsddmm_bcast_kernel(const EdgeArgs a) 
         const int g = lane / L, li = lane % L;
         for (int f0 = 0; f0 < FV; f0 += L) {
             const bool in_row = f0 + li < FV;
-            const int f = (in_row ? f0 + li : FV - 1) * V;
+            const int f = first_feature<V>(in_row ? f0 + li : FV - 1, a.F);
             const int l = kUsesLhs<OP> ? (a.lhs_off ? a.lhs_off[f] : f) : 0;
             const int r = kUsesRhs<OP> ? (a.rhs_off ? a.rhs_off[f] : f) : 0;
             for (int tb = 0; tb < n; tb += G * U) {
@@ -794,7 +807,7 @@ __global__ __launch_bounds__(kBlock) void gsddmm_dot_kernel(const EdgeArgs a) {
 
 template <int OP>
 void launch_sddmm(int vec, dim3 grid, hipStream_t st, EdgeArgs a) {
-    const int FV = vec ? a.F / 4 : a.F;
+    const int FV = vec ? (a.F + 3) / 4 : a.F;
     a.vec_magic = FV > 1 ? (uint32_t)((0x100000000ull + FV - 1) / FV) : 0;
     const bool flat = !(kUsesLhs<OP> && a.lhs_off) && !(kUsesRhs<OP> && a.rhs_off) && FV < 8192;
     // a wavefront's 64 edges fill eight steps; 3 M edges, u_add_v with eight / four: F=4 35 / 25 us, F=8 38 / 29, F=16 49 / 43
@@ -853,9 +866,13 @@ int gspmm_bcast_run(fg_spmm_plan *pl, const int32_t *pos_dev, const int32_t *idx
     if (int rc = fg::ensure_scratch(pl, need, stream)) return rc;
     hipStream_t st = (hipStream_t)stream;
     const BcastScratch b = bcast_scratch(pl, out_len, arg_dev != nullptr);
-    const int lmode = vector_mode(uses_l, lhs_dev, lhs_len, lhs_off_dev, flags, FG_BCAST_LHS_VEC4, FG_BCAST_LHS_SPLAT4);
-    const int rmode = vector_mode(uses_r, rhs_dev, rhs_len, rhs_off_dev, flags, FG_BCAST_RHS_VEC4, FG_BCAST_RHS_SPLAT4);
-    const int vec = vector_variant(out_len % 4 == 0 && (((uintptr_t)out_dev | (uintptr_t)arg_dev) & 15) == 0, lmode, rmode);
+    const int lmode = vector_mode(uses_l, lhs_len, lhs_off_dev, out_len, flags, FG_BCAST_LHS_VEC4, FG_BCAST_LHS_SPLAT4);
+    const int rmode = vector_mode(uses_r, rhs_len, rhs_off_dev, out_len, flags, FG_BCAST_RHS_VEC4, FG_BCAST_RHS_SPLAT4);
+    const bool streams = (uses_l && lhs_target == FG_TARGET_E && lmode == 1) || (uses_r && rhs_target == FG_TARGET_E && rmode == 1);
+    // An operand streamed from the edges in short rows of an odd length: one feature per lane, whose loads walk consecutive words (u_mul_e
+    // sum, one / 4 features per lane, 20,000 rows of 200 elements F=9 / 13 / 17 52 / 67, 57 / 81, 99 / 98 us; 100,000 of 8 30 / 33, 31 / 37, 47 / 47).
+    const bool short_odd = streams && out_len % 4 != 0 && out_len <= 16;
+    const int vec = vector_variant(out_len >= 4 && !short_odd, lmode, rmode);
     const int V = vec ? 4 : 1;
     float *const values = pl->partial_dev;                                          // [P][pieces] then [P][buffers]
     int32_t *const positions = reinterpret_cast<int32_t *>(pl->partial_dev + b.half);
@@ -881,11 +898,16 @@ int gspmm_bcast_run(fg_spmm_plan *pl, const int32_t *pos_dev, const int32_t *idx
     // degree 15 4287 -> 4385 / 8284 -> 8528 / 16374 -> 16879; F=192 / 320 at degree 200 313 -> 338 / 605 -> 614.  Below 2^15 edges
     // launches are all there is, and either is the other's time.  u_add_e max, which instructions bound, 12.5M edges on 58,000 nodes 669 -> 683 / 1132 -> 1270 / 2573 -> 2403, 8M on 200,000 509 -> 549 / 1101 -> 1030 / 2320 -> 2198.)
     const bool gathers = (uses_l && lhs_target == FG_TARGET_U) || (uses_r && rhs_target == FG_TARGET_U);
-    const bool streams = (uses_l && lhs_target == FG_TARGET_E && lmode == 1) || (uses_r && rhs_target == FG_TARGET_E && rmode == 1);
     int T = (V == 4 && gathers && !streams && out_len >= 128 && out_len % 64 == 0) ? out_len / 64 : 1;
     if (arg_dev && !(op == FG_BIN_COPY_LHS && (T & (T - 1)) == 0 && pl->nnz >= 32 * pl->n_dst) && pl->nnz >= (1 << 15)) T = 1;
     a.n_tiles = T; a.tile_vecs = T > 1 ? 16 : (out_len + V - 1) / V;
-    a.F = out_len; a.L = lanes_for(T > 1 ? 16 : out_len / V);
+    a.F = out_len; a.L = lanes_for(T > 1 ? 16 : (out_len + V - 1) / V);
+    // Lane groups that hold several rows at once: see GenArgs.  Spread over as many groups as there are, rows take the fewest
+    // steps; kept closer together, uneven rows leave fewer groups idle and streamed operands are read in longer runs.  1 / 2 / 4, us: copy_u max on 100,000 rows
+    // of 40, F=4 44 / 58 / -, F=16 62 / 67 / -, F=32 87 / 82 / -; of 8, F=16 31 / 24 / -; u_mul_e sum with F edge features on rows of 8, F=8 34 / 28 / 30,
+    // F=32 61 / 57 / 47, F=64 - / 79 / 76, of 16, F=16 64 / 52 / 55, F=32 89 / 79 / 72.  With a row either in one group or in all of them F=4 115, F=16 112 and 74,
+    // F=32 115; u_mul_e F=8 98, F=16 91, F=32 56 and 79.
+    a.spread = streams ? (out_len > 16 ? 4 : 2) : (out_len <= 8 ? 1 : 2);
     a.item_off = pl->item_off_dev; a.edge_pos = edge_pos_dev; a.n_parts = P; a.final = P == 1;
     a.ordered = !edge_pos_dev || (flags & FG_BCAST_EDGES_ASCEND) != 0;
     a.pos_stride = pl->n_dst + 1; a.col_width = (pl->n_src + P - 1) / P;
@@ -1023,9 +1045,9 @@ extern "C" int fg_gsddmm_bcast_f32(const int32_t *row_dev, const int32_t *col_de
     const bool any_u = (uses_l && lhs_target == FG_TARGET_U) || (uses_r && rhs_target == FG_TARGET_U);
     const bool any_v = (uses_l && lhs_target == FG_TARGET_V) || (uses_r && rhs_target == FG_TARGET_V);
     if (!out_dev || (any_u && !col_dev) || (any_v && !row_dev)) return fail(FG_ERR_ARG, "null device pointer");
-    const int lmode = vector_mode(uses_l, lhs_dev, lhs_len, lhs_off_dev, flags, FG_BCAST_LHS_VEC4, FG_BCAST_LHS_SPLAT4);
-    const int rmode = vector_mode(uses_r, rhs_dev, rhs_len, rhs_off_dev, flags, FG_BCAST_RHS_VEC4, FG_BCAST_RHS_SPLAT4);
-    const int vec = vector_variant(op != FG_BIN_DOT && out_len % 4 == 0 && ((uintptr_t)out_dev & 15) == 0, lmode, rmode);
+    const int lmode = vector_mode(uses_l, lhs_len, lhs_off_dev, out_len, flags, FG_BCAST_LHS_VEC4, FG_BCAST_LHS_SPLAT4);
+    const int rmode = vector_mode(uses_r, rhs_len, rhs_off_dev, out_len, flags, FG_BCAST_RHS_VEC4, FG_BCAST_RHS_SPLAT4);
+    const int vec = vector_variant(op != FG_BIN_DOT && out_len >= 4, lmode, rmode);
     const int V = vec ? 4 : 1;
     // every lane reads its operands' row indices without a branch: an operand on the edges reads (and discards) an
     // index array that exists, or the start of out when the call has none
@@ -1036,7 +1058,7 @@ extern "C" int fg_gsddmm_bcast_f32(const int32_t *row_dev, const int32_t *col_de
     a.n_edges = n_edges;
     a.lhs = lhs_dev; a.rhs = rhs_dev; a.lhs_off = lhs_off_dev; a.rhs_off = rhs_off_dev;
     a.lhs_len = lhs_len; a.rhs_len = rhs_len; a.lhs_target = lhs_target; a.rhs_target = rhs_target;
-    a.out = out_dev; a.F = out_len; a.L = lanes_for(out_len / V); a.R = R;
+    a.out = out_dev; a.F = out_len; a.L = lanes_for((out_len + V - 1) / V); a.R = R;
     const int64_t waves = (n_edges + 63) / 64;
     const int64_t blocks = (waves + kWavesPerBlock - 1) / kWavesPerBlock;
     if (blocks > 0x7fffffffLL) return fail(FG_ERR_SHAPE, "grid of %lld workgroups is too large", (long long)blocks);
