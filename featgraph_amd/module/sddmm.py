@@ -258,7 +258,7 @@ class SDDMMbase(object):
         tiled = None
         nnz = self._adj_row_indices.shape[0]
         if order in ('auto', 'tiled') and nnz > 0:
-            tiled = tuning.choose_sddmm(self._num_rows, self._num_cols, nnz, H, D, self._graph_stats() if H == 1 else None,
+            tiled = tuning.choose_sddmm(self._num_rows, self._num_cols, nnz, H, D, self._graph_stats() if H == 1 else self._degree_stats(),
                                         given_len=getattr(self, '_pad_from', None), scattered=not self._row_sorted)
             if H > 1 and getattr(self, '_pad_from', None) is not None and tiled is not None and tiled[0] == 1:
                 # padded heads without source partitions: the edge-list kernel reads them unpadded (40,000 nodes of degree 4, 8 x 48:
@@ -284,6 +284,15 @@ class SDDMMbase(object):
             dv, dm = np.unique(degs, return_counts=True)
             self._stats = tuning.GraphStats(self._num_rows, self._num_cols, len(self._adj_col_indices), cv, cm, dv, dm)
         return self._stats
+
+    def _degree_stats(self):
+        """The same from the row degrees alone, which stand for the columns' too (None: the edges are in no order)."""
+        if not self._row_sorted:
+            return None
+        if getattr(self, '_deg_stats', None) is None:
+            vals, mult = np.unique(np.diff(self._adj_indptr), return_counts=True)
+            self._deg_stats = tuning.GraphStats(self._num_rows, self._num_cols, len(self._adj_col_indices), vals, mult, vals, mult)
+        return self._deg_stats
 
     def _tune(self, phs, compute_args, schedule_args, how_many):
         """Times the stored-order kernel(s) and the cost model's `how_many` most promising tiled traversals on

@@ -401,7 +401,13 @@ def choose_sddmm(n_rows, n_cols, nnz, heads, head_len, stats=None, given_len=Non
             # 1 x 1; 2.45M-node graph at F = 512: 1 x 2 tiles 22.5 ms, stored order 20.1 ms; uniform 1M-node graph: 23.3 / 22.7 ms).
             return None
         return ranked[0]
-    return _choose_sddmm_heads(n_rows, n_cols, nnz, heads, head_len)
+    first = _choose_sddmm_heads(n_rows, n_cols, nnz, heads, head_len)
+    if stats is None:
+        stats = GraphStats(n_rows, n_cols, nnz)
+    # (heads that would be padded: the edge list reads them as they are, and the rule below rarely asks for more)
+    if nnz > 0 and _is_small(stats) and given_len is None and 8 <= head_len <= 64 and _is_pow2(head_len):
+        return _choose_sddmm_heads_small(stats, heads, head_len, first)
+    return first
 
 
 def _is_pow2(v):
@@ -419,6 +425,35 @@ def _partitions(n_src, row_bytes, nnz, n_rows, slice_bytes, min_segment):
     while p > 1 and avg_deg / p < min_segment:
         p //= 2
     return max(1, min(64, p))
+
+
+# Several heads on a small graph: seconds of the edge list (factor on the model's time of it, launch) and of the tiled walk (the same, per byte of results that
+# are staged, per byte of those that are scattered, a last kernel, per row segment and tile).  Fitted to 336 graphs and shapes (6,000 to
+# 150,000 nodes, degrees 6 to 90, uniform and power-law, 2 to 16 heads of 8 to 64 floats): 4 % behind the best of edge list and 1 to 8 partitions on average, where
+# the rule for large graphs below is 12 %.  us, that rule's choice / this: 40,000 nodes of degree 90, 8 x 32 493 / 325, 4 x 32 217 / 116, 2 x 64 213 / 111; of degree
+# 25, 16 x 32 316 / 196; 150,000 of degree 6, 3 x 16 89 / 38, 8 x 64 461 / 303.
+_HEADS_SMALL = dict(edges=1.527, edges_launch=1.2e-6, tiled=1.718, staged=0.177e-12, scattered=0.145e-12, launch=3.6e-6, last=4.3e-6, segment=0.023e-10)
+
+
+def _choose_sddmm_heads_small(stats, heads, head_len, first):
+    """The choice of this model, or `first` where that is a candidate and the model sees less than 5 % more time for it."""
+    feat_len, out_bytes, c = heads * head_len, 4.0 * stats.nnz * heads, _HEADS_SMALL
+
+    def tiled(p, t):
+        tile = feat_len // t
+        per_tile, segments = tile // head_len, stats.segments(p)
+        s = c['tiled'] * (_gather_seconds(stats, feat_len, p, t, SDDMM_SMALL_COEF) + segments * 4.0 * feat_len / SDDMM_SMALL_COEF['stream'])
+        s += c['launch'] + segments * t * c['segment']
+        if per_tile == 1 and heads >= 4 and t > 1:
+            return s + out_bytes * c['staged'] + c['last']
+        return s + out_bytes * c['scattered'] * max(1.0, 8.0 / per_tile)
+
+    edges = c['edges'] * predict_sddmm(stats, feat_len, 1, 1, SDDMM_SMALL_COEF) + c['edges_launch']
+    cands = [(p, feat_len // w) for w in (32, 64, 128, 256) if feat_len % w == 0 and w % head_len == 0 for p in (1, 2, 4, 8) if p <= max(1, stats.n_src)]
+    costs = {c: tiled(*c) for c in cands}
+    costs[None] = edges
+    best = min(costs, key=costs.get)
+    return first if first in costs and costs[best] > 0.95 * costs[first] else best
 
 
 def _choose_sddmm_heads(n_rows, n_cols, nnz, heads, head_len):
@@ -509,7 +544,7 @@ def sum_gradients_in_one_sweep(num_rows, num_cols, nnz, heads, head_len):
     feat_len = heads * head_len
     if heads == 1:
         return nnz < 1 << 20 or head_len > 16 and (head_len != 32 or nnz >= 24 * num_rows)
-    if head_len >= 64 or not _is_pow2(feat_len) and choose_sddmm(num_rows, num_cols, nnz, heads, head_len) is None:
+    if head_len >= 64 or not _is_pow2(feat_len) and _choose_sddmm_heads(num_rows, num_cols, nnz, heads, head_len) is None:
         return True
     if head_len == 16:
         if heads % 4:

@@ -18,3 +18,16 @@ def test_scattered_edges_take_the_tiled_walk_sooner():
                     assert F % scattered[1] == 0 and 16 <= tile <= 256 and tile & (tile - 1) == 0
     assert tuning.choose_sddmm(140000, 140000, 5_600_000, 1, 256, None, 222, scattered=True) is not None
     assert tuning.choose_sddmm(30000, 30000, 240_000, 1, 32, None, None, scattered=True) is None
+
+
+def test_heads_on_small_graphs_get_tiles_that_the_kernel_takes():
+    for n, deg in ((6000, 6), (6000, 90), (40000, 25), (150000, 90)):
+        for heads in (2, 3, 4, 6, 8, 12, 16):
+            for head_len in (8, 16, 32, 64):
+                got = tuning.choose_sddmm(n, n, n * deg, heads, head_len)
+                if got is not None:
+                    tile = heads * head_len // got[1]
+                    assert heads * head_len % got[1] == 0 and 16 <= tile <= 256 and tile & (tile - 1) == 0
+                    assert tile % head_len == 0 or head_len % tile == 0 and heads == 1
+    assert tuning.choose_sddmm(150000, 150000, 900_000, 8, 64) is None          # degree 6: the edge list
+    assert tuning.choose_sddmm(40000, 40000, 3_600_000, 4, 32) is not None
