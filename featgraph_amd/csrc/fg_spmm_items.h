@@ -459,6 +459,78 @@ __device__ __forceinline__ void spmm_items_body(const SpmmArgs &a) {
 #pragma unroll
             for (int i = 0; i < kOwnTouch; ++i) asm volatile("" ::"v"(own_touched[i]));
         }
+        // Rows in the middle: many at a time, `share` neighbouring groups (a power of two) to a row, the fewest that are spread / nrows of
+        // all.  Wide apart (a small spread) rows take fewer steps, together uneven rows leave fewer groups idle.  us with every such row on all
+        // groups, or from 2 * G rows on one group each / spread 2 / 4: 120,000 rows of 8, F=16 31 / 16 / 16, power-law 30 / 20 / 16, F=32 22 / 22 / 22, 32 / 32 /
+        // 23; of 16, F=8 34 / 21 / 23, F=16 36 / 26 / 26; of 60, power-law, F=8 56 / 63 / 57, F=128 300 / 311 / 293; 20,000 of 8, F=16 11 / 8 / 10, of 60, power-law, F=64
+        // 29 / 29 / 27.
+        const int spread = L <= 4 && it.len <= 48 * nrows ? 2 : 4;
+        int share = 1;
+        while (share < G && share * nrows < spread * G) share *= 2;
+        if (share > 1 && share < G) {
+            const int sub = g & (share - 1);
+            for (int q0 = 0; q0 < nrows; q0 += G / share) {
+                const int q = q0 + g / share;
+                const bool mine = q < nrows;
+                const int b = mine && q ? s_end[wave][q - 1] : 0, e = mine ? s_end[wave][q] : 0;
+#pragma unroll
+                for (int k = 0; k < K; ++k) acc[k] = vzero(vec());
+                load_own(it.row + min(q, nrows - 1));
+                if (ACC && e > b) {
+                    const float *src = out_p + (int64_t)(it.row + q) * F + f_lo;
+#pragma unroll
+                    for (int k = 0; k < K; ++k)
+                        if (FULL || on[k]) old[k] = *reinterpret_cast<const vec *>(src + k * L * V);
+                }
+                for (int j = b + sub; j < e; j += share * U) {
+                    int2 cw[U];
+                    vec xv[U][K];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const int t = j + u * share, at = t < e ? t : j;      // beyond the row: its element once more, replaced by zeros
+                        cw[u] = edge[at];
+                        if (HPT > 1) cw[u].y = __float_as_int(wrow[at]);
+                        if (t >= e) cw[u].y = 0;
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+#pragma unroll
+                        for (int k = 0; k < K; ++k)
+                            if (FULL || on[k])
+                                xv[u][k] = *reinterpret_cast<const vec *>(row_ptr<OFF32>(x_p, lane_bytes, F, cw[u].x) + k * L * V);
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+#pragma unroll
+                        for (int k = 0; k < K; ++k)
+                            if (FULL || on[k]) {
+                                const int t = j + u * share;
+                                if (u > 0) xv[u][k] = vkeep(t < e, xv[u][k]);
+                                vfma(acc[k], __int_as_float(cw[u].y), xv[u][k]);
+                                const int at = t < e ? t : j;
+                                dots.put(lane, xv[u][k], t < e, HPT > 1 ? reinterpret_cast<int32_t *>(wrow + at) : &edge[at].y);
+                            }
+                }
+                for (int off = L; off < L * share; off <<= 1)
+#pragma unroll
+                    for (int k = 0; k < K; ++k) vadd(acc[k], vshfl_xor(acc[k], off));
+                if (mine && sub == 0 && (!ACC || e > b)) {
+                    if constexpr (SHORT) {
+                        store_short<V, L, K, FULL>(a, acc, on, out_p + (int64_t)(it.row + q) * a.out_ld, f_lo);
+                    } else {
+                        float *dst = out_p + (int64_t)(it.row + q) * F + f_lo;
+#pragma unroll
+                        for (int k = 0; k < K; ++k)
+                            if (FULL || on[k]) {
+                                vec r = acc[k];
+                                if (ACC) vadd(r, old[k]);
+                                *reinterpret_cast<vec *>(dst + k * L * V) = r;
+                            }
+                    }
+                }
+            }
+            flush_dots(it.start, it.len);
+            return;
+        }
         if (nrows < 2 * G) {
             // Few, longer rows: all lane groups share each row in turn.
             int b = 0;
