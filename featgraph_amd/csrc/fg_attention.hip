@@ -179,17 +179,21 @@ __device__ __forceinline__ Running load_state(const float *out_row, const float 
     return old;
 }
 
-// Merges the lane groups' running sums (every group ends with the row's), then, in later passes, the
-// row's state from the earlier partitions, and stores the row.
-template <int L, bool FIRST>
-__device__ __forceinline__ void finish_row(Running r, const Running &old, int g, int li, float *out_row, float *state_row) {
-#pragma unroll
-    for (int off = L; off < 64; off <<= 1) {
+// Merges the running sums of lanes `from`, 2 * from, .. below `to` apart (powers of two).
+__device__ __forceinline__ void merge_groups(Running &r, int from, int to) {
+    for (int off = from; off < to; off <<= 1) {
         Running o;
         o.m = __shfl_xor(r.m, off); o.l = __shfl_xor(r.l, off);
         o.acc = make_float4(__shfl_xor(r.acc.x, off), __shfl_xor(r.acc.y, off), __shfl_xor(r.acc.z, off), __shfl_xor(r.acc.w, off));
         running_merge(r, o);
     }
+}
+
+// Merges the lane groups' running sums (every group ends with the row's), then, in later passes, the
+// row's state from the earlier partitions, and stores the row.
+template <int L, bool FIRST>
+__device__ __forceinline__ void finish_row(Running r, const Running &old, int g, int li, float *out_row, float *state_row) {
+    merge_groups(r, L, 64);
     if (g != 0) return;
     if (!FIRST) running_merge(r, old);
     if constexpr (FIRST) {
@@ -306,6 +310,40 @@ __global__ __launch_bounds__(kBlock) void attention_items_kernel(const AttnArgs 
                 if (!done && j < e) {
                     own_batch<L>(cols, j, e, k_p, v_p, lane_bytes, q, a.scale, run);
                     j += kU;
+                }
+            }
+            return;
+        }
+        const int share = fg::groups_per_row<L>(nrows, it.len);
+        if (share < G) {
+            // Rows in the middle: many at a time, `share` neighbouring lane groups to a row, so that fewer parts are merged (each level of
+            // it takes two exponentials and six exchanges).  Whole steps with the same in the gradients, every such row on all groups -> so, us:
+            // 100,000 nodes of degree 8, 1 x 16 164 -> 105, 1 x 32 173 -> 141, 4 x 16 421 -> 378, 2 x 64 453 -> 437; of 16, power-law, 1 x 16 199 -> 149,
+            // 4 x 16 571 -> 525; 60,000 of 60, power-law, 1 x 16 260 -> 211, 8 x 32 1953 -> 1964.
+            const int sub = g & (share - 1);
+            for (int r0 = 0; r0 < nrows; r0 += G / share) {
+                const int r = r0 + g / share;
+                const bool mine = r < nrows;
+                const int64_t row = it.row + min(r, nrows - 1);
+                const int b = mine && r ? s_end[wave][r - 1] : 0, e = mine ? s_end[wave][r] : 0;
+                const float4 q = own_q(row);
+                const Running old = load_state<FIRST>(out_row(row), state_row(row));
+                Running run = running_empty();
+                for (int j = b + sub; j < e; j += share * kU) {
+                    int32_t c[kU];
+                    bool valid[kU];
+#pragma unroll
+                    for (int u = 0; u < kU; ++u) {
+                        valid[u] = j + u * share < e;
+                        c[u] = cols[valid[u] ? j + u * share : j];
+                    }
+                    update<L, kU>(c, valid, k_p, v_p, lane_bytes, q, a.scale, run);
+                }
+                merge_groups(run, L, L * share);
+                if (mine && sub == 0 && (FIRST || e > b)) {
+                    if (!FIRST) running_merge(run, old);
+                    *reinterpret_cast<float4 *>(out_row(row)) = run.acc;
+                    if (li == 0) { float *st = state_row(row); st[0] = run.m; st[1] = run.l; }
                 }
             }
             return;

@@ -291,6 +291,38 @@ __global__ __launch_bounds__(kBlock) void attention_backward_kernel(const BwdArg
             flush(it.start, it.len);
             return;
         }
+        const int share = fg::groups_per_row<L>(nrows, it.len);
+        if (share < G) {
+            // Rows in the middle: many at a time, `share` neighbouring lane groups to a row.
+            const int sub = g & (share - 1);
+            for (int r0 = 0; r0 < nrows; r0 += G / share) {
+                const int r = r0 + g / share;
+                const bool mine = r < nrows;
+                const int64_t row = it.row + min(r, nrows - 1);
+                const int b = mine && r ? s_end[wave][r - 1] : 0, e = mine ? s_end[wave][r] : 0;
+                row_inputs(row, o0, o1, c1, delta, oldA, oldB);
+                float4 accA = zero4(), accB = zero4();
+                for (int j = b + sub; j < e; j += share * KU) {
+                    W w[KU];
+                    int at[KU];
+                    bool ok[KU];
+#pragma unroll
+                    for (int u = 0; u < KU; ++u) {
+                        ok[u] = j + u * share < e;
+                        at[u] = ok[u] ? j + u * share : j;
+                        w[u] = far[at[u]];
+                    }
+                    apply(std::integral_constant<int, KU>(), w, at, ok, o0, o1, c1, delta, accA, accB);
+                }
+                for (int off = L; off < L * share; off <<= 1) {
+                    shfl_add(accA, off);
+                    if (BY_COLUMN) shfl_add(accB, off);
+                }
+                if (mine && sub == 0 && (!ACC || e > b)) store(row, accA, accB, oldA, oldB);
+            }
+            flush(it.start, it.len);
+            return;
+        }
         int b = 0;
         for (int r = 0; r < nrows; ++r) {
             const int e = __builtin_amdgcn_readfirstlane(s_end[wave][r]);

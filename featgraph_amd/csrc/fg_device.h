@@ -139,4 +139,15 @@ __device__ __forceinline__ void each_piece(int first, int n, Load load, Use use)
     }
 }
 
+// How many neighbouring lane groups (of L lanes) share a row of an item of `nrows` rows and `len` elements that are walked many at a
+// time: the fewest, a power of two, that are spread / nrows of all 64 / L groups.  Wide apart (a small spread) rows take fewer steps,
+// together uneven rows leave fewer groups idle.
+template <int L>
+__device__ __forceinline__ int groups_per_row(int nrows, int len) {
+    constexpr int G = 64 / L;
+    const int spread = L <= 4 && len <= 48 * nrows ? 2 : 4;
+    int share = 1;
+    while (share < G && share * nrows < spread * G) share *= 2;
+    return share;
+}
 }  // namespace fg

@@ -459,14 +459,10 @@ __device__ __forceinline__ void spmm_items_body(const SpmmArgs &a) {
 #pragma unroll
             for (int i = 0; i < kOwnTouch; ++i) asm volatile("" ::"v"(own_touched[i]));
         }
-        // Rows in the middle: many at a time, `share` neighbouring groups (a power of two) to a row, the fewest that are spread / nrows of
-        // all.  Wide apart (a small spread) rows take fewer steps, together uneven rows leave fewer groups idle.  us with every such row on all
-        // groups, or from 2 * G rows on one group each / spread 2 / 4: 120,000 rows of 8, F=16 31 / 16 / 16, power-law 30 / 20 / 16, F=32 22 / 22 / 22, 32 / 32 /
-        // 23; of 16, F=8 34 / 21 / 23, F=16 36 / 26 / 26; of 60, power-law, F=8 56 / 63 / 57, F=128 300 / 311 / 293; 20,000 of 8, F=16 11 / 8 / 10, of 60, power-law, F=64
-        // 29 / 29 / 27.
-        const int spread = L <= 4 && it.len <= 48 * nrows ? 2 : 4;
-        int share = 1;
-        while (share < G && share * nrows < spread * G) share *= 2;
+        // Rows in the middle: many at a time, `share` neighbouring groups to a row.  us with every such row on all groups, or from 2 * G rows on one
+        // group each / as here: 120,000 rows of 8, F=16 31 / 16, power-law 30 / 19, F=32 22 / 22, 32 / 22; of 16, F=8 34 / 21, F=16 36 / 26; of 60, power-law, F=8 56 /
+        // 60, F=128 300 / 293; 20,000 of 8, F=16 11 / 8, of 60, power-law, F=64 29 / 27.
+        const int share = fg::groups_per_row<L>(nrows, it.len);
         if (share > 1 && share < G) {
             const int sub = g & (share - 1);
             for (int q0 = 0; q0 < nrows; q0 += G / share) {
