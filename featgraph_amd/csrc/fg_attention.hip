@@ -314,11 +314,11 @@ __global__ __launch_bounds__(kBlock) void attention_items_kernel(const AttnArgs 
             }
             return;
         }
-        const int share = fg::groups_per_row<L>(nrows, it.len);
+        const int share = L <= 8 ? fg::groups_per_row<L>(nrows, it.len) : G;      // (heads of 64 floats: nothing gained, and 5 to 15 registers more)
         if (share < G) {
             // Rows in the middle: many at a time, `share` neighbouring lane groups to a row, so that fewer parts are merged (each level of
             // it takes two exponentials and six exchanges).  Whole steps with the same in the gradients, every such row on all groups -> so, us:
-            // 100,000 nodes of degree 8, 1 x 16 164 -> 105, 1 x 32 173 -> 141, 4 x 16 421 -> 378, 2 x 64 453 -> 437; of 16, power-law, 1 x 16 199 -> 149,
+            // 100,000 nodes of degree 8, 1 x 16 164 -> 105, 1 x 32 173 -> 141, 4 x 16 421 -> 378; of 16, power-law, 1 x 16 199 -> 149,
             // 4 x 16 571 -> 525; 60,000 of 60, power-law, 1 x 16 260 -> 211, 8 x 32 1953 -> 1964.
             const int sub = g & (share - 1);
             for (int r0 = 0; r0 < nrows; r0 += G / share) {

@@ -291,7 +291,7 @@ __global__ __launch_bounds__(kBlock) void attention_backward_kernel(const BwdArg
             flush(it.start, it.len);
             return;
         }
-        const int share = fg::groups_per_row<L>(nrows, it.len);
+        const int share = L <= 8 ? fg::groups_per_row<L>(nrows, it.len) : G;      // (heads of 64 floats: nothing gained, and 5 to 15 registers more)
         if (share < G) {
             // Rows in the middle: many at a time, `share` neighbouring lane groups to a row.
             const int sub = g & (share - 1);
