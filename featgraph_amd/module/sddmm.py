@@ -260,10 +260,6 @@ class SDDMMbase(object):
         if order in ('auto', 'tiled') and nnz > 0:
             tiled = tuning.choose_sddmm(self._num_rows, self._num_cols, nnz, H, D, self._graph_stats() if H == 1 else self._degree_stats(),
                                         given_len=getattr(self, '_pad_from', None), scattered=not self._row_sorted)
-            if H > 1 and getattr(self, '_pad_from', None) is not None and tiled is not None and tiled[0] == 1:
-                # padded heads without source partitions: the edge-list kernel reads them unpadded (40,000 nodes of degree 4, 8 x 48:
-                # 131 -> 44 us; 193,000 of degree 17 1289 -> 706; 172,000 of degree 16, 2 x 20 141 -> 81)
-                tiled = None
             p_arg, t_arg = schedule_args.get('num_src_partitions'), schedule_args.get('num_feat_tiles')
             if t_arg is None and knob_tiles is not None and order != 'coo' and order != 'csr':
                 t_arg = knob_tiles

@@ -403,12 +403,16 @@ def choose_sddmm(n_rows, n_cols, nnz, heads, head_len, stats=None, given_len=Non
             # 1 x 1; 2.45M-node graph at F = 512: 1 x 2 tiles 22.5 ms, stored order 20.1 ms; uniform 1M-node graph: 23.3 / 22.7 ms).
             return None
         return ranked[0]
-    first = _choose_sddmm_heads(n_rows, n_cols, nnz, heads, head_len)
+    first = _choose_sddmm_heads(n_rows, n_cols, nnz, heads, head_len, scattered)
     if stats is None:
         stats = GraphStats(n_rows, n_cols, nnz)
-    # (heads that would be padded: the edge list reads them as they are, and the rule below rarely asks for more)
-    if nnz > 0 and _is_small(stats) and given_len is None and 8 <= head_len <= 64 and _is_pow2(head_len):
-        return _choose_sddmm_heads_small(stats, heads, head_len, first)
+    padded = given_len is not None and given_len != head_len
+    if nnz > 0 and _is_small(stats) and (scattered or not padded) and 8 <= head_len <= 64 and _is_pow2(head_len):
+        return _choose_sddmm_heads_small(stats, heads, head_len, first, given_len if padded else None, scattered)
+    if padded and not scattered and first is not None and first[0] == 1:
+        # padded heads without source partitions: the edge-list kernel reads them unpadded (40,000 nodes of degree 4, 8 x 48:
+        # 131 -> 44 us; 193,000 of degree 17 1289 -> 706; 172,000 of degree 16, 2 x 20 141 -> 81)
+        return None
     return first
 
 
@@ -437,28 +441,48 @@ def _partitions(n_src, row_bytes, nnz, n_rows, slice_bytes, min_segment):
 _HEADS_SMALL = dict(edges=1.527, edges_launch=1.2e-6, tiled=1.718, staged=0.177e-12, scattered=0.145e-12, launch=3.6e-6, last=4.3e-6, segment=0.023e-10)
 
 
-def _choose_sddmm_heads_small(stats, heads, head_len, first):
-    """The choice of this model, or `first` where that is a candidate and the model sees less than 5 % more time for it."""
+# The same where the edges are stored in no order: the edge list gathers both operands (shares of the model's time for row-ordered edges and of one
+# operand's gather), the tiled walk's results go to random places (more per byte).  Fitted to 294 graphs and shapes (6,000 to 500,000 nodes, degrees 6 to
+# 200, 2 to 16 heads of 8 to 128 floats), 5 % behind the best of edge list and 1 to 8 partitions on average; the rule for large graphs is 13 % behind, and the
+# numbers above, which know nothing of the second gather, 16 %.  us, edge list / (1, 1) / this: 140,000 nodes of degree 40, 8 x 16 811 / 456 / 456, 4 x 32 767 /
+# 433 / 368, 8 x 64 3037 / - / 1624; 60,000 of 20, 8 x 8 85 / 60 / 60; 200,000 of 16, power-law, 8 x 64 1749 / - / 1102; 150,000 of 6, power-law, 2 x 16 34 / 48 / 34.
+_HEADS_SCATTERED = dict(ordered=0.5, gather=1.4, staged=0.5e-12, scattered=0.25e-12)
+
+
+def _choose_sddmm_heads_small(stats, heads, head_len, first, given_len=None, scattered=False):
+    """The choice of this model, or `first` where that is a candidate and the model sees less than 5 % (10 % for scattered edges, whose times
+    it knows less well) more time for it.  given_len (scattered edges): the heads' length where head_len is what the tiled walk would pad them to."""
     feat_len, out_bytes, c = heads * head_len, 4.0 * stats.nnz * heads, _HEADS_SMALL
+    more = _HEADS_SCATTERED if scattered else dict(staged=0.0, scattered=0.0)
+    copies = 0.0 if given_len is None else _padding_seconds(stats, heads * given_len, feat_len)
 
     def tiled(p, t):
         tile = feat_len // t
         per_tile, segments = tile // head_len, stats.segments(p)
         s = c['tiled'] * (_gather_seconds(stats, feat_len, p, t, SDDMM_SMALL_COEF) + segments * 4.0 * feat_len / SDDMM_SMALL_COEF['stream'])
-        s += c['launch'] + segments * t * c['segment']
+        s += c['launch'] + segments * t * c['segment'] + copies
         if per_tile == 1 and heads >= 4 and t > 1:
-            return s + out_bytes * c['staged'] + c['last']
-        return s + out_bytes * c['scattered'] * max(1.0, 8.0 / per_tile)
+            return s + out_bytes * (c['staged'] + more['staged']) + c['last']
+        return s + out_bytes * (c['scattered'] + more['scattered']) * max(1.0, 8.0 / per_tile)
 
-    edges = c['edges'] * predict_sddmm(stats, feat_len, 1, 1, SDDMM_SMALL_COEF) + c['edges_launch']
+    def edge_list():
+        length = feat_len if given_len is None else heads * given_len + (EDGES_MISALIGNED if heads * given_len % 32 else 0)
+        s = predict_sddmm(stats, length, 1, 1, SDDMM_SMALL_COEF)
+        if scattered:
+            s = more['ordered'] * s + more['gather'] * _gather_seconds(stats, length, 1, 1, SDDMM_SMALL_COEF)
+        # (unpadded against padded: 90,000 nodes of degree 30, power-law, edge list / tiled: 2 x 20 144 / 126, 3 x 20 217 / 228, 8 x 48 1072 / 740; 100,000 of 12
+        # 70 / 85, 105 / 150, 532 / 529; 500,000 of 8 281 / 367, 389 / 707, 1928 / 2602)
+        return (1.0 if given_len is None else 1.1) * c['edges'] * s + c['edges_launch']
+
     cands = [(p, feat_len // w) for w in (32, 64, 128, 256) if feat_len % w == 0 and w % head_len == 0 for p in (1, 2, 4, 8) if p <= max(1, stats.n_src)]
     costs = {c: tiled(*c) for c in cands}
-    costs[None] = edges
+    costs[None] = edge_list()
     best = min(costs, key=costs.get)
-    return first if first in costs and costs[best] > 0.95 * costs[first] else best
+    margin = 0.1 if scattered and given_len is None else 0.05
+    return first if first in costs and costs[best] > (1.0 - margin) * costs[first] else best
 
 
-def _choose_sddmm_heads(n_rows, n_cols, nnz, heads, head_len):
+def _choose_sddmm_heads(n_rows, n_cols, nnz, heads, head_len, scattered=False):
     """Several heads per edge.  What an (edge, tile) pair writes decides the tile: the memory system writes whole 32-byte
     sectors, so a tile that holds fewer than 8 heads and scatters them to `out` pays a sector for its 8 or 16 bytes
     (232,965-node graph, counted at the fabric: 8.0 GB written for 3.67 GB of results at H=8, D=32 with 128-float tiles,
@@ -495,7 +519,13 @@ def _choose_sddmm_heads(n_rows, n_cols, nnz, heads, head_len):
         # at least one partition per XCD (a single launch covers them all) -- unless that leaves the segments too short
         p = 8 // t if nnz / max(1, n_rows) / (8 // t) >= min_segment else 1
     if p == 1 and (t == 1 or feat_len <= 256 and _is_pow2(feat_len)):
-        # the edge-list kernel, which needs no positions: 36,608 nodes of degree 11, 8x32 69 -> 61 us; 124,691 of degree 67, 8x8 322 -> 315
+        # Row-ordered edges: the edge-list kernel, which needs no positions (36,608 nodes of degree 11, 8x32 69 -> 61 us; 124,691 of degree 67, 8x8
+        # 322 -> 315; 2,450,000 of degree 25, power-law, 8x32 11672 -> 10827; 1,000,000 of 60, 8x16 4435 -> 4522).  Scattered ones: one tile, which gathers
+        # one operand and reads a destination row once per segment, where the edge list gathers both (edge list / one tile: 1,000,000 of 60, 8x32 20831
+        # / 12795, 4x16 4257 / 3932; 700,000 of 50, power-law, 8x32 9642 / 5475, 2x16 1259 / 1084) -- unless rows are short and few edges share
+        # one (2,450,000 of 25, power-law, 8x32 20995 / 13765, but 4x16 4371 / 4814, 2x16 2322 / 3062).
+        if scattered and 16 <= feat_len <= 256 and _is_pow2(feat_len) and (feat_len > 64 or nnz >= 32 * n_rows or nnz < SMALL_NNZ):
+            return 1, 1
         return None
     return p, t
 

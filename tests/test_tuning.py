@@ -31,3 +31,23 @@ def test_heads_on_small_graphs_get_tiles_that_the_kernel_takes():
                     assert tile % head_len == 0 or head_len % tile == 0 and heads == 1
     assert tuning.choose_sddmm(150000, 150000, 900_000, 8, 64) is None          # degree 6: the edge list
     assert tuning.choose_sddmm(40000, 40000, 3_600_000, 4, 32) is not None
+
+
+def test_scattered_edges_of_several_heads_take_the_tiled_walk_sooner():
+    for n in (5000, 30000, 140000, 1_000_000):
+        for deg in (6, 16, 40, 160):
+            if n * deg > 6.5e7:
+                continue
+            for heads, head_len, given in ((2, 16, None), (8, 8, None), (4, 32, None), (8, 32, None), (2, 64, None), (8, 64, None), (8, 64, 48), (2, 32, 20)):
+                args = (n, n, n * deg, heads, head_len, None, given)
+                ordered, scattered = tuning.choose_sddmm(*args), tuning.choose_sddmm(*args, scattered=True)
+                assert scattered is not None or ordered is None, args
+                if scattered is not None:
+                    tile = heads * head_len // scattered[1]
+                    assert heads * head_len % scattered[1] == 0 and 16 <= tile <= 256 and tile & (tile - 1) == 0 and tile % head_len == 0
+    # where the edge list, which gathers both operands, takes 1.2 to 2.1 times as long
+    for n, deg, heads, head_len in ((140000, 40, 8, 16), (140000, 40, 2, 64), (60000, 20, 4, 16), (60000, 20, 8, 8), (36608, 11, 4, 32), (150000, 6, 8, 32),
+                                    (200000, 16, 8, 64), (1_000_000, 60, 8, 32)):
+        assert tuning.choose_sddmm(n, n, n * deg, heads, head_len, scattered=True) is not None
+    assert tuning.choose_sddmm(40000, 40000, 1_000_000, 8, 64, given_len=48, scattered=True) is not None
+    assert tuning.choose_sddmm(6000, 6000, 120_000, 2, 16, scattered=True) is None              # everything in the caches
