@@ -264,7 +264,7 @@ class SDDMMbase(object):
             if t_arg is None and knob_tiles is not None and order != 'coo' and order != 'csr':
                 t_arg = knob_tiles
             if order == 'tiled' or p_arg is not None or t_arg is not None:
-                base = tiled or (1, 1)
+                base = tiled or tuning.complete_tiled_sddmm(self._num_rows, self._num_cols, nnz, H, D, self._graph_stats() if H == 1 else None)
                 tiled = (int(p_arg) if p_arg is not None else base[0], int(t_arg) if t_arg is not None else base[1])
             if tiled is not None:
                 notes.append("tiled traversal: %d source-column partitions x %d feature tiles; results are "

@@ -416,6 +416,25 @@ def choose_sddmm(n_rows, n_cols, nnz, heads, head_len, stats=None, given_len=Non
     return first
 
 
+def complete_tiled_sddmm(n_rows, n_cols, nnz, heads, head_len, stats=None):
+    """(num_src_partitions, num_feat_tiles) for a caller who asks for the tiled traversal, or for one of the two numbers, where choose_sddmm
+    would take an edge-list kernel: tiles that the kernel takes, (1, 1) where there are none."""
+    feat_len = heads * head_len
+    takes = lambda tile: 16 <= tile <= 256 and _is_pow2(tile) and (heads == 1 or tile % head_len == 0 and head_len % 4 == 0 and head_len >= 8)
+    if heads == 1:
+        if takes(feat_len) or nnz == 0 or feat_len % 4 != 0:
+            return 1, 1
+        if stats is None:
+            stats = GraphStats(n_rows, n_cols, nnz)
+        cands = [(p, t) for p, t in _candidates(feat_len) if feat_len % t == 0 and takes(feat_len // t)]
+        ranked = _rank(stats, feat_len, predict_sddmm, cands, _sddmm_tie, SDDMM_COEF)
+        return ranked[0] if ranked else (1, 1)
+    first = _choose_sddmm_heads(n_rows, n_cols, nnz, heads, head_len, scattered=True)
+    if first is not None:
+        return first
+    return 1, next((feat_len // tile for tile in (256, 128, 64, 32, 16) if feat_len % tile == 0 and takes(tile)), 1)
+
+
 def _is_pow2(v):
     return v > 0 and (v & (v - 1)) == 0
 

@@ -1,0 +1,34 @@
+"""Schedules of the SDDMM modules that name a part of the tiled traversal's shape: the rest is completed to a shape that the kernel takes."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+from helpers import assert_sum_close
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,deg,shape", [(60000, 8, (8, 64)), (60000, 8, (16, 32)), (140000, 16, (320,)), (40000, 9, (8, 48)), (3000, 5, (4, 16)), (3000, 5, (512,)),
+                                         (3000, 5, (64,))])
+@pytest.mark.parametrize("schedule", [{"order": "tiled"}, {"num_src_partitions": 2}, {"order": "tiled", "num_src_partitions": 3}])
+def test_partial_schedules_are_completed(n, deg, shape, schedule):
+    import torch
+    from featgraph_amd.module import MultiHeadSDDMMhip, VanillaSDDMMhip, placeholder
+    rng = np.random.default_rng(n + len(shape))
+    row = np.repeat(np.arange(n), deg)
+    col = np.sort(rng.integers(0, n, (n, deg)), axis=1).ravel()
+    keep = np.r_[True, (row[1:] != row[:-1]) | (col[1:] != col[:-1])]
+    adj = sp.csr_matrix((np.ones(int(keep.sum()), np.float32), (row[keep], col[keep])), shape=(n, n))
+    adj.sort_indices()
+    row, col = np.repeat(np.arange(n), np.diff(adj.indptr)), adj.indices
+    x, y = (rng.standard_normal((n,) + shape, dtype=np.float32) for _ in range(2))
+    m = (MultiHeadSDDMMhip if len(shape) == 2 else VanillaSDDMMhip)(adj)
+    m.build([placeholder(x.shape)] * 2, {}, dict(schedule))
+    assert m._tiled is not None and m._tiled[0]["P"] == schedule.get("num_src_partitions", m._tiled[0]["P"])
+    m.out_tvm.fill_(float("nan"))
+    got = m.run([torch.from_numpy(x).cuda(), torch.from_numpy(y).cuda()]).cpu().numpy()
+    at = rng.choice(len(col), 2000)                 # (all of them in float64 would take minutes)
+    assert np.isfinite(got).all()
+    prod = (x[col[at]].astype("f8") * y[row[at]]).reshape((2000,) + (shape if len(shape) == 2 else (1,) + shape))
+    want, mass = prod.sum(-1), np.abs(prod).sum(-1)
+    assert_sum_close(got[at].reshape(want.shape), want, mass, str((n, shape, schedule)))

@@ -51,3 +51,12 @@ def test_scattered_edges_of_several_heads_take_the_tiled_walk_sooner():
         assert tuning.choose_sddmm(n, n, n * deg, heads, head_len, scattered=True) is not None
     assert tuning.choose_sddmm(40000, 40000, 1_000_000, 8, 64, given_len=48, scattered=True) is not None
     assert tuning.choose_sddmm(6000, 6000, 120_000, 2, 16, scattered=True) is None              # everything in the caches
+
+
+def test_a_tiled_traversal_that_is_asked_for_gets_tiles_that_the_kernel_takes():
+    for n, nnz in ((1000, 5000), (60000, 480000), (140000, 2240000), (2_000_000, 40_000_000)):
+        for heads, head_len in ((8, 64), (16, 32), (1, 320), (8, 48 + 16), (12, 16), (1, 512), (1, 2048), (1, 64), (2, 8), (3, 8 * 4)):
+            p, t = tuning.complete_tiled_sddmm(n, n, nnz, heads, head_len)
+            tile = heads * head_len // t
+            assert p >= 1 and heads * head_len % t == 0 and 16 <= tile <= 256 and tile & (tile - 1) == 0 and (heads == 1 or tile % head_len == 0)
+    assert tuning.complete_tiled_sddmm(1000, 1000, 5000, 3, 20) == (1, 1)            # nothing fits: the kernel refuses, as ever
