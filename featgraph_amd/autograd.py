@@ -47,6 +47,7 @@ class Graph(object):
         # scratch); later ones of the same orientation use them too: every operator of a Graph runs on the caller's one
         # stream, one after the other, so one scratch per orientation is enough
         self._layout_owner = {}
+        self._sweeps_do_not_fit = set()         # (transposed, row length) of the sweeps of _sweep_selected
 
     def _gspmm_module(self, transposed):
         m = GSpMMhip(self._tr if transposed else self._csr)
@@ -168,16 +169,23 @@ class Graph(object):
         """The unpartitioned layout of one orientation with scratch for sweeps over rows of `feat_len`, and (transposed) its
         elements' CSR positions."""
         key = ('sweep', transposed)
-        if key not in self._mods:
-            m = self._gspmm_module(transposed)
-            m.set_weight_order(self._tr_pos_host if transposed else None)
-            m.swept = set()
-            self._mods[key] = m
-        m = self._mods[key]
-        lay = m._layout(1)
-        if transposed and feat_len not in m.swept:
-            common.reserve(lay['plan'], common.OP_GSPMM_BCAST, 1, feat_len, 0, m.ctx)
-            m.swept.add(feat_len)
+        m = self._mods.get(key) or self._gspmm_module(transposed)
+        made = 1 not in m._layouts
+        try:
+            if key not in self._mods:
+                m.set_weight_order(self._tr_pos_host if transposed else None)
+                m.swept = set()
+            lay = m._layout(1)
+            if transposed and feat_len not in m.swept:
+                common.reserve(lay['plan'], common.OP_GSPMM_BCAST, 1, feat_len, 0, m.ctx)
+                m.swept.add(feat_len)
+        except Exception:                       # what does not fit leaves no layout behind
+            if made and 1 in m._layouts:
+                m._destroy_layout(m._layouts.pop(1))
+            if key not in self._mods and self._layout_owner[transposed] is m:
+                del self._layout_owner[transposed]
+            raise
+        self._mods[key] = m
         return lay, m._weight_perm
 
     def _sweep_selected(self, message, side, arg, other, dout, grads, shape):
@@ -189,6 +197,8 @@ class Graph(object):
         sources, own_len = sweep[0] == 'u', (message.lhs_len, message.rhs_len)[side]
         if not tuning.select_by_sweep(self.nnz, self.shape[0], message.out_len, sweep[0], own_len, sweep[2]):
             return False
+        if (sources, message.out_len) in self._sweeps_do_not_fit:
+            return False
         try:
             layout, edge_pos = self._sweep_layout(sources, message.out_len)
             grad = torch.empty(shape, dtype=dout.dtype, device=dout.device)
@@ -196,7 +206,9 @@ class Graph(object):
                 message.select_sources(sweep, layout, edge_pos, arg, other, dout, grad)
             else:
                 message.select_edges(sweep, layout, arg, other, dout, grad, own_len)
-        except MemoryError:
+        except (MemoryError, torch.cuda.OutOfMemoryError):
+            # a failed attempt costs a layout's preparation and device synchronisations: not at every step
+            self._sweeps_do_not_fit.add((sources, message.out_len))
             return False
         grads[side] = grad
         return True

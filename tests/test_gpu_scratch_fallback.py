@@ -153,3 +153,51 @@ def test_additive_attention_without_memory_for_the_kept_sums(monkeypatch, where)
             # either way within 2e-6 of float64 on such rows
             assert float((a - b).norm()) <= 4e-6 * float(b.norm())
     assert len(calls) == 1
+
+
+@pytest.mark.parametrize("where", ["positions", "layout", "scratch", "call"])
+@pytest.mark.parametrize("op", ["copy", "mul"])
+def test_max_gradients_without_memory_for_the_sweeps(monkeypatch, where, op):
+    """The sweep's layout, its positions, its scratch or the library's own buffers do not fit: the gradient result by result, from then on
+    without another attempt, and nothing of the attempt stays."""
+    import torch
+    from featgraph_amd import _lib, ops, tuning
+    from featgraph_amd.autograd import Graph
+    from featgraph_amd.module import GSpMMhip, common
+    adj = _graph()
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    normal = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    leaves = [normal(adj.shape[1], 64).requires_grad_()] + ([normal(adj.nnz, 64).requires_grad_()] if op == "mul" else [])
+    dy = normal(adj.shape[0], 64)
+    g = Graph(adj)
+
+    def step():
+        out = g.aggregate(leaves[0], "max") if op == "copy" else ops.gspmm(g, "mul", "max", *leaves)
+        return torch.autograd.grad(out, leaves, dy)
+
+    monkeypatch.setattr(tuning, "select_by_sweep", lambda *a: False)
+    ref = step()
+    monkeypatch.setattr(tuning, "select_by_sweep", lambda *a: True)
+    calls = []
+
+    def no(error):
+        def fail(*a, **kw):
+            calls.append(1)
+            raise error
+        return fail
+    if where == "positions":
+        monkeypatch.setattr(GSpMMhip, "set_weight_order", no(torch.cuda.OutOfMemoryError("positions")))
+    elif where == "layout":
+        monkeypatch.setattr(GSpMMhip, "_layout", no(torch.cuda.OutOfMemoryError("layout")))
+    elif where == "scratch":
+        monkeypatch.setattr(common, "reserve", no(MemoryError("scratch")))
+    else:
+        monkeypatch.setattr(_lib.lib(), "fg_select_sources_f32", _failing(calls))
+        monkeypatch.setattr(_lib.lib(), "fg_select_edges_f32", _failing(calls))
+    for _ in range(2):
+        for a, b in zip(step(), ref):
+            # float sums of up to 400 results in two orders
+            assert float((a - b).norm()) <= 400 * 2.0 ** -24 * float(b.norm())
+    assert len(calls) == (1 if op == "copy" or where == "scratch" else 2)          # each operand's sweep (the edges' has no scratch), once
+    if where == "scratch":
+        assert 1 not in getattr(g._layout_owner.get(True), "_layouts", {})
