@@ -211,7 +211,23 @@ class SDDMMbase(object):
             raise ValueError("SrcFeat / DstFeat must be 2-D, got %s and %s" % (src_ph.shape, dst_ph.shape))
         return 1, src_ph.shape[1]
 
-    def _resolve(self, input_placeholders, compute_args, schedule_args):
+    def _padded(self, given, compute_args, schedule_args):
+        """(placeholders, schedule_args, pad_from): what the kernels are chosen for, and the rows' given length where that is
+        another one (else None).  Single-head rows of an awkward length run at the next friendly one (tuning.padded_feature_len), heads at one that
+        fills whole lane groups (tuning.padded_head_len): the extra columns add zeros to every dot product.  The tiled traversal reads
+        them from zero-padded copies of both operands; the edge-list kernels read the operands as they are and fill up in registers."""
+        pads = len(given) == 2 and len(given[0].shape) in (2, 3) and tuple(given[0].shape[1:]) == tuple(given[1].shape[1:]) \
+            and schedule_args.get('pad_features', True) and not compute_args.get('num_feat_partitions') \
+            and not any(schedule_args.get(k) for k in ('num_feat_partitions', 'num_feat_tiles'))
+        schedule_args = {k: v for k, v in schedule_args.items() if k != 'pad_features'}
+        if pads:
+            heads, length = given[0].shape[1:-1], given[0].shape[-1]
+            want = tuning.padded_head_len(length) if heads else tuning.padded_feature_len(length)
+            if want != length and self._adj_row_indices.shape[0] * int(np.prod(given[0].shape[1:])) >= tuning.PAD_MIN_GATHERED:
+                return [common.placeholder((g.shape[0],) + tuple(heads) + (want,)) for g in given], schedule_args, length
+        return given, schedule_args, None
+
+    def _resolve(self, input_placeholders, compute_args, schedule_args, pad_from=None):
         compute_args = common.take_args(compute_args, self._compute_keys, "compute_func")
         schedule_args = common.take_args(schedule_args, self._schedule_keys, "schedule_func")
         if len(input_placeholders) != 2:
@@ -259,7 +275,7 @@ class SDDMMbase(object):
         nnz = self._adj_row_indices.shape[0]
         if order in ('auto', 'tiled') and nnz > 0:
             tiled = tuning.choose_sddmm(self._num_rows, self._num_cols, nnz, H, D, self._graph_stats() if H == 1 else self._degree_stats(),
-                                        given_len=getattr(self, '_pad_from', None), scattered=not self._row_sorted)
+                                        given_len=pad_from, scattered=not self._row_sorted)
             p_arg, t_arg = schedule_args.get('num_src_partitions'), schedule_args.get('num_feat_tiles')
             if t_arg is None and knob_tiles is not None and order != 'coo' and order != 'csr':
                 t_arg = knob_tiles
@@ -269,6 +285,8 @@ class SDDMMbase(object):
             if tiled is not None:
                 notes.append("tiled traversal: %d source-column partitions x %d feature tiles; results are "
                              "written back in the stored edge order" % tiled)
+                if pad_from is not None:
+                    notes.append("rows of %d floats run as rows of %d on zero-padded copies" % (pad_from, D))
         return [src_ph, dst_ph], H, D, use_csr, tiled, notes
 
     def _graph_stats(self):
@@ -348,35 +366,13 @@ class SDDMMbase(object):
                 and (compute_args.get('num_feat_partitions', 1) or 1) == 1 and self._adj_row_indices.shape[0] > 0:
             schedule_args = self._tune(list(input_placeholders), dict(compute_args), dict(schedule_args), 6 if tune is True else int(tune))
         schedule_args = {k: v for k, v in schedule_args.items() if k != 'tune'}
-        # Single-head rows of an awkward length run at the next friendly one (tuning.padded_feature_len): the extra columns
-        # add zeros to every dot product.  The tiled traversal reads them from zero-padded copies of both operands; the
-        # edge-list kernel reads the operands as they are and fills up in registers.
-        self._pad_from = None
         given = list(input_placeholders)
-        if len(given) == 2 and len(given[0].shape) == 2 and len(given[1].shape) == 2 and given[0].shape[1] == given[1].shape[1] \
-                and schedule_args.get('pad_features', True) and not compute_args.get('num_feat_partitions') \
-                and not any(schedule_args.get(k) for k in ('num_feat_partitions', 'num_feat_tiles')):
-            D0 = given[0].shape[1]
-            want = tuning.padded_feature_len(D0)
-            if want != D0 and self._adj_row_indices.shape[0] * D0 >= tuning.PAD_MIN_GATHERED:
-                self._pad_from = D0
-                input_placeholders = [common.placeholder((given[0].shape[0], want)), common.placeholder((given[1].shape[0], want))]
-        elif len(given) == 2 and len(given[0].shape) == 3 and tuple(given[0].shape[1:]) == tuple(given[1].shape[1:]) \
-                and schedule_args.get('pad_features', True) and not compute_args.get('num_feat_partitions') \
-                and not any(schedule_args.get(k) for k in ('num_feat_partitions', 'num_feat_tiles')):
-            # several heads: every head padded to a length that fills whole lane groups (tuning.padded_head_len)
-            H0, D0 = given[0].shape[1], given[0].shape[2]
-            want = tuning.padded_head_len(D0)
-            if want != D0 and self._adj_row_indices.shape[0] * H0 * D0 >= tuning.PAD_MIN_GATHERED:
-                self._pad_from = D0
-                input_placeholders = [common.placeholder((given[0].shape[0], H0, want)), common.placeholder((given[1].shape[0], H0, want))]
-        schedule_args = {k: v for k, v in schedule_args.items() if k != 'pad_features'}
-        phs, H, D, use_csr, tiled, notes = self._resolve(input_placeholders, compute_args, schedule_args)
+        input_placeholders, schedule_args, self._pad_from = self._padded(given, compute_args, schedule_args)
+        phs, H, D, use_csr, tiled, notes = self._resolve(input_placeholders, compute_args, schedule_args, self._pad_from)
         self._src_pad = self._dst_pad = None
         if self._pad_from is not None:
             phs = given
         if self._pad_from is not None and tiled is not None:
-            notes.append("rows of %d floats run as rows of %d on zero-padded copies" % (self._pad_from, D))
             tail = (D,) if len(given[0].shape) == 2 else (H, D)
             self._src_pad = torch.zeros((self._num_cols,) + tail, dtype=torch.float32, device=self._ctx)
             self._dst_pad = torch.zeros((self._num_rows,) + tail, dtype=torch.float32, device=self._ctx)
@@ -398,7 +394,10 @@ class SDDMMbase(object):
 
     def lower_to_ir(self, input_placeholders, compute_args, schedule_args):
         """Return a text description of the launch. This can be useful for debug."""
-        _, H, D, use_csr, tiled, notes = self._resolve(input_placeholders, compute_args, schedule_args)
+        phs, schedule_args, pad_from = self._padded(list(input_placeholders), compute_args, schedule_args)
+        _, H, D, use_csr, tiled, notes = self._resolve(phs, compute_args, schedule_args, pad_from)
+        if pad_from is not None and tiled is None:
+            D = pad_from                       # the edge-list kernels read the rows as they are
         nnz = self._adj_row_indices.shape[0]
         text = "featgraph-hip SDDMM (gfx950)\n"
         text += "  adjacency        : %d x %d, %d stored edges, %d x %d partition blocks\n" % (

@@ -32,3 +32,23 @@ def test_partial_schedules_are_completed(n, deg, shape, schedule):
     prod = (x[col[at]].astype("f8") * y[row[at]]).reshape((2000,) + (shape if len(shape) == 2 else (1,) + shape))
     want, mass = prod.sum(-1), np.abs(prod).sum(-1)
     assert_sum_close(got[at].reshape(want.shape), want, mass, str((n, shape, schedule)))
+
+
+@pytest.mark.parametrize("shapes", [((100,), (512,)), ((8, 48), (8, 64)), ((512,), (100,))])
+def test_descriptions_do_not_depend_on_what_was_built_before(shapes):
+    """lower_to_ir() describes what build() would take for its own arguments, padded rows included, whatever the module was built for."""
+    from featgraph_amd.module import MultiHeadSDDMMhip, VanillaSDDMMhip, placeholder
+    rng = np.random.default_rng(1)
+    n, deg = 60000, 40
+    col = rng.integers(0, n, (n, deg)).ravel()
+    adj = sp.coo_matrix((np.ones(n * deg, np.float32), (np.repeat(np.arange(n), deg), col)), shape=(n, n)).tocsr()
+    adj.sort_indices()
+    make = MultiHeadSDDMMhip if len(shapes[0]) == 2 else VanillaSDDMMhip
+    phs = [[placeholder((n,) + s)] * 2 for s in shapes]
+    m = make(adj)
+    m.build(phs[0], {}, {})
+    assert m.lower_to_ir(phs[1], {}, {}) == make(adj).lower_to_ir(phs[1], {}, {})
+    text = m.lower_to_ir(phs[0], {}, {})
+    assert ("sddmm_tiled_kernel" in text) == (m._tiled is not None) and ("zero-padded" in text) == (m._src_pad is not None)
+    if m._tiled is not None:
+        assert "%d source-column partition(s) x %d feature tile(s)" % (m._tiled[0]["P"], m._tiled[1]) in text
