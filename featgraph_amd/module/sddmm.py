@@ -274,7 +274,8 @@ class SDDMMbase(object):
         tiled = None
         nnz = self._adj_row_indices.shape[0]
         if order in ('auto', 'tiled') and nnz > 0:
-            tiled = tuning.choose_sddmm(self._num_rows, self._num_cols, nnz, H, D, self._graph_stats() if H == 1 else self._degree_stats(),
+            stats = self._graph_stats() if H == 1 or nnz < tuning.SMALL_NNZ else None          # (several heads on large graphs: sizes decide)
+            tiled = tuning.choose_sddmm(self._num_rows, self._num_cols, nnz, H, D, stats,
                                         given_len=pad_from, scattered=not self._row_sorted)
             p_arg, t_arg = schedule_args.get('num_src_partitions'), schedule_args.get('num_feat_tiles')
             if t_arg is None and knob_tiles is not None and order != 'coo' and order != 'csr':
@@ -293,20 +294,11 @@ class SDDMMbase(object):
         """Column reference counts and row degrees of the adjacency, as the tuning model reads them (once per object)."""
         if getattr(self, '_stats', None) is None:
             counts = np.bincount(self._adj_col_indices, minlength=self._num_cols) if len(self._adj_col_indices) else np.zeros(self._num_cols, np.int64)
-            degs = np.bincount(self._adj_row_indices, minlength=self._num_rows) if len(self._adj_row_indices) else np.zeros(self._num_rows, np.int64)
+            degs = np.diff(self._adj_indptr) if self._row_sorted else np.bincount(self._adj_row_indices, minlength=self._num_rows)
             cv, cm = np.unique(counts, return_counts=True)
             dv, dm = np.unique(degs, return_counts=True)
             self._stats = tuning.GraphStats(self._num_rows, self._num_cols, len(self._adj_col_indices), cv, cm, dv, dm)
         return self._stats
-
-    def _degree_stats(self):
-        """The same from the row degrees alone, which stand for the columns' too (None: the edges are in no order)."""
-        if not self._row_sorted:
-            return None
-        if getattr(self, '_deg_stats', None) is None:
-            vals, mult = np.unique(np.diff(self._adj_indptr), return_counts=True)
-            self._deg_stats = tuning.GraphStats(self._num_rows, self._num_cols, len(self._adj_col_indices), vals, mult, vals, mult)
-        return self._deg_stats
 
     def _tune(self, phs, compute_args, schedule_args, how_many):
         """Times the stored-order kernel(s) and the cost model's `how_many` most promising tiled traversals on

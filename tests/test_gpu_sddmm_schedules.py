@@ -52,3 +52,18 @@ def test_descriptions_do_not_depend_on_what_was_built_before(shapes):
     assert ("sddmm_tiled_kernel" in text) == (m._tiled is not None) and ("zero-padded" in text) == (m._src_pad is not None)
     if m._tiled is not None:
         assert "%d source-column partition(s) x %d feature tile(s)" % (m._tiled[0]["P"], m._tiled[1]) in text
+
+
+def test_several_heads_on_a_rectangular_adjacency_are_chosen_for_its_own_column_counts():
+    """Far fewer sources than destinations: every column is referenced far more often than a row is long."""
+    from featgraph_amd import tuning
+    from featgraph_amd.module import MultiHeadSDDMMhip, placeholder
+    rng = np.random.default_rng(2)
+    rows, cols, deg = 300000, 20000, 20
+    col = np.sort(rng.integers(0, cols, (rows, deg)), axis=1)
+    adj = sp.csr_matrix((np.ones(rows * deg, np.float32), col.ravel(), np.arange(0, rows * deg + 1, deg)), shape=(rows, cols))
+    adj.sum_duplicates()
+    m = MultiHeadSDDMMhip(adj)
+    m.build([placeholder((cols, 8, 32)), placeholder((rows, 8, 32))], {}, {})
+    want = tuning.choose_sddmm(rows, cols, adj.nnz, 8, 32, tuning.GraphStats.from_csr(adj.indptr, adj.indices, cols))
+    assert want is not None and m._tiled is not None and (m._tiled[0]["P"], m._tiled[1]) == want
