@@ -47,12 +47,15 @@ SPMM_COEF = dict(cache=2.12, hit=24.0e12, miss=7.07e12, span=0.011, seg=1.64e-11
 SDDMM_COEF = dict(cache=2.26, hit=23.5e12, miss=6.58e12, span=0.0, seg=3.82e-11, edge=0.0, stream=3.86e12)
 
 # Below this many stored elements the launches, the sums that follow them and the caches' real size weigh more.  A second set of
-# coefficients is fitted to sweeps of P (1 .. 16) x T on 23 graphs of 3,000 to 390,000 nodes and 100,000 to 22 M elements (degrees 7 to 430,
-# power-law and uniform; feature lengths 16 .. 512) and overrules the first where it sees 15 % (SpMM) or 5 % (SDDMM) less time for
-# its own choice: over the sweeps the time falls by 4.3 % (SpMM) and 8.7 % (SDDMM) on average, the worst point loses 6 % and 8 %, and
-# what is left to the best is 1.5 % and 3.8 %.  With the second set alone: 3.7 % and 9.2 %, the worst 54 % and 14 %.  The largest, us: 17,600 nodes of
-# degree 266, uniform, F=512: SpMM 723 -> 360, SDDMM 1128 -> 400; 12,000 of degree 200, F=512: SpMM 232 -> 190, SDDMM 473 -> 195.
+# coefficients, fitted to sweeps of P (1 .. 16) x T on 23 graphs, overrules the first where it sees 15 % (SpMM) or 5 % (SDDMM) less time for its own
+# choice; from more than 200,000 sources on 30 % and 10 %, where the first set is the nearer one.  Held against 276 other graphs (4,000 to 400,000
+# nodes, degrees 6 to 260, uniform and power-law, feature lengths 16 .. 512, P 1 .. 8 with every T): the choice's time against the first set's, mean / worst,
+# SpMM 0.972 / 1.17 (beyond 200,000 sources 0.999 / 1.00), SDDMM 0.935 / 1.17 (0.996 / 1.07); against the best of the sweep SpMM 1.031 (first set 1.061), SDDMM
+# 1.038 (1.110).  With 15 % and 5 % everywhere the worst beyond 200,000 sources are 1.23 (250,000 of degree 50, uniform, F=128, SpMM 719 -> 886 us) and
+# 1.21 (280,000 of 32, power-law, F=256, SDDMM 1053 -> 1278); without the second set there, uniform, SpMM 320,000 of 32, F=64 365 -> 408, SDDMM 250,000 of 20, F=32 99 -> 125.
+# The largest, us: 17,600 nodes of degree 266, uniform, F=512: SpMM 723 -> 360, SDDMM 1128 -> 400; 12,000 of degree 200, F=512: 232 -> 190, 473 -> 195.
 SMALL_NNZ = 1 << 25
+MANY_SOURCES = 200_000
 # pass / sum: seconds that a second pass over the graph (SpMM) and the sum of the tiles' scores (SDDMM) cost whatever their size;
 # seg_tiled: per row segment and tile where there are several; edges_dst: the edge-list kernel's reads of destination rows, as
 # a share of the gathered bytes at the hit rate.
@@ -63,9 +66,7 @@ SDDMM_SMALL_COEF = dict(cache=1.32, hit=24.7e12, miss=8.49e12, span=0.006, seg=2
 
 
 def _is_small(stats):
-    # (not the long rows of many nodes, which lie outside the fit: uniform, 385,603 nodes of degree 62, F=128, sum and SDDMM: 3213 us by the other
-    # coefficients, 3570 by these)
-    return stats.nnz < SMALL_NNZ and not (stats.n_src > 200_000 and stats.nnz >= 40 * stats.n_dst)
+    return stats.nnz < SMALL_NNZ
 
 
 # legacy names (attention module): per-XCD slice that two L2s' worth of slices add up to
@@ -274,12 +275,12 @@ def rank_spmm(stats, feat_len):
         # short rows: 32-float tiles, which the model likes for their hit rate, are behind (30,000 nodes of degree 30, us with tiles of 64 / 32
         # floats: F=64 25 / 28, F=256 65 / 78, F=512 116 / 150; 60,000 of degree 40, F=512 385 / 333)
         cands = [(p, t) for p, t in cands if feat_len // t >= 64]
-    return _overrule(stats, feat_len, predict_spmm, ranked, cands, SPMM_SMALL_COEF, 0.15)
+    return _overrule(stats, feat_len, predict_spmm, ranked, cands, SPMM_SMALL_COEF, 0.15 if stats.n_src <= MANY_SOURCES else 0.3)
 
 
-def rank_sddmm(stats, feat_len):
+def rank_sddmm(stats, feat_len, pieces=None):
     """(num_src_partitions, num_feat_tiles) candidates of the tiled traversal, most promising first;
-    (1, 1) stands for the edge-list kernel."""
+    (1, 1) stands for the edge-list kernel.  pieces: see below."""
     cands = [(p, t) for p, t in _candidates(feat_len) if not (t == 1 and p > 1 and feat_len > 256)]
     ranked = _rank(stats, feat_len, predict_sddmm, cands, _sddmm_tie, SDDMM_COEF)
     if not ranked or not _is_small(stats):
@@ -288,7 +289,15 @@ def rank_sddmm(stats, feat_len):
     ranked = [c for c in ranked if c in takes]
     if 4.0 * stats.n_src * feat_len <= N_XCD * L2_BYTES / 4 or ranked[0][0] == 1:
         ranked = [(1, 1)]
-    return _overrule(stats, feat_len, predict_sddmm, ranked, takes, SDDMM_SMALL_COEF, 0.05)
+    # Several partitions and one tile write each row's results in pieces, 4 bytes at a time where a row has few elements per partition, which the model does
+    # not price: only from `pieces` of them on, or where the first set is for it too (edge list / 2 x 1: 40,000 nodes of degree 20, power-law, F=128
+    # 45 / 66, F=64 24 / 32; 25,000 of 32 37 / 54; 15,000 of 12, uniform, F=256 22 / 31; 200,000 of 32, uniform, F=128 2 x 4 460, 2 x 1 570; 40,000 of
+    # 32, uniform, F=64 39 / 37).  Over the 276 graphs 93 of 1539 choices are more than 5 % behind the first set's and 34 more than 15 % without this line,
+    # 22 and 1 with it.
+    if pieces is None:
+        pieces = 20 if feat_len <= 64 else 32
+    takes = [(p, t) for p, t in takes if p == 1 or t > 1 or ranked[0][0] > 1 == ranked[0][1] or stats.nnz >= pieces * p * stats.n_dst]
+    return _overrule(stats, feat_len, predict_sddmm, ranked, takes, SDDMM_SMALL_COEF, 0.05 if stats.n_src <= MANY_SOURCES else 0.1)
 
 
 def choose_spmm(n_dst, n_src, nnz, feat_len, stats=None):
@@ -351,18 +360,19 @@ def _choose_sddmm_scattered(stats, feat_len, given_len):
     tiled traversal scatters its results.  us, edge list / tiled, uniform graphs unless said: 30,000 nodes of degree 8, F=128 33 / 30
     (power-law 28 / 37), F=512 125 / 74; of degree 40, F=64 66 / 41, F=222 333 / 127; of degree 160, F=16 52 / 71, F=37 194 / 137;
     140,000 of degree 8, F=37 79 / 93, F=64 79 / 74, F=128 157 / 119, F=256 330 / 213; of degree 40, F=222 1642 / 763."""
-    # (partitions with one tile scatter from short segments: 30,000 nodes of degree 8, power-law, F=256 edge list 52, 2 x 1 63)
-    takes = [(p, t) for p, t in rank_sddmm(stats, feat_len) if (p, t) != (1, 1) and (t > 1 or stats.nnz >= 12 * stats.n_dst)]
-    if not takes:
-        return None
-    coef, tiled = SDDMM_SMALL_COEF, takes[0]
-    best = predict_sddmm(stats, feat_len, *tiled, coef) + 12e-6 + 7e-12 * stats.nnz
-    edges_len = feat_len
+    # (partitions with one tile: from 12 elements per row on -- 30,000 nodes of degree 8, power-law, F=256 edge list 52, 2 x 1 63 --, and above 64 floats only
+    # where nothing else is ahead of the edge list: 40,000 of 16, power-law, F=128 1 x 2 43, 2 x 1 62; 20,000 of 16, F=128 edge list 42, 2 x 1 27; 40,000 of
+    # 16, F=64 41, 32)
+    coef, edges_len, more = SDDMM_SMALL_COEF, feat_len, 12e-6 + 7e-12 * stats.nnz
     if given_len is not None and given_len != feat_len:
         edges_len = given_len + EDGES_MISALIGNED
-        best += _padding_seconds(stats, given_len, feat_len)
+        more += _padding_seconds(stats, given_len, feat_len)
     edges = 1.15 * (predict_sddmm(stats, edges_len, 1, 1, coef) + _gather_seconds(stats, edges_len, 1, 1, coef))
-    return tiled if best < edges else None
+    for pieces in (0,) if feat_len <= 64 else (32, 0):
+        takes = [(p, t) for p, t in rank_sddmm(stats, feat_len, pieces) if (p, t) != (1, 1) and (t > 1 or stats.nnz >= 12 * stats.n_dst)]
+        if takes and predict_sddmm(stats, feat_len, *takes[0], coef) + more < edges:
+            return takes[0]
+    return None
 
 
 def _padding_seconds(stats, given_len, feat_len):

@@ -60,3 +60,18 @@ def test_a_tiled_traversal_that_is_asked_for_gets_tiles_that_the_kernel_takes():
             tile = heads * head_len // t
             assert p >= 1 and heads * head_len % t == 0 and 16 <= tile <= 256 and tile & (tile - 1) == 0 and (heads == 1 or tile % head_len == 0)
     assert tuning.complete_tiled_sddmm(1000, 1000, 5000, 3, 20) == (1, 1)            # nothing fits: the kernel refuses, as ever
+
+
+def test_choices_on_small_graphs_that_were_measured():
+    """Where the fitted model is known to be wrong by more than the measurements' noise, on both sides of the rules that say so (uniform degrees)."""
+    def sddmm(n, deg, feat_len, **kw):
+        return tuning.choose_sddmm(n, n, n * deg, 1, feat_len, **kw)
+    # partitions with one tile: results in pieces of a few elements (40,000 nodes of degree 20 and the like: 1.3 to 1.5 times the edge list's time)
+    for n, deg, feat_len in ((25000, 20, 128), (15000, 12, 256), (40000, 12, 64), (200000, 32, 128)):
+        got = sddmm(n, deg, feat_len)
+        assert got is None or got[1] > 1 or got[0] == 1, (n, deg, feat_len)
+    assert sddmm(150000, 62, 32) == (4, 1) and sddmm(140000, 62, 16)[1] == 1
+    # from 200,000 sources on the second set of coefficients has to see more of a gain
+    for n, deg, feat_len in ((250000, 50, 128), (400000, 62, 128), (250000, 40, 256)):
+        assert tuning.choose_spmm(n, n, n * deg, feat_len) == (4, feat_len // 32), (n, deg, feat_len)
+    assert tuning.choose_spmm(320000, 320000, 320000 * 32, 64)[0] == 1
