@@ -123,12 +123,16 @@ struct Spread {
     static __device__ __forceinline__ bool stores(int i) { return i % lanes == 0; }
 };
 
-// The staged units [0, n) of `unit` (x / y: the operands' rows, as byte offsets with OFF32, else as column and row ids whose
-// block of heads is in `block`; valid entries up to the next multiple of a batch); unit j's results go to out[j * side ..], or with
-// `edge_pos` (of the edge of unit 0, whose block is first_block) to the place of its edge.  ONE: a head is one chunk at most.
-template <int L, bool OFF32, bool ONE>
-__device__ __forceinline__ void dot_units(const uint2 *unit, const uint32_t *block, int n, int lane, const SddmmArgs &a, float *out,
-                                          const int32_t *edge_pos, int first_block) {
+// The byte offsets of a unit's rows of src and dst.
+template <bool OFF32> using Offset = std::conditional_t<OFF32, uint32_t, uint64_t>;
+template <bool OFF32> struct alignas(2 * sizeof(Offset<OFF32>)) Unit { Offset<OFF32> x, y; };
+
+// The staged units [0, n) (valid entries up to the next multiple of a batch); unit j's results go to out[j * side ..], or, PLACED, to the
+// place of its edge, edge_pos (of the edge of unit 0, whose block is first_block).  ONE: a head is one chunk at most.
+template <int L, bool OFF32, bool ONE, bool PLACED>
+__device__ __forceinline__ void dot_units(const Unit<OFF32> *unit, int n, int lane, const SddmmArgs &a, float *out, const int32_t *edge_pos,
+                                          int first_block) {
+    using off = Offset<OFF32>;
     constexpr int U = batch_steps(L), CH = 4 * L;
     using S = Spread<L, U>;
     const int li = lane % L;
@@ -140,24 +144,19 @@ __device__ __forceinline__ void dot_units(const uint2 *unit, const uint32_t *blo
     // the lane's words of the last chunk: read from `from`, words below `skip` belong to an earlier lane (or to nobody)
     const int c0 = full_chunks * CH + 4 * li;
     const int from = min(c0, a.D - 4), skip = c0 - from;
-    const uint32_t head_bytes = (uint32_t)(head * a.D) * 4u;
-    auto at = [&](const char *base, uint32_t row, uint32_t b, uint32_t bytes) -> const W4 * {
-        if (OFF32) return reinterpret_cast<const W4 *>(base + (row + bytes));
-        return reinterpret_cast<const W4 *>(base + ((int64_t)row * a.H + (int64_t)b * a.side) * a.D * 4 + bytes);
-    };
+    const uint32_t head_at = (uint32_t)(head * a.D);
+    auto at = [&](const char *base, off row, uint32_t word) { return reinterpret_cast<const W4 *>(base + (row + (off)word * 4)); };
     for (int s0 = 0; s0 < n; s0 += G * U) {
-        uint2 rc[U];
-        uint32_t rb[U];
-        uint32_t differ = 0;
+        Unit<OFF32> rc[U];
+        off differ = 0;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int j = s0 + u * G + g;      // past the end: the last unit again; no result is stored
             rc[u] = unit[j];
-            rb[u] = OFF32 ? 0u : block[j];
-            differ |= (rc[u].y ^ rc[0].y) | (rb[u] ^ rb[0]);
+            differ |= rc[u].y ^ rc[0].y;
         }
         int place[S::per_lane];
-        if (edge_pos) {                        // the results' places, on their way while the dot products are formed
+        if constexpr (PLACED) {                // the results' places, on their way while the dot products are formed
 #pragma unroll
             for (int i = 0; i < S::per_lane; ++i) {
                 const int j = min(s0 + (S::kept(li) + i) * G + g, n - 1);
@@ -165,67 +164,71 @@ __device__ __forceinline__ void dot_units(const uint2 *unit, const uint32_t *blo
             }
         }
         float p[U];
-        auto batch = [&](auto one_row) {
+        // N units from u0 on, with one read of the destination row that they share (SAME: all their gathers of a chunk in flight together) or
+        // one each (half a batch at a time: as many loads in flight, in half the registers)
+        auto batch = [&](auto units, int u0, auto one_row) {
+            constexpr int N = decltype(units)::value;
             constexpr bool SAME = decltype(one_row)::value;
-            float4 acc[ONE ? 1 : U];
+            float4 acc[ONE ? 1 : N];
             if constexpr (!ONE) {
 #pragma unroll
-                for (int u = 0; u < U; ++u) acc[u] = vzero4();
+                for (int u = 0; u < N; ++u) acc[u] = vzero4();
             }
-            auto chunk = [&](uint32_t bytes, auto last_one) {
+            auto chunk = [&](uint32_t word, auto last_one) {
                 auto words = [&](const W4 &w) {
                     return decltype(last_one)::value ? make_float4(0 >= skip ? w.v[0] : 0.f, 1 >= skip ? w.v[1] : 0.f,
                                                                    2 >= skip ? w.v[2] : 0.f, 3 >= skip ? w.v[3] : 0.f)
                                                      : make_float4(w.v[0], w.v[1], w.v[2], w.v[3]);
                 };
-                auto use = [&](int u, const W4 &s, const float4 &d) {
-                    const float4 x = words(s);
-                    if constexpr (ONE) p[u] = vdot(x, d);
-                    else { acc[u].x += x.x * d.x; acc[u].y += x.y * d.y; acc[u].z += x.z * d.z; acc[u].w += x.w * d.w; }
-                };
-                if constexpr (SAME) {
-                    W4 s[U];
-                    const W4 d = *at(db, rc[0].y, rb[0], bytes);
+                constexpr int M = SAME ? N : U / 2;
 #pragma unroll
-                    for (int u = 0; u < U; ++u) s[u] = *at(sb, rc[u].x, rb[u], bytes);
-                    const float4 dv = words(d);
+                for (int h = 0; h < N; h += M) {
+                    W4 s[M], d[SAME ? 1 : M];
+                    if constexpr (SAME) d[0] = *at(db, rc[u0].y, word);
 #pragma unroll
-                    for (int u = 0; u < U; ++u) use(u, s[u], dv);
-                } else {
-                    // half a batch at a time: as many loads in flight, in half the registers
-#pragma unroll
-                    for (int h = 0; h < U; h += U / 2) {
-                        W4 s[U / 2], d[U / 2];
-#pragma unroll
-                        for (int u = 0; u < U / 2; ++u) {
-                            s[u] = *at(sb, rc[h + u].x, rb[h + u], bytes);
-                            d[u] = *at(db, rc[h + u].y, rb[h + u], bytes);
-                        }
-#pragma unroll
-                        for (int u = 0; u < U / 2; ++u) use(h + u, s[u], words(d[u]));
-                        __builtin_amdgcn_sched_barrier(0);      // the compiler would issue both halves' loads first
+                    for (int u = 0; u < M; ++u) {
+                        s[u] = *at(sb, rc[u0 + h + u].x, word);
+                        if constexpr (!SAME) d[u] = *at(db, rc[u0 + h + u].y, word);
                     }
+#pragma unroll
+                    for (int u = 0; u < M; ++u) {
+                        const float4 x = words(s[u]), y = words(d[SAME ? 0 : u]);
+                        if constexpr (ONE) p[u0 + h + u] = vdot(x, y);
+                        else { acc[h + u].x += x.x * y.x; acc[h + u].y += x.y * y.y; acc[h + u].z += x.z * y.z; acc[h + u].w += x.w * y.w; }
+                    }
+                    if (M < N) __builtin_amdgcn_sched_barrier(0);      // the compiler would issue both halves' loads first
                 }
             };
             if constexpr (ONE) {
-                if (ragged) chunk(head_bytes + (uint32_t)from * 4u, std::true_type());
-                else chunk(head_bytes + (uint32_t)li * 16u, std::false_type());
+                if (ragged) chunk(head_at + (uint32_t)from, std::true_type());
+                else chunk(head_at + (uint32_t)li * 4u, std::false_type());
             } else {
 #pragma unroll 1
-                for (int k = 0; k < full_chunks; ++k) chunk(head_bytes + (uint32_t)(k * CH + 4 * li) * 4u, std::false_type());
-                if (ragged) chunk(head_bytes + (uint32_t)from * 4u, std::true_type());
+                for (int k = 0; k < full_chunks; ++k) chunk(head_at + (uint32_t)(k * CH + 4 * li), std::false_type());
+                if (ragged) chunk(head_at + (uint32_t)from, std::true_type());
 #pragma unroll
-                for (int u = 0; u < U; ++u) p[u] = (acc[u].x + acc[u].y) + (acc[u].z + acc[u].w);
+                for (int u = 0; u < N; ++u) p[u0 + u] = (acc[u].x + acc[u].y) + (acc[u].z + acc[u].w);
             }
         };
-        if (!__any(differ != 0)) batch(std::true_type());
-        else batch(std::false_type());
+        if (!__any(differ != 0)) {
+            batch(std::integral_constant<int, U>(), 0, std::true_type());
+        } else if constexpr (OFF32) {
+            batch(std::integral_constant<int, U>(), 0, std::false_type());
+        } else {
+            // Matrices that need 64 bits lie outside the caches: one half's rows from end to end, the next chunk's loads before this one's
+            // products, then the other half's (2,450,000 nodes, 20 M edges, F=448 / 512 / 600: 6558 / 7547 / 8899 us chunk by chunk, 5773 / 6644 / 8316
+            // so; with rows numbered by block of heads and multiplied out at every load, 184 registers, 8454 / 9736 / 11284; 104,000 nodes, 530,000 edges, in
+            // the caches, F=256 80, 91, 103).
+            batch(std::integral_constant<int, U / 2>(), 0, std::false_type());
+            __builtin_amdgcn_sched_barrier(0);
+            batch(std::integral_constant<int, U / 2>(), U / 2, std::false_type());
+        }
         spread_sums<L, U>(p, lane);
 #pragma unroll
         for (int i = 0; i < S::per_lane; ++i) {
             const int j = s0 + (S::kept(li) + i) * G + g;
             if (S::stores(li) && j < n) {
-                if (edge_pos) out[(int64_t)place[i] * a.H + (blocks == 1 ? 0 : (first_block + j) % blocks * a.side) + head] = p[i];
+                if constexpr (PLACED) out[(int64_t)place[i] * a.H + (blocks == 1 ? 0 : (first_block + j) % blocks * a.side) + head] = p[i];
                 else out[j * a.side + head] = p[i];
             }
         }
@@ -234,12 +237,17 @@ __device__ __forceinline__ void dot_units(const uint2 *unit, const uint32_t *blo
 
 // Stages the units of n_edges consecutive edges and multiplies them.  Edge e's column is col[e]; its row is row[e] (COO), or, without
 // `row`, row_of(e).  OFF32: row numbers and the bytes of a unit's row fit 24 bits, their product 32.
-template <int L, bool OFF32, bool ONE, typename RowOf>
-__device__ __forceinline__ void dot_run(uint2 *unit, uint32_t *block, int n_edges, int lane, const SddmmArgs &a, const int32_t *col,
-                                        const int32_t *row, float *out, const int32_t *edge_pos, RowOf row_of) {
+template <int L, bool OFF32, bool ONE, bool PLACED, typename RowOf>
+__device__ __forceinline__ void dot_run(Unit<OFF32> *unit, int n_edges, int lane, const SddmmArgs &a, const int32_t *col, const int32_t *row,
+                                        float *out, const int32_t *edge_pos, RowOf row_of) {
+    using off = Offset<OFF32>;
     const uint32_t blocks = (uint32_t)(a.H / a.side);
     const int batch = 64 / L / a.side * batch_steps(L);
-    const uint32_t row_bytes = (uint32_t)(a.side * a.D) * 4u;
+    const off row_bytes = (off)(a.side * a.D) * 4;
+    auto unit_at = [&](uint32_t r, uint32_t b) -> off {
+        if constexpr (OFF32) return __umul24(__umul24(r, blocks) + b, row_bytes);
+        else return ((uint64_t)r * blocks + b) * row_bytes;
+    };
     const int64_t n_units = (int64_t)n_edges * blocks;
     for (int64_t v0 = 0; v0 < n_units; v0 += kStageUnits) {
         // more units than are staged at a time: one edge's (COO), or those of many (CSR)
@@ -251,45 +259,36 @@ __device__ __forceinline__ void dot_run(uint2 *unit, uint32_t *block, int n_edge
             fg::load_four(col + v0, n, lane, 1, c);
             fg::load_four(row + v0, n, lane, 1, r);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (OFF32) { c[i] = (int)__umul24((uint32_t)c[i], row_bytes); r[i] = (int)__umul24((uint32_t)r[i], row_bytes); }
-                else block[4 * lane + i] = 0;
-            }
-            uint4 *u4 = reinterpret_cast<uint4 *>(unit);
-            u4[2 * lane] = make_uint4((uint32_t)c[0], (uint32_t)r[0], (uint32_t)c[1], (uint32_t)r[1]);
-            u4[2 * lane + 1] = make_uint4((uint32_t)c[2], (uint32_t)r[2], (uint32_t)c[3], (uint32_t)r[3]);
+            for (int i = 0; i < 4; ++i) unit[4 * lane + i] = {unit_at((uint32_t)c[i], 0), unit_at((uint32_t)r[i], 0)};
         } else {
             e0 = blocks == 1 ? (uint32_t)v0 : (uint32_t)(v0 / blocks); b0 = (uint32_t)(v0 - (int64_t)e0 * blocks);
             for (int t = lane; t < (n + batch - 1) / batch * batch; t += 64) {
                 const uint32_t v = b0 + (uint32_t)min(t, n - 1), q = blocks == 1 ? v : v / blocks, e = e0 + q, b = v - q * blocks;
                 const uint32_t c = (uint32_t)col[e], r = (uint32_t)(row ? row[e] : row_of((int)e));
-                if (OFF32) unit[t] = make_uint2(__umul24(__umul24(c, blocks) + b, row_bytes), __umul24(__umul24(r, blocks) + b, row_bytes));
-                else { unit[t] = make_uint2(c, r); block[t] = b; }
+                unit[t] = {unit_at(c, b), unit_at(r, b)};
             }
         }
         wave_lds_sync();
-        dot_units<L, OFF32, ONE>(unit, block, n, lane, a, edge_pos ? out : out + v0 * a.side, edge_pos ? edge_pos + e0 : nullptr, (int)b0);
+        dot_units<L, OFF32, ONE, PLACED>(unit, n, lane, a, PLACED ? out : out + v0 * a.side, PLACED ? edge_pos + e0 : nullptr, (int)b0);
     }
 }
 
-// A wavefront takes edges_per_wave consecutive edges.
-template <int L, bool OFF32, bool ONE>
+// A wavefront takes edges_per_wave consecutive edges.  PLACED: the results go through a.edge_pos.
+template <int L, bool OFF32, bool ONE, bool PLACED>
 __global__ __launch_bounds__(kBlock) void sddmm_coo_kernel(const SddmmArgs a) {
-    __shared__ __align__(16) uint2 s_unit[kWavesPerBlock][kStageUnits];
-    __shared__ uint32_t s_block[kWavesPerBlock][OFF32 ? 1 : kStageUnits];
+    __shared__ Unit<OFF32> s_unit[kWavesPerBlock][kStageUnits];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t e_begin = ((int64_t)blockIdx.x * kWavesPerBlock + wave) * a.edges_per_wave;
     if (e_begin >= a.n_edges) return;
     const int n = (int)min((int64_t)a.edges_per_wave, a.n_edges - e_begin);
-    dot_run<L, OFF32, ONE>(s_unit[wave], s_block[wave], n, lane, a, a.col + e_begin, a.row + e_begin,
-                           a.edge_pos ? a.out : a.out + e_begin * a.H, a.edge_pos ? a.edge_pos + e_begin : nullptr, [](int) { return 0; });
+    dot_run<L, OFF32, ONE, PLACED>(s_unit[wave], n, lane, a, a.col + e_begin, a.row + e_begin, PLACED ? a.out : a.out + e_begin * a.H,
+                                   PLACED ? a.edge_pos + e_begin : nullptr, [](int) { return 0; });
 }
 
 // CSR-order kernel over plan items: a run of whole rows, one row, or a piece of a long row.
 template <int L, bool OFF32, bool ONE>
 __global__ __launch_bounds__(kBlock) void sddmm_csr_kernel(const SddmmArgs a) {
-    __shared__ __align__(16) uint2 s_unit[kWavesPerBlock][kStageUnits];
-    __shared__ uint32_t s_block[kWavesPerBlock][OFF32 ? 1 : kStageUnits];
+    __shared__ Unit<OFF32> s_unit[kWavesPerBlock][kStageUnits];
     __shared__ int32_t s_end[kWavesPerBlock][fg::kItemRows];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t item_id = (int64_t)blockIdx.x * kWavesPerBlock + wave;
@@ -299,7 +298,7 @@ __global__ __launch_bounds__(kBlock) void sddmm_csr_kernel(const SddmmArgs a) {
     const int nrows = it.info < -1 ? -it.info : 1;
     if (lane < nrows) s_end[wave][lane] = nrows > 1 ? a.pos[it.row + lane + 1] - it.start : it.len;
     wave_lds_sync();
-    dot_run<L, OFF32, ONE>(s_unit[wave], s_block[wave], it.len, lane, a, a.col + it.start, nullptr, a.out + (int64_t)it.start * a.H, nullptr,
+    dot_run<L, OFF32, ONE, false>(s_unit[wave], it.len, lane, a, a.col + it.start, nullptr, a.out + (int64_t)it.start * a.H, nullptr,
                            [&](int e) {
         // the row of the item's edge e: the first whose end exceeds it
         int lo = 0, hi = nrows - 1;
@@ -810,9 +809,14 @@ void launch_units(bool csr, dim3 grid, hipStream_t st, const SddmmArgs &a) {
     if (csr) {
         if (one) hipLaunchKernelGGL((sddmm_csr_kernel<L, OFF32, true>), grid, dim3(kBlock), 0, st, a);
         else hipLaunchKernelGGL((sddmm_csr_kernel<L, OFF32, false>), grid, dim3(kBlock), 0, st, a);
+    } else if (a.edge_pos) {
+        if constexpr (!OFF32) {                // (one set of kernels for placed results)
+            if (one) hipLaunchKernelGGL((sddmm_coo_kernel<L, false, true, true>), grid, dim3(kBlock), 0, st, a);
+            else hipLaunchKernelGGL((sddmm_coo_kernel<L, false, false, true>), grid, dim3(kBlock), 0, st, a);
+        }
     } else {
-        if (one) hipLaunchKernelGGL((sddmm_coo_kernel<L, OFF32, true>), grid, dim3(kBlock), 0, st, a);
-        else hipLaunchKernelGGL((sddmm_coo_kernel<L, OFF32, false>), grid, dim3(kBlock), 0, st, a);
+        if (one) hipLaunchKernelGGL((sddmm_coo_kernel<L, OFF32, true, false>), grid, dim3(kBlock), 0, st, a);
+        else hipLaunchKernelGGL((sddmm_coo_kernel<L, OFF32, false, false>), grid, dim3(kBlock), 0, st, a);
     }
 }
 
@@ -861,7 +865,7 @@ int sddmm_run(const fg_spmm_plan *pl, const int32_t *row, const int32_t *col, co
         if (blocks > 0x7fffffffLL) return fail(FG_ERR_SHAPE, "grid too large");
         const uint64_t row_bytes = (uint64_t)H * D * 4u;
         const uint64_t rows = (uint64_t)std::max(n_src, n_dst);
-        const bool off32 = n_src > 0 && n_dst > 0 && rows * row_bytes < (1ull << 32) && rows * blocks_per_edge < (1u << 24) &&
+        const bool off32 = !edge_pos && n_src > 0 && n_dst > 0 && rows * row_bytes < (1ull << 32) && rows * blocks_per_edge < (1u << 24) &&
                            row_bytes < (1u << 24);
         if (off32) launch_units_l<true>(L, csr, dim3((unsigned)blocks), st, a);
         else launch_units_l<false>(L, csr, dim3((unsigned)blocks), st, a);

@@ -58,3 +58,21 @@ def test_edges_match_float64(H, D, n_edges):
         assert np.array_equal(got[~finite & ~np.isnan(want)], want[~finite & ~np.isnan(want)].astype(np.float32)), what
         assert_sum_close(got[finite], want[finite], mass[finite], what)
 
+
+@pytest.mark.parametrize("H,D", [(1, 3), (1, 5), (1, 16), (1, 31), (1, 64), (1, 100), (1, 127), (1, 338), (1, 512), (2, 8), (3, 16), (6, 20), (5, 32), (300, 4)])
+def test_rows_addressed_with_64_bits_give_the_same_results(H, D):
+    """Without the operands' row counts (and for operands of 4 GiB or more) rows are addressed with 64 bits and walked half a batch at a time; every dot
+    product adds up in the same order."""
+    import torch
+    from featgraph_amd import _lib
+    rng = np.random.default_rng(D)
+    ptr, stream = _lib.dev_ptr, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for n_edges in (1, 255, 3001):
+        row, col = rng.integers(0, 23, n_edges), rng.integers(0, 37, n_edges)
+        row[: n_edges // 2] = np.sort(row[: n_edges // 2])
+        r, c = (torch.from_numpy(a.astype(np.int32)).cuda() for a in (row, col))
+        src, dst = (torch.from_numpy(rng.standard_normal((n, H, D), dtype=np.float32)).cuda() for n in (37, 23))
+        narrow, wide = (torch.full((n_edges, H), float("nan"), device="cuda") for _ in range(2))
+        _lib.check(_lib.lib().fg_sddmm_edges_f32(ptr(r), ptr(c), None, n_edges, 37, 23, ptr(src), ptr(dst), ptr(narrow), H, D, stream))
+        _lib.check(_lib.lib().fg_sddmm_coo_f32(ptr(r), ptr(c), n_edges, ptr(src), ptr(dst), ptr(wide), H, D, stream))
+        assert torch.equal(narrow, wide)
