@@ -1047,7 +1047,9 @@ extern "C" int fg_gsddmm_bcast_f32(const int32_t *row_dev, const int32_t *col_de
     if (!out_dev || (any_u && !col_dev) || (any_v && !row_dev)) return fail(FG_ERR_ARG, "null device pointer");
     const int lmode = vector_mode(uses_l, lhs_len, lhs_off_dev, out_len, flags, FG_BCAST_LHS_VEC4, FG_BCAST_LHS_SPLAT4);
     const int rmode = vector_mode(uses_r, rhs_len, rhs_off_dev, out_len, flags, FG_BCAST_RHS_VEC4, FG_BCAST_RHS_SPLAT4);
-    const int vec = vector_variant(op != FG_BIN_DOT && out_len >= 4, lmode, rmode);
+    // results over an operand of theirs: no lane may read what another has written, as the two vectors that share features would
+    const bool in_place = (uses_l && lhs_target == FG_TARGET_E && lhs_dev == out_dev) || (uses_r && rhs_target == FG_TARGET_E && rhs_dev == out_dev);
+    const int vec = vector_variant(op != FG_BIN_DOT && out_len >= 4 && !(in_place && out_len % 4 != 0), lmode, rmode);
     const int V = vec ? 4 : 1;
     // every lane reads its operands' row indices without a branch: an operand on the edges reads (and discards) an
     // index array that exists, or the start of out when the call has none

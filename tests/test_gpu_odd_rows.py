@@ -89,3 +89,23 @@ def test_per_edge(F):
         got = ops.gsddmm(g, op, _odd(values[lhs]), _odd(values[rhs]), lhs.replace("1", "e"), rhs.replace("1", "e")).cpu().numpy()
         want = BIN[op](values[lhs][at[lhs]], values[rhs][at[rhs]])
         assert np.array_equal(got, want) if op != "div" else np.allclose(got, want, rtol=3e-7, atol=0), (op, lhs, rhs)
+
+
+@pytest.mark.parametrize("F", [5, 32, 33, 65, 257])
+@pytest.mark.parametrize("targets", [("e", "v"), ("u", "e"), ("e", "e")])
+def test_per_edge_over_an_operand_of_its_own(F, targets):
+    """Results written over the edge operand they are formed from."""
+    import torch
+    from featgraph_amd.module import GSDDMMhip, placeholder
+    rng = np.random.default_rng(F)
+    adj = _graph(rng, "mixed")
+    n, m = adj.shape
+    at = {"u": adj.indices, "v": np.repeat(np.arange(n), np.diff(adj.indptr)), "e": slice(None)}
+    x, y = (rng.standard_normal(({"u": m, "v": n, "e": adj.nnz}[t], F), dtype=np.float32) for t in targets)
+    mod = GSDDMMhip(adj)
+    mod.build([placeholder(x.shape), placeholder(y.shape)], {"op": "sub", "lhs_target": targets[0], "rhs_target": targets[1]}, {})
+    own = 0 if targets[0] == "e" else 1
+    mod.out_tvm.copy_(torch.from_numpy((x, y)[own]))
+    args = [torch.from_numpy(a).cuda() for a in (x, y)]
+    args[own] = mod.out_tvm
+    assert np.array_equal(mod.run(args).cpu().numpy(), x[at[targets[0]]] - y[at[targets[1]]])
