@@ -162,7 +162,7 @@ class BroadcastOp(object):
         library's operator, features of the other operand or 0), or None where there is no sweep for it."""
         operands = [(self.lhs_target, self.lhs_len, self.lhs_off), (self.rhs_target, self.rhs_len, self.rhs_off)]
         (target, own_len, own_off), (other_target, other_len, other_off) = operands[side], operands[1 - side]
-        if self.out_len < 4 or self.op == 'div' and side == 1 or self.op not in ('add', 'sub', 'mul', 'div', 'copy_lhs'):
+        if target not in ('u', 'e') or self.out_len < 4 or self.op == 'div' and side == 1 or self.op not in ('add', 'sub', 'mul', 'div', 'copy_lhs'):
             return None
         if own_len != self.out_len and not (target == 'e' and own_len == 1 and self.out_len <= 256) or own_len == self.out_len and own_off is not None:
             return None

@@ -177,3 +177,18 @@ def test_oracle_edge_operators(oracle):
             for j in range(5):
                 want = sum(float(a[row[e], i, 0, k]) * float(b[e, j, k]) for k in range(4))
                 assert abs(out[e, i, j] - want) < 1e-12
+
+
+def test_sweeps_are_for_operands_on_sources_and_edges():
+    """The sweeps that form a max / min aggregation's gradient write one row per source or per edge: an operand on the destinations has none."""
+    from featgraph_amd.module import placeholder
+    rows = {"u": 7, "v": 5, "e": 20}
+    for op in ("add", "sub", "mul", "div"):
+        for lt in "uve":
+            for rt in "uve":
+                bop = general.BroadcastOp(op, lt, rt, placeholder((rows[lt], 8)), placeholder((rows[rt], 8)), 5, 7, 20, "cpu", allow_v=True)
+                for side, t in ((0, lt), (1, rt)):
+                    sweep = bop.sweep_of(side)
+                    assert sweep is None or t in "ue" and sweep[0] == t
+                    if t == "v":
+                        assert sweep is None
