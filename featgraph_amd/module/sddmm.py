@@ -274,8 +274,7 @@ class SDDMMbase(object):
         tiled = None
         nnz = self._adj_row_indices.shape[0]
         if order in ('auto', 'tiled') and nnz > 0:
-            stats = self._graph_stats() if H == 1 or nnz < tuning.SMALL_NNZ else None          # (several heads on large graphs: sizes decide)
-            tiled = tuning.choose_sddmm(self._num_rows, self._num_cols, nnz, H, D, stats,
+            tiled = tuning.choose_sddmm(self._num_rows, self._num_cols, nnz, H, D, self._graph_stats,
                                         given_len=pad_from, scattered=not self._row_sorted)
             p_arg, t_arg = schedule_args.get('num_src_partitions'), schedule_args.get('num_feat_tiles')
             if t_arg is None and knob_tiles is not None and order != 'coo' and order != 'csr':

@@ -383,13 +383,16 @@ def _padding_seconds(stats, given_len, feat_len):
 def choose_sddmm(n_rows, n_cols, nnz, heads, head_len, stats=None, given_len=None, scattered=False):
     """(num_src_partitions, num_feat_tiles) for the tiled traversal, or None when the plain
     kernels should be used (small feature matrices, or a shape the tiled kernel does not take).  given_len: the rows' length where
-    head_len is what the tiled traversal would pad them to.  scattered: the edges are stored in no order of their rows."""
+    head_len is what the tiled traversal would pad them to.  scattered: the edges are stored in no order of their rows.
+    stats: GraphStats, or a function that returns them, called where they are read."""
     feat_len = heads * head_len
     if heads == 1:
         if nnz == 0 or feat_len % 4 != 0:
             return None
         if stats is None:
             stats = GraphStats(n_rows, n_cols, nnz)
+        elif callable(stats):
+            stats = stats()
         if _is_small(stats) and scattered:
             return _choose_sddmm_scattered(stats, feat_len, given_len)
         if _is_small(stats):
@@ -414,10 +417,9 @@ def choose_sddmm(n_rows, n_cols, nnz, heads, head_len, stats=None, given_len=Non
             return None
         return ranked[0]
     first = _choose_sddmm_heads(n_rows, n_cols, nnz, heads, head_len, scattered)
-    if stats is None:
-        stats = GraphStats(n_rows, n_cols, nnz)
     padded = given_len is not None and given_len != head_len
-    if nnz > 0 and _is_small(stats) and (scattered or not padded) and 8 <= head_len <= 64 and _is_pow2(head_len):
+    if 0 < nnz < SMALL_NNZ and (scattered or not padded) and 8 <= head_len <= 64 and _is_pow2(head_len):
+        stats = GraphStats(n_rows, n_cols, nnz) if stats is None else stats() if callable(stats) else stats
         return _choose_sddmm_heads_small(stats, heads, head_len, first, given_len if padded else None, scattered)
     if padded and not scattered and first is not None and first[0] == 1:
         # padded heads without source partitions: the edge-list kernel reads them unpadded (40,000 nodes of degree 4, 8 x 48:
