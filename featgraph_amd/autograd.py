@@ -584,8 +584,8 @@ class _GSpMMExtreme(torch.autograd.Function):
 
 
 def _wants_torch_grads():
-    """Whether a max / min gradient has to come from torch's operators: it is differentiated again (create_graph) or must
-    add in a fixed order; one kernel with float atomics gives neither."""
+    """Whether a max / min gradient has to come from torch's operators: it is differentiated again (create_graph), or must add in a fixed
+    order, which the sweeps do but the kernel with float atomics, which takes what they do not, does not."""
     return torch.is_grad_enabled() or torch.are_deterministic_algorithms_enabled()
 
 

@@ -62,7 +62,7 @@ __device__ __forceinline__ float segment_sum(float v) {
 //   104,000, 530,000: F=64 22.5 -> 21.5, F=71 95 -> 35, 8x32 94 -> 90;  58,000, 12.5 M: F=16 76 -> 74, 4x48 3691 -> 1056
 
 // Units per lane group and batch.  Heads of a few lanes are bound by vector instructions and want wavefronts, not loads, in
-// flight: with 8 units on 4 lanes (96 registers, 4 units: 72) rows of 16 floats take 79.9 us for 74.3 on 12.5 M edges of 58,000 nodes.
+// flight: with 8 units on 4 lanes rows of 16 floats take 79.9 us for 74.3 on 12.5 M edges of 58,000 nodes.
 __host__ __device__ constexpr int batch_steps(int L) { return L <= 4 ? 4 : 8; }
 constexpr int kStageUnits = fg::kItemEdges;    // most units staged per wavefront at a time
 constexpr int kMinDot = 4;                     // shorter heads: sddmm_short_kernel

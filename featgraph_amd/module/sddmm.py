@@ -64,7 +64,7 @@ class SDDMMbase(object):
         # below -- so a module that only ever runs the tiled traversal holds the partitioned copy only)
         self._share_from = None
         # Stored order with non-decreasing row ids is CSR order: row pieces from the SpMM plan
-        # then replace the per-edge row array and dst rows are fetched once per piece.
+        # can then replace the per-edge row array.
         self._plan = ctypes.c_void_p()
         self._adj_indptr_dev = None
         self._row_sorted = bool(nnz == 0 or (np.diff(adj_row_indices) >= 0).all())
@@ -397,7 +397,7 @@ class SDDMMbase(object):
             self._num_rows, self._num_cols, nnz, self._num_row_partitions, self._num_col_partitions)
         text += "  features         : %d head(s) x %d floats\n" % (H, D)
         text += "  kernel           : %s\n" % ("sddmm_tiled_kernel over a source-column-partitioned edge list" if tiled
-                                               else "sddmm_csr_kernel over row pieces (dst row held in registers)"
+                                               else "sddmm_csr_kernel over row pieces"
                                                if use_csr else "sddmm_coo_kernel over runs of consecutive stored edges")
         if tiled:
             P, T = tiled

@@ -312,8 +312,8 @@ int fg_sddmm_edges_f32(const int32_t *row_dev, const int32_t *col_dev, const int
 
 /*
  * Same result for edges in CSR order (edge e of row v at position indptr[v] + k), using the
- * SpMM plan's row items so that dst[v] is fetched once per row piece and no row-id array
- * is read.  The plan must have num_col_partitions == 1.
+ * SpMM plan's row items, so that no row-id array is read; dst[v] is read once per batch of edges (8 .. 128 of them) that
+ * share it, and once per edge in a batch of several rows.  The plan must have num_col_partitions == 1.
  */
 int fg_sddmm_csr_f32(const fg_spmm_plan *plan, const int32_t *indptr_dev,
                      const int32_t *indices_dev, const float *src_dev, const float *dst_dev,
@@ -361,7 +361,8 @@ int fg_gsddmm_elementwise_f32(const int32_t *row_dev, const int32_t *col_dev, in
  *     into 64-float tiles that different workgroups take (the tiling the reference applies to the weighted sum,
  *     python/featgraph/op/vanilla_spmm.py:43-60).  Otherwise, with 256 output features or more (64 without
  *     128-bit accesses), a row's sum is formed in stored element order (rows longer than the split threshold:
- *     piece by piece).
+ *     piece by piece); with fewer, several lane groups may take every so many elements of a row each and their sums are
+ *     added, in a fixed order.
  *   fg_gspmm_bcast_dds_f32 : the same result over a source-column-partitioned (DDS) copy of the adjacency, so that
  *     an operand gathered from the source nodes is read partition by partition and its rows stay in the L2s
  *     (the reference's 1-D graph partitioning, python/featgraph/op/vanilla_spmm.py:198-222, applied to these
@@ -377,7 +378,8 @@ int fg_gsddmm_elementwise_f32(const int32_t *row_dev, const int32_t *col_dev, in
  *     one partition (s1_pos / s1_idx = indptr / indices) edge_pos may be NULL for the identity.
  *   fg_gsddmm_bcast_f32 : out[e, f] = lhs[.., lhs_off[f]] op rhs[.., rhs_off[f]], or, with FG_BIN_DOT,
  *     out[e, f] = sum_{i < reduce_len} lhs[.., lhs_off[f] * reduce_len + i] * rhs[.., rhs_off[f] * reduce_len + i];
- *     row_dev / col_dev give each stored edge's row and column (needed for the targets that are used).
+ *     row_dev / col_dev give each stored edge's row and column (needed for the targets that are used).  out may be an operand on
+ *     the elements of out_len features without an offset array.
  */
 typedef enum {
     FG_BIN_ADD = 0, FG_BIN_SUB = 1, FG_BIN_MUL = 2, FG_BIN_DIV = 3, FG_BIN_COPY_LHS = 4, FG_BIN_COPY_RHS = 5,
@@ -385,8 +387,9 @@ typedef enum {
 } fg_binary_op;
 typedef enum { FG_TARGET_U = 0, FG_TARGET_E = 1, FG_TARGET_V = 2 } fg_target;
 /* flags: what the caller knows about an offset array, which lets the kernels use 128-bit accesses when out_len
- * is a multiple of 4 and the arrays are 16-byte aligned (0 is always valid; an operand without an offset array
- * needs no flag).  _VEC4: every aligned group of 4 output features reads 4 consecutive operand features that
+ * is a multiple of 4 (0 is always valid).  An operand without an offset array, or of one feature, needs no flag: where all operands are
+ * such, 128-bit accesses are used from 4 output features on, at any length and 4-byte alignment (but in short odd rows with an operand
+ * streamed from the elements, and at odd lengths where out_dev is an operand).  _VEC4: every aligned group of 4 output features reads 4 consecutive operand features that
  * start at a multiple of 4.  _SPLAT4: every such group reads one operand feature 4 times.
  * FG_BCAST_EDGES_ASCEND: edge_pos ascends along every row segment of the layout (it does for the positions that
  * fg_csr_to_dds gives), which lets max / min with positions skip comparing positions on ties. */
