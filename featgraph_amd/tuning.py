@@ -296,7 +296,8 @@ def rank_sddmm(stats, feat_len, pieces=None):
     # 22 and 1 with it.
     if pieces is None:
         pieces = 20 if feat_len <= 64 else 32
-    takes = [(p, t) for p, t in takes if p == 1 or t > 1 or ranked[0][0] > 1 == ranked[0][1] or stats.nnz >= pieces * p * stats.n_dst]
+    if not (ranked[0][0] > 1 and ranked[0][1] == 1):
+        takes = [(p, t) for p, t in takes if p == 1 or t > 1 or stats.nnz >= pieces * p * stats.n_dst]
     return _overrule(stats, feat_len, predict_sddmm, ranked, takes, SDDMM_SMALL_COEF, 0.05 if stats.n_src <= MANY_SOURCES else 0.1)
 
 
